@@ -304,7 +304,7 @@ struct XcdCfg {
     int n_ht, gpx, n_groups;   // members of a group, groups per XCD, groups of the launch
     int ks;                    // k-steps of the contraction
     int lds;
-    size_t xslot;              // bytes of one exchange slot (the kernels use two)
+    size_t xslot;              // bytes of one exchange slot (of kXchgSlots)
 };
 
 // The XCD-local kernels apply when the device deals workgroups to XCDs in turn, the shape fits
@@ -349,13 +349,11 @@ bool select_xcd(int T, int B_all, int H, int dtype, bool backward, size_t ws_byt
     c->n_groups = cdiv(B, bt);
     if (copies * c->n_groups > kNumXcd * c->gpx) return false;   // (the tile loop above guarantees it; the kernels index counters by group)
     c->xslot = (size_t)c->n_groups * c->ntw * c->ks * kFragBytes;
-    if (ws_bytes < kWsHeaderBytes + kWsCounterBytes + 2 * (size_t)copies * c->xslot) return false;
-    const int gseg = ht * s;
-    const int red_blocks = backward ? 8 * c->mt * c->ntw : 4 * c->mt * c->ntw;
-    c->lds = red_blocks * kFragBytes + bt * (4 * gseg + 16) + 2 * bt * (gseg + 16);
-#ifdef FASTLSTM_TIMELINE
-    c->lds += 4096;
-#endif
+    if (ws_bytes < kWsHeaderBytes + kWsCounterBytes + kXchgSlots * (size_t)copies * c->xslot) return false;
+    // partial sums of the K-shares, gates tile(s), two state tiles (as the kernels lay them out)
+    const int gseg = ht * s, gates = bt * (4 * gseg + 16), states = 2 * bt * (gseg + 16);
+    const int shares = backward || (c->nwv == 8 && c->ntw == 1) ? 8 : 4;
+    c->lds = shares * c->mt * c->ntw * kFragBytes + (backward ? c->ntw * (gates + states) : 2 * gates + states);
     return true;
 }
 
@@ -435,7 +433,7 @@ int try_fwd_xcd(void *ifgo, void *out, void *cell, const void *Wh, unsigned char
     XcdCfg c;
     const int copies = (second && !x) ? 2 + o.n_more : 1;   // independent recurrences side by side
     if (!select_xcd(T, B, H, dtype, false, ws_bytes, &c, o.rows, copies)) return copies > 1 ? 2 : 1;
-    if (second && ws_bytes < kWsHeaderBytes + kWsCounterBytes + 2 * 2 * c.xslot) return 2;   // both layers' slots side by side
+    if (second && ws_bytes < kWsHeaderBytes + kWsCounterBytes + kXchgSlots * 2 * c.xslot) return 2;   // both layers' slots side by side
     FwdXcdParams p{};
     p.ifgo = ifgo; p.out = out; p.cell = cell; p.Wh = Wh;
     p.hdr = reinterpret_cast<WsHeader *>(wsb);
@@ -451,7 +449,7 @@ int try_fwd_xcd(void *ifgo, void *out, void *cell, const void *Wh, unsigned char
     if (second && !x) {   // independent recurrences of this shape side by side (their projections are done)
         const int n = 2 + o.n_more;
         if (n > kMaxSideBySide || n * c.n_groups > kNumXcd * c.gpx) return 2;   // every group needs its CUs on one XCD
-        if (ws_bytes < kWsHeaderBytes + kWsCounterBytes + 2 * (size_t)n * c.xslot) return 2;
+        if (ws_bytes < kWsHeaderBytes + kWsCounterBytes + kXchgSlots * (size_t)n * c.xslot) return 2;
         p.n_layers = n;
         p.ifgo2 = second->ifgo; p.out2 = second->out; p.cell2 = second->cell; p.Wh2 = second->Wh;
         for (int i = 0; i < o.n_more; ++i) {
@@ -848,7 +846,7 @@ int try_bwd_xcd(const void *dout, void *dh, void *dc, const void *ifgo, const vo
     XcdCfg c;
     const int copies = (lower && !extras) ? 2 + o.n_more : 1;   // independent recurrences side by side
     if (!select_xcd(T, B, H, dtype, true, ws_bytes, &c, o.rows, copies)) return copies > 1 ? 2 : 1;
-    if (lower && ws_bytes < kWsHeaderBytes + kWsCounterBytes + 2 * 2 * c.xslot) return 2;   // both layers' slots side by side
+    if (lower && ws_bytes < kWsHeaderBytes + kWsCounterBytes + kXchgSlots * 2 * c.xslot) return 2;   // both layers' slots side by side
     BwdXcdParams p{};
     p.dout = dout; p.dh = dh; p.dc = dc; p.ifgo = ifgo; p.cell = cell; p.d_ifgo = d_ifgo; p.Wh = Wh;
     p.hdr = reinterpret_cast<WsHeader *>(wsb);
@@ -863,7 +861,7 @@ int try_bwd_xcd(const void *dout, void *dh, void *dc, const void *ifgo, const vo
         const int n = 2 + o.n_more;
         // (32-row groups of the 16-k-step reverse kernel, H > 512, cost 1.9 x a 16-row step: no gain over one after the other)
         if (n > kMaxSideBySide || n * c.n_groups > kNumXcd * c.gpx || (c.ntw == 2 && c.nkw == 16)) return 2;
-        if (ws_bytes < kWsHeaderBytes + kWsCounterBytes + 2 * (size_t)n * c.xslot) return 2;
+        if (ws_bytes < kWsHeaderBytes + kWsCounterBytes + kXchgSlots * (size_t)n * c.xslot) return 2;
         p.n_layers = n;
         for (int i = 0; i < o.n_more; ++i) {
             p.dout_more[i] = o.more[i][0]; p.dh_more[i] = o.more[i][1]; p.dc_more[i] = o.more[i][2]; p.ifgo_more[i] = o.more[i][3];

@@ -150,6 +150,7 @@ inline int *ws_chunk_counters(WsHeader *hdr, int which) { return reinterpret_cas
 constexpr size_t kWsHeaderBytes = 1024;
 static_assert(sizeof(WsHeader) + 3 * kMaxChunks * sizeof(int) <= kWsHeaderBytes, "chunk counters fit the header block");
 constexpr size_t kWsCounterBytes = 65536;
+constexpr int kXchgSlots = 4;   // exchange slots of the XCD-local kernels (recurrent_fwd_xcd.hpp); the other families use two
 
 long long spin_limit_ticks();
 

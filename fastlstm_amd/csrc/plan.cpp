@@ -222,7 +222,7 @@ extern "C" size_t fastlstm_recurrent_workspace_bytes(const fastlstm_plan *plan, 
     if (!plan || T <= 0 || H <= 0 || !dtype_ok(dtype)) return 0;
     if (plan->wave_split == 2 || plan->wave_split == 3) return plan->ws_bytes;
     const size_t slot = recurrent_slot_bytes(H, dtype, plan->bt, plan->n_btiles, backward != 0);
-    const int slots = 2;   // every kernel exchanges through two slots, whatever T is
+    const int slots = kXchgSlots;   // whatever T is
     size_t ws = plan->ws_bytes;
     // the XCD-local kernels lay their ring out for batch tiles of 16 or 32 rows, which covers at most
     // 16 rows (one operand block per k-step) more than the tiles of the plan

@@ -1,15 +1,14 @@
 // Persistent reverse-time kernel, XCD-local form: the hidden tiles of one batch tile run on one XCD
 // and exchange d_ifgo[t] through that XCD's L2.  Same mathematics and results as
 // lstm_bwd_persistent_kernel (which replaces fastlstm/kernels.py:1201-1409); placement, exchange
-// ring, L2 counter barrier and the register-resident weight slice follow lstm_fwd_xcd_kernel.
+// slots whose data carries the synchronisation, and the register-resident weight slice follow lstm_fwd_xcd_kernel.
 //
 // Per reverse step s (timestep t = T-1-s) a workgroup of NWV waves, owning 16*MT hidden units and
 // 16*NTW batch rows:
-//   gate backward for its (unit, row) items -> d_ifgo[t] tile (LDS) and exchange slot s (L2)
-//   counter barrier over the group
+//   gate backward for its (unit, row) items -> exchange slot s % 4 (L2) and d_ifgo[t] tile (LDS)
 //   dh_rec(units, rows) = Wh[:, units]^T . d_ifgo[t](rows, :)^T over K = 4H:
 //       the waves split K NWV ways; wave w holds A fragments (MT unit tiles x NKW k-steps
-//       w, w + NWV, ...) of Wh^T in registers and requests its NKW*NTW operand blocks at once
+//       w, w + NWV, ...) of Wh^T in registers and repeats the loads of its operand blocks until they have been written
 //   cross-wave sum of the NWV partials through LDS
 // K index = 4 * source unit + gate, as in the general kernel.
 #pragma once
@@ -27,8 +26,8 @@ struct BwdXcdParams {
     void *d_ifgo;       // [T,B,4H]
     const void *Wh;     // [4H,H]
     WsHeader *hdr;
-    int *counters;         // [groups][kXcdReplicas][kXcdCounterStride], zero at launch
-    unsigned char *xbuf;   // [2 slots][groups][NT][KSB] operand blocks; reverse step s uses slot s % 2
+    int *counters;         // [groups][kXcdReplicas][kXcdCounterStride], zero at launch (XCD-local kernels: the barrier of their prologue)
+    unsigned char *xbuf;   // [kXchgSlots][groups][NT][KSB] operand blocks; reverse step s uses slot s % kXchgSlots
     int T, B, H;
     int n_ht, gpx, n_groups;
     int b_base;         // first batch row of this launch (a large batch runs as several launches over row ranges)
@@ -39,7 +38,7 @@ struct BwdXcdParams {
     // chunk_done[c] counts the recurrence workgroups (n_active) whose part of chunk c is in memory.
     GemmParams k5;      // M = T*B, N = I, K = 4H, A = d_ifgo, B = Wx (K-major), C = dx
     // Bias gradient inside the launch (HELP instantiations, db_part != nullptr): every recurrence workgroup sums the
-    // d_ifgo values it produces over all timesteps -- thread-private fp32 slots in LDS, updated behind the publish of
+    // d_ifgo values it produces over all timesteps -- thread-private fp32 slots in LDS, updated behind the exchange stores of
     // each step, while the workgroup waits for its peers anyway -- and writes the sums of its 16-row batch tiles to
     // db_part[batch tile][4H] at the end; a small kernel adds the batch tiles up.  The separate column-sum pass
     // over d_ifgo (one more read of T*B*4H elements) is not needed then.
@@ -307,7 +306,7 @@ __global__ __launch_bounds__(kWave * NWV) void lstm_bwd_xcd_kernel(const BwdXcdP
     constexpr int GROW = 4 * GSEG + 16, SROW = GSEG + 16;
     constexpr int PPSEG = GSEG / 16;
     constexpr int GPIECES = BT * 4 * PPSEG, SPIECES = BT * PPSEG;
-    constexpr int IOT = NTHR - kWave;                  // wave 0 polls, the others move the tiles
+    constexpr int IOT = NTHR - kWave;                  // waves 1 .. move the tiles (wave 0 does the waits for chunks)
     constexpr int GPT = (GPIECES + IOT - 1) / IOT, SPT = (SPIECES + IOT - 1) / IOT;
 
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -396,7 +395,7 @@ __global__ __launch_bounds__(kWave * NWV) void lstm_bwd_xcd_kernel(const BwdXcdP
     float dc_state[IPT], dh_rec[IPT], c1v[IPT];
     size_t off_h[IPT];
     int xoff[IPT], roff[IPT], goff[IPT], soff[IPT];
-    bool valid[IPT], pair_lead[IPT];
+    bool valid[IPT], stores[IPT];   // stores: this lane writes exchange words (zeros for rows past the batch)
     const size_t BH = (size_t)B * H, B4H = (size_t)B * 4 * H;
 #pragma unroll
     for (int m = 0; m < IPT; ++m) {
@@ -407,7 +406,7 @@ __global__ __launch_bounds__(kWave * NWV) void lstm_bwd_xcd_kernel(const BwdXcdP
         valid[m] = nt < NT && b < B;
         off_h[m] = valid[m] ? (size_t)b * H + unit : (size_t)b0 * H + u0;
         xoff[m] = (nt < NT ? nt : 0) * KSB * kFragBytes + frag_offset<T>(n, unit * 4);
-        pair_lead[m] = valid[m] && ((ul & 1) == 0);
+        stores[m] = nt < NT && (E::BYTES == 4 || (ul & 1) == 0);
         const int a = ul >> 4, ur = ul & 15;
         roff[m] = ((a * NT + (nt < NT ? nt : 0)) * kWave + (ur >> 2) * 16 + n) * 4 + (ur & 3);
         goff[m] = ((nt < NT ? nt : 0) * 16 + n) * GROW + ul * E::BYTES;
@@ -419,26 +418,40 @@ __global__ __launch_bounds__(kWave * NWV) void lstm_bwd_xcd_kernel(const BwdXcdP
 
     const unsigned xgrp = (unsigned)vg * NT * KSB * kFragBytes;
     const size_t xslot = (size_t)p.n_groups * n_layers * NT * KSB * kFragBytes;
+    auto xslot_of = [&](int v) { return XchgL2(p.xbuf + (size_t)(v % kXchgSlots) * xslot, (unsigned)xslot); };
     int *grp_counters = p.counters + (size_t)vg * kXcdGroupStride;
-    int *my_counter = grp_counters + (j % kXcdReplicas) * kXcdCounterStride;
+    bool dead = false;   // the launch has given up (see poll_blocks)
+    auto unwrite = [&](const XchgL2 &x) {
+#pragma unroll
+        for (int m = 0; m < IPT; ++m)
+            if (stores[m]) x.store16(xgrp + xoff[m], u32x4{kUnwritten, kUnwritten, kUnwritten, kUnwritten});
+    };
+    // every member has marked its part of the slots unwritten before any member stores or reads one
+    for (int v = 0; v < kXchgSlots; ++v) unwrite(xslot_of(v));
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (tid < kXcdReplicas)
+        __hip_atomic_fetch_add(grp_counters + tid * kXcdCounterStride, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    if (wave == 0) wait_counter(grp_counters + (j % kXcdReplicas) * kXcdCounterStride, p.n_ht, p.hdr, p.spin_limit, vg, 0);
+    __syncthreads();
 
     // ---- coalesced tile I/O: ifgo[t], cell[t], dout[t] in, d_ifgo[t] out --------------------
     // Buffer loads / stores: the step's base addresses in scalar registers, per-lane byte offsets that never change.
-    // Groups of 16 rows keep two sets of tile pieces in flight in registers: the tiles of step s + 2 are requested
-    // right after step s's tile went out and go to the LDS behind step s + 1's K loop -- almost two steps later,
-    // which also covers the memory latency while the workgroups without a role in the recurrence stream their
-    // GEMM operands.  Groups of 32 rows have no registers for that (the pieces were spilled right behind their
-    // loads, and a spill waits for its load): there the three tiles go global -> LDS tiles with LDS-direct loads,
-    // one step ahead, slot by slot (a padded tile row is a whole number of 16-byte slots; lane l of wave
-    // instruction w fills slot 64 w + l of its tile; pad slots and rows past B stay untouched), and the d_ifgo tile
-    // leaves by the slots the same wave filled.
+    // The tiles of reverse step s + 2 are requested in step s behind the arrival of d_ifgo[t].  Groups of 16 rows hold
+    // them in registers until d_ifgo has arrived in step s + 1 -- those loads were issued later, so nothing waits for
+    // the tiles -- and put them into the LDS there.  Groups of 32 rows have no registers for that (the pieces were spilled right
+    // behind their loads, and a spill waits for its load): there the three tiles go global -> LDS with LDS-direct
+    // loads into the set of step s (two sets in turn), slot by slot (a padded tile row is a whole number of 16-byte
+    // slots; lane l of wave instruction w fills slot 64 w + l of its tile; pad slots and rows past B stay untouched), and
+    // the d_ifgo tile leaves by the slots the same wave filled.
     constexpr bool DMA = NTW == 2;
-    constexpr int DIST = DMA ? 1 : 2;                    // steps between the request of a tile and its use
+    constexpr int DIST = 2;                              // steps between the request of a tile and its use
+    constexpr int SET = DMA ? BT * GROW + 2 * BT * SROW : 0;   // bytes from one set of LDS tiles to the next
     constexpr int SPRG = GROW / 16, SPRS = SROW / 16;    // slots per padded row
     constexpr int NG = (BT * SPRG + kWave - 1) / kWave, NS = (BT * SPRS + kWave - 1) / kWave;   // wave instructions per tile
     constexpr int DT = (NG + 2 * NS + NWV - 2) / (NWV - 1);                                     // per moving wave
     constexpr int GD = DMA ? DT : GPT, SD = DMA ? 1 : SPT;
-    u32x4 gpre[DMA ? 1 : 2][DMA ? 1 : GPT], cpre[DMA ? 1 : 2][DMA ? 1 : SPT], dpre[DMA ? 1 : 2][DMA ? 1 : SPT];
+    u32x4 gpre[DMA ? 1 : GPT], cpre[DMA ? 1 : SPT], dpre[DMA ? 1 : SPT];
     unsigned g_off[GD], s_off[SD];
     int g_lds[GD], s_lds[SD], g_kind[GD];   // DMA: tile of item d (0 gates, 1 c, 2 dout; uniform), g_lds = byte inside that tile
     bool g_ok[GD], s_ok[SD];
@@ -478,44 +491,52 @@ __global__ __launch_bounds__(kWave * NWV) void lstm_bwd_xcd_kernel(const BwdXcdP
         s_lds[i] = s_ok[i] ? row * SROW + k * 16 : 0;
         s_off[i] = s_ok[i] ? (unsigned)(((size_t)row * H + k * (16 / E::BYTES)) * E::BYTES) : 0u;
     }
-    auto fetch_tiles = [&](int t, u32x4(&gp)[DMA ? 1 : GPT], u32x4(&cp)[DMA ? 1 : SPT], u32x4(&dp)[DMA ? 1 : SPT]) {
+    const unsigned tiles_addr = (unsigned)(size_t)((FASTLSTM_LDS_PTR unsigned char *)tiles);
+    auto fetch_tiles = [&](int t) __attribute__((always_inline)) {   // of timestep t >= 0
         if (io_tid < 0) return;
-        const __amdgpu_buffer_rsrc_t rg = __builtin_amdgcn_make_buffer_rsrc(const_cast<T *>(ifgo) + (size_t)t * B4H + tile_org, 0, g_bytes, 0x00020000);
-        const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc(const_cast<T *>(cell) + (size_t)t * BH + state_org, 0, s_bytes, 0x00020000);
-        const __amdgpu_buffer_rsrc_t rd = __builtin_amdgcn_make_buffer_rsrc(const_cast<T *>(dout) + (size_t)t * BH + state_org, 0, s_bytes, 0x00020000);
+        const T *ig = ifgo + (size_t)t * B4H + tile_org, *ic = cell + (size_t)t * BH + state_org, *id = dout + (size_t)t * BH + state_org;
         if constexpr (DMA) {
+            auto rsrc = [](const T *ptr, unsigned bytes) {
+                const unsigned long long addr = reinterpret_cast<unsigned long long>(uniform_ptr(ptr));
+                return u32x4{(unsigned)addr, (unsigned)(addr >> 32) & 0xffffu, bytes, 0x00020000u};
+            };
+            const u32x4 rg = rsrc(ig, g_bytes), rc = rsrc(ic, s_bytes), rd = rsrc(id, s_bytes);
+            const unsigned base = (unsigned)uniform_int((int)(tiles_addr + ((T_ - 1 - t) & 1) * SET));
 #pragma unroll
             for (int i = 0; i < GD; ++i) {
                 const int w = (wave - 1) + (NWV - 1) * i;
                 if (g_kind[i] == 0) {
-                    if (g_ok[i]) load_block_to_lds(rg, tiles + (size_t)w * kFragBytes, g_off[i], 0);
+                    if (g_ok[i]) dma_block_asm<false>(rg, base + w * kFragBytes, g_off[i], 0u);
                 } else if (g_kind[i] == 1) {
-                    if (g_ok[i]) load_block_to_lds(rc, tiles + BT * GROW + (size_t)(w - NG) * kFragBytes, g_off[i], 0);
+                    if (g_ok[i]) dma_block_asm<false>(rc, base + BT * GROW + (w - NG) * kFragBytes, g_off[i], 0u);
                 } else {
-                    if (g_ok[i]) load_block_to_lds(rd, tiles + BT * GROW + BT * SROW + (size_t)(w - NG - NS) * kFragBytes, g_off[i], 0);
+                    if (g_ok[i]) dma_block_asm<false>(rd, base + BT * GROW + BT * SROW + (w - NG - NS) * kFragBytes, g_off[i], 0u);
                 }
             }
         } else {
+            const __amdgpu_buffer_rsrc_t rg = __builtin_amdgcn_make_buffer_rsrc(const_cast<T *>(ig), 0, g_bytes, 0x00020000);
+            const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc(const_cast<T *>(ic), 0, s_bytes, 0x00020000);
+            const __amdgpu_buffer_rsrc_t rd = __builtin_amdgcn_make_buffer_rsrc(const_cast<T *>(id), 0, s_bytes, 0x00020000);
 #pragma unroll
-            for (int i = 0; i < GPT; ++i) gp[i] = __builtin_amdgcn_raw_buffer_load_b128(rg, g_off[i], 0, 0);   // (pieces that do not exist read the tile's first bytes)
+            for (int i = 0; i < GPT; ++i) gpre[i] = __builtin_amdgcn_raw_buffer_load_b128(rg, g_off[i], 0, 0);   // (pieces that do not exist read the tile's first bytes)
 #pragma unroll
             for (int i = 0; i < SPT; ++i) {
-                cp[i] = __builtin_amdgcn_raw_buffer_load_b128(rc, s_off[i], 0, 0);
-                dp[i] = __builtin_amdgcn_raw_buffer_load_b128(rd, s_off[i], 0, 0);
+                cpre[i] = __builtin_amdgcn_raw_buffer_load_b128(rc, s_off[i], 0, 0);
+                dpre[i] = __builtin_amdgcn_raw_buffer_load_b128(rd, s_off[i], 0, 0);
             }
         }
     };
-    auto tiles_to_lds = [&](const u32x4(&gp)[DMA ? 1 : GPT], const u32x4(&cp)[DMA ? 1 : SPT], const u32x4(&dp)[DMA ? 1 : SPT]) {
+    auto tiles_to_lds = [&]() __attribute__((always_inline)) {
         if constexpr (!DMA) {
             unsigned char *stc = tiles + BT * GROW, *std_ = stc + BT * SROW;
 #pragma unroll
             for (int i = 0; i < GPT; ++i)
-                if (g_ok[i]) *reinterpret_cast<u32x4 *>(tiles + g_lds[i]) = gp[i];
+                if (g_ok[i]) *reinterpret_cast<u32x4 *>(tiles + g_lds[i]) = gpre[i];
 #pragma unroll
             for (int i = 0; i < SPT; ++i)
                 if (s_ok[i]) {
-                    *reinterpret_cast<u32x4 *>(stc + s_lds[i]) = cp[i];
-                    *reinterpret_cast<u32x4 *>(std_ + s_lds[i]) = dp[i];
+                    *reinterpret_cast<u32x4 *>(stc + s_lds[i]) = cpre[i];
+                    *reinterpret_cast<u32x4 *>(std_ + s_lds[i]) = dpre[i];
                 }
         }
     };
@@ -527,7 +548,7 @@ __global__ __launch_bounds__(kWave * NWV) void lstm_bwd_xcd_kernel(const BwdXcdP
 #pragma unroll
         for (int i = 0; i < GD; ++i)
             if (g_kind[i] == 0 && g_ok[i]) {
-                const u32x4 v = *reinterpret_cast<const u32x4 *>(tiles + g_lds[i]);
+                const u32x4 v = *reinterpret_cast<const u32x4 *>(tiles + ((T_ - 1 - t) & 1) * SET + g_lds[i]);
                 if (k5_live) __builtin_amdgcn_raw_buffer_store_b128(v, rg, g_off[i], 0, 16);
                 else __builtin_amdgcn_raw_buffer_store_b128(v, rg, g_off[i], 0, 0);
             }
@@ -535,42 +556,38 @@ __global__ __launch_bounds__(kWave * NWV) void lstm_bwd_xcd_kernel(const BwdXcdP
     if (follows) {   // the latest chunk(s) of this layer's dout have to be there
         if (wave == 0) {
             wait_dout(T_ - 1);
-            if (DIST > 1 && T_ > 1) wait_dout(T_ - 2);
+            if (T_ > 1) wait_dout(T_ - 2);
         }
         __syncthreads();
     }
-    fetch_tiles(T_ - 1, gpre[0], cpre[0], dpre[0]);
-    if constexpr (DMA) {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // every wave's share of the tiles has landed before anyone reads them
-    } else {
-        if (T_ > 1) fetch_tiles(T_ - 2, gpre[1], cpre[1], dpre[1]);
-        tiles_to_lds(gpre[0], cpre[0], dpre[0]);   // step 0 works on the LDS tiles right away
-    }
+    fetch_tiles(T_ - 1);
+    tiles_to_lds();   // step 0 works on the LDS tiles right away
+    if (T_ > 1) fetch_tiles(T_ - 2);
+    if constexpr (DMA) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // every wave's share of the tiles has landed before anyone reads them
     __syncthreads();
 
-    // one reverse step; PAR = s % 2 picks the register sets at compile time
-    auto step = [&](const int s, auto par) __attribute__((always_inline)) {
-        constexpr int PAR = DMA ? 0 : decltype(par)::value, PARN = DMA ? 0 : (PAR ^ 1);
+    for (int s = 0; s < T_; ++s) {
         const int t = T_ - 1 - s;
-        const XchgL2 xch(p.xbuf + (size_t)(s & 1) * xslot, (unsigned)xslot);
-        // the dout of timestep t - DIST is requested behind this step's publish barrier: when it is the
+        const XchgL2 xch = xslot_of(s);
+        unsigned char *const set = tiles + (s & 1) * SET;
+        // the dout of timestep t - DIST is requested behind a workgroup barrier of this step: when it is the
         // latest timestep of a chunk, that chunk of the upper layer's dx must be complete
         if (follows && wave == 0 && t >= DIST && (t - DIST) % p.k5_chunk_steps == p.k5_chunk_steps - 1) wait_dout(t - DIST);
 
         // ---- point-wise gate backward for this thread's items --------------------------
-        u32x2 d_kept[IPT];   // the items' four stored gate gradients, for the bias sums behind the publish
+        u32x2 d_kept[IPT];   // the items' four stored gate gradients, for the bias sums behind the exchange stores
 #pragma unroll
         for (int m = 0; m < IPT; ++m) {
             T st_d[4];
             if (valid[m]) {
-                T *gl_ = reinterpret_cast<T *>(tiles + goff[m]);   // the item's 4 gates in the LDS tile
+                T *gl_ = reinterpret_cast<T *>(set + goff[m]);   // the item's 4 gates in the LDS tile
                 const float si = sigmoidf_<ACC>(E::to_f32(gl_[0]));
                 const float sf = sigmoidf_<ACC>(E::to_f32(gl_[HT]));
                 const float tg = tanhf_<ACC>(E::to_f32(gl_[2 * HT]));
                 const float so = sigmoidf_<ACC>(E::to_f32(gl_[3 * HT]));
                 const float tc = tanhf_<ACC>(c1v[m]);
-                const float c0 = E::to_f32(*reinterpret_cast<const T *>(tiles + BT * GROW + soff[m]));
-                const float dh = dh_rec[m] + E::to_f32(*reinterpret_cast<const T *>(tiles + BT * GROW + BT * SROW + soff[m]));
+                const float c0 = E::to_f32(*reinterpret_cast<const T *>(set + BT * GROW + soff[m]));
+                const float dh = dh_rec[m] + E::to_f32(*reinterpret_cast<const T *>(set + BT * GROW + BT * SROW + soff[m]));
                 const float dc1 = dc_state[m] + dh * so * (1.f - tc * tc);
                 const float d_o = dh * tc * so * (1.f - so);
                 const float d_f = dc1 * c0 * sf * (1.f - sf);
@@ -594,25 +611,21 @@ __global__ __launch_bounds__(kWave * NWV) void lstm_bwd_xcd_kernel(const BwdXcdP
             // exchange copy: 4 consecutive k = (unit, gate 0..3).  16-bit types: lanes l and l+16
             // own units u and u+1 of the same batch row; the even-unit lane writes both (16 bytes)
             if constexpr (E::BYTES == 2) {
-                const u32x2 mine = *reinterpret_cast<u32x2 *>(st_d);
-                u32x2 other;
+                u32x2 mine = *reinterpret_cast<u32x2 *>(st_d), other;
+                mine[0] = written_word(mine[0]);
+                mine[1] = written_word(mine[1]);
                 other[0] = (unsigned)__shfl_down((int)mine[0], 16);
                 other[1] = (unsigned)__shfl_down((int)mine[1], 16);
-                if (pair_lead[m])
-                    __builtin_amdgcn_raw_buffer_store_b128(u32x4{mine[0], mine[1], other[0], other[1]}, xch.rsrc,
-                                                           xgrp + xoff[m], 0, 0);
+                if (stores[m]) xch.store16(xgrp + xoff[m], u32x4{mine[0], mine[1], other[0], other[1]});
             } else {
-                if (valid[m])
-                    __builtin_amdgcn_raw_buffer_store_b128(*reinterpret_cast<u32x4 *>(st_d), xch.rsrc, xgrp + xoff[m], 0, 0);
+                u32x4 mine = *reinterpret_cast<u32x4 *>(st_d);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) mine[e] = written_word(mine[e]);
+                if (stores[m]) xch.store16(xgrp + xoff[m], mine);
             }
         }
-        // ---- publish: stores acknowledged by the L2, then the group's counters ----------------
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        __syncthreads();
-        if (tid < kXcdReplicas)
-            __hip_atomic_fetch_add(grp_counters + tid * kXcdCounterStride, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        __syncthreads();   // the d_ifgo tile is complete (and everyone has read the partial sums of the step before)
         tile_to_global(t);
-        if (s + DIST < T_) fetch_tiles(t - DIST, gpre[PAR], cpre[PAR], dpre[PAR]);
         if constexpr (HELP != 0 && E::BYTES == 2) {
             if (db_part) {   // (the rounded values, as they were stored: db is the column sum of d_ifgo)
 #pragma unroll
@@ -625,51 +638,46 @@ __global__ __launch_bounds__(kWave * NWV) void lstm_bwd_xcd_kernel(const BwdXcdP
             }
         }
 
-        if (wave == 0) wait_counter(my_counter, p.n_ht * (s + 1), p.hdr, p.spin_limit, vg, s);
-        __syncthreads();
-        // Every workgroup of the group has passed this step's publish point, where its stores of the
-        // previous steps (the written-through d_ifgo tiles included) were acknowledged: they are in
-        // memory.  When the previous step closed a chunk, ONE workgroup hands the group's share of it to
-        // the helpers on the other XCDs and counts for all n_ht workgroups.
-        if (k5_live && j == 0 && tid == kWave && s > 0 && (t + 1) % p.k5_chunk_steps == 0)
-            __hip_atomic_fetch_add(chunk_done + (t + 1) / p.k5_chunk_steps, p.n_ht, __ATOMIC_RELAXED,
-                                   __HIP_MEMORY_SCOPE_AGENT);
-
         // ---- dh_rec(units, rows) = Wh[:, units]^T . d_ifgo[t](rows, :)^T over this wave's k-steps
         f32x4 acc[MT][NTW];
 #pragma unroll
         for (int a = 0; a < MT; ++a)
 #pragma unroll
             for (int i = 0; i < NTW; ++i) acc[a][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-        // the operand blocks of the wave are requested in batches of at most 8 k-steps (registers):
-        // all loads of a batch are issued before its first MFMA -- one round trip per batch
-        constexpr int KB = NKW > 8 ? 8 : NKW;   // (all 16 at once: slower, the L2 is the bound, not the round trips)
+        // the operand blocks of the wave come in batches of at most 8 k-steps (registers)
+        constexpr int KB = NKW > 8 ? 8 : NKW;
 #pragma unroll
         for (int k0 = 0; k0 < NKW; k0 += KB) {
-            u32x4 bq[KB][NTW];
-#pragma unroll
-            for (int kk = 0; kk < KB; ++kk) {
-                const int ks = min(wave + NWV * (k0 + kk), KSB - 1);   // past the end: any valid block (its weights are zero)
-#pragma unroll
-                for (int i = 0; i < NTW; ++i)
-                    bq[kk][i] = xch.load16_l2(xgrp + (unsigned)((i * KSB + ks) * kWave + lane) * 16u);
+            u32x4 bq[KB * NTW];
+            poll_blocks(bq, [&](int i) {
+                const int ks = min(wave + NWV * (k0 + i / NTW), KSB - 1);   // past the end: any valid block (its weights are zero)
+                return xch.load16_l2(xgrp + (unsigned)(((i % NTW) * KSB + ks) * kWave + lane) * 16u);
+            }, dead, p.hdr, p.spin_limit, vg, s);
+            if (k0 + KB >= NKW) {   // the tile has left for memory: the next step's inputs take its place
+                if (s + 1 < T_) tiles_to_lds();
+                if (s + DIST < T_) fetch_tiles(t - DIST);
             }
-            __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int kk = 0; kk < KB; ++kk)
 #pragma unroll
                 for (int a = 0; a < MT; ++a)
 #pragma unroll
-                    for (int i = 0; i < NTW; ++i) acc[a][i] = mfma_kstep<T>(wreg[a][k0 + kk], bq[kk][i], acc[a][i]);
+                    for (int i = 0; i < NTW; ++i) acc[a][i] = mfma_kstep<T>(wreg[a][k0 + kk], bq[kk * NTW + i], acc[a][i]);
             __builtin_amdgcn_sched_barrier(0);
         }
 #pragma unroll
         for (int a = 0; a < MT; ++a)
 #pragma unroll
             for (int i = 0; i < NTW; ++i) red[((wave * MT + a) * NT + i) * kWave + lane] = acc[a][i];
-        // the tile was drained before the barrier above: the next step's inputs take its place
-        if (s + 1 < T_) tiles_to_lds(gpre[PARN], cpre[PARN], dpre[PARN]);
         __syncthreads();
+        // Every wave of this workgroup has seen its part of d_ifgo[t].  So every member has stored it, i.e. finished step
+        // s-1, where the data of its loads had arrived -- and what each of its waves had stored before those loads
+        // was acknowledged: its written-through d_ifgo tile of that step is in memory.  When step s-1 closed a chunk,
+        // ONE workgroup hands the group's share of it to the helpers on the other XCDs and counts for all n_ht workgroups.
+        if (k5_live && j == 0 && tid == kWave && s > 0 && (t + 1) % p.k5_chunk_steps == 0)
+            __hip_atomic_fetch_add(chunk_done + (t + 1) / p.k5_chunk_steps, p.n_ht, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT);
+        if (s > 0) unwrite(xslot_of(s + kXchgSlots - 1));   // every member has read what was exchanged in step s-1
         const float *redf = reinterpret_cast<const float *>(red);
 #pragma unroll
         for (int m = 0; m < IPT; ++m) {
@@ -678,11 +686,7 @@ __global__ __launch_bounds__(kWave * NWV) void lstm_bwd_xcd_kernel(const BwdXcdP
             for (int pp = 1; pp < NWV; ++pp) v += redf[roff[m] + pp * MT * NT * kWave * 4];
             dh_rec[m] = v;
         }
-        // the next step's publish barrier orders these reads before the next writes to `red`
-    };
-    for (int s = 0; s < T_; s += 2) {
-        step(s, std::integral_constant<int, 0>{});
-        if (s + 1 < T_) step(s + 1, std::integral_constant<int, 1>{});
+        // the next step's first workgroup barrier orders these reads before the next writes to `red`
     }
 
     if (k5_live) {   // the last chunk (timesteps 0 ..)
