@@ -644,16 +644,26 @@ __global__ __launch_bounds__(kWave * NWV) void lstm_bwd_xcd_kernel(const BwdXcdP
         for (int a = 0; a < MT; ++a)
 #pragma unroll
             for (int i = 0; i < NTW; ++i) acc[a][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-        // the operand blocks of the wave come in batches of at most 8 k-steps (registers)
-        constexpr int KB = NKW > 8 ? 8 : NKW;
+        // The operand blocks of the wave come in batches of four: the loads of a batch are under way while the one before
+        // is multiplied, and repeated in the rare case that a member was late.  Few at a time, because what a CU
+        // fetches per step (128 KiB for 16 rows at H = 1024) keeps its path to the L2 busy for most of the step and every
+        // repeated block adds to that: H = 1024, B = 64 / 256, us per step: batches of 4 2.47 / 4.4, of 8 2.56 / 6.6
+        // (spilled), of 16 2.88 / 12.8; with a counter barrier before the fetch 3.07 / 6.5.
+        constexpr int KB = 4 / NTW, NBATCH = NKW / KB;
+        static_assert(NKW % KB == 0, "whole batches");
+        u32x4 bq[2][KB * NTW];
+        auto block = [&](int k0, int i) {
+            const int ks = min(wave + NWV * (k0 + i / NTW), KSB - 1);   // past the end: any valid block (its weights are zero)
+            return xch.load16_l2(xgrp + (unsigned)(((i % NTW) * KSB + ks) * kWave + lane) * 16u);
+        };
+        poll_blocks(bq[0], [&](int i) { return block(0, i); }, dead, p.hdr, p.spin_limit, vg, s);
 #pragma unroll
-        for (int k0 = 0; k0 < NKW; k0 += KB) {
-            u32x4 bq[KB * NTW];
-            poll_blocks(bq, [&](int i) {
-                const int ks = min(wave + NWV * (k0 + i / NTW), KSB - 1);   // past the end: any valid block (its weights are zero)
-                return xch.load16_l2(xgrp + (unsigned)(((i % NTW) * KSB + ks) * kWave + lane) * 16u);
-            }, dead, p.hdr, p.spin_limit, vg, s);
-            if (k0 + KB >= NKW) {   // the tile has left for memory: the next step's inputs take its place
+        for (int n = 0; n < NBATCH; ++n) {
+            if (n + 1 < NBATCH) {
+#pragma unroll
+                for (int i = 0; i < KB * NTW; ++i) bq[(n + 1) & 1][i] = block((n + 1) * KB, i);
+                __builtin_amdgcn_sched_barrier(0);
+            } else {   // the tile has left for memory: the next step's inputs take its place
                 if (s + 1 < T_) tiles_to_lds();
                 if (s + DIST < T_) fetch_tiles(t - DIST);
             }
@@ -662,8 +672,10 @@ __global__ __launch_bounds__(kWave * NWV) void lstm_bwd_xcd_kernel(const BwdXcdP
 #pragma unroll
                 for (int a = 0; a < MT; ++a)
 #pragma unroll
-                    for (int i = 0; i < NTW; ++i) acc[a][i] = mfma_kstep<T>(wreg[a][k0 + kk], bq[kk * NTW + i], acc[a][i]);
+                    for (int i = 0; i < NTW; ++i) acc[a][i] = mfma_kstep<T>(wreg[a][n * KB + kk], bq[n & 1][kk * NTW + i], acc[a][i]);
             __builtin_amdgcn_sched_barrier(0);
+            if (n + 1 < NBATCH && any_unwritten(bq[(n + 1) & 1]))
+                poll_blocks(bq[(n + 1) & 1], [&](int i) { return block((n + 1) * KB, i); }, dead, p.hdr, p.spin_limit, vg, s);
         }
 #pragma unroll
         for (int a = 0; a < MT; ++a)

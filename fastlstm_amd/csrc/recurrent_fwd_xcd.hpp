@@ -112,6 +112,16 @@ struct XchgL2 {
     __device__ __forceinline__ void store16(unsigned off, u32x4 v) const { __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, off, 0, 0); }
 };
 
+// Some word of the wave's blocks is kUnwritten (uniform in the wave).
+template <int N> __device__ __forceinline__ bool any_unwritten(const u32x4 (&b)[N]) {
+    unsigned m = 0;   // (the largest unsigned value is kUnwritten)
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) m = m > b[i][e] ? m : b[i][e];
+    return __any(m == kUnwritten);
+}
+
 // b[i] = load(i), i < N, repeated until no word of them is kUnwritten.  All loads of a round are requested before the
 // first is looked at, and none is in flight behind the loop: what the compiler issues next needs no wait for them.
 // (Repeating only the blocks that were not there was slower, 1.85 against 1.79 us per step.)  Bounded like
@@ -123,12 +133,7 @@ __device__ __forceinline__ void poll_blocks(u32x4 (&b)[N], Load load, bool &dead
     for (int polls = 0;;) {
 #pragma unroll
         for (int i = 0; i < N; ++i) b[i] = load(i);
-        unsigned m = 0;   // (the largest unsigned value is kUnwritten)
-#pragma unroll
-        for (int i = 0; i < N; ++i)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) m = m > b[i][e] ? m : b[i][e];
-        if (!__any(m == kUnwritten) || dead) break;
+        if (!any_unwritten(b) || dead) break;
         if (++polls >= 64 || spin_limit <= 1) {
             polls = 0;
             if (__hip_atomic_load(&hdr->abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) dead = true;
