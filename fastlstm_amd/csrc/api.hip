@@ -11,6 +11,7 @@
 #include "recurrent_bwd_wide.hpp"
 #include "recurrent_bwd_wide_split.hpp"
 #include "recurrent_fwd_xcd.hpp"
+#include "recurrent_step.hpp"
 #include "recurrent_stream.hpp"
 
 using namespace fastlstm;
@@ -1635,6 +1636,82 @@ int fastlstm_fwd_layer_infer(const void *x, const void *Wx, const void *bx, cons
     if (int rc = begin_recurrent(stream)) return rc;
     return finish_recurrent(fwd_layer_impl(x, Wx, bx, bh, Wh, ifgo, out, cell, ws, ws_bytes, T, B, I, H, dtype, stream, 0), ws,
                             stream, poison_fwd(dtype, T, B, H, out, cell));
+}
+
+// ---- a few timesteps of inference, one kernel per step (recurrent_step.hpp) ----------------------------------
+// 1 where that is the faster form.  A launch takes about 3 us plus the operands its workgroups read through the L2s at about
+// 7.5 TB/s; the persistent path about 40 us per layer (its small launches and the host's work for them) and 0.6 us
+// per step more.  Measured on either side of the line, us per call of the module, persistent / one kernel per step:
+// 1 layer, B = 1, I = 80, H = 128 fp16 T = 8 52 / 34, T = 16 51 / 65; 2 layers, B = 4, I = H = 512 T = 16 108 / 91, T = 24
+// 108 / 134; B = 64, I = 1024, H = 2048 T = 1 53 / 22, T = 4 59 / 86.
+int fastlstm_infer_short_applies(int layers, int T, int B, int I, int H, int dtype) {
+    if (layers <= 0 || !dtype_ok(dtype) || check_dims(T, B, I, H)) return 0;
+    if (T > 64 || B > 64) return 0;
+    const int at_once = std::min(std::min(layers, T), kStepJobs);
+    const int rows = B <= 16 ? 32 : B <= 32 || at_once * cdiv(H, 4) >= 512 ? 48 : 80;   // operand rows read per 4 units
+    const double mb = (double)at_once * cdiv(H, 4) * rows * ((double)std::max(I, H) + H) * elem_bytes(dtype) * 1e-6;
+    const double step_us = (3.0 + mb / 7.5) * cdiv(layers, at_once);
+    return (T + layers - 1) * step_us + 10.0 < layers * (40.0 + 0.6 * T);
+}
+
+size_t fastlstm_infer_short_scratch_bytes(int layers, int T, int B, int H, int dtype) {
+    if (layers <= 0 || !dtype_ok(dtype) || check_dims(T, B, H, H)) return 0;
+    if (T == 1) return 0;   // (a lower layer's out is its h_n, and no c is carried)
+    return align_up((size_t)(layers - 1) * T * B * H * elem_bytes(dtype), 256) + (size_t)layers * B * H * sizeof(float);
+}
+
+int fastlstm_infer_short(int layers, const void *const *weights, const void *x, const void *h0, const void *c0, void *out,
+                         void *h_n, void *c_n, void *scratch, size_t scratch_bytes, int T, int B, int I, int H, int dtype,
+                         void *stream) {
+    if (!weights || !x || !out || !h_n || !c_n || (!h0) != (!c0)) return FASTLSTM_ERR_NULL;
+    if (!dtype_ok(dtype)) return FASTLSTM_ERR_DTYPE;
+    if (layers <= 0) return FASTLSTM_ERR_DIM;
+    if (int rc = check_dims(T, B, I, H)) return rc;
+    if (cdiv(B, 64) > 65535) return FASTLSTM_ERR_DIM;
+    if (scratch_bytes < fastlstm_infer_short_scratch_bytes(layers, T, B, H, dtype) || (T > 1 && !scratch)) return FASTLSTM_ERR_WORKSPACE;
+    if (T > 1 && !aligned16(scratch)) return FASTLSTM_ERR_ALIGN;
+    if (int rc = take_pending_status()) return rc;
+    const size_t es = elem_bytes(dtype), bh = (size_t)B * H;
+    // whole 16-byte pieces in every row of every operand
+    bool vec = (I * es) % 16 == 0 && (H * es) % 16 == 0 && aligned16(x) && aligned16(h0) && aligned16(out) && aligned16(h_n);
+    for (int l = 0; l < layers; ++l) {
+        if (!weights[4 * l] || !weights[4 * l + 2]) return FASTLSTM_ERR_NULL;
+        vec = vec && aligned16(weights[4 * l]) && aligned16(weights[4 * l + 2]);
+    }
+    unsigned char *lower = static_cast<unsigned char *>(scratch);   // [layers - 1][T][B][H]
+    float *run = T > 1 ? reinterpret_cast<float *>(lower + align_up((size_t)(layers - 1) * T * bh * es, 256)) : nullptr;
+    auto at = [](const void *p, size_t bytes) { return p ? static_cast<const unsigned char *>(p) + bytes : nullptr; };
+    auto out_of = [&](int l, int t) -> void * {   // where step t of layer l puts its h
+        if (l == layers - 1) return static_cast<unsigned char *>(out) + (size_t)t * bh * es;
+        return T == 1 ? static_cast<unsigned char *>(h_n) + (size_t)l * bh * es : lower + ((size_t)l * T + t) * bh * es;
+    };
+    for (int k = 0; k < T + layers - 1; ++k) {
+        StepParams p{};
+        p.B = B; p.H = H;
+        int jobs = 0;
+        for (int l = std::max(0, k - T + 1); l <= std::min(k, layers - 1); ++l) {
+            const int t = k - l;
+            StepJob &j = p.job[jobs++];
+            j.K = l ? H : I;
+            j.x = l ? out_of(l - 1, t) : at(x, (size_t)t * B * I * es);
+            j.h = t ? out_of(l, t - 1) : at(h0, (size_t)l * bh * es);
+            j.Wx = weights[4 * l]; j.bx = weights[4 * l + 1]; j.Wh = weights[4 * l + 2]; j.bh = weights[4 * l + 3];
+            j.first = t == 0;
+            j.c_in = at(c0, (size_t)l * bh * es);
+            j.c_run = run ? run + (size_t)l * bh : nullptr;
+            j.h_out = out_of(l, t);
+            if (t == T - 1) {
+                void *hn = static_cast<unsigned char *>(h_n) + (size_t)l * bh * es;
+                j.h_out2 = hn != j.h_out ? hn : nullptr;
+                j.c_out = static_cast<unsigned char *>(c_n) + (size_t)l * bh * es;
+            }
+            if (jobs == kStepJobs || l == std::min(k, layers - 1)) {
+                if (launch_step(dtype, p, jobs, vec, static_cast<hipStream_t>(stream)) != hipSuccess) return FASTLSTM_ERR_HIP;
+                jobs = 0;
+            }
+        }
+    }
+    return FASTLSTM_OK;
 }
 
 // ---- fastlstm_fwd_layer for callers that cannot allocate ---------------------------------------

@@ -1158,6 +1158,13 @@ def _padded_hidden_size_cached(T, B, H, code, device_index, training, families):
     return 0
 
 
+@functools.lru_cache(maxsize=4096)
+def _short_scratch_bytes(L, T, B, I, H, code):
+    """Scratch bytes of fastlstm_infer_short for this call, or -1 where the persistent path is the faster form."""
+    lib = _lib.load()
+    return lib.fastlstm_infer_short_scratch_bytes(L, T, B, H, code) if lib.fastlstm_infer_short_applies(L, T, B, I, H, code) else -1
+
+
 class _GatherRows(torch.autograd.Function):
     """src[take]; the gradient of src is the rows `back` of the result's gradient -- for a gather in which every
     row of src has one slot that counts (back[p]) and the other slots' gradients are zero by construction."""
@@ -1186,6 +1193,9 @@ class _TakeRows(torch.autograd.Function):
     def backward(ctx, g):
         idx, = ctx.saved_tensors
         return g.new_zeros(ctx.n, g.shape[1]).index_copy(0, idx, g), None
+
+
+_LAYER_PARAMETERS = ("weight_ih_l", "bias_ih_l", "weight_hh_l", "bias_hh_l")   # in the order of _layer_operands
 
 
 class FastLSTM(nn.Module):
@@ -1360,7 +1370,53 @@ class FastLSTM(nn.Module):
                 x = F.dropout(x, self.dropout, True)
         return x, h_n, c_n
 
+    def _forward_short(self, x, h_c_0):
+        """A few timesteps without gradients (the steps of a stream, the state carried from call to call):
+        fastlstm_infer_short, one library call for all layers.  None where it does not apply."""
+        if type(x) is not torch.Tensor or x.dim() != 3 or not x.is_contiguous() or torch.is_autocast_enabled():
+            return None
+        T, B, I = x.shape
+        dt, idx, L, H = x.dtype, x.get_device(), self.num_layers, self.hidden_size
+        if T > 64 or idx < 0 or dt not in _DTYPE_CODE or I != self.input_size or self.batch_first or self.bidirectional:
+            return None
+        if self.version != "persistent" or (self.dropout and self.training):
+            return None
+        scratch_bytes = _short_scratch_bytes(L, T, B, I, H, _DTYPE_CODE[dt])
+        if scratch_bytes < 0:
+            return None
+        h0 = c0 = None
+        if h_c_0 is not None:
+            h_0, c_0 = h_c_0
+            for t in (h_0, c_0):
+                if type(t) is not torch.Tensor or t.dtype != dt or t.shape != (L, B, H) or t.get_device() != idx or not t.is_contiguous():
+                    return None
+            h0, c0 = h_0.data_ptr(), c_0.data_ptr()
+        params, pointers = self._parameters, []
+        for layer in range(L):
+            for name in _LAYER_PARAMETERS if self.bias else _LAYER_PARAMETERS[::2]:
+                p = params.get(name + str(layer))   # (missing: parametrized, say; then the general path asks for the attribute)
+                if p is None or p.dtype != dt or p.get_device() != idx or not p.is_contiguous():
+                    return None
+                pointers.append(p.data_ptr())
+                if not self.bias:
+                    pointers.append(None)
+        if idx != torch.cuda.current_device():
+            with torch.cuda.device(idx):
+                return self._forward_short(x, h_c_0)
+        out, h_n, c_n = x.new_empty((T, B, H)), x.new_empty((L, B, H)), x.new_empty((L, B, H))
+        scratch = torch.empty(scratch_bytes, dtype=torch.uint8, device=x.device) if scratch_bytes else None
+        status = _lib.load().fastlstm_infer_short(
+            L, (ctypes.c_void_p * (4 * L))(*pointers), x.data_ptr(), h0, c0, out.data_ptr(), h_n.data_ptr(), c_n.data_ptr(),
+            scratch.data_ptr() if scratch_bytes else None, scratch_bytes, T, B, I, H, _DTYPE_CODE[dt], _stream())
+        if status != _lib.OK:
+            _lib.check(status, "an earlier fastlstm launch on %s" % (x.device,) if status == _lib.ERR_TIMEOUT else "fastlstm_infer_short")
+        return out, (h_n, c_n)
+
     def forward(self, x, h_c_0=None):
+        if not torch.is_grad_enabled():
+            short = self._forward_short(x, h_c_0)
+            if short is not None:
+                return short
         directions = 2 if self.bidirectional else 1
         if h_c_0 is None:
             h_0, c_0 = [None] * (self.num_layers * directions), [None] * (self.num_layers * directions)
@@ -1587,6 +1643,9 @@ class _OperandsPadded:
         return self._module.parameters()
 
     def _operand_padding(self, x):
+        return None
+
+    def _forward_short(self, x, h_c_0):
         return None
 
     def _layer_operands(self, layer, suffix=""):

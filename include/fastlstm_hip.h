@@ -148,6 +148,19 @@ int fastlstm_fwd_layer_noalloc(const void *x, const void *Wx, const void *bx, co
                                void *stream);
 size_t fastlstm_noalloc_scratch_bytes(void);
 
+/* A few timesteps of inference through `layers` stacked layers of one direction (the loop of fastlstm/lstm.py:685-696
+ * over lstm_persistent_fwd, :31-146), one kernel per timestep and no workspace: for steps of a stream whose state is carried
+ * from call to call.  weights: 4 * layers device pointers on the host, (Wx, bx, Wh, bh) per layer, bx and bh may be
+ * null; x[T,B,I]; h0, c0 [layers,B,H] or both null (zeros); out[T,B,H], h_n, c_n [layers,B,H]; scratch:
+ * fastlstm_infer_short_scratch_bytes device bytes on a 16-byte boundary (0 for T = 1).  Any alignment of the other pointers; results
+ * as fastlstm_fwd_layer_infer up to the rounding of the projection, which is not stored here.
+ * fastlstm_infer_short_applies: 1 where this is the faster form of the call. */
+int fastlstm_infer_short(int layers, const void *const *weights, const void *x, const void *h0, const void *c0, void *out,
+                         void *h_n, void *c_n, void *scratch, size_t scratch_bytes, int T, int B, int I, int H,
+                         int dtype, void *stream);
+size_t fastlstm_infer_short_scratch_bytes(int layers, int T, int B, int H, int dtype);
+int fastlstm_infer_short_applies(int layers, int T, int B, int I, int H, int dtype);
+
 /* fastlstm_fwd_layer for a forward pass that no reverse pass follows (the reference decides this per
  * call from torch.is_grad_enabled / requires_grad and still stores everything, fastlstm/lstm.py:
  * 507-522): out[1..T] and cell[T] are the same bits as fastlstm_fwd_layer writes; the recurrence
