@@ -54,6 +54,8 @@ SIGNATURES = {
     "fastlstm_fwd_persistent": (_i, [_vp, _vp, _vp, _vp, _vp, _sz, _i, _i, _i, _i, _vp]),
     "fastlstm_fwd_layer": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _i, _i, _i, _i, _i, _vp]),
     "fastlstm_fwd_layer_infer": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _i, _i, _i, _i, _i, _vp]),
+    "fastlstm_copy_blocks": (_i, [_i, _vp, _i, _i, _vp, _vp, _vp, _vp]),
+    "fastlstm_upload_ints": (_i, [_vp, _i, _vp, _vp]),
     "fastlstm_infer_short": (_i, [_i] + [_vp] * 8 + [_sz, _i, _i, _i, _i, _i, _vp]),
     "fastlstm_infer_short_scratch_bytes": (_sz, [_i, _i, _i, _i, _i]),
     "fastlstm_infer_short_applies": (_i, [_i, _i, _i, _i, _i, _i]),

@@ -1159,6 +1159,31 @@ def _padded_hidden_size_cached(T, B, H, code, device_index, training, families):
 
 
 @functools.lru_cache(maxsize=4096)
+def _operand_padding_cached(T, B, I, H, num_layers, bidirectional, whole_rows, code, idx, training, families):
+    fp32 = code == _DTYPE_CODE[torch.float32]
+    Hp = _padded_hidden_size(T, B, H, code, idx, training) or H
+    # Where H is padded anyway and stacked layers read it as the K of their input projection: a multiple of 64, which
+    # the MFMA tile kernel takes (2 x (T = 256, B = 32): H = 704 forward + backward 2.19 ms, H = 672 2.32).  (Two
+    # directions make K = 2H; below 512 the projection is too small to matter.)
+    if (Hp != H and num_layers > 1 and not bidirectional and not fp32 and Hp % 64 == 32
+            and Hp >= 512 and _recurrent_kind(T, B, Hp + 32, code, idx) in (1, 2)):
+        Hp += 32
+    Ip = -(-I // 64) * 64 if not fp32 and T * B >= 1024 and whole_rows else I
+    if Hp <= 64 and I <= 64 and I % 16 == 0:   # a narrow layer's streaming products take any multiple of 16
+        Ip = I
+    return (Hp, Ip) if (Hp, Ip) != (H, I) else None
+
+
+@functools.lru_cache(maxsize=4096)
+def _rows_per_launch(T, B, H, code, idx, families):
+    """fastlstm_recurrent_rows_per_launch of the forward call for the workspace this module allocates."""
+    lib = _lib.load()
+    with torch.cuda.device(idx):
+        plan = _plan(torch.device("cuda", idx), B, H, code, False)
+        return lib.fastlstm_recurrent_rows_per_launch(T, B, H, code, 0, lib.fastlstm_recurrent_workspace_bytes(plan, T, H, code, 0))
+
+
+@functools.lru_cache(maxsize=4096)
 def _short_scratch_bytes(L, T, B, I, H, code):
     """Scratch bytes of fastlstm_infer_short for this call, or -1 where the persistent path is the faster form."""
     lib = _lib.load()
@@ -1252,6 +1277,21 @@ class FastLSTM(nn.Module):
         return (stack2_runs_in_one_launch(T, B, I, self.hidden_size, dt, x.device)
                 or stack2_wavefront_chunks(T, B, self.hidden_size, dt, x.device) > 0)
 
+    def _plan_layers(self, x, h_c_0):
+        return layers.plan(self, x, h_c_0)
+
+    def _operand_list(self):
+        """The parameters in the order (Wx, bx, Wh, bh) (without biases: Wx, Wh) per layer and direction."""
+        names = self.__dict__.get("_operand_names")
+        if names is None:
+            names = self.__dict__["_operand_names"] = [
+                name + str(layer) + suffix for layer in range(self.num_layers)
+                for suffix in ("", "_reverse")[:2 if self.bidirectional else 1]
+                for name in (_LAYER_PARAMETERS if self.bias else _LAYER_PARAMETERS[::2])]
+        params = self._parameters
+        # (a parametrized parameter is no entry of _parameters but an attribute)
+        return [params[n] if n in params else getattr(self, n) for n in names]
+
     def _layer_operands(self, layer, suffix=""):
         """(Wx, bx, Wh, bh) of one layer and direction; zero biases when the module has none."""
         Wx = getattr(self, f"weight_ih_l{layer}{suffix}")
@@ -1317,23 +1357,27 @@ class FastLSTM(nn.Module):
             h_n, c_n = h_n.index_select(1, packed.unsorted_indices), c_n.index_select(1, packed.unsorted_indices)
         return out, (h_n, c_n)
 
-    def _packed_range_rows(self, T, B, lengths, data):
+    def _packed_range_rows(self, T, B, lengths, data, H=None):
         """Rows per range for a packed batch of B rows sorted by length (descending, lengths on the CPU): the rows
         the library takes per launch where it runs this batch as several launches
         (fastlstm_recurrent_rows_per_launch) and cutting there saves at least an eighth of the steps; else 0."""
         dt = torch.get_autocast_dtype("cuda") if torch.is_autocast_enabled() else data.dtype
         if not data.is_cuda or dt not in _DTYPE_CODE or B < 32:
             return 0
-        lib = _lib.load()
-        code, H = _DTYPE_CODE[dt], self.hidden_size
-        with torch.cuda.device(data.device):
-            plan = _plan(data.device, B, H, code, False)
-            rows = lib.fastlstm_recurrent_rows_per_launch(T, B, H, code, 0,
-                                                          lib.fastlstm_recurrent_workspace_bytes(plan, T, H, code, 0))
+        rows = _rows_per_launch(T, B, H or self.hidden_size, _DTYPE_CODE[dt], data.get_device(), _families())
         if rows <= 0 or rows >= B:
             return 0
         saved = sum((T - int(lengths[r0])) * (min(B, r0 + rows) - r0) for r0 in range(0, B, rows))
         return rows if saved * 8 >= T * B else 0
+
+    def _packed_range_rows_of(self, packed, H):
+        """_packed_range_rows of a PackedSequence whose layers run with H hidden units."""
+        T, B, dev = packed.batch_sizes.numel(), int(packed.batch_sizes[0]), packed.data.get_device()
+        dt = torch.get_autocast_dtype("cuda") if torch.is_autocast_enabled() else packed.data.dtype
+        if not 0 < _rows_per_launch(T, B, H, _DTYPE_CODE[dt], dev, _families()) < B:
+            return 0
+        lengths = (packed.batch_sizes[:, None] > torch.arange(B)[None, :]).sum(0)
+        return self._packed_range_rows(T, B, lengths, packed.data, H)
 
     def _run_padded(self, x, lengths_dev, h_0, c_0):
         """All layers over a padded batch x [T,B,I] with T = max(lengths); lengths_dev [B] on x's device; h_0, c_0:
@@ -1428,6 +1472,9 @@ class FastLSTM(nn.Module):
         data = x.data if isinstance(x, nn.utils.rnn.PackedSequence) else x
         if data.is_cuda and not torch.cuda.is_current_stream_capturing():
             _raise_pending(data.device)   # a failed earlier launch is reported before new work goes behind it
+        call = self._plan_layers(x, h_c_0)
+        if call is not None:
+            return layers.run(self, call, x, h_c_0)
         padding = self._operand_padding(x)
         if padding:
             return self._forward_operands_padded(x, h_c_0, *padding)
@@ -1571,23 +1618,12 @@ class FastLSTM(nn.Module):
         if dt not in _DTYPE_CODE:
             return None
         if packed:
-            T, B = int(x.batch_sizes.numel()), int(x.batch_sizes[0])
+            T, B = x.batch_sizes.numel(), int(x.batch_sizes[0])
         else:
             T, B = (data.shape[1], data.shape[0]) if self.batch_first else (data.shape[0], data.shape[1])
-        idx = data.device.index if data.device.index is not None else torch.cuda.current_device()
-        H, I = self.hidden_size, self.input_size
-        training = torch.is_grad_enabled() and (data.requires_grad or any(p.requires_grad for p in self.parameters()))
-        Hp = _padded_hidden_size(T, B, H, _DTYPE_CODE[dt], idx, training) or H
-        # Where H is padded anyway and stacked layers read it as the K of their input projection: a multiple of 64, which
-        # the MFMA tile kernel takes (2 x (T = 256, B = 32): H = 704 forward + backward 2.19 ms, H = 672 2.32).  (Two
-        # directions make K = 2H; below 512 the projection is too small to matter.)
-        if (Hp != H and self.num_layers > 1 and not self.bidirectional and dt != torch.float32 and Hp % 64 == 32
-                and Hp >= 512 and _recurrent_kind(T, B, Hp + 32, _DTYPE_CODE[dt], idx) in (1, 2)):
-            Hp += 32
-        Ip = -(-I // 64) * 64 if dt != torch.float32 and T * B >= 1024 and data.shape[-1] == I else I
-        if Hp <= 64 and I <= 64 and I % 16 == 0:   # a narrow layer's streaming products take any multiple of 16
-            Ip = I
-        return (Hp, Ip) if (Hp, Ip) != (H, I) else None
+        training = torch.is_grad_enabled() and (data.requires_grad or any(p.requires_grad for p in self._operand_list()))
+        return _operand_padding_cached(T, B, self.input_size, self.hidden_size, self.num_layers, self.bidirectional,
+                                       data.shape[-1] == self.input_size, _DTYPE_CODE[dt], data.get_device(), training, _families())
 
     def _forward_operands_padded(self, x, h_c_0, Hp, Ip):
         H, D = self.hidden_size, 2 if self.bidirectional else 1
@@ -1648,6 +1684,9 @@ class _OperandsPadded:
     def _forward_short(self, x, h_c_0):
         return None
 
+    def _plan_layers(self, x, h_c_0):
+        return None
+
     def _layer_operands(self, layer, suffix=""):
         if (layer, suffix) not in self._operands:
             H, Hp, D = self._module.hidden_size, self.hidden_size, 2 if self.bidirectional else 1
@@ -1679,3 +1718,6 @@ class _OperandsPadded:
                 cache[key] = (stamp, ops)
             self._operands[(layer, suffix)] = ops
         return self._operands[(layer, suffix)]
+
+
+from . import layers  # noqa: E402  (reads this module's functions at call time)

@@ -148,6 +148,32 @@ int fastlstm_fwd_layer_noalloc(const void *x, const void *Wx, const void *bx, co
                                void *stream);
 size_t fastlstm_noalloc_scratch_bytes(void);
 
+/* n copies in one launch (more than 32: several): zero-padding, cutting, converting and reordering of the operands and results
+ * of a call (the counterparts of the torch operators around the layers, fastlstm/lstm.py:509-515, 685-698).
+ * descriptors: n * FASTLSTM_COPY_FIELDS 64-bit integers on the host, per copy: src, src2 (addresses; 0: zeros, nothing to
+ * add), dst, src mode, src2 mode, dst mode, groups, rows_src, rows_dst, blocks, cols_src, cols_dst, ld_src, ld_src2,
+ * ld_dst (elements), dtype of src and src2 + 16 * dtype of dst.
+ * All modes 0: dst[g][r][k][c] = r < rows_src and c < cols_src ? src[g][r][k][c] : 0 for g < groups, r < rows_dst, k < blocks,
+ * c < cols_dst, where row (g, r) starts at (g * rows + r) * ld and block k of a row at k * cols.
+ * Otherwise (groups = rows = 0, blocks = 1) row by row over the steps t < T and rows b < B of a batch, each tensor addressed in
+ * its own mode; elements c < cols_src, zeros up to cols_dst.  lens [B], offs [T]: length of row b, first packed row of step t
+ * (both null: T steps each, t * B); order [B] or null: row of b in the caller's order.  Device pointers. */
+#define FASTLSTM_COPY_FIELDS 16
+enum {
+    FASTLSTM_ROWS_PADDED = 1,            /* t * B + b */
+    FASTLSTM_ROWS_PADDED_REVERSED = 2,   /* (len - 1 - t) * B + b; behind the end of the row as PADDED */
+    FASTLSTM_ROWS_PACKED = 3,            /* offs[t] + b; behind the end of the row: reads zeros, writes nothing */
+    FASTLSTM_ROWS_PACKED_REVERSED = 4,   /* offs[len - 1 - t] + b */
+    FASTLSTM_ROWS_LAST = 5,              /* (len - 1) * B + b, for each b once (as dst), as are the following */
+    FASTLSTM_ROWS_ORDERED = 6,           /* order[b] */
+    FASTLSTM_ROWS_BATCH = 7              /* b */
+};
+int fastlstm_copy_blocks(int n, const long long *descriptors, int T, int B, const int *lens, const int *offs,
+                         const long long *order, void *stream);
+/* n host integers to device memory through the arguments of a launch: no pinned buffer, no synchronisation; the host
+ * memory may be reused at once. */
+int fastlstm_upload_ints(const int *host, int n, int *dev, void *stream);
+
 /* A few timesteps of inference through `layers` stacked layers of one direction (the loop of fastlstm/lstm.py:685-696
  * over lstm_persistent_fwd, :31-146), one kernel per timestep and no workspace: for steps of a stream whose state is carried
  * from call to call.  weights: 4 * layers device pointers on the host, (Wx, bx, Wh, bh) per layer, bx and bh may be

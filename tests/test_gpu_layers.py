@@ -1,0 +1,101 @@
+"""What surrounds the layers of a call: the copy launch (fastlstm_copy_blocks) against torch indexing, and the one-node form of
+a call (fastlstm_amd.layers) against the layer loop of the module."""
+import pytest
+import torch
+from torch.nn.utils.rnn import PackedSequence, pack_padded_sequence
+
+import fastlstm_amd.layers as layers
+import fastlstm_amd.lstm as L
+from fastlstm_amd import FastLSTM
+
+pytestmark = pytest.mark.gpu
+CODE = L._DTYPE_CODE
+
+
+class _Ctx:
+    def __init__(self, T=0, B=0, lens=None, offs=None, order=None):
+        self.T, self.B, self.stream = T, B, L._stream()
+        self.lens, self.offs, self.order = (None if t is None else t.data_ptr() for t in (lens, offs, order))
+
+
+@pytest.mark.parametrize("src,dst", [(torch.float32, torch.bfloat16), (torch.float16, torch.float32), (torch.float16, torch.float16)])
+@pytest.mark.parametrize("G,rs,rd,blocks,cs,cd", [(1, 1, 1, 1, 1, 1), (4, 5, 8, 1, 7, 16), (4, 8, 5, 2, 16, 9), (3, 33, 33, 2, 65, 65), (4, 1, 1, 1, 257, 288)])
+def test_padding_cutting_and_converting_copies(G, rs, rd, blocks, cs, cd, src, dst):
+    a = torch.randn(G, rs, blocks, cs, device="cuda").to(src)
+    out, zero = (torch.full((G, rd, blocks, cd), 7.0, device="cuda", dtype=dst) for _ in range(2))
+    c = layers._Copies()
+    c.matrix(a.data_ptr(), out.data_ptr(), G, (rs, rd), (cs, cd), CODE[src] + 16 * CODE[dst], blocks=blocks)
+    c.matrix(None, zero.data_ptr(), G, (rs, rd), (cs, cd), CODE[src] + 16 * CODE[dst], blocks=blocks)
+    c.run(_Ctx())
+    want = torch.zeros_like(out)
+    r, k = min(rs, rd), min(cs, cd)
+    want[:, :r, :, :k] = a[:, :r, :, :k].to(dst)
+    assert torch.equal(out, want) and not zero.any()
+
+
+@pytest.mark.parametrize("n", [1, 9, 40])   # (more sequences than descriptors fit a launch have nothing to do with it; 40 copies do)
+def test_row_modes_of_the_copies(n):
+    T, B, I = 7, 5, 11
+    lens = torch.tensor([7, 7, 4, 2, 1])
+    sizes = torch.tensor([int((lens > t).sum()) for t in range(T)])
+    offs = torch.cumsum(sizes, 0) - sizes
+    order = torch.tensor([3, 0, 4, 1, 2], device="cuda")
+    packed, padded = torch.randn(int(sizes.sum()), I, device="cuda"), torch.randn(T, B, I, device="cuda")
+    ints = torch.cat((lens, offs)).int().cuda()
+    ctx = _Ctx(T, B, ints[:B], ints[B:], order)
+    f32 = CODE[torch.float32] * 17
+    outs = [torch.full((T, B, 16), 7.0, device="cuda") for _ in range(n)]
+    back, last, state = torch.zeros_like(packed), torch.zeros(B, I, device="cuda"), torch.zeros(B, I, device="cuda")
+    c = layers._Copies()
+    for o in outs:
+        c.rows(packed.data_ptr(), layers.PACKED_REVERSED, I, o.data_ptr(), layers.PADDED, 16, (I, 16), f32)
+    c.rows(padded.data_ptr(), layers.REVERSED, I, back.data_ptr(), layers.PACKED, I, (I, I), f32, packed.data_ptr(), layers.PACKED, I)
+    c.rows(padded.data_ptr(), layers.LAST, I, last.data_ptr(), layers.ORDERED, I, (I, I), f32)
+    c.rows(last.data_ptr(), layers.ORDERED, I, state.data_ptr(), layers.BATCH, I, (I, I), f32)
+    c.run(ctx)
+    for b in range(B):
+        ln = int(lens[b])
+        for t in range(T):
+            row = packed[int(offs[ln - 1 - t]) + b] if t < ln else torch.zeros(I, device="cuda")
+            assert all(torch.equal(o[t, b, :I], row) and not o[t, b, I:].any() for o in outs)
+            if t < ln:
+                assert torch.equal(back[int(offs[t]) + b], padded[ln - 1 - t, b] + packed[int(offs[t]) + b])
+        assert torch.equal(last[int(order[b])], padded[ln - 1, b]) and torch.equal(state[b], padded[ln - 1, b])
+
+
+@pytest.mark.parametrize("kw,T,B,I,H,dt,autocast,packed", [
+    (dict(num_layers=2), 35, 20, 90, 150, torch.float32, torch.bfloat16, False),              # converted and padded parameters
+    (dict(num_layers=2, bidirectional=True), 40, 12, 50, 100, torch.float16, None, True),     # both directions between layers, packed
+    (dict(num_layers=3, bias=False, batch_first=True), 33, 9, 24, 65, torch.float32, None, False),
+    (dict(num_layers=2), 130, 16, 64, 512, torch.float16, None, True),                        # a wavefront of two layers, packed
+    (dict(), 12, 5, 16, 48, torch.float32, torch.float16, False),
+])
+def test_one_node_call_against_the_layer_loop(kw, T, B, I, H, dt, autocast, packed, monkeypatch):
+    torch.manual_seed(T)
+    m = FastLSTM(I, H, **kw).to("cuda", dt)
+    D = 2 if kw.get("bidirectional") else 1
+    x = torch.randn(*((B, T) if kw.get("batch_first") else (T, B)), I, device="cuda").to(dt)
+    if packed:
+        lengths = torch.randint(1, T + 1, (B,))
+        lengths[B // 2] = T
+        x = pack_padded_sequence(x, lengths, enforce_sorted=False)
+    s = tuple((torch.randn(m.num_layers * D, B, H, device="cuda") * 0.3).to(dt) for _ in range(2))
+    plan, taken, results = layers.plan, [], []
+    for node in (False, True):
+        monkeypatch.setattr(layers, "plan", (lambda *a: (taken.append(plan(*a)), taken[-1])[1]) if node else (lambda *a: None))
+        m.zero_grad(set_to_none=True)
+        leaf = (x.data if packed else x).detach().clone().requires_grad_(True)
+        st = tuple(t.clone().requires_grad_(True) for t in s)
+        arg = PackedSequence(leaf, x.batch_sizes, x.sorted_indices, x.unsorted_indices) if packed else leaf
+        with torch.autocast("cuda", dtype=autocast or torch.float16, enabled=autocast is not None):
+            y, (h, c) = m(arg, st)
+        y = y.data if packed else y
+        w = torch.randn(y.shape, generator=torch.Generator("cuda").manual_seed(3), device="cuda").to(y.dtype)
+        loss = (y * w).sum() + (h.float().sum() if packed else 0.0)   # (packed: h_n carries a gradient)
+        loss.backward()
+        results.append([y, h, c, leaf.grad, st[0].grad, st[1].grad] + [p.grad for p in m.parameters()])
+    assert taken and taken[0] is not None
+    tol = 2e-5 if (autocast or dt) == torch.float32 else 1.2e-2
+    for a, b in zip(*results):
+        assert a.shape == b.shape and a.dtype == b.dtype
+        assert (a.float() - b.float()).abs().max() <= tol * a.float().abs().max()
