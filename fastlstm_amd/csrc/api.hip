@@ -375,6 +375,11 @@ struct SecondLayer {
     void *ifgo, *out, *cell;
 };
 
+// Products inside a recurrent launch overlap with it chunk by chunk, all but the first chunk (forward: the time loop starts behind
+// it) or the last one (reverse).  A layer of fewer than four chunks (reverse: of one) has little to overlap, and launches of
+// their own are the better tiles (T = 35, B = 20, I = H = 704, one chunk: forward 134 us inside, 103 as two launches).
+constexpr int kMinChunks = 4;
+
 bool plan_k1_helpers(const XcdCfg &c, const void *x, const void *Wx, const void *bx, const void *bh, void *ifgo, int T,
                      int B, int I, int H, int dtype, FwdXcdParams *p, const SecondLayer *second = nullptr) {
     if (dtype == FASTLSTM_FP32 || c.nwv != 8 || c.mt != 8 || c.nkw != 8) return false;
@@ -385,10 +390,10 @@ bool plan_k1_helpers(const XcdCfg &c, const void *x, const void *Wx, const void 
     const int max_chunks = kMaxChunks;
     const int M = T * B, N = 4 * H;
     if (!gemm16_eligible(dtype, M, N, I, I, I, false, false) || N % 8) return false;
-    if (!second && !helpers_keep_up(2.0 * M * N * I, n_helpers, T * (c.ntw == 1 ? 2.3e-3 : 3.8e-3))) return false;
+    if (!second && !helpers_keep_up(2.0 * M * N * I, n_helpers, T * (c.ntw == 1 ? 1.85e-3 : 3.8e-3))) return false;
     // two layers: both projections on the helpers; past 1.25 x the time of the two time loops side by side the layers
     // are better run one by one, each with more helpers (config E: 1.0)
-    if (second && 2.0 * M * N * (I + H) / (n_helpers * 3.5e9) > 1.25 * T * 2.4e-3) return false;
+    if (second && 2.0 * M * N * (I + H) / (n_helpers * 3.5e9) > 1.25 * T * 1.95e-3) return false;
     const int tiles_m = cdiv(M, 256), tiles_n = cdiv(N, 256);
     // a chunk: whole timesteps, about one round of the helpers, at most kMaxChunks chunks
     int base = 1;
@@ -400,6 +405,7 @@ bool plan_k1_helpers(const XcdCfg &c, const void *x, const void *Wx, const void 
     while (cdiv(tiles_m, ct) > max_chunks) ct += base;
     const int steps = ct * 256 / B;
     if (steps < 2) return false;
+    if (!second && cdiv(tiles_m, ct) < kMinChunks) return false;
     p->n_layers = layers;
     p->n_active = c.n_groups * c.n_ht;
     if (second) {
@@ -722,9 +728,9 @@ bool plan_bwd_helpers(const XcdCfg &c, const void *d_ifgo, const BwdExtras &e, i
     // A weight-gradient tile is one helper's from the first timestep to the last (2 * 256 * 256 * T * B flop), so with
     // fewer tiles than helpers (H = 384: 24 tiles) most helpers have none and the launch lasts as long as one tile.
     // Of {dx and the weight gradients inside, dx inside, nothing inside} the fastest by this estimate is taken.
-    bool wgrad_inside = true;
+    bool wgrad_inside = true, lower_wgrad_inside = true;
     if (!lower) {
-        const double per_cu = 3.5e9, rec_ms = T * (c.ntw == 1 ? 3.0e-3 : 5.4e-3);   // flop per ms and CU inside a launch
+        const double per_cu = 3.5e9, rec_ms = T * (c.ntw == 1 ? 2.5e-3 : 4.4e-3);   // flop per ms and CU inside a launch
         // (e.dx null: the caller wants no dx; e.dWx null: no weight gradients)
         const double dx_flop = e.dx ? 2.0 * M * K * I : 0.0, wg_flop = e.dWx ? 2.0 * M * K * (I + H) : 0.0;
         const int wg_tiles = cdiv(K, 256) * (cdiv(I, 256) + cdiv(H, 256));
@@ -749,19 +755,24 @@ bool plan_bwd_helpers(const XcdCfg &c, const void *d_ifgo, const BwdExtras &e, i
     if (lower) {
         // the lower layer runs two chunks behind the upper one: no more than 64 timesteps per chunk
         ct = std::min(ct, std::max(1, 64 * B / 256 / base) * base);
-        // dx, dW_x and dW_h of both layers on the helpers: see plan_k1_helpers (config E: 1.0).  Where that is too much
-        // for them, both dx alone (the upper one is the lower recurrence's operand and has to be inside): the weight
-        // gradients then follow as launches of their own on the whole device (T = 512, B = 64, I = 256, H = 768 bf16,
-        // two layers: reverse pass 3.6 ms as a wavefront of launches, 2.8 ms this way).
+        // Which of dx, dW_x and dW_h of both layers the helpers take: both dx always (the upper one is the lower
+        // recurrence's operand), then by estimate all of them, all but the lower layer's weight gradients, or no weight
+        // gradients; what is left out follows on the whole device.  A CU sustains about 3.7 TFLOP/s inside the launch and
+        // 4.2 outside, and the launch lasts as long as the longer of its two sides.  2 x (T = 2048, B = 32, I = H = 1024):
+        // reverse pass 7.03 ms with all of them inside (128 helpers: 7.0 ms of products), 6.3 with the lower layer's
+        // weight gradients behind; T = 512, B = 64, I = 256, H = 768 bf16: both dx alone 2.8 ms, 3.6 as a wavefront of launches.
         const double dx_flop = 2.0 * M * K * I + (lower->dx ? 2.0 * M * K * lower->I : 0.0);
-        const double flop = dx_flop + 2.0 * M * K * (I + H) + 2.0 * M * K * (lower->I + H);
-        const double budget_ms = 1.25 * T * 3.6e-3;
-        if (flop / (n_helpers * 3.5e9) > budget_ms) {
-            if (dx_flop / (n_helpers * 3.5e9) > budget_ms) return false;
-            wgrad_inside = false;
-        }
+        const double up_flop = 2.0 * M * K * (I + H), lo_flop = 2.0 * M * K * (lower->I + H);
+        const double rec_ms = (T + 128) * 2.5e-3, in = n_helpers * 3.7e9, out = 256 * 4.2e9;
+        const double all_ms = std::max(rec_ms, (dx_flop + up_flop + lo_flop) / in);
+        const double upper_ms = std::max(rec_ms, (dx_flop + up_flop) / in) + lo_flop / out;
+        const double dx_ms = std::max(rec_ms, dx_flop / in) + (up_flop + lo_flop) / out;
+        if (dx_flop / in > 1.5 * rec_ms) return false;
+        wgrad_inside = std::min(all_ms, upper_ms) <= dx_ms;
+        lower_wgrad_inside = all_ms <= upper_ms;
     }
     while (cdiv(tiles_m, ct) > max_chunks) ct += base;
+    if (!lower && cdiv(tiles_m, ct) < 2) return false;   // (see kMinChunks)
     p->n_layers = layers;
     if (lower) {
         if (e.I != H) return false;   // the upper layer's dx is the lower layer's dout
@@ -807,7 +818,7 @@ bool plan_bwd_helpers(const XcdCfg &c, const void *d_ifgo, const BwdExtras &e, i
             if (upper_bytes > lower->scratch_bytes) {
                 p->wg_tiles = 0;
                 *wgrad_fused = false;
-            } else if (lower->dWx && lower->dWh && lower->x && lower->h && lower_wgrad_fused &&
+            } else if (lower_wgrad_inside && lower->dWx && lower->dWh && lower->x && lower->h && lower_wgrad_fused &&
                        gemm16_eligible(dtype, K, lower->I, M, K, lower->I, true, true) && lower->I % 8 == 0) {
                 // the lower layer's weight gradients the same way, its tiles parked behind the upper layer's
                 GemmParams lo{};
@@ -830,7 +841,8 @@ bool plan_bwd_helpers(const XcdCfg &c, const void *d_ifgo, const BwdExtras &e, i
     const int ipt = cdiv(16 * c.mt * 16 * c.ntw, kWave * 8);   // (unit, row) items per thread of the reverse kernel
     const bool slots_fit = p->db_lds_off + ipt * kWave * 8 * 16 <= Gemm16Cfg<256, 256, 2, 2, 4, 2>::LDS_BYTES;
     p->db_part = (*wgrad_fused && slots_fit) ? e.db_part : nullptr;
-    p->db_part_lo = (lower && lower_wgrad_fused && *lower_wgrad_fused && slots_fit) ? lower->db_part : nullptr;
+    // (the lower layer's too where its weight gradients follow behind the launch: the sums are the same either way)
+    p->db_part_lo = (lower && *wgrad_fused && slots_fit) ? lower->db_part : nullptr;
     return true;
 }
 
@@ -2013,8 +2025,12 @@ static int bwd_stack2_impl(const void *dout, void *dh1, void *dc1, const void *i
                        ? FASTLSTM_OK
                        : FASTLSTM_ERR_HIP;
         }
-        if (rc == 0 || rc == 3)
-            return fastlstm_gemm_wgrad(d_ifgo0, x, out0, dWx0, dWh0, db0, wgrad_ws, wgrad_ws_bytes, T, B, I, H, dtype, stream);
+        if (rc == 0 || rc == 3) {
+            if (int r2 = fastlstm_gemm_wgrad(d_ifgo0, x, out0, dWx0, dWh0, db0, wgrad_ws, park_bytes, T, B, I, H, dtype, stream))
+                return r2;
+            if ((db_done & 2) && launch_colsum_final(dtype, dbp0, db0, 4 * H, cdiv(B, 16), s) != hipSuccess) return FASTLSTM_ERR_HIP;
+            return FASTLSTM_OK;
+        }
     }
     // one layer after the other; the workspace is cleared in between
     if (int rc = bwd_layer_impl(dout, dh1, dc1, ifgo1, cell1, d_ifgo1, Wh1, Wx1, x1, out1, dx1, dWx1, dWh1, db1, ws, ws_bytes,

@@ -225,7 +225,7 @@ def forward(c, x, h_0, c_0, params, keep):
                 width -= 1
             if width >= 3:
                 acts = L.lstm_persistent_fwd_stack(cur, operands[layer:layer + width], **kw)
-            elif width == 2 and (L.stack2_runs_in_one_launch(T, B, cur.shape[2], Hp, c.dt, dev)
+            elif width == 2 and ((L._stack2_overlaps(T, B) and L.stack2_runs_in_one_launch(T, B, cur.shape[2], Hp, c.dt, dev))
                                  or L.stack2_wavefront_chunks(T, B, Hp, c.dt, dev)):
                 r = L.lstm_persistent_fwd_stack2(cur, *operands[layer], *operands[layer + 1], **kw)
                 acts = [r[:3], r[3:]]
