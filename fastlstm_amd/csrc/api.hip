@@ -12,7 +12,7 @@
 #include "recurrent_bwd_wide_split.hpp"
 #include "recurrent_fwd_xcd.hpp"
 #include "recurrent_step.hpp"
-#include "recurrent_stream.hpp"
+#include "recurrent_bwd_big.hpp"
 
 using namespace fastlstm;
 
@@ -1165,12 +1165,11 @@ static int fwd_persistent_impl(void *ifgo, void *out, void *cell, const void *Wh
     const int rs = (!sync && tile_io && pl.ht == 64 && pl.bt == 16) ? one_tile_row_split(B, 1 + n_others, pl.num_cus) : 0;
     const int kstep = dtype == FASTLSTM_FP32 ? 16 : 32;
     unsigned char *wsb = static_cast<unsigned char *>(ws);
-    if (pl.wave_split == 3) {   // W_h does not fit on chip: pack it once, then stream it every step
+    if (pl.wave_split == 3) {   // beyond the register-resident kernels
         const StreamLayout l = stream_layout(pl, H, dtype, false);
         hipStream_t s = static_cast<hipStream_t>(stream);
-        if (launch_pack_wh(dtype, false, Wh, wsb + l.wpack_off, H, l.KS, l.KSP, l.mt, pl.n_htiles, s) != hipSuccess)
-            return FASTLSTM_ERR_HIP;
         FwdStreamParams p{};
+        p.Wh = Wh;
         p.ifgo = ifgo; p.out = out; p.cell = cell;
         p.wpack = wsb + l.wpack_off;
         p.hdr = reinterpret_cast<WsHeader *>(wsb);
@@ -1180,6 +1179,15 @@ static int fwd_persistent_impl(void *ifgo, void *out, void *cell, const void *Wh
         p.KS = l.KS; p.KSP = l.KSP;
         p.keep = keep;
         p.spin_limit = spin_limit_ticks();
+        // 16-bit up to H = 4096: the slice of 16 units of a workgroup stays on its CU for the whole launch
+        bool resident = dtype != FASTLSTM_FP32 && pl.ht == 16 && H % 16 == 0 && l.KSP >= 80 && l.KSP <= 128 && (g_families.load() & 2);
+        if (resident) {
+            int occ = 0;
+            if (launch_fwd_big(dtype, p, l.KSP / 4, pl.bt / 16, 0, nullptr, &occ) != hipSuccess) return FASTLSTM_ERR_HIP;
+            resident = (long long)occ * pl.num_cus >= (long long)pl.n_btiles * pl.n_htiles;
+        }
+        if (!resident && launch_pack_wh(dtype, false, Wh, wsb + l.wpack_off, H, l.KS, l.KSP, l.mt, pl.n_htiles, s) != hipSuccess)
+            return FASTLSTM_ERR_HIP;
         const int n_bt_total = cdiv(B, pl.bt);
         for (int c = 0, bt0 = 0; bt0 < n_bt_total; ++c, bt0 += pl.n_btiles) {
             const int n_bt = std::min(pl.n_btiles, n_bt_total - bt0);
@@ -1189,6 +1197,10 @@ static int fwd_persistent_impl(void *ifgo, void *out, void *cell, const void *Wh
             p.b_base = bt0 * pl.bt;
             const int grid = n_bt * pl.n_htiles;
             int occ = 0;
+            if (resident) {
+                if (launch_fwd_big(dtype, p, l.KSP / 4, pl.bt / 16, grid, s, nullptr) != hipSuccess) return FASTLSTM_ERR_HIP;
+                continue;
+            }
             if (launch_fwd_stream(dtype, p, l.mt, pl.bt / 16, 0, pl.lds_bytes, nullptr, &occ) != hipSuccess) return FASTLSTM_ERR_HIP;
             if ((long long)occ * pl.num_cus < grid) return FASTLSTM_ERR_RESIDENCY;
             if (launch_fwd_stream(dtype, p, l.mt, pl.bt / 16, grid, pl.lds_bytes, s, nullptr) != hipSuccess) return FASTLSTM_ERR_HIP;
@@ -1308,11 +1320,9 @@ static int bwd_persistent_impl(const void *dout, void *dh, void *dc, const void 
     if (n_others && (sync || n_others > 3)) return FASTLSTM_ERR_DIM;
     const int kstep = dtype == FASTLSTM_FP32 ? 16 : 32;
     unsigned char *wsb = static_cast<unsigned char *>(ws);
-    if (pl.wave_split == 3) {   // W_h does not fit on chip: pack Wh[:, units]^T once, then stream it every step
+    if (pl.wave_split == 3) {   // beyond the register-resident kernels
         const StreamLayout l = stream_layout(pl, H, dtype, true);
         hipStream_t s = static_cast<hipStream_t>(stream);
-        if (launch_pack_wh(dtype, true, Wh, wsb + l.wpack_off, H, l.KS, l.KSP, l.mt, pl.n_htiles, s) != hipSuccess)
-            return FASTLSTM_ERR_HIP;
         BwdStreamParams p{};
         p.dout = dout; p.dh = dh; p.dc = dc; p.ifgo = ifgo; p.cell = cell; p.d_ifgo = d_ifgo;
         p.wpack = wsb + l.wpack_off;
@@ -1322,6 +1332,23 @@ static int bwd_persistent_impl(const void *dout, void *dh, void *dc, const void 
         p.flag_stride = (int)align_up((size_t)pl.n_htiles, 64);
         p.KSB = l.KS; p.KSBP = l.KSP;
         p.spin_limit = spin_limit_ticks();
+        // 16-bit up to H = 4096: teams of 4 workgroups keep the slices of 64 units on their CUs for the whole launch; the
+        // place of the packed weights holds the team's partial sums
+        DeviceInfo di;
+        const int teams = H / (16 * kBigTeam), grid_big = kNumXcd * cdiv(teams, kNumXcd) * kBigTeam, kw = cdiv(l.KS, 64) * 4;
+        bool resident = dtype != FASTLSTM_FP32 && pl.ht == 16 && pl.n_btiles == 1 && H % (16 * kBigTeam) == 0 && kw >= 20 && kw <= 32 && (g_families.load() & 2) &&
+                        device_info(-1, &di) == FASTLSTM_OK && di.xcd_round_robin == 1 && di.num_cus >= kNumXcd * 32 &&
+                        grid_big <= kNumXcd * 32;
+        if (resident) {
+            p.Wh = Wh;
+            p.team_flags = reinterpret_cast<int *>(wsb + kWsHeaderBytes);
+            p.partials = wsb + l.wpack_off;
+            int occ = 0;
+            if (launch_bwd_big(dtype, p, kw, pl.bt / 16, 0, nullptr, &occ) != hipSuccess) return FASTLSTM_ERR_HIP;
+            resident = occ >= 1;
+        }
+        if (!resident && launch_pack_wh(dtype, true, Wh, wsb + l.wpack_off, H, l.KS, l.KSP, l.mt, pl.n_htiles, s) != hipSuccess)
+            return FASTLSTM_ERR_HIP;
         const int n_bt_total = cdiv(B, pl.bt);
         for (int c = 0, bt0 = 0; bt0 < n_bt_total; ++c, bt0 += pl.n_btiles) {
             const int n_bt = std::min(pl.n_btiles, n_bt_total - bt0);
@@ -1331,6 +1358,11 @@ static int bwd_persistent_impl(const void *dout, void *dh, void *dc, const void 
             p.b_base = bt0 * pl.bt;
             const int grid = n_bt * pl.n_htiles;
             int occ = 0;
+            if (resident) {
+                if (c && !clear_xcd_counters(wsb, s)) return FASTLSTM_ERR_HIP;   // (the team flags lie there)
+                if (launch_bwd_big(dtype, p, kw, pl.bt / 16, grid_big, s, nullptr) != hipSuccess) return FASTLSTM_ERR_HIP;
+                continue;
+            }
             if (launch_bwd_stream(dtype, p, l.mt, pl.bt / 16, 0, pl.lds_bytes, nullptr, &occ) != hipSuccess) return FASTLSTM_ERR_HIP;
             if ((long long)occ * pl.num_cus < grid) return FASTLSTM_ERR_RESIDENCY;
             if (launch_bwd_stream(dtype, p, l.mt, pl.bt / 16, grid, pl.lds_bytes, s, nullptr) != hipSuccess) return FASTLSTM_ERR_HIP;

@@ -73,6 +73,8 @@ struct FwdStreamParams;
 struct BwdStreamParams;
 hipError_t launch_fwd_stream(int dtype, const FwdStreamParams &p, int mt, int nt, int grid, int lds, hipStream_t s,
                              int *max_blocks_per_cu);
+hipError_t launch_fwd_big(int dtype, const FwdStreamParams &p, int kw, int nt, int grid, hipStream_t s, int *max_blocks_per_cu);
+hipError_t launch_bwd_big(int dtype, const BwdStreamParams &p, int kw, int nt, int grid, hipStream_t s, int *max_blocks_per_cu);
 hipError_t launch_bwd_stream(int dtype, const BwdStreamParams &p, int mtb, int nt, int grid, int lds, hipStream_t s,
                              int *max_blocks_per_cu);
 hipError_t launch_pack_wh(int dtype, bool backward, const void *Wh, unsigned char *wpack, int H, int KS, int KSP, int mt,

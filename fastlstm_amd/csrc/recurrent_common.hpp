@@ -44,6 +44,10 @@ struct XchgGlobal {
         if constexpr (COHERENT) return __builtin_amdgcn_raw_buffer_load_b128(rsrc, off, 0, kAuxDevice);
         else return __builtin_amdgcn_raw_buffer_load_b128(rsrc, off, 0, 0);
     }
+    // device-scope load at a per-lane plus a uniform offset (in a scalar register)
+    __device__ __forceinline__ u32x4 load16(unsigned lane_off, unsigned uniform_off) const {
+        return __builtin_amdgcn_raw_buffer_load_b128(rsrc, lane_off, uniform_off, kAuxDevice);
+    }
     template <typename T> __device__ __forceinline__ void store_elem(unsigned off, T v) const {
         if constexpr (sizeof(T) == 2) {
             __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, v), rsrc, off, 0, kAuxDevice);

@@ -3,9 +3,9 @@
 //
 // The reference does the same above H = 64 (fp32) / 128 (16-bit): RELOAD_WEIGHTS, fastlstm/lstm.py:70-72,
 // fastlstm/kernels.py:464, 550-626 (forward) and 1362-1383 (reverse, always).  Here the resident kernels
-// cover everything up to 32 MiB of W_h (H = 2048 in 16 bits, 1024 in fp32); these kernels take over beyond
-// that, so that no hidden size is refused.  Mathematics, stored values and rounding points are those of
-// lstm_fwd_persistent_kernel / lstm_bwd_persistent_kernel.
+// cover everything up to 32 MiB of W_h (H = 2048 in 16 bits, 1024 in fp32) and, in 16 bits, multiples of 64 up to H = 4096
+// (recurrent_fwd_big.hpp, recurrent_bwd_big.hpp); these kernels take the rest, so that no hidden size is refused.
+// Mathematics, stored values and rounding points are those of lstm_fwd_persistent_kernel / lstm_bwd_persistent_kernel.
 //
 // What bounds a step here is the stream itself: all of W_h (4H x H elements) crosses the memory system once
 // per timestep and direction (H = 4096 in fp16: 128 MiB, 16 us at 8 TB/s), so the design keeps that stream
@@ -34,6 +34,7 @@ struct FwdStreamParams {
     void *ifgo;        // [T,B,4H]
     void *out, *cell;  // [T+1,B,H]
     const unsigned char *wpack;   // [n_ht][MT][KSP] operand blocks, rows (unit, gate), zero past H
+    const void *Wh;    // [4H,H] (lstm_fwd_big_kernel)
     WsHeader *hdr;
     int *flags;        // [n_bt][flag_stride]
     unsigned char *xbuf;   // [2 slots][n_bt][NT][KSP] operand blocks
@@ -50,6 +51,10 @@ struct BwdStreamParams {
     const void *ifgo, *cell;
     void *d_ifgo;
     const unsigned char *wpack;   // [n_ht][MTB][KSBP] operand blocks of Wh[:, units]^T, K = (unit', gate)
+    // lstm_bwd_big_kernel:
+    const void *Wh;    // [4H,H]
+    int *team_flags;   // [n_ht]
+    unsigned char *partials;   // [n_ht receivers][4 senders][NT] blocks of fp32 sums
     WsHeader *hdr;
     int *flags;
     unsigned char *xbuf;   // [2 slots][n_bt][NT][KSBP]

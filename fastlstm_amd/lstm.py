@@ -1141,6 +1141,10 @@ def _padded_hidden_size_cached(T, B, H, code, device_index, training, families):
     # The launches that pad and cut cost ~0.1 ms forward and ~0.2 ms forward + backward whatever the shape: a few steps
     # repay them only with many rows and units (T = 16, B = 128, H = 1150 bf16 forward + backward 0.82 ms as it is,
     # 0.59 ms as 1280; B = 64, H = 650 0.48 against 0.68).
+    # 16-bit between 2048 and 4096: the kernels that keep all of W_h on chip take multiples of 64, any other size streams
+    # W_h from memory every step -- ~10 us more per step (H = 2500, B = 32: 15 instead of 6), against ~0.1 ms for the copies.
+    if not fp32 and 2048 < H < 4096 and H % 64:
+        return -(-H // 64) * 64 if T >= 16 else 0
     if T < 32 and (H <= 64 or T * B * H < (1_200_000 if fp32 else 2_000_000)):
         return 0
     if H <= 64:
