@@ -9,7 +9,7 @@
 #include "recurrent_fwd.hpp"
 #include "recurrent_bwd_xcd.hpp"
 #include "recurrent_bwd_wide.hpp"
-#include "recurrent_bwd_wide_split.hpp"
+#include "recurrent_bwd_wide.hpp"
 #include "recurrent_fwd_xcd.hpp"
 #include "recurrent_step.hpp"
 #include "recurrent_bwd_big.hpp"
@@ -33,7 +33,7 @@ struct LaunchOpts {
 
 static long long *g_rec_trace = nullptr;
 static std::atomic<long long> g_spin_limit{400000000ll};  // 4 s of the 100 MHz clock
-static std::atomic<int> g_families{7};   // diagnostics: bit 0 = XCD-local kernels allowed, bit 1 = register-resident wide kernels, bit 2 = their reverse form with teams
+static std::atomic<int> g_families{7};   // diagnostics: bit 0 = XCD-local kernels allowed, bit 1 = register-resident wide kernels, bit 2 = their forms with 32 units per workgroup
 long long spin_limit_ticks() { return g_spin_limit.load(); }
 
 namespace {
@@ -542,11 +542,12 @@ static bool clear_xcd_counters(unsigned char *wsb, hipStream_t s) {
 }
 
 // Shape of a launch of the register-resident kernels whose barrier groups span several XCDs
-// (recurrent_fwd_wide.hpp): 16 units x 16 nt batch rows per workgroup, H / 16 workgroups per group.
+// (recurrent_fwd_wide.hpp): 16 units x 16 nt batch rows per workgroup, H / 16 workgroups per group; or, 16-bit, 32 units per
+// workgroup (recurrent_fwd_big.hpp).
 struct WideCfg {
     int nkw, n_ht, xpg, n_groups, ks, lds;
     int nt;   // batch tiles of 16 rows per group: the smallest of 1, 2, 4 with which the launch holds the batch
-    int v;    // reverse kernel, 64-row groups: members of a team that splits K (lstm_bwd_wide_split_kernel); 0 = no teams
+    int big;  // batch tiles per group of the kernels with 32 units per workgroup (recurrent_fwd_big.hpp), else 0
     size_t xslot;
 };
 // copies > 1: that many recurrences of this shape share the launch (groups of 16 or 32 rows only).
@@ -559,7 +560,29 @@ bool select_wide(int T, int B_all, int H, int dtype, bool backward, size_t ws_by
     // 640, 768, 896, 1024 with fp32
     const int es = elem_bytes(dtype), kstep = dtype == FASTLSTM_FP32 ? 16 : 32;
     if ((H * es) % 512 || H * es <= 2048 || H * es > 4096) return false;
-    c->nkw = (backward ? 4 * H : H) / kstep / 8;
+    c->ks = (backward ? 4 * H : H) / kstep;
+    c->big = 0;
+    if (es == 2 && copies == 1 && (g_families.load() & 4)) {
+        // 32 units per workgroup: groups of H / 32 workgroups, more of them, so fewer rows and operand bytes per CU.  The reverse
+        // pass gains at every batch size (us per step, 16 units / 32: H = 2048, B = 32 6.4 / 5.3, 64 9.0 / 6.2, 128
+        // 11.0 / 8.6; H = 1280, B = 128 8.7 / 7.0): groups of 16 rows where the batch fits the launch that way, else of 32.
+        // The forward pass gains with groups of 16 rows where the 16-unit form needs more (H = 2048, B = 64 4.57 / 4.39, H = 1280
+        // 3.99 / 3.31); with 32 rows there is no difference (H = 2048, B = 128 7.1 / 7.3), and where 16-row groups of
+        // 16-unit workgroups fit, their half as many products per CU count for more (H = 2048, B = 32 3.4 / 3.8).
+        const int n_ht = H / 32, max_groups = kNumXcd * 32 / n_ht;
+        const int nt = cdiv(B, 16) <= max_groups ? 1 : 2, groups = cdiv(B, 16 * nt);
+        const bool faster = backward || (nt == 1 && cdiv(B, 16) * cdiv(H / 16, 32) > kNumXcd);
+        const size_t xslot = (size_t)groups * nt * c->ks * kFragBytes;
+        const size_t partials = backward ? (size_t)groups * n_ht * kBigTeam * 2 * nt * kFragBytes : 0;
+        if (faster && groups <= max_groups && ws_bytes >= kWsHeaderBytes + kWsCounterBytes + 2 * xslot + partials) {
+            c->big = nt;
+            c->n_ht = n_ht;
+            c->n_groups = groups;
+            c->xslot = xslot;
+            return true;
+        }
+    }
+    c->nkw = c->ks / 8;
     c->n_ht = H / 16;
     if (c->n_ht > kXcdGroupStride) return false;
     c->xpg = cdiv(c->n_ht, 32);   // XCDs per group (the last one partly used when H is not a multiple of 512)
@@ -576,22 +599,12 @@ bool select_wide(int T, int B_all, int H, int dtype, bool backward, size_t ws_by
     // instead of 5.7 us per step; the reverse step, with four times the operand bytes, gains at every size)
     // (a remainder of rows behind full launches still runs here: the general kernel would take the whole batch)
     if (dtype == FASTLSTM_FP32 && !backward && copies * c->n_groups * c->xpg < 6 && B == B_all) return false;
-    c->ks = (backward ? 4 * H : H) / kstep;
     c->xslot = (size_t)c->n_groups * c->nt * c->ks * kFragBytes;
     if (ws_bytes < kWsHeaderBytes + kWsCounterBytes + 2 * (size_t)copies * c->xslot) return false;
     const int gr = 16 * c->nt;
     const int gseg = 16 * es;
     const int tiles = gr * (4 * gseg + 16) + 2 * gr * (gseg + 16);   // gates + two state tiles of `gr` rows x 16 units
     c->lds = backward ? 8 * c->nt * kFragBytes + tiles + 8 * kWideRing * kFragBytes : 8 * 4 * c->nt * kFragBytes + tiles;
-    c->v = 0;
-    if (backward && c->nt == 4 && (g_families.load() & 4)) {
-        const int v = 4;   // divides the k-steps per wave (20 ... 32) and the workgroups of an XCD
-        const size_t partials = (size_t)c->n_groups * c->n_ht * v * 4 * kFragBytes;
-        if (c->n_ht % v == 0 && ws_bytes >= kWsHeaderBytes + kWsCounterBytes + 2 * c->xslot + partials) {
-            c->v = v;
-            c->lds = 4 * kFragBytes + tiles + 8 * 4 * v * kFragBytes;   // the waves' sums take the place of their rings
-        }
-    }
     return true;
 }
 
@@ -599,7 +612,9 @@ bool select_wide(int T, int B_all, int H, int dtype, bool backward, size_t ws_by
 // (fp32: 32-row groups) on all XCDs.
 static int wide_rows_per_launch(int T, int B, int H, int dtype, bool backward, size_t ws_bytes) {
     const int xpg = cdiv(H / 16, 32);
-    const int rows = (dtype == FASTLSTM_FP32 ? 32 : 64) * (kNumXcd / std::max(1, xpg));
+    const int rows = backward && dtype != FASTLSTM_FP32 && H >= 32 && (g_families.load() & 4)
+                         ? 32 * (kNumXcd * 32 / (H / 32))   // (groups of the 32-unit form)
+                         : (dtype == FASTLSTM_FP32 ? 32 : 64) * (kNumXcd / std::max(1, xpg));
     if (rows >= B || rows <= 0) return 0;
     WideCfg c;
     if (!select_wide(T, B, H, dtype, backward, ws_bytes, &c, rows)) return 0;
@@ -615,6 +630,24 @@ int try_fwd_wide(void *ifgo, void *out, void *cell, const void *Wh, unsigned cha
     WideCfg c;
     const int copies = second ? 2 + o.n_more : 1;
     if (copies > kMaxSideBySide || !select_wide(T, B, H, dtype, false, ws_bytes, &c, o.rows, copies)) return 1;
+    if (c.big) {
+        FwdStreamParams q{};
+        q.ifgo = ifgo; q.out = out; q.cell = cell; q.Wh = Wh;
+        q.hdr = reinterpret_cast<WsHeader *>(wsb);
+        q.flags = reinterpret_cast<int *>(wsb + kWsHeaderBytes);
+        q.flag_stride = kXcdGroupStride;
+        q.xbuf = wsb + kWsHeaderBytes + kWsCounterBytes;
+        q.T = T; q.B = B; q.H = H;
+        q.b_base = o.row0; q.n_bt = c.n_groups; q.n_ht = c.n_ht;
+        q.KS = q.KSP = c.ks;
+        q.keep = o.keep;
+        q.spin_limit = spin_limit_ticks();
+        int occ = 0;
+        if (launch_fwd_big(dtype, q, H / 128, 8, c.big, 0, nullptr, &occ) != hipSuccess) return FASTLSTM_ERR_HIP;
+        if (occ < 1) return 1;
+        if (!dry_run && launch_fwd_big(dtype, q, H / 128, 8, c.big, c.n_groups * c.n_ht, stream, nullptr) != hipSuccess) return FASTLSTM_ERR_HIP;
+        return FASTLSTM_OK;
+    }
     FwdXcdParams p{};
     p.n_layers = copies;
     if (second) {
@@ -649,7 +682,26 @@ int try_bwd_wide(const void *dout, void *dh, void *dc, const void *ifgo, const v
     WideCfg c;
     const int copies = second ? 2 + o.n_more : 1;
     if (copies > kMaxSideBySide || !select_wide(T, B, H, dtype, true, ws_bytes, &c, o.rows, copies)) return 1;
-    if (copies > 1) c.v = 0;   // (never set: the team form is for 64-row groups)
+    if (c.big) {
+        BwdStreamParams q{};
+        q.dout = dout; q.dh = dh; q.dc = dc; q.ifgo = ifgo; q.cell = cell; q.d_ifgo = d_ifgo; q.Wh = Wh;
+        q.hdr = reinterpret_cast<WsHeader *>(wsb);
+        q.flags = reinterpret_cast<int *>(wsb + kWsHeaderBytes);
+        q.flag_stride = kXcdGroupStride;
+        q.team_flags = q.flags + kNumXcd * kXcdGroupStride;
+        q.xbuf = wsb + kWsHeaderBytes + kWsCounterBytes;
+        q.partials = q.xbuf + 2 * c.xslot;
+        q.T = T; q.B = B; q.H = H;
+        q.b_base = o.row0; q.n_bt = c.n_groups; q.n_ht = c.n_ht;
+        q.KSB = q.KSBP = c.ks;
+        q.spin_limit = spin_limit_ticks();
+        int occ = 0;
+        if (launch_bwd_big(dtype, q, H / 128, 8, c.big, 0, nullptr, &occ) != hipSuccess) return FASTLSTM_ERR_HIP;
+        if (occ < 1) return 1;
+        const int grid = kNumXcd * cdiv(c.n_groups * c.n_ht / kBigTeam, kNumXcd) * kBigTeam;
+        if (!dry_run && launch_bwd_big(dtype, q, H / 128, 8, c.big, grid, stream, nullptr) != hipSuccess) return FASTLSTM_ERR_HIP;
+        return FASTLSTM_OK;
+    }
     BwdXcdParams p{};
     p.n_layers = copies;
     if (second) {
@@ -669,15 +721,12 @@ int try_bwd_wide(const void *dout, void *dh, void *dc, const void *ifgo, const v
     p.n_ht = c.n_ht; p.gpx = c.xpg; p.n_groups = c.n_groups; p.KSB = c.ks;
     p.b_base = o.row0;
     p.spin_limit = spin_limit_ticks();
-    p.partials = p.xbuf + 2 * c.xslot;
-    auto launch = c.v ? (dtype == FASTLSTM_FP16 ? launch_bwd_wide_split_f16 : launch_bwd_wide_split_bf16)
-                      : (dtype == FASTLSTM_FP16 ? launch_bwd_wide_f16 : dtype == FASTLSTM_BF16 ? launch_bwd_wide_bf16 : launch_bwd_wide_f32);
-    const int form = c.v ? c.v : c.nt;
+    auto launch = dtype == FASTLSTM_FP16 ? launch_bwd_wide_f16 : dtype == FASTLSTM_BF16 ? launch_bwd_wide_bf16 : launch_bwd_wide_f32;
     int occ = 0;
-    if (launch(p, c.nkw, form, 0, c.lds, nullptr, &occ) != hipSuccess) return FASTLSTM_ERR_HIP;
+    if (launch(p, c.nkw, c.nt, 0, c.lds, nullptr, &occ) != hipSuccess) return FASTLSTM_ERR_HIP;
     if (occ < 1) return 1;
     if (dry_run) return FASTLSTM_OK;
-    if (launch(p, c.nkw, form, kNumXcd * 32, c.lds, stream, nullptr) != hipSuccess) return FASTLSTM_ERR_HIP;
+    if (launch(p, c.nkw, c.nt, kNumXcd * 32, c.lds, stream, nullptr) != hipSuccess) return FASTLSTM_ERR_HIP;
     return FASTLSTM_OK;
 }
 
@@ -1183,7 +1232,7 @@ static int fwd_persistent_impl(void *ifgo, void *out, void *cell, const void *Wh
         bool resident = dtype != FASTLSTM_FP32 && pl.ht == 16 && H % 16 == 0 && l.KSP >= 80 && l.KSP <= 128 && (g_families.load() & 2);
         if (resident) {
             int occ = 0;
-            if (launch_fwd_big(dtype, p, l.KSP / 4, pl.bt / 16, 0, nullptr, &occ) != hipSuccess) return FASTLSTM_ERR_HIP;
+            if (launch_fwd_big(dtype, p, l.KSP / 4, 4, pl.bt / 16, 0, nullptr, &occ) != hipSuccess) return FASTLSTM_ERR_HIP;
             resident = (long long)occ * pl.num_cus >= (long long)pl.n_btiles * pl.n_htiles;
         }
         if (!resident && launch_pack_wh(dtype, false, Wh, wsb + l.wpack_off, H, l.KS, l.KSP, l.mt, pl.n_htiles, s) != hipSuccess)
@@ -1198,7 +1247,7 @@ static int fwd_persistent_impl(void *ifgo, void *out, void *cell, const void *Wh
             const int grid = n_bt * pl.n_htiles;
             int occ = 0;
             if (resident) {
-                if (launch_fwd_big(dtype, p, l.KSP / 4, pl.bt / 16, grid, s, nullptr) != hipSuccess) return FASTLSTM_ERR_HIP;
+                if (launch_fwd_big(dtype, p, l.KSP / 4, 4, pl.bt / 16, grid, s, nullptr) != hipSuccess) return FASTLSTM_ERR_HIP;
                 continue;
             }
             if (launch_fwd_stream(dtype, p, l.mt, pl.bt / 16, 0, pl.lds_bytes, nullptr, &occ) != hipSuccess) return FASTLSTM_ERR_HIP;
@@ -1344,7 +1393,7 @@ static int bwd_persistent_impl(const void *dout, void *dh, void *dc, const void 
             p.team_flags = reinterpret_cast<int *>(wsb + kWsHeaderBytes);
             p.partials = wsb + l.wpack_off;
             int occ = 0;
-            if (launch_bwd_big(dtype, p, kw, pl.bt / 16, 0, nullptr, &occ) != hipSuccess) return FASTLSTM_ERR_HIP;
+            if (launch_bwd_big(dtype, p, kw, 4, pl.bt / 16, 0, nullptr, &occ) != hipSuccess) return FASTLSTM_ERR_HIP;
             resident = occ >= 1;
         }
         if (!resident && launch_pack_wh(dtype, true, Wh, wsb + l.wpack_off, H, l.KS, l.KSP, l.mt, pl.n_htiles, s) != hipSuccess)
@@ -1360,7 +1409,7 @@ static int bwd_persistent_impl(const void *dout, void *dh, void *dc, const void 
             int occ = 0;
             if (resident) {
                 if (c && !clear_xcd_counters(wsb, s)) return FASTLSTM_ERR_HIP;   // (the team flags lie there)
-                if (launch_bwd_big(dtype, p, kw, pl.bt / 16, grid_big, s, nullptr) != hipSuccess) return FASTLSTM_ERR_HIP;
+                if (launch_bwd_big(dtype, p, kw, 4, pl.bt / 16, grid_big, s, nullptr) != hipSuccess) return FASTLSTM_ERR_HIP;
                 continue;
             }
             if (launch_bwd_stream(dtype, p, l.mt, pl.bt / 16, 0, pl.lds_bytes, nullptr, &occ) != hipSuccess) return FASTLSTM_ERR_HIP;

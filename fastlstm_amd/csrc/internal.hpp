@@ -60,21 +60,20 @@ hipError_t launch_small_k1(int dtype, const void *x, const void *Wx, const void 
     hipError_t launch_fwd_wide_##SUF(const FwdXcdParams &p, int nkw, int nt, int grid, int lds, hipStream_t s, \
                                      int *max_blocks_per_cu);                                    \
     hipError_t launch_bwd_wide_##SUF(const BwdXcdParams &p, int nkw, int nt, int grid, int lds, hipStream_t s, \
-                                     int *max_blocks_per_cu);                                    \
-    hipError_t launch_bwd_wide_split_##SUF(const BwdXcdParams &p, int nkw, int v, int grid, int lds, hipStream_t s, \
-                                           int *max_blocks_per_cu);
+                                     int *max_blocks_per_cu);
 FASTLSTM_DECL_REC(f32)
 FASTLSTM_DECL_REC(f16)
 FASTLSTM_DECL_REC(bf16)
 #undef FASTLSTM_DECL_REC
 
-// streamed-weights kernels (recurrent_stream.hpp): plans with wave_split == 3
+// streamed-weights kernels (recurrent_stream.hpp) and the kernels that keep up to 512 KiB of weights per CU
+// (recurrent_fwd_big.hpp, recurrent_bwd_big.hpp)
 struct FwdStreamParams;
 struct BwdStreamParams;
 hipError_t launch_fwd_stream(int dtype, const FwdStreamParams &p, int mt, int nt, int grid, int lds, hipStream_t s,
                              int *max_blocks_per_cu);
-hipError_t launch_fwd_big(int dtype, const FwdStreamParams &p, int kw, int nt, int grid, hipStream_t s, int *max_blocks_per_cu);
-hipError_t launch_bwd_big(int dtype, const BwdStreamParams &p, int kw, int nt, int grid, hipStream_t s, int *max_blocks_per_cu);
+hipError_t launch_fwd_big(int dtype, const FwdStreamParams &p, int kw, int mt, int nt, int grid, hipStream_t s, int *max_blocks_per_cu);
+hipError_t launch_bwd_big(int dtype, const BwdStreamParams &p, int kw, int mt, int nt, int grid, hipStream_t s, int *max_blocks_per_cu);
 hipError_t launch_bwd_stream(int dtype, const BwdStreamParams &p, int mtb, int nt, int grid, int lds, hipStream_t s,
                              int *max_blocks_per_cu);
 hipError_t launch_pack_wh(int dtype, bool backward, const void *Wh, unsigned char *wpack, int H, int KS, int KSP, int mt,

@@ -83,7 +83,6 @@ struct BwdXcdParams {
     // Without helpers, n_layers = 3 or 4 independent recurrences: recurrence r >= 2 is described by entry r - 2.
     const void *dout_more[2], *ifgo_more[2], *cell_more[2], *Wh_more[2];
     void *dh_more[2], *dc_more[2], *d_ifgo_more[2];
-    unsigned char *partials;   // lstm_bwd_wide_split_kernel: the teams' partial sums (see there)
 };
 
 #ifndef FASTLSTM_HELPER_PP

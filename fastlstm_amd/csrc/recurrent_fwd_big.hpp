@@ -1,12 +1,12 @@
-// Persistent forward kernel for 16-bit elements and 2048 < H <= 4096: a workgroup keeps the weights of 16 hidden
-// units -- up to 512 KiB -- on its CU for the whole launch, three quarters of them in registers, the rest in LDS.
+// Persistent forward kernel for 16-bit elements and 1280 <= H <= 4096: a workgroup keeps up to 512 KiB of weights -- those of
+// 16 hidden units, or of 32 where H <= 2048 -- on its CU for the whole launch, three quarters of them in registers, the rest in LDS.
 //
 // Same mathematics, stored values and rounding points as lstm_fwd_persistent_kernel (which replaces
 // fastlstm/kernels.py:414-663).  lstm_fwd_stream_kernel reads all of W_h (H = 4096: 128 MiB) from memory every timestep;
 // here it is read once per launch.
 //  * one wave per SIMD with all of its 512 registers: the 4 waves split K (k-step ks = wave + 4 ki), a wave holds
-//    4 unit tiles x KW k-steps: up to 24 k-steps in registers (384), the others, spread evenly over the k-steps so
-//    that an LDS read has the MFMAs of the k-steps between to arrive, in LDS (32 KiB per wave);
+//    MT unit tiles (4 units each) x KW k-steps: 96 blocks in registers (384 per lane), the others in LDS, spread evenly over
+//    the k-steps so that an LDS read has the MFMAs of the k-steps between to arrive;
 //  * the batch tiles of 16 rows are multiplied one after the other.  Operand blocks go through a ring of R blocks of
 //    registers, refilled as they are consumed, across the tiles of a step;
 //  * behind each tile the four partial sums meet in LDS and the gates of its rows are computed while the next tile's operand
@@ -15,7 +15,9 @@
 // What bounds a step now: the operand blocks, 512 KiB per CU at H = 4096 and 64 rows (16 MiB through the L2 of an XCD at about
 // 2.1 TB/s), and the exchange.  us per step of lstm_fwd_stream_kernel and here: H = 4096, 64 rows 24.8 -> 11.0, 16 rows
 // 20.9 -> 4.8; H = 3072, 32 rows 14.1 -> 5.5; H = 2560, 64 rows 15.4 -> 8.7; and no packed copy of W_h per call (118 us at 4096).
-// Requirements (host): H a multiple of 16, ceil(H / 16) workgroups co-resident, LDS for KW.
+// Up to H = 2048, with 32 units, there are twice as many barrier groups as lstm_fwd_wide_kernel has: half the rows per group, half
+// the operand bytes per CU (H = 1280, B = 64 3.99 -> 3.31).
+// Requirements (host): H a multiple of MT * 4 (and of 8), the workgroups of all groups co-resident.
 #pragma once
 #include <type_traits>
 
@@ -24,13 +26,18 @@
 
 namespace fastlstm {
 
-constexpr int kBigRegSteps = 24;  // k-steps per wave whose weights stay in registers,
-constexpr int kBigAccSteps = 16;  // the first of them in the accumulator half of the register file
+constexpr int kBigRegBlocks = 96;   // blocks of weights per wave (of 4 registers per lane) that stay in registers,
+constexpr int kBigAccBlocks = 64;   // the first of them in the accumulator half of the register file
 
-constexpr int big_ring(int kw) { return kw <= 20 ? 16 : kw <= 24 ? 12 : 10; }   // operand blocks in flight per wave: what the registers hold
-constexpr int big_lds_bytes(int kw, int nt, int elem_bytes) {
-    const int bt = 16 * nt, gseg = 16 * elem_bytes, kl = kw > kBigRegSteps ? kw - kBigRegSteps : 0;
-    return 4 * kl * 4 * kFragBytes + 4 * 4 * kFragBytes + bt * (4 * gseg + 16) + 2 * bt * (gseg + 16);
+constexpr int big_ring(int kw, int mt) {   // operand blocks in flight per wave: what the registers hold
+    return mt == 8 ? (kw <= 10 ? 16 : kw <= 12 ? 12 : kw <= 14 ? 6 : 8) : kw <= 20 ? 16 : kw <= 24 ? 12 : 10;
+}
+constexpr int big_lds_steps(int kw, int mt) { return kw > kBigRegBlocks / mt ? kw - kBigRegBlocks / mt : 0; }
+// tiles whose partial sums meet in LDS at a time: all, or four where the weights leave room for no more
+constexpr int big_sum_tiles(int kw, int mt) { return 4 * big_lds_steps(kw, mt) * mt > 48 ? 4 : mt; }
+constexpr int big_lds_bytes(int kw, int mt, int nt) {   // (16-bit elements)
+    const int bt = 16 * nt, gseg = 4 * mt * 2;
+    return 4 * (big_lds_steps(kw, mt) * mt + big_sum_tiles(kw, mt)) * kFragBytes + bt * (4 * gseg + 16) + 2 * bt * (gseg + 16);
 }
 
 // acc (+)= A . B with the A block in the accumulator half of the register file (ACC_HALF) or in the ordinary one.  Inline assembly:
@@ -52,26 +59,29 @@ __device__ __forceinline__ void mfma_resident(f32x4 &acc, const u32x4 &a, const 
 }
 // The wait states between these MFMAs and the first other reader of their results (8 passes: at most 11 + 8).
 template <int N> __device__ __forceinline__ void mfma_results(f32x4 (&acc)[N]) {
-    static_assert(N == 4, "one operand per tile");
-    asm volatile("s_nop 15\n\ts_nop 7" : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]));
+    asm volatile("s_nop 15\n\ts_nop 7");
+#pragma unroll
+    for (int a = 0; a < N; a += 4) asm volatile("" : "+v"(acc[a]), "+v"(acc[a + 1]), "+v"(acc[a + 2]), "+v"(acc[a + 3]));
 }
 
-template <typename T, int KW, int NT>
+template <typename T, int KW, int MT, int NT>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))) void lstm_fwd_big_kernel(const FwdStreamParams p) {
     using E = Elem<T>;
     static_assert(E::BYTES == 2, "16-bit element types");
-    constexpr int NWV = 4, MT = 4;
-    constexpr int KR = KW < kBigRegSteps ? KW : kBigRegSteps, KL = KW - KR;
+    constexpr int NWV = 4, TPW = MT / NWV;                 // waves, unit tiles whose cells a wave takes
+    constexpr int KL = big_lds_steps(KW, MT), KR = KW - KL, ACC_STEPS = kBigAccBlocks / MT;
+    constexpr int ST = big_sum_tiles(KW, MT);
     constexpr int HT = 4 * MT, BT = 16 * NT;
-    constexpr int NB = KW * NT, R = big_ring(KW);              // operand blocks of a step, in flight
+    constexpr int NB = KW * NT, R = big_ring(KW, MT);              // operand blocks of a step, in flight
     constexpr int GSEG = HT * E::BYTES, GROW = 4 * GSEG + 16, SROW = GSEG + 16, PPSEG = GSEG / 16;
     static_assert(BT * PPSEG <= kThreads, "one state piece per thread");
-    constexpr auto in_lds = [](int ki) { return (ki + 1) * KL / KW > ki * KL / KW; };
+    constexpr auto in_lds = [](int ki) { return ki * KL % KW < KL; };   // evenly spread, the first k-step among them
+    constexpr auto reg_of = [](int ki) { return KL ? ki - ki * KL / KW - 1 : ki; };
 
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     unsigned char *wl = smem;                                                             // [wave][KL][MT] blocks
-    f32x4 *red = reinterpret_cast<f32x4 *>(smem + NWV * KL * MT * kFragBytes);            // [wave][MT][64]
-    unsigned char *tiles = reinterpret_cast<unsigned char *>(red + NWV * MT * kWave);     // gates, h, c tiles
+    f32x4 *red = reinterpret_cast<f32x4 *>(smem + NWV * KL * MT * kFragBytes);            // [wave][ST][64]
+    unsigned char *tiles = reinterpret_cast<unsigned char *>(red + NWV * ST * kWave);     // gates, h, c tiles
     unsigned char *const sth = tiles + BT * GROW, *const stc = sth + BT * SROW;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int q = lane >> 4, n = lane & 15;
@@ -94,31 +104,31 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
         if (k0 >= H) v = u32x4{0u, 0u, 0u, 0u};
         return v;
     };
+    // (whole 4-register tuples in the half that they are used from; the loads of a k-step are under way together)
+    static_for<0, KW>([&](auto kc) __attribute__((always_inline)) {
+        constexpr int ki = decltype(kc)::value, k = in_lds(ki) ? 0 : reg_of(ki);
+        u32x4 f[MT];
 #pragma unroll
-    for (int ki = 0; ki < KW; ++ki)
-#pragma unroll
-        for (int a = 0; a < MT; ++a) {
-            if (in_lds(ki)) *reinterpret_cast<u32x4 *>(wl + ((wave * KL + ki * KL / KW) * MT + a) * kFragBytes + lane * 16) = fragment(ki, a);
-            else wreg[ki - ki * KL / KW][a] = fragment(ki, a);
-        }
-    // (from here on whole 4-register tuples in the half that they are used from)
-#pragma unroll
-    for (int k = 0; k < KR; ++k)
+        for (int a = 0; a < MT; ++a) f[a] = fragment(ki, a);
 #pragma unroll
         for (int a = 0; a < MT; ++a) {
-            if (k < kBigAccSteps) asm volatile("" : "+a"(wreg[k][a]));
-            else asm volatile("" : "+v"(wreg[k][a]));
+            if constexpr (in_lds(ki)) *reinterpret_cast<u32x4 *>(wl + ((wave * KL + ki * KL / KW) * MT + a) * kFragBytes + lane * 16) = f[a];
+            else if constexpr (k < ACC_STEPS) asm volatile("" : "+a"(f[a]));
+            else asm volatile("" : "+v"(f[a]));
+            if constexpr (!in_lds(ki)) wreg[k][a] = f[a];
         }
+    });
 
-    // ---- this lane's cells: unit tile `wave`, row 16 i + n of batch tile i -------------
-    float c_state[NT];
+    // ---- this lane's cells: unit tiles wave + 4 h, row 16 i + n of batch tile i -------------
+    float c_state[NT][TPW];
     bool valid[NT];
-    const int unit = u0 + wave * 4 + q;
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
         const int b = b0 + i * 16 + n;
         valid[i] = b < B;
-        c_state[i] = valid[i] ? E::to_f32(cell[(size_t)b * H + unit]) : 0.f;
+#pragma unroll
+        for (int h = 0; h < TPW; ++h)
+            c_state[i][h] = valid[i] ? E::to_f32(cell[(size_t)b * H + u0 + (wave + NWV * h) * 4 + q]) : 0.f;
     }
     const int goff = n * GROW + (wave * 4 + q) * E::BYTES, soff = n * SROW + (wave * 4 + q) * E::BYTES;
 
@@ -184,62 +194,80 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
         if (wave == 0) wait_versions(grp_flags, p.n_ht, t + 1, p.hdr, p.spin_limit, g, t);
         __syncthreads();
 
-        u32x4 ring[R], wf[MT];
+        u32x4 ring[R], wf[4];
         auto request = [&](int b) {   // (past KS: zero weights times some block)
             const int ks = min(wave + NWV * (b % KW), KS - 1);
             ring[b % R] = xch.load16(lane * 16u, xb + (unsigned)((b / KW) * p.KSP + ks) * kFragBytes);
         };
-        auto read_weights = [&](int l) {
+        auto read_weights = [&](int l, int half) {   // four tiles at a time
 #pragma unroll
-            for (int a = 0; a < MT; ++a)
-                wf[a] = *reinterpret_cast<const u32x4 *>(wl + ((wave * KL + l) * MT + a) * kFragBytes + lane * 16);
+            for (int a = 0; a < 4; ++a)
+                wf[a] = *reinterpret_cast<const u32x4 *>(wl + ((wave * KL + l) * MT + half * 4 + a) * kFragBytes + lane * 16);
         };
 #pragma unroll
         for (int b = 0; b < R; ++b) request(b);
-        if constexpr (KL > 0) read_weights(0);
+        if constexpr (KL > 0) read_weights(0, 0);
 #pragma unroll
         for (int i = 0; i < NT; ++i) {
             f32x4 acc[MT];
             static_for<0, KW>([&](auto kc) __attribute__((always_inline)) {
                 constexpr int ki = decltype(kc)::value, l = ki * KL / KW;
+                constexpr bool halves_ = KL > 0 && MT == 8;   // the upper tiles of a k-step in LDS follow behind the next k-step
                 const int b = i * KW + ki;
                 if constexpr (in_lds(ki)) {
 #pragma unroll
-                    for (int a = 0; a < MT; ++a) mfma_resident<T, false, ki == 0>(acc[a], wf[a], ring[b % R]);
-                    if (i + 1 < NT || l + 1 < KL) read_weights((l + 1) % (KL > 0 ? KL : 1));
+                    for (int a = 0; a < 4; ++a) mfma_resident<T, false, ki == 0>(acc[a], wf[a], ring[b % R]);
+                    if constexpr (halves_) read_weights(l, 1);
+                    else if (i + 1 < NT || l + 1 < KL) read_weights((l + 1) % (KL > 0 ? KL : 1), 0);
                 } else {
 #pragma unroll
-                    for (int a = 0; a < MT; ++a) mfma_resident<T, (ki - l < kBigAccSteps), ki == 0>(acc[a], wreg[ki - l][a], ring[b % R]);
+                    for (int a = 0; a < MT; ++a) {
+                        if (halves_ && ki == 1 && a >= 4) mfma_resident<T, (reg_of(ki) < ACC_STEPS), true>(acc[a], wreg[reg_of(ki)][a], ring[b % R]);
+                        else mfma_resident<T, (reg_of(ki) < ACC_STEPS), ki == 0>(acc[a], wreg[reg_of(ki)][a], ring[b % R]);
+                    }
+                    if constexpr (halves_ && in_lds(ki - 1)) {
+#pragma unroll
+                        for (int a = 4; a < MT; ++a) mfma_resident<T, false, false>(acc[a], wf[a - 4], ring[(b - 1) % R]);
+                        if (i + 1 < NT || l + 1 < KL) read_weights((l + 1) % KL, 0);
+                        if (b - 1 + R < NB) request(b - 1 + R);
+                    }
                 }
-                if (b + R < NB) request(b + R);
+                if (!(halves_ && in_lds(ki)) && b + R < NB) request(b + R);
                 __builtin_amdgcn_sched_barrier(0);   // (the order above is the schedule)
             });
             mfma_results(acc);
 #pragma unroll
-            for (int a = 0; a < MT; ++a) red[(wave * MT + a) * kWave + lane] = acc[a];
-            __syncthreads();
-            f32x4 s = red[wave * kWave + lane];
+            for (int a0 = 0; a0 < MT; a0 += ST) {
 #pragma unroll
-            for (int pp = 1; pp < NWV; ++pp) s += red[(pp * MT + wave) * kWave + lane];
-            if (valid[i]) {
-                T *gl_ = reinterpret_cast<T *>(tiles + i * 16 * GROW + goff);
-                const float pi = E::to_f32(gl_[0]) + s[0];
-                const float pf = E::to_f32(gl_[HT]) + s[1];
-                const float pg = E::to_f32(gl_[2 * HT]) + s[2];
-                const float po = E::to_f32(gl_[3 * HT]) + s[3];
-                const float c1 = sigmoidf_<false>(pf) * c_state[i] + sigmoidf_<false>(pi) * tanhf_<false>(pg);
-                const float h1 = sigmoidf_<false>(po) * tanhf_<false>(c1);
-                c_state[i] = c1;
-                if (keep) {
-                    gl_[0] = E::from_f32(pi);
-                    gl_[HT] = E::from_f32(pf);
-                    gl_[2 * HT] = E::from_f32(pg);
-                    gl_[3 * HT] = E::from_f32(po);
+                for (int a = 0; a < ST; ++a) red[(wave * ST + a) * kWave + lane] = acc[a0 + a];
+                __syncthreads();
+#pragma unroll
+                for (int h = a0 / NWV; h < (a0 + ST) / NWV; ++h) {   // unit tile wave + 4 h
+                    const int tl = wave + NWV * h - a0;
+                    f32x4 s = red[tl * kWave + lane];
+#pragma unroll
+                    for (int pp = 1; pp < NWV; ++pp) s += red[(pp * ST + tl) * kWave + lane];
+                    if (valid[i]) {
+                        T *gl_ = reinterpret_cast<T *>(tiles + i * 16 * GROW + goff) + h * NWV * 4;
+                        const float pi = E::to_f32(gl_[0]) + s[0];
+                        const float pf = E::to_f32(gl_[HT]) + s[1];
+                        const float pg = E::to_f32(gl_[2 * HT]) + s[2];
+                        const float po = E::to_f32(gl_[3 * HT]) + s[3];
+                        const float c1 = sigmoidf_<false>(pf) * c_state[i][h] + sigmoidf_<false>(pi) * tanhf_<false>(pg);
+                        const float h1 = sigmoidf_<false>(po) * tanhf_<false>(c1);
+                        c_state[i][h] = c1;
+                        if (keep) {
+                            gl_[0] = E::from_f32(pi);
+                            gl_[HT] = E::from_f32(pf);
+                            gl_[2 * HT] = E::from_f32(pg);
+                            gl_[3 * HT] = E::from_f32(po);
+                        }
+                        *(reinterpret_cast<T *>(sth + i * 16 * SROW + soff) + h * NWV * 4) = E::from_f32(h1);
+                        *(reinterpret_cast<T *>(stc + i * 16 * SROW + soff) + h * NWV * 4) = E::from_f32(c1);
+                    }
                 }
-                *reinterpret_cast<T *>(sth + i * 16 * SROW + soff) = E::from_f32(h1);
-                *reinterpret_cast<T *>(stc + i * 16 * SROW + soff) = E::from_f32(c1);
+                __syncthreads();   // `red` is read; behind the last tile: the state tiles are complete
             }
-            __syncthreads();   // `red` is read; behind the last tile: the state tiles are complete
         }
         if (t + 1 < T_) {
             if (st_ok) xch.store16(xn + x_off, *reinterpret_cast<const u32x4 *>(sth + st_lds));

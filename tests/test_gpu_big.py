@@ -1,4 +1,4 @@
-"""The kernels that keep up to 128 MiB of W_h on the chip (16-bit, 2048 < H <= 4096) against the oracle: every number of
+"""The kernels that keep up to 512 KiB of weights per CU (16-bit, 1280 <= H <= 4096) against the oracle: every number of
 k-steps per wave, hidden sizes with padded k-steps and with uneven numbers of teams per XCD, every number of batch tiles, launches
 over row ranges, the first steps."""
 import pytest
@@ -18,6 +18,10 @@ pytestmark = pytest.mark.gpu
     (4, 48, 3136, torch.bfloat16),   # 28
     (5, 64, 3648, torch.float16),    # 32, padded
     (3, 65, 4096, torch.bfloat16),   # two launches, the second of one row
+    (2, 97, 1280, torch.float16),    # 32 units per workgroup: groups of 32 rows, the last one ragged
+    (3, 161, 1536, torch.bfloat16),  # ... a launch over 160 rows and one row
+    (2, 15, 1792, torch.float16),    # ... one group of 16 rows, the weights' sums four tiles at a time
+    (1, 128, 2048, torch.float16),   # ... all CUs
     (3, 33, 2064, torch.float16),    # no multiple of 64: the forward kernel only
 ])
 def test_big_layers_vs_oracle(oracle, T, B, H, dt):
