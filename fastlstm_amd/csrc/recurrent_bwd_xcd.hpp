@@ -291,6 +291,53 @@ __device__ __forceinline__ void bwd_helper(const BwdXcdParams &p, unsigned char 
         }
 }
 
+// Operand blocks of W_h[:, col0 ...]^T for the reverse recurrence (16-bit): for i < N, a < MT, put(i, a, f) with lane (q, r) of f
+// holding row r = unit col0 + 16 a + r and k = 32 ks_of(i) + 8 q + e, e < 8, k = 4 * source unit + gate; zeros from k-step `ks_end`
+// on.  Called by a whole wave with MT KiB of LDS of its own.  A k-step is 32 rows of W_h: they come in with 16 bytes per
+// lane and are transposed on the way out of LDS.  Gathered element by element (8 two-byte loads
+// per block) the 256 KiB of a CU took ~40 us: a reverse launch of 4 steps, B = 64, H = 1024, 72.9 -> 35.3 us; 256 steps 643 -> 582.
+// (Tried in lstm_bwd_big_kernel: the 512 KiB per CU spilled there, H = 2048 and 128 rows 8.9 -> 20 us per step.)
+template <typename T, int MT, int N, typename KStep, typename Put>
+__device__ __forceinline__ void load_wh_transposed(const T *Wh, int H, int col0, unsigned char *buf, int ks_end, KStep ks_of, Put put) {
+    constexpr int G = MT >= 4 ? 1 : 8 / MT;   // k-steps under way together
+    constexpr int PPR = 2 * MT, LD = 16 * PPR;   // 16-byte pieces, bytes per row
+    const int lane = threadIdx.x & 63, q = lane >> 4, r = lane & 15;
+    static_for<0, (N + G - 1) / G>([&](auto bc) __attribute__((always_inline)) {
+        constexpr int i0 = decltype(bc)::value * G;
+        u32x4 v[G][MT];
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                const int p = lane + kWave * m, kk = p / PPR, ks = i0 + g < N ? ks_of(i0 + g) : ks_end;
+                v[g][m] = u32x4{0u, 0u, 0u, 0u};
+                if (ks < ks_end)
+                    v[g][m] = *reinterpret_cast<const u32x4 *>(Wh + ((size_t)(kk & 3) * H + ks * 8 + (kk >> 2)) * H + col0 + (p % PPR) * 8);
+            }
+        static_for<0, G>([&](auto gc) __attribute__((always_inline)) {
+            constexpr int g = decltype(gc)::value;
+            if constexpr (i0 + g < N) {
+#pragma unroll
+                for (int m = 0; m < MT; ++m) *reinterpret_cast<u32x4 *>(buf + (lane + kWave * m) * 16) = v[g][m];
+                asm volatile("" ::: "memory");
+                u32x4 f[MT];
+#pragma unroll
+                for (int a = 0; a < MT; ++a) {
+                    const unsigned char *src = buf + (q * 8 + (r >> 2)) * LD + a * 32 + (r & 3) * 8;
+                    const u32x2 lo = lds_read_tr16<0>(src), hi = lds_read_tr16<4 * LD>(src);
+                    f[a] = u32x4{lo[0], lo[1], hi[0], hi[1]};
+                }
+#pragma unroll
+                for (int a = 0; a < MT; ++a) lds_reads_landed_but<0>(f[a]);
+                static_for<0, MT>([&](auto ac) __attribute__((always_inline)) {
+                    put(std::integral_constant<int, i0 + g>{}, ac, f[decltype(ac)::value]);
+                });
+                asm volatile("" ::: "memory");
+            }
+        });
+    });
+}
+
 // HELP: 0 = recurrence only; 1 = the workgroups without a role compute dx and the weight gradients;
 // 2 = the same for two stacked layers that share the launch.
 template <typename T, int MT, int NKW, int NTW, int NWV, int HELP = 0>
@@ -369,26 +416,32 @@ __global__ __launch_bounds__(kWave * NWV) void lstm_bwd_xcd_kernel(const BwdXcdP
 #pragma unroll
         for (int m = 0; m < IPT; ++m) db_slots[m * NTHR] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    // ---- prologue: this wave's fragments of Wh[:, units]^T, gathered from global memory ----
+    // ---- prologue: this wave's fragments of Wh[:, units]^T (fp32: gathered from global memory) ----
     // fragment (unit tile a, k-step ks): lane (q, r) holds row r = unit u0 + 16a + r and
     // k = ks*KSTEP + q*EPL + e, e < EPL, with k = 4 * source unit + gate
     u32x4 wreg[MT][NKW];
+    if constexpr (E::BYTES == 2) {
+        load_wh_transposed<T, MT, NKW>(Wh, H, u0, reinterpret_cast<unsigned char *>(red) + wave * MT * kFragBytes, KSB,
+                                       [&](int ki) { return wave + NWV * ki; },
+                                       [&](auto ki, auto a, u32x4 f) { wreg[decltype(a)::value][decltype(ki)::value] = f; });
+    } else {
 #pragma unroll
-    for (int a = 0; a < MT; ++a)
+        for (int a = 0; a < MT; ++a)
 #pragma unroll
-        for (int ki = 0; ki < NKW; ++ki) {
-            const int ks = wave + NWV * ki;
-            T tmp[E::EPL];
+            for (int ki = 0; ki < NKW; ++ki) {
+                const int ks = wave + NWV * ki;
+                T tmp[E::EPL];
 #pragma unroll
-            for (int e = 0; e < E::EPL; ++e) {
-                const int k = ks * E::KSTEP + q * E::EPL + e;
-                const int uk = k >> 2, gate = k & 3;
-                const bool ok = ks < KSB && uk < H;
-                const T v = Wh[ok ? ((size_t)gate * H + uk) * H + u0 + a * 16 + r : 0];
-                tmp[e] = ok ? v : E::from_f32(0.f);
+                for (int e = 0; e < E::EPL; ++e) {
+                    const int k = ks * E::KSTEP + q * E::EPL + e;
+                    const int uk = k >> 2, gate = k & 3;
+                    const bool ok = ks < KSB && uk < H;
+                    const T v = Wh[ok ? ((size_t)gate * H + uk) * H + u0 + a * 16 + r : 0];
+                    tmp[e] = ok ? v : E::from_f32(0.f);
+                }
+                wreg[a][ki] = *reinterpret_cast<u32x4 *>(tmp);
             }
-            wreg[a][ki] = *reinterpret_cast<u32x4 *>(tmp);
-        }
+    }
 
     // ---- per-thread items: it = tid + NTHR*m -> (row n, unit ul, n-tile nt) ----------------
     float dc_state[IPT], dh_rec[IPT], c1v[IPT];
