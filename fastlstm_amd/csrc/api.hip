@@ -9,7 +9,6 @@
 #include "recurrent_fwd.hpp"
 #include "recurrent_bwd_xcd.hpp"
 #include "recurrent_bwd_wide.hpp"
-#include "recurrent_bwd_wide.hpp"
 #include "recurrent_fwd_xcd.hpp"
 #include "recurrent_step.hpp"
 #include "recurrent_bwd_big.hpp"
@@ -562,7 +561,13 @@ bool select_wide(int T, int B_all, int H, int dtype, bool backward, size_t ws_by
     if ((H * es) % 512 || H * es <= 2048 || H * es > 4096) return false;
     c->ks = (backward ? 4 * H : H) / kstep;
     c->big = 0;
-    if (es == 2 && copies == 1 && (g_families.load() & 4)) {
+    // Two recurrences side by side: the reverse kernel of a call by itself for a pair too (other kernels take the sums in another
+    // order: dh_0 and dc_0 of the two ways would differ in their last bits), where the forward pass of the pair is one launch
+    // (below: groups of at most 32 rows of the 16-unit form) -- a caller finds a pair fused in both directions or in neither.
+    // Such a forward pass is on the 16-unit form by itself as well: two groups of 32 rows for each of the pair leave room for
+    // 16-row groups of one.
+    const bool both = copies == 2 && backward && 2 * cdiv(B, 32) * cdiv(H / 16, 32) <= kNumXcd;
+    if (es == 2 && (copies == 1 || both) && (g_families.load() & 4)) {
         // 32 units per workgroup: groups of H / 32 workgroups, more of them, so fewer rows and operand bytes per CU.  The reverse
         // pass gains at every batch size (us per step, 16 units / 32: H = 2048, B = 32 6.4 / 5.3, 64 9.0 / 6.2, 128
         // 11.0 / 8.6; H = 1280, B = 128 8.7 / 7.0): groups of 16 rows where the batch fits the launch that way, else of 32.
@@ -570,11 +575,11 @@ bool select_wide(int T, int B_all, int H, int dtype, bool backward, size_t ws_by
         // 3.99 / 3.31); with 32 rows there is no difference (H = 2048, B = 128 7.1 / 7.3), and where 16-row groups of
         // 16-unit workgroups fit, their half as many products per CU count for more (H = 2048, B = 32 3.4 / 3.8).
         const int n_ht = H / 32, max_groups = kNumXcd * 32 / n_ht;
-        const int nt = cdiv(B, 16) <= max_groups ? 1 : 2, groups = cdiv(B, 16 * nt);
+        const int nt = copies * cdiv(B, 16) <= max_groups ? 1 : 2, groups = cdiv(B, 16 * nt);
         const bool faster = backward || (nt == 1 && cdiv(B, 16) * cdiv(H / 16, 32) > kNumXcd);
         const size_t xslot = (size_t)groups * nt * c->ks * kFragBytes;
         const size_t partials = backward ? (size_t)groups * n_ht * kBigTeam * 2 * nt * kFragBytes : 0;
-        if (faster && groups <= max_groups && ws_bytes >= kWsHeaderBytes + kWsCounterBytes + 2 * xslot + partials) {
+        if (faster && copies * groups <= max_groups && ws_bytes >= kWsHeaderBytes + kWsCounterBytes + copies * (2 * xslot + partials)) {
             c->big = nt;
             c->n_ht = n_ht;
             c->n_groups = groups;
@@ -690,7 +695,12 @@ int try_bwd_wide(const void *dout, void *dh, void *dc, const void *ifgo, const v
         q.flag_stride = kXcdGroupStride;
         q.team_flags = q.flags + kNumXcd * kXcdGroupStride;
         q.xbuf = wsb + kWsHeaderBytes + kWsCounterBytes;
-        q.partials = q.xbuf + 2 * c.xslot;
+        q.partials = q.xbuf + 2 * copies * c.xslot;
+        q.n_rec = copies;
+        if (second) {
+            q.dout2 = second[0]; q.dh2 = second[1]; q.dc2 = second[2]; q.ifgo2 = second[3]; q.cell2 = second[4];
+            q.d_ifgo2 = second[5]; q.Wh2 = second[6];
+        }
         q.T = T; q.B = B; q.H = H;
         q.b_base = o.row0; q.n_bt = c.n_groups; q.n_ht = c.n_ht;
         q.KSB = q.KSBP = c.ks;
@@ -698,7 +708,7 @@ int try_bwd_wide(const void *dout, void *dh, void *dc, const void *ifgo, const v
         int occ = 0;
         if (launch_bwd_big(dtype, q, H / 128, 8, c.big, 0, nullptr, &occ) != hipSuccess) return FASTLSTM_ERR_HIP;
         if (occ < 1) return 1;
-        const int grid = kNumXcd * cdiv(c.n_groups * c.n_ht / kBigTeam, kNumXcd) * kBigTeam;
+        const int grid = kNumXcd * cdiv(copies * c.n_groups * c.n_ht / kBigTeam, kNumXcd) * kBigTeam;
         if (!dry_run && launch_bwd_big(dtype, q, H / 128, 8, c.big, grid, stream, nullptr) != hipSuccess) return FASTLSTM_ERR_HIP;
         return FASTLSTM_OK;
     }
@@ -1390,6 +1400,7 @@ static int bwd_persistent_impl(const void *dout, void *dh, void *dc, const void 
                         grid_big <= kNumXcd * 32;
         if (resident) {
             p.Wh = Wh;
+            p.n_rec = 1;
             p.team_flags = reinterpret_cast<int *>(wsb + kWsHeaderBytes);
             p.partials = wsb + l.wpack_off;
             int occ = 0;

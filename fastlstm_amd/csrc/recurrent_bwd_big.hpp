@@ -17,6 +17,9 @@
 // lstm_bwd_stream_kernel and here: H = 4096, 64 rows 33.6 -> 12.8, 16 rows 21.1 -> 6.7; H = 3072, 32 rows 16.8 -> 7.2;
 // H = 2560, 64 rows 22.6 -> 9.5.  Of the form with 16 units and 8 waves per CU for H <= 2048 and here: H = 2048, 128 rows 11.0 -> 8.6,
 // 64 rows 9.0 -> 6.2, 32 rows 6.4 -> 5.3; H = 1280, 128 rows 8.7 -> 7.0.
+// Up to H = 2048 a second recurrence of the same shape may share the launch (the directions of a bidirectional layer, the chunks of
+// a wavefront): the sums are those of a launch of its own, bit by bit.  us per step of a pair on lstm_bwd_wide_kernel and here:
+// H = 2048, B = 16 6.8 -> 5.2, B = 32 9.8 -> 6.5; H = 1536, B = 32 7.7 -> 5.6; H = 1280, B = 20 6.6 -> 5.9.
 // Requirements (host): H a multiple of 16 MT, workgroup ids dealt to the XCDs in turn, all teams co-resident.
 #pragma once
 #include <type_traits>
@@ -51,17 +54,19 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
     const int KSB = p.KSB, H = p.H, B = p.B, T_ = p.T;
 
     // ---- placement: whole teams on one XCD (hardware deals workgroup i to XCD i % 8), teams spread evenly ------
-    const int tpg = p.n_ht / V, teams = p.n_bt * tpg, tpx = (teams + kNumXcd - 1) / kNumXcd;
+    const int n_groups = p.n_rec * p.n_bt;   // (the groups of the second recurrence behind those of the first)
+    const int tpg = p.n_ht / V, teams = n_groups * tpg, tpx = (teams + kNumXcd - 1) / kNumXcd;
     const int slot = blockIdx.x / kNumXcd, id = (int)(blockIdx.x % kNumXcd) * tpx + slot / V;
     if (slot / V >= tpx || id >= teams) return;
     check_xcd_placement(p.hdr);
     const int g = id / tpg, team = id % tpg, mem = slot % V, j = team * V + mem;
-    const int u0 = j * HT, b0 = p.b_base + g * BT;
-    const T *dout = static_cast<const T *>(p.dout);
-    const T *ifgo = static_cast<const T *>(p.ifgo);
-    const T *cell = static_cast<const T *>(p.cell);
-    T *d_ifgo = static_cast<T *>(p.d_ifgo);
-    const T *Wh = static_cast<const T *>(p.Wh);
+    const bool second = g >= p.n_bt;
+    const int u0 = j * HT, b0 = p.b_base + (second ? g - p.n_bt : g) * BT;
+    const T *dout = static_cast<const T *>(second ? p.dout2 : p.dout);
+    const T *ifgo = static_cast<const T *>(second ? p.ifgo2 : p.ifgo);
+    const T *cell = static_cast<const T *>(second ? p.cell2 : p.cell);
+    T *d_ifgo = static_cast<T *>(second ? p.d_ifgo2 : p.d_ifgo);
+    const T *Wh = static_cast<const T *>(second ? p.Wh2 : p.Wh);
 
     // ---- Wh[k-part, team units]^T, gathered: fragment (unit tile v, k-step ks = (mem KW + ki) 4 + wave): lane (q, n) holds
     // row n = unit team*16*MT + 16 v + n and k = ks*KSTEP + q*EPL + e, e < EPL, with k = 4 * source unit + gate
@@ -106,12 +111,12 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
         return *reinterpret_cast<u32x2 *>(o);
     };
     if (valid) {
-        dh_rec = halves(*reinterpret_cast<const u32x2 *>(static_cast<const T *>(p.dh) + off_h));
-        dc_state = halves(*reinterpret_cast<const u32x2 *>(static_cast<const T *>(p.dc) + off_h));
+        dh_rec = halves(*reinterpret_cast<const u32x2 *>(static_cast<const T *>(second ? p.dh2 : p.dh) + off_h));
+        dc_state = halves(*reinterpret_cast<const u32x2 *>(static_cast<const T *>(second ? p.dc2 : p.dc) + off_h));
         c1v = *reinterpret_cast<const u32x2 *>(cell + (size_t)T_ * BH + off_h);
     }
     const int goff = (ci * 16 + n) * GROW + (16 * ut + 4 * q) * E::BYTES, soff = (ci * 16 + n) * SROW + (16 * ut + 4 * q) * E::BYTES;
-    const unsigned xslot = (unsigned)p.n_bt * NT * p.KSBP * kFragBytes, xgrp = (unsigned)g * NT * p.KSBP * kFragBytes;
+    const unsigned xslot = (unsigned)n_groups * NT * p.KSBP * kFragBytes, xgrp = (unsigned)g * NT * p.KSBP * kFragBytes;
     const XchgGlobal xch(p.xbuf, 2u * xslot);
     const unsigned x_off = mine ? xgrp + (unsigned)(ci * p.KSBP * kFragBytes + frag_offset<T>(n, (u0 + 16 * ut + 4 * q) * 4)) : 0u;
     int *grp_flags = p.flags + (size_t)g * p.flag_stride, *team_flags = p.team_flags + (size_t)g * p.flag_stride + team * V;
@@ -119,7 +124,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
     // partial sums in the workspace: [receiver][sender][UT][NT][64] f32x4, one set (a sender passes the next step's group
     // barrier only after the receiver published that step, i.e. after it read this one)
     constexpr unsigned kSetBytes = UT * NT * kFragBytes;
-    const XchgGlobal part(p.partials, (unsigned)(p.n_bt * p.n_ht) * V * kSetBytes);
+    const XchgGlobal part(p.partials, (unsigned)(n_groups * p.n_ht) * V * kSetBytes);
     const unsigned part_team = (unsigned)(g * p.n_ht + team * V) * V * kSetBytes;
     auto part_to = [&](int v, int i) {   // unit tile v of the team is tile v % UT of member v / UT
         return part_team + (unsigned)((v / UT) * V + mem) * kSetBytes + (unsigned)((v % UT) * NT + i) * kFragBytes;
@@ -299,8 +304,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
         }
     }
     if (valid) {
-        *reinterpret_cast<u32x2 *>(static_cast<T *>(p.dh) + off_h) = packed(dh_rec);
-        *reinterpret_cast<u32x2 *>(static_cast<T *>(p.dc) + off_h) = packed(dc_state);
+        *reinterpret_cast<u32x2 *>(static_cast<T *>(second ? p.dh2 : p.dh) + off_h) = packed(dh_rec);
+        *reinterpret_cast<u32x2 *>(static_cast<T *>(second ? p.dc2 : p.dc) + off_h) = packed(dc_state);
     }
 }
 

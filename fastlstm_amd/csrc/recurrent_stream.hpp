@@ -53,8 +53,11 @@ struct BwdStreamParams {
     const unsigned char *wpack;   // [n_ht][MTB][KSBP] operand blocks of Wh[:, units]^T, K = (unit', gate)
     // lstm_bwd_big_kernel:
     const void *Wh;    // [4H,H]
-    int *team_flags;   // [n_ht]
-    unsigned char *partials;   // [n_ht receivers][4 senders][NT] blocks of fp32 sums
+    int *team_flags;   // [n_rec n_bt][flag_stride]
+    unsigned char *partials;   // [n_rec n_bt][n_ht receivers][4 senders][unit tiles][NT] blocks of fp32 sums
+    int n_rec;         // 2: a second, independent recurrence of this shape side by side, its operands here
+    const void *dout2, *ifgo2, *cell2, *Wh2;
+    void *dh2, *dc2, *d_ifgo2;
     WsHeader *hdr;
     int *flags;
     unsigned char *xbuf;   // [2 slots][n_bt][NT][KSBP]

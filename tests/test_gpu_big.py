@@ -6,7 +6,7 @@ import torch
 
 import fastlstm_amd.lstm as L
 from test_gpu_parity import FWD_KEYS, HALF_TOL, RM, dev, make_problem, npy, to_np, within
-from fastlstm_amd import FastLSTM
+from fastlstm_amd import FastLSTM, _lib
 
 pytestmark = pytest.mark.gpu
 
@@ -57,3 +57,47 @@ def test_module_pads_to_a_multiple_of_64(oracle):
     pr["h0"] = pr["c0"] = zeros
     want, _, _ = oracle.forward(*to_np(pr, FWD_KEYS), round_mode=RM[torch.float16])
     within(out, want[1:], HALF_TOL, "out")
+
+
+@pytest.mark.parametrize("T,B,H,dt,whole", [
+    (1, 20, 1280, torch.float16, True),      # two ragged groups of 16 rows each, 20 teams on the XCDs unevenly
+    (3, 32, 1792, torch.bfloat16, True),     # ... full groups
+    (4, 17, 2048, torch.float16, True),      # all CUs
+    (2, 9, 1536, torch.bfloat16, True),      # one partly filled group each
+    (3, 32, 2048, torch.bfloat16, False),    # no room for the teams' partial sums: the 16-unit form, alone and as a pair
+])
+def test_pair_of_reverse_recurrences_equals_two_calls(T, B, H, dt, whole):
+    """fastlstm_bwd_persistent_pair on the whole-CU kernel: d_ifgo and the state gradients of both recurrences are the bits of
+    two calls of their own (the same kernel adds in the same order, whichever workgroup a group is on)."""
+    lib, code = _lib.load(), RM[dt]
+    st = torch.cuda.current_stream().cuda_stream
+    plan = _lib.Plan()
+    _lib.check(lib.fastlstm_plan_device(0, B, H, code, 1, plan), "plan")
+    gen = torch.Generator(device="cuda").manual_seed(T * H + B)
+    rnd = lambda *shape, s=1.0: (torch.randn(*shape, device="cuda", generator=gen) * s).to(dt)
+    sides = [dict(dout=rnd(T, B, H), dh=rnd(B, H), dc=rnd(B, H), ifgo=rnd(T, B, 4 * H), cell=rnd(T + 1, B, H, s=0.5), Wh=rnd(4 * H, H, s=H ** -0.5))
+             for _ in range(2)]
+    one, two = (lib.fastlstm_recurrent_workspace_bytes(plan, T, H, code, 1), lib.fastlstm_stack2_bwd_workspace_bytes(plan, T, H, code))
+    if not whole:
+        one, two = plan.ws_bytes, 2 * plan.ws_bytes
+    assert lib.fastlstm_pair_fused(T, B, H, code, 1, two) == 1
+
+    def operands(o, d_ifgo):
+        return [o[k].data_ptr() for k in ("dout", "dh", "dc", "ifgo", "cell")] + [d_ifgo.data_ptr(), o["Wh"].data_ptr()]
+
+    def fresh():
+        return [dict(o, dh=o["dh"].clone(), dc=o["dc"].clone()) for o in sides], [torch.empty(T, B, 4 * H, device="cuda", dtype=dt) for _ in sides]
+
+    got, d_got = fresh()
+    ws = torch.zeros(two, dtype=torch.uint8, device="cuda")
+    _lib.check(lib.fastlstm_bwd_persistent_pair(*operands(got[0], d_got[0]), *operands(got[1], d_got[1]), ws.data_ptr(), two, T, B, H, code, st), "pair")
+    torch.cuda.synchronize()
+    assert lib.fastlstm_ws_status(ws[:64].cpu().numpy().tobytes()) == _lib.OK
+    want, d_want = fresh()
+    for o, d in zip(want, d_want):
+        ws = torch.zeros(one, dtype=torch.uint8, device="cuda")
+        _lib.check(lib.fastlstm_bwd_persistent(*operands(o, d), ws.data_ptr(), one, T, B, H, code, st), "single")
+    torch.cuda.synchronize()
+    for g, w, dg, dw in zip(got, want, d_got, d_want):
+        assert torch.equal(dg, dw) and torch.equal(g["dh"], w["dh"]) and torch.equal(g["dc"], w["dc"])
+        assert torch.isfinite(dg.float()).all()
