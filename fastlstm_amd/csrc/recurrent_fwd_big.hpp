@@ -57,11 +57,16 @@ __device__ __forceinline__ void mfma_resident(f32x4 &acc, const u32x4 &a, const 
     }
 #undef FASTLSTM_MFMA
 }
-// The wait states between these MFMAs and the first other reader of their results (8 passes: at most 11 + 8).
+// The wait states between these MFMAs and the first other reader of their results (4 passes: 8 of them).  The results go through
+// the statement, so that no reader moves in front of it; that no copy of them does either -- the compiler does not see MFMAs
+// here, and would not wait -- is checked in the machine code (tests/test_mfma_wait_states.py).
 template <int N> __device__ __forceinline__ void mfma_results(f32x4 (&acc)[N]) {
-    asm volatile("s_nop 15\n\ts_nop 7");
-#pragma unroll
-    for (int a = 0; a < N; a += 4) asm volatile("" : "+v"(acc[a]), "+v"(acc[a + 1]), "+v"(acc[a + 2]), "+v"(acc[a + 3]));
+    static_assert(N == 4 || N == 8, "unit tiles of the whole-CU kernels");
+    if constexpr (N == 4)
+        asm volatile("s_nop 15\n\ts_nop 7" : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]));
+    else
+        asm volatile("s_nop 15\n\ts_nop 7"
+                     : "+v"(acc[0]), "+v"(acc[1]), "+v"(acc[2]), "+v"(acc[3]), "+v"(acc[4]), "+v"(acc[5]), "+v"(acc[6]), "+v"(acc[7]));
 }
 
 template <typename T, int KW, int MT, int NT>
