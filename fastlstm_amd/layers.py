@@ -41,18 +41,27 @@ class _Copies:
         self.n += 1
         self.fields += (src or 0, src2, dst, mode, mode2, dmode, 0, 0, 0, 1, cols[0], cols[1], ld, ld2, dld, types)
 
-    def run(self, call):
+    def run(self, at):
         if self.n:
             _lib.check(_lib.load().fastlstm_copy_blocks(
-                self.n, (ctypes.c_longlong * len(self.fields))(*self.fields), call.T, call.B, call.lens, call.offs, call.order,
-                call.stream), "fastlstm_copy_blocks")
+                self.n, (ctypes.c_longlong * len(self.fields))(*self.fields), at.T, at.B, at.lens, at.offs, at.order, at.stream),
+                "fastlstm_copy_blocks")
+
+
+class _Pass:
+    """What the copy launches of one pass (forward, or one of several backward passes) take besides their descriptors."""
+    __slots__ = ("T", "B", "lens", "offs", "order", "stream")
+
+    def __init__(self, c, order, stream):
+        self.T, self.B, self.lens, self.offs, self.stream = c.T, c.B, c.lens, c.offs, stream
+        self.order = None if order is None else order.data_ptr()
 
 
 class _Call:
-    """Sizes and options of one call; what the node keeps of it."""
-    __slots__ = ("T", "B", "I", "H", "Hp", "Ip", "L", "D", "dt", "code", "es", "device", "packed", "N", "lens", "offs", "order",
-                 "index_memory", "stream", "copy_weights", "copy_x", "bias", "x_dtype", "held", "states", "inputs", "acts",
-                 "weights", "groups")
+    """Sizes and options of one call.  Written by plan() and forward() alone: the graph's node keeps it, and several threads may
+    run backward over one graph."""
+    __slots__ = ("T", "B", "I", "H", "Hp", "Ip", "L", "D", "dt", "code", "es", "device", "packed", "N", "lens", "offs",
+                 "index_memory", "copy_weights", "copy_x", "bias", "x_dtype", "held", "states", "groups")
 
     def view(self, base, offset, shape):
         strides, n = [], 1
@@ -114,11 +123,11 @@ def plan(module, x, h_c_0):
         return None   # a batch of several launches, each range of rows to its own length
     c.es = 4 if c.dt == torch.float32 else 2
     c.device, c.x_dtype = data.device, data.dtype
-    c.lens = c.offs = c.order = c.index_memory = None
+    c.lens = c.offs = c.index_memory = None
     return c
 
 
-def _upload_lengths(c, x):
+def _upload_lengths(c, x, stream):
     """Row lengths and first packed rows on the device, through the arguments of a launch."""
     sizes = x.batch_sizes.numpy()
     ints = np.empty(c.B + c.T, dtype=np.int32)
@@ -126,11 +135,8 @@ def _upload_lengths(c, x):
     ints[c.B] = 0
     np.cumsum(sizes[:-1], out=ints[c.B + 1:])
     dev = torch.empty(c.B + c.T, dtype=torch.int32, device=c.device)
-    _lib.check(_lib.load().fastlstm_upload_ints(ints.ctypes.data, ints.size, dev.data_ptr(), c.stream), "fastlstm_upload_ints")
-    c.lens, c.offs = dev.data_ptr(), dev.data_ptr() + 4 * c.B
-    order = x.sorted_indices
-    c.order = order.data_ptr() if order is not None else None
-    c.index_memory = (dev, order)
+    _lib.check(_lib.load().fastlstm_upload_ints(ints.ctypes.data, ints.size, dev.data_ptr(), stream), "fastlstm_upload_ints")
+    c.lens, c.offs, c.index_memory = dev.data_ptr(), dev.data_ptr() + 4 * c.B, dev
 
 
 def _weights(c, copies, params):
@@ -168,18 +174,18 @@ def _weights(c, copies, params):
     return out
 
 
-def _states(c, copies, h_0, c_0):
+def _states(c, copies, h_0, c_0, order):
     """Per layer and direction (h0 [B,Hp], c0) in the compute type and the kernels' row order, or (None, None)."""
     n = c.L * c.D
     if h_0 is None:
         return [(None, None)] * n
     h_0, c_0 = h_0.contiguous(), c_0.contiguous()
-    if c.Hp == c.H and c.order is None and c.states == (c.dt, c.dt):
+    if c.Hp == c.H and order is None and c.states == (c.dt, c.dt):
         return [(h_0[k], c_0[k]) for k in range(n)]
     buf = torch.empty((2, n, c.B, c.Hp), dtype=c.dt, device=c.device)
     for i, s in enumerate((h_0, c_0)):
         types, src, dst = L._DTYPE_CODE[s.dtype] + 16 * c.code, s.data_ptr(), buf.data_ptr() + i * n * c.B * c.Hp * c.es
-        if c.order is None:
+        if order is None:
             copies.matrix(src, dst, 1, (n * c.B, n * c.B), (c.H, c.Hp), types)
         else:
             for k in range(n):
@@ -188,17 +194,19 @@ def _states(c, copies, h_0, c_0):
 
 
 def forward(c, x, h_0, c_0, params, keep):
-    """(out, h_n, c_n) of the call; with `keep` what the reverse pass reads is left in c."""
-    data = x.data if c.packed else x
-    c.stream = L._stream()
+    """(out, h_n, c_n) of the call and, per layer and direction, what the reverse pass reads (with `keep`): the inputs, the
+    (out, cell, ifgo), the weights."""
+    data, order = (x.data, x.sorted_indices) if c.packed else (x, None)
+    stream = L._stream()
     if c.packed:
-        _upload_lengths(c, x)
+        _upload_lengths(c, x, stream)
         keep = True   # (a row's last cell state is read out of the history)
+    here = _Pass(c, order, stream)
     T, B, H, Hp, D, es = c.T, c.B, c.H, c.Hp, c.D, c.es
     dev, new = c.device, lambda *shape: torch.empty(shape, dtype=c.dt, device=c.device)
     copies = _Copies()
-    c.weights = _weights(c, copies, params)
-    states = _states(c, copies, h_0, c_0)
+    weights = _weights(c, copies, params)
+    states = _states(c, copies, h_0, c_0, order)
     data = data.contiguous()
     types = L._DTYPE_CODE[c.x_dtype] + 16 * c.code
     cur, cur_r = data, None
@@ -211,11 +219,11 @@ def forward(c, x, h_0, c_0, params, keep):
     if D == 2:
         cur_r = new(T, B, c.Ip)
         copies.rows(data.data_ptr(), PACKED_REVERSED if c.packed else REVERSED, c.I, cur_r.data_ptr(), PADDED, c.Ip, (c.I, c.Ip), types)
-    copies.run(c)
+    copies.run(here)
 
     kw = {} if keep else {"keep_activations": False}
-    c.inputs, c.acts, c.groups = [], [], []    # per layer and direction; groups: (first layer, layers) of a host call
-    operands = [states[k] + tuple(c.weights[k]) for k in range(c.L * D)]
+    inputs, kept, c.groups = [], [], []    # groups: (first layer, layers) of a host call
+    operands = [states[k] + tuple(weights[k]) for k in range(c.L * D)]
     row, own = B * Hp * es, c.code + 16 * c.code
     layer = 0
     while layer < c.L:
@@ -232,8 +240,8 @@ def forward(c, x, h_0, c_0, params, keep):
             else:
                 width, acts = 1, [L.lstm_persistent_fwd(cur, *operands[layer], **kw)]
             for a in acts:
-                c.inputs.append(cur)
-                c.acts.append(a)
+                inputs.append(cur)
+                kept.append(a)
                 cur = a[0][1:]
             c.groups.append((layer, width))
             layer += width
@@ -244,8 +252,8 @@ def forward(c, x, h_0, c_0, params, keep):
             acts = [r[:3], r[3:]]
         else:
             acts = [L.lstm_persistent_fwd(cur, *a, **kw), L.lstm_persistent_fwd(cur_r, *b, **kw)]
-        c.inputs += [cur, cur_r]
-        c.acts += acts
+        inputs += [cur, cur_r]
+        kept += acts
         c.groups.append((layer, 1))
         layer += 1
         if layer < c.L:   # both directions' h side by side, in time order and reversed
@@ -255,7 +263,7 @@ def forward(c, x, h_0, c_0, params, keep):
             for dst, ma, mb in ((cur.data_ptr(), PADDED, REVERSED), (cur_r.data_ptr(), REVERSED, PADDED)):
                 copies.rows(pa, ma, Hp, dst, PADDED, 2 * Hp, (Hp, Hp), own)
                 copies.rows(pb, mb, Hp, dst + Hp * es, PADDED, 2 * Hp, (Hp, Hp), own)
-            copies.run(c)
+            copies.run(here)
 
     copies = _Copies()
     out_mode = PACKED if c.packed else PADDED
@@ -264,24 +272,25 @@ def forward(c, x, h_0, c_0, params, keep):
     else:
         out = new(c.N, D * H) if c.packed else new(T, B, D * H)
         for d in range(D):
-            copies.rows(c.acts[-D + d][0].data_ptr() + row, REVERSED if d else PADDED, Hp, out.data_ptr() + d * H * es, out_mode, D * H,
+            copies.rows(kept[-D + d][0].data_ptr() + row, REVERSED if d else PADDED, Hp, out.data_ptr() + d * H * es, out_mode, D * H,
                         (H, H), own)
     h_n, c_n = new(c.L * D, B, H), new(c.L * D, B, H)
-    for k, a in enumerate(c.acts):
+    for k, a in enumerate(kept):
         for src, dst in ((a[0], h_n), (a[1], c_n)):
             to = dst.data_ptr() + k * B * H * es
             if c.packed:
                 copies.rows(src.data_ptr() + row, LAST, Hp, to, ORDERED, H, (H, H), own)
             else:
                 copies.matrix(src.data_ptr() + T * row, to, 1, (B, B), (Hp, H), own)
-    copies.run(c)
-    return out, h_n, c_n
+    copies.run(here)
+    return (out, h_n, c_n), (inputs, kept, weights)
 
 
-def backward(c, dout, dh_n, need_x, need_states, need_w):
+def backward(c, kept, order, dout, dh_n, need_x, need_states, need_w):
     """Gradients of (x, h_0, c_0, params) for the gradient of out (and, packed input, of h_n; either may be None)."""
     T, B, H, Hp, D, es = c.T, c.B, c.H, c.Hp, c.D, c.es
-    c.stream = L._stream()
+    inputs, acts_of, weights_of = kept
+    here = _Pass(c, order, L._stream())
     new = lambda *shape, dtype=c.dt: torch.empty(shape, dtype=dtype, device=c.device)
     own, row = c.code + 16 * c.code, B * Hp * es
     copies = _Copies()
@@ -295,7 +304,7 @@ def backward(c, dout, dh_n, need_x, need_states, need_w):
             mode = (PACKED_REVERSED if d else PACKED) if c.packed else (REVERSED if d else PADDED)
             ptr, types = (0, own) if dout is None else (dout.data_ptr() + d * H * dout.element_size(), L._DTYPE_CODE[dout.dtype] + 16 * c.code)
             copies.rows(ptr, mode, D * H, dh[d].data_ptr(), PADDED, Hp, (H, Hp), types)
-    copies.run(c)
+    copies.run(here)
 
     def add_state_gradient(layer):   # packed input: h_n is out at each row's last step
         if dh_n is None:
@@ -306,7 +315,7 @@ def backward(c, dout, dh_n, need_x, need_states, need_w):
         for d in range(D):
             more.rows(g.data_ptr() + (layer * D + d) * B * H * es, ORDERED, H, dh[d].data_ptr(), LAST, Hp, (H, H), own,
                       src2=dh[d].data_ptr(), mode2=LAST, ld2=Hp)
-        more.run(c)
+        more.run(here)
 
     n = c.L * D
     dh0, dc0, dw = [None] * n, [None] * n, [None] * n
@@ -317,9 +326,9 @@ def backward(c, dout, dh_n, need_x, need_states, need_w):
         need_dx = need_x or layer > 0
         k = layer * D
         if D == 1:
-            x = c.inputs[layer]
+            x = inputs[layer]
             add_state_gradient(layer)
-            acts, weights = c.acts[layer:layer + width], [(w[0], w[2]) for w in c.weights[layer:layer + width]]
+            acts, weights = acts_of[layer:layer + width], [(w[0], w[2]) for w in weights_of[layer:layer + width]]
             if width >= 3:
                 res = L.lstm_persistent_bwd_stack(dh[0], x, acts, weights, None, need_dx)
             elif width == 2:
@@ -329,7 +338,7 @@ def backward(c, dout, dh_n, need_x, need_states, need_w):
             dh = [res[0][0]]
         else:
             add_state_gradient(layer)
-            a, b = (c.inputs[k], *c.acts[k], c.weights[k][0], c.weights[k][2]), (c.inputs[k + 1], *c.acts[k + 1], c.weights[k + 1][0], c.weights[k + 1][2])
+            a, b = (inputs[k], *acts_of[k], weights_of[k][0], weights_of[k][2]), (inputs[k + 1], *acts_of[k + 1], weights_of[k + 1][0], weights_of[k + 1][2])
             if L.pair_runs_in_one_launch(T, B, Hp, c.dt, c.device, backward=True):
                 res = L.lstm_persistent_bwd_pair(dh[0], None, *a, dh[1], None, *b, need_dx=(need_dx, need_dx))
             else:
@@ -341,7 +350,7 @@ def backward(c, dout, dh_n, need_x, need_states, need_w):
                 copies = _Copies()
                 copies.rows(pa, PADDED, 2 * Hp, dh[0].data_ptr(), PADDED, Hp, (Hp, Hp), own, pb, REVERSED, 2 * Hp)
                 copies.rows(pa + Hp * es, REVERSED, 2 * Hp, dh[1].data_ptr(), PADDED, Hp, (Hp, Hp), own, pb + Hp * es, PADDED, 2 * Hp)
-                copies.run(c)
+                copies.run(here)
             else:
                 dh = dx
         for i, r in enumerate(res):
@@ -387,7 +396,7 @@ def backward(c, dout, dh_n, need_x, need_states, need_w):
                 d_params += (gx, gbx, gh, gbh)
             else:
                 d_params += (gx, gh)
-    copies.run(c)
+    copies.run(here)
     return d_x, d_states[0], d_states[1], d_params
 
 
@@ -398,15 +407,15 @@ class Layersfn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, c, packed, data, h_0, c_0, *params):
         with torch.cuda.device(data.device):
-            out, h_n, c_n = forward(c, packed if c.packed else data, h_0, c_0, params, True)
-        ctx.call, ctx.count = c, (len(c.inputs), len(c.acts))
-        flat = list(c.inputs)
-        for a in c.acts:
+            (out, h_n, c_n), (inputs, acts, weights) = forward(c, packed if c.packed else data, h_0, c_0, params, True)
+        ctx.call, ctx.count = c, (len(inputs), len(acts))
+        flat = list(inputs)
+        for a in acts:
             flat += a
-        for w in c.weights:
+        for w in weights:
             flat += (w[0], w[2])
         ctx.save_for_backward(*flat)
-        c.inputs = c.acts = c.weights = None
+        ctx.order = packed.sorted_indices if c.packed else None
         ctx.set_materialize_grads(False)
         ctx.mark_non_differentiable(*((c_n,) if c.packed else (h_n, c_n)))
         return out, h_n, c_n
@@ -419,13 +428,11 @@ class Layersfn(torch.autograd.Function):
         L._raise_pending_before_backward(dout if dout is not None else dh_n)   # a failed forward launch is reported before its gradients are computed
         t = ctx.saved_tensors
         ni, na = ctx.count
-        c.inputs = list(t[:ni])
-        c.acts = [tuple(t[ni + 3 * k:ni + 3 * k + 3]) for k in range(na)]
+        acts = [tuple(t[ni + 3 * k:ni + 3 * k + 3]) for k in range(na)]
         w = t[ni + 3 * na:]
-        c.weights = [(w[2 * k], None, w[2 * k + 1], None) for k in range(na)]
+        kept = t[:ni], acts, [(w[2 * k], None, w[2 * k + 1], None) for k in range(na)]
         with torch.cuda.device(c.device):
-            d_x, d_h, d_c, d_params = backward(c, dout, dh_n if c.packed else None, need[2], need[3:5], any(need[5:]))
-        c.inputs = c.acts = c.weights = None
+            d_x, d_h, d_c, d_params = backward(c, kept, ctx.order, dout, dh_n if c.packed else None, need[2], need[3:5], any(need[5:]))
         if not d_params:
             d_params = [None] * (len(need) - 5)
         return (None, None, d_x, d_h, d_c, *d_params)
@@ -444,7 +451,7 @@ def run(module, c, x, h_c_0):
         out, h_n, c_n = Layersfn.apply(c, x if c.packed else None, data, h_0, c_0, *params)
     else:
         with torch.cuda.device(data.device):
-            out, h_n, c_n = forward(c, x if c.packed else data, h_0, c_0, params, False)
+            (out, h_n, c_n), _ = forward(c, x if c.packed else data, h_0, c_0, params, False)
     if c.packed:
         return PackedSequence(out, x.batch_sizes, x.sorted_indices, x.unsorted_indices), (h_n, c_n)
     return (out.transpose(0, 1) if module.batch_first else out), (h_n, c_n)

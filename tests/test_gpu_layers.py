@@ -101,3 +101,32 @@ def test_one_node_call_against_the_layer_loop(kw, T, B, I, H, dt, autocast, pack
     for a, b in zip(*results):
         assert a.shape == b.shape and a.dtype == b.dtype
         assert (a.float() - b.float()).abs().max() <= tol * a.float().abs().max()
+
+
+def test_backward_passes_over_one_graph_do_not_share_state(monkeypatch):
+    """A second backward pass over a retained graph while the first is under way (here: from inside its first layer) leaves the
+    first one's tensors alone."""
+    torch.manual_seed(0)
+    m = FastLSTM(24, 72, num_layers=3, bidirectional=True).cuda()
+    x = torch.randn(9, 6, 24, device="cuda", requires_grad=True)
+    assert layers.plan(m, x, None) is not None
+    y, _ = m(x)
+    inputs, dout = [x, *m.parameters()], torch.randn_like(y)
+    want = torch.autograd.grad(y, inputs, dout, retain_graph=True)
+    names, inner = ("lstm_persistent_bwd", "lstm_persistent_bwd_pair"), []
+
+    def nested(call):
+        def run(*args, **kw):
+            r = call(*args, **kw)
+            if not inner:
+                inner.append(None)
+                inner[0] = torch.autograd.grad(y, inputs, dout, retain_graph=True)
+            return r
+        return run
+
+    for name in names:
+        monkeypatch.setattr(L, name, nested(getattr(L, name)))
+    got = torch.autograd.grad(y, inputs, dout, retain_graph=True)
+    assert inner
+    for a, b, c in zip(want, got, inner[0]):
+        assert torch.equal(a, b) and torch.equal(a, c)
