@@ -414,8 +414,7 @@ class Layersfn(torch.autograd.Function):
             flat += a
         for w in weights:
             flat += (w[0], w[2])
-        ctx.save_for_backward(*flat)
-        ctx.order = packed.sorted_indices if c.packed else None
+        ctx.save_for_backward(packed.sorted_indices if c.packed else None, *flat)   # (the caller's tensor: a change in place is noticed)
         ctx.set_materialize_grads(False)
         ctx.mark_non_differentiable(*((c_n,) if c.packed else (h_n, c_n)))
         return out, h_n, c_n
@@ -426,13 +425,13 @@ class Layersfn(torch.autograd.Function):
         if dout is None and dh_n is None:
             return (None,) * len(need)
         L._raise_pending_before_backward(dout if dout is not None else dh_n)   # a failed forward launch is reported before its gradients are computed
-        t = ctx.saved_tensors
+        order, *t = ctx.saved_tensors
         ni, na = ctx.count
         acts = [tuple(t[ni + 3 * k:ni + 3 * k + 3]) for k in range(na)]
         w = t[ni + 3 * na:]
         kept = t[:ni], acts, [(w[2 * k], None, w[2 * k + 1], None) for k in range(na)]
         with torch.cuda.device(c.device):
-            d_x, d_h, d_c, d_params = backward(c, kept, ctx.order, dout, dh_n if c.packed else None, need[2], need[3:5], any(need[5:]))
+            d_x, d_h, d_c, d_params = backward(c, kept, order, dout, dh_n if c.packed else None, need[2], need[3:5], any(need[5:]))
         if not d_params:
             d_params = [None] * (len(need) - 5)
         return (None, None, d_x, d_h, d_c, *d_params)

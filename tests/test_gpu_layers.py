@@ -130,3 +130,13 @@ def test_backward_passes_over_one_graph_do_not_share_state(monkeypatch):
     assert inner
     for a, b, c in zip(want, got, inner[0]):
         assert torch.equal(a, b) and torch.equal(a, c)
+
+
+def test_sorted_indices_changed_in_place_after_forward_are_an_error():
+    m = FastLSTM(24, 72, num_layers=2).cuda()
+    x = pack_padded_sequence(torch.randn(7, 4, 24, device="cuda"), torch.tensor([3, 7, 5, 1]), enforce_sorted=False)
+    assert layers.plan(m, x, None) is not None
+    y, _ = m(x)
+    x.sorted_indices.copy_(torch.arange(4, device="cuda"))
+    with pytest.raises(RuntimeError, match="inplace"):
+        y.data.sum().backward()
