@@ -83,17 +83,19 @@ __device__ __forceinline__ f32x4 mfma_kstep<float>(const u32x4 a, const u32x4 b,
 // shape's outputs and gradients against nn.LSTM at 0.29 of the bar, 0.39 over the reference's test grid -- 0.43 with
 // the library forms: the fp32 summation order sets it, not the activations).
 // -DFASTLSTM_FP32_LIBM brings the library forms back.
-// 1 / d for d >= 1: the hardware reciprocal and one Newton step (what an IEEE division spends 10 instructions on)
+// 1 / d for d >= 1: the hardware reciprocal and one Newton step (what an IEEE division spends 10 instructions on).  d may be inf,
+// whose reciprocal 0 times d is no number: the minimum takes that one, and the step adds 0 times 1.  (The bound is here and not
+// on the argument of the exponential, where the minimum drops a NaN: its gate would be 0 or 1.  Here a NaN goes through r.)
 __device__ __forceinline__ float rcp_refined(float d) {
     const float r = __builtin_amdgcn_rcpf(d);
-    return __builtin_fmaf(r, __builtin_fmaf(-d, r, 1.0f), r);
+    return __builtin_fmaf(r, fminf(__builtin_fmaf(-d, r, 1.0f), 1.0f), r);
 }
 template <bool ACCURATE> __device__ __forceinline__ float sigmoidf_(float x) {
     if constexpr (ACCURATE) {
 #ifdef FASTLSTM_FP32_LIBM
         return 1.0f / (1.0f + expf(-x));
 #else
-        return rcp_refined(1.0f + __expf(fminf(-x, 80.0f)));   // (e^80 is finite: the Newton step has no inf x 0)
+        return rcp_refined(1.0f + __expf(-x));
 #endif
     } else {
         return __builtin_amdgcn_rcpf(1.0f + __expf(-x));
@@ -104,7 +106,7 @@ template <bool ACCURATE> __device__ __forceinline__ float tanhf_(float x) {
 #ifdef FASTLSTM_FP32_LIBM
         return tanhf(x);
 #else
-        return 1.0f - 2.0f * rcp_refined(1.0f + __expf(fminf(2.0f * x, 80.0f)));
+        return 1.0f - 2.0f * rcp_refined(1.0f + __expf(2.0f * x));
 #endif
     } else {
         // 1 - 2/(1+e^{2x}); saturates correctly at +-inf of the exponential

@@ -211,3 +211,51 @@ def test_padded_operand_cache_is_opt_in_and_follows_the_version_counters():
         assert next(iter(kept.values()))[1][0] is not first
         m.cache_padded_operands = False
         assert torch.equal(y3, m(x)[0]) and not torch.equal(y3, y2)
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.float16])
+@pytest.mark.parametrize("T,B,H", [(5, 7, 48), (5, 7, 64), (5, 7, 72), (5, 20, 256), (5, 70, 1024), (3, 5, 2100), (1, 4, 96)])
+def test_a_nan_of_the_input_reaches_the_results(T, B, H, dt):
+    """x[t, b] = NaN: out of that row is NaN from step t on and so are its last states, on every kernel family (and in the
+    gradients of the row); all other rows keep their bits."""
+    m = _module(24, H, 1, dt, 4)
+    x = torch.randn(T, B, 24, generator=torch.Generator().manual_seed(2)).to(dt).cuda()
+    t, b, others = T // 2, B - 2, [r for r in range(B) if r != B - 2]
+    bad = x.clone()
+    bad[t, b, 5] = float("nan")
+
+    def run(x, grads):
+        if not grads:
+            with torch.no_grad():
+                y, (h, c) = m(x)
+            return [y, h, c]
+        x = x.clone().requires_grad_(True)
+        y, (h, c) = m(x)
+        y.sum().backward()
+        return [y.detach(), h, c, x.grad]
+
+    for grads in (False, True):
+        want, got = run(x, grads), run(bad, grads)
+        for w, g in zip(want, got):
+            assert torch.equal(w[:, others], g[:, others])
+        assert torch.equal(want[0][:t, b], got[0][:t, b])
+        assert got[0][t:, b].isnan().all() and all(g[0, b].isnan().all() for g in got[1:3])
+        if grads:
+            assert got[3][:, b].isnan().all()
+    assert fastlstm_amd.pending_status() == _lib.OK
+
+
+@pytest.mark.parametrize("H", [64, 256])
+def test_saturated_fp32_gates(H):
+    """Pre-activations from -1e4 to 1e4, where the exponential is 0 or inf: forward and backward against nn.LSTM in 64 bits."""
+    m = _module(8, H, 1, torch.float32, 6)
+    ref = torch.nn.LSTM(8, H).double()
+    ref.load_state_dict({k: v.double().cpu() for k, v in m.state_dict().items()})
+    x = torch.randn(6, 5, 8, generator=torch.Generator().manual_seed(1)) * torch.logspace(0, 5, 6)[:, None, None]
+    a, b = x.cuda().requires_grad_(True), x.double().requires_grad_(True)
+    (y, _), (z, _) = m(a), ref(b)
+    y.sum().backward()
+    z.sum().backward()
+    # fp32 rounding of a sum of eight terms of 1e4 / 3 is about 1e-3, and a gate that is not saturated takes it with a slope of up to 1
+    torch.testing.assert_close(y.double().cpu(), z, rtol=2e-3, atol=2e-3)
+    torch.testing.assert_close(a.grad.double().cpu(), b.grad, rtol=2e-3, atol=2e-3)
