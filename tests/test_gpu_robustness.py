@@ -259,3 +259,39 @@ def test_saturated_fp32_gates(H):
     # fp32 rounding of a sum of eight terms of 1e4 / 3 is about 1e-3, and a gate that is not saturated takes it with a slope of up to 1
     torch.testing.assert_close(y.double().cpu(), z, rtol=2e-3, atol=2e-3)
     torch.testing.assert_close(a.grad.double().cpu(), b.grad, rtol=2e-3, atol=2e-3)
+
+
+@pytest.mark.parametrize("T,B,I,H,dt", [(6, 20, 32, 256, torch.float32),       # four waves, a ragged second group
+                                        (5, 9, 32, 80, torch.float32),
+                                        (6, 20, 32, 1024, torch.float16),      # eight waves, K split eight ways
+                                        (6, 40, 32, 512, torch.bfloat16),
+                                        (5, 300, 32, 256, torch.float16),      # groups of 32 rows
+                                        (4, 200, 32, 1024, torch.bfloat16),    # ... LDS-direct tiles
+                                        (96, 64, 1024, 1024, torch.float16)])  # products inside the launches
+def test_values_that_look_like_an_unwritten_exchange_word(T, B, I, H, dt):
+    """The XCD-local kernels mark exchange words as unwritten with all ones, which in h_0 or in a gradient is a NaN like any
+    other: it ends no launch and stays in its batch row, whose results are NaN; every other row keeps its bits."""
+    g = torch.Generator().manual_seed(H + B)
+    k = 1.0 / H ** 0.5
+    u = lambda *s: ((torch.rand(*s, generator=g) * 2 - 1) * k).to(dt).cuda()
+    n = lambda *s: torch.randn(*s, generator=g).to(dt).cuda()
+    x, h0, c0, dout = n(T, B, I), u(B, H), u(B, H), n(T, B, H)
+    Wx, bx, Wh, bh = u(4 * H, I), u(4 * H), u(4 * H, H), u(4 * H)
+    ones = torch.full((H,), -1, device="cuda", dtype=torch.int32 if dt == torch.float32 else torch.int16).view(dt)
+    rows, others = [3, B - 1], [b for b in range(B) if b not in (3, B - 1)]
+    z = lambda: torch.zeros(B, H, device="cuda", dtype=dt)
+    out, cell, ifgo = L.lstm_persistent_fwd(x, h0, c0, Wx, bx, Wh, bh)
+    clean = L.lstm_persistent_bwd(dout, z(), z(), x, out, cell, ifgo, Wx, Wh)
+    bad_h, bad_dout, at = h0.clone(), dout.clone(), T // 2
+    bad_h[rows], bad_dout[at, rows] = ones, ones
+    got = L.lstm_persistent_fwd(x, bad_h, c0, Wx, bx, Wh, bh)
+    grads = L.lstm_persistent_bwd(bad_dout, z(), z(), x, out, cell, ifgo, Wx, Wh)
+    torch.cuda.synchronize()
+    assert fastlstm_amd.pending_status() == _lib.OK
+    for a, b in zip(got, (out, cell, ifgo)):
+        assert torch.equal(a[:, others], b[:, others])
+    assert got[0][1:, rows].isnan().all() and got[1][1:, rows].isnan().all()
+    for a, b in zip(grads[:3], clean[:3]):
+        assert torch.equal(a.view(-1, B, a.shape[-1])[:, others], b.view(-1, B, b.shape[-1])[:, others])
+    assert grads[0][:at + 1, rows].isnan().all() and grads[1][rows].isnan().all() and grads[2][rows].isnan().all()
+    assert torch.equal(grads[0][at + 1:], clean[0][at + 1:])
