@@ -76,8 +76,9 @@ typedef struct {
     int wave_split;   /* 0: waves split K, 1: waves split batch tiles, 2: waves split W rows (H <= 64, no cross-CU sync),
                          3: W_h does not fit on chip -- waves split K and the weight slice is streamed every step */
     int lds_bytes;    /* LDS the kernel will request */
-    size_t ws_bytes;  /* smallest workspace the recurrent call accepts (2 exchange slots; wave_split 3: plus W_h once
-                         in operand order, which the call itself writes) */
+    size_t ws_bytes;  /* smallest workspace the recurrent call accepts (2 exchange slots of the general kernels;
+                         wave_split 3: plus W_h once in operand order, which the call itself writes).  The faster kernels
+                         need more: fastlstm_recurrent_workspace_bytes */
     size_t ws_zero_bytes; /* leading bytes of the workspace that must be zero (header + counters + flags) */
     int ring_needs_zero;  /* 1: B or H leave padding in the exchange blocks -> zero the whole workspace */
 } fastlstm_plan;
@@ -95,11 +96,13 @@ int fastlstm_plan_for(int num_cus, int lds_limit, int B, int H, int dtype, int b
  * used on a device where that was seen.  The launch calls below never synchronise. */
 int fastlstm_plan_device(int device, int B, int H, int dtype, int backward, fastlstm_plan *plan);
 
-/* Workspace of a recurrent call for this plan: header, barrier counters, flags and TWO exchange slots in the
- * layout of whichever kernel family the call may choose (fastlstm_recurrent_kernel_kind) -- a few hundred KiB,
- * independent of T (h_t / d_ifgo[t] of step t live in slot t % 2; plans that stream W_h add one packed copy of
- * it).  At least plan->ws_bytes.  The first plan->ws_zero_bytes bytes must be zero; the rest only if
- * plan->ring_needs_zero. */
+/* Workspace of a recurrent call for this plan: header, barrier counters, flags and the exchange slots of whichever
+ * kernel family the call may choose (fastlstm_recurrent_kernel_kind), independent of T: FOUR slots for the XCD-local
+ * kernels (h_v / the d_ifgo of reverse step s in slot v % 4 / s % 4), two for the others, the teams' partial sums of the
+ * 16-bit reverse pass at H = 1280 ... 2048 (8 MiB); plans that stream W_h add one packed copy of it.  B = 64, H = 1024,
+ * 16-bit: 705 KiB forward, 2.6 MiB reverse.  At least plan->ws_bytes; a call accepts anything from there on, and with less
+ * than this runs the kernels that fit, down to the general ones (B = 64, H = 1024, fp16: 3.1 instead of 1.75 us per
+ * step).  The first plan->ws_zero_bytes bytes must be zero; the rest only if plan->ring_needs_zero. */
 size_t fastlstm_recurrent_workspace_bytes(const fastlstm_plan *plan, int T, int H, int dtype, int backward);
 
 /* K1 -- ifgo[T*B,4H] = x[T*B,I] . Wx[4H,I]^T + (bx + bh).
@@ -133,7 +136,7 @@ int fastlstm_fwd_layer(const void *x, const void *Wx, const void *bx, const void
  * own copy until the process ends); the call clears the part it needs zeroed itself and calls no
  * hipMalloc/hipFree.  Same results as fastlstm_fwd_layer with a zeroed workspace of
  * min(16 MiB, fastlstm_recurrent_workspace_bytes(forward plan)) bytes -- the kernel choice follows the
- * workspace size as it does there (XCD-local kernels while a slot per timestep fits, else the general
+ * workspace size as it does there (XCD-local kernels while their four slots fit, else the general
  * ones).  FASTLSTM_ERR_WORKSPACE if the smallest workspace of the shape (plan.ws_bytes) exceeds the array.
  * All calls on one GPU share the array: calls that overlap in time on one GPU (two streams, two threads)
  * race; serialise them.  The XCD-local kernels are only chosen on a device that fastlstm_plan_device has

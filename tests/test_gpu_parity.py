@@ -1843,3 +1843,18 @@ def test_config_E_two_layers_fp16():
     assert rel_err(cn, cr) < HALF_TOL
     for n, prm in m.named_parameters():
         assert rel_err(prm.grad, getattr(ref, n).grad) < HALF_TOL, n
+
+
+@pytest.mark.parametrize("B,H,dt,kinds", [(64, 1024, torch.float16, (1, 1)), (100, 256, torch.float32, (1, 1)), (128, 2048, torch.bfloat16, (2, 2))])
+def test_workspace_size_and_kernel_family(B, H, dt, kinds):
+    """fastlstm_recurrent_workspace_bytes is enough for the fast kernels; plan.ws_bytes is accepted and may run slower ones."""
+    lib, code, T = _lib.load(), RM[dt], 5
+    for bw in (0, 1):
+        plan = _lib.Plan()
+        _lib.check(lib.fastlstm_plan_device(0, B, H, code, bw, plan), "plan")
+        full = lib.fastlstm_recurrent_workspace_bytes(plan, T, H, code, bw)
+        assert lib.fastlstm_recurrent_kernel_kind(T, B, H, code, bw, full) == kinds[bw]
+        if kinds[bw] == 1:
+            assert lib.fastlstm_recurrent_kernel_kind(T, B, H, code, bw, plan.ws_bytes) == 0
+    assert lib.fastlstm_plan_device(0, 64, 1024, 1, 0, plan) == _lib.OK and plan.ws_bytes == 322 << 10
+    assert lib.fastlstm_recurrent_workspace_bytes(plan, T, 1024, 1, 0) == 705 << 10
