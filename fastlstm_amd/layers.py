@@ -89,8 +89,9 @@ def plan(module, x, h_c_0):
     params = module._operand_list()
     c.held = params[0].dtype
     idx = data.get_device()
-    for p in params:
-        if p.dtype != c.held or p.get_device() != idx or not p.is_contiguous():
+    shapes = L._parameter_shapes(module.num_layers, 2 if module.bidirectional else 1, module.input_size, module.hidden_size, module.bias)
+    for p, (_, shape) in zip(params, shapes):
+        if p.dtype != c.held or p.get_device() != idx or p.shape != shape or not p.is_contiguous():
             return None
     if c.held not in L._DTYPE_CODE or (c.held != c.dt and not autocast):
         return None

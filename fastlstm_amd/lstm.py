@@ -187,6 +187,7 @@ def lstm_persistent_fwd(x, h0, c0, Wx, bx, Wh, bh, version=None, keep_activation
     assert x.is_contiguous()  # fastlstm/lstm.py:49-50
     assert Wh.is_contiguous()
     assert Wx.shape == (4 * hidden_size, input_size) and Wh.shape == (4 * hidden_size, hidden_size)
+    assert bx.numel() == bh.numel() == 4 * hidden_size
     for w in (Wx, bx, Wh, bh):
         if w.dtype != x.dtype:
             raise TypeError("weights must have the dtype of x (%s), got %s" % (x.dtype, w.dtype))
@@ -472,6 +473,7 @@ def lstm_persistent_fwd_stack(x, layers, keep_activations=True):
     assert x.is_contiguous()
     for l, (_, _, Wx, bx, Wh, bh) in enumerate(layers):
         assert Wx.shape == (4 * H, I if l == 0 else H) and Wh.shape == (4 * H, H) and Wh.is_contiguous()
+        assert bx.numel() == bh.numel() == 4 * H
         for w in (Wx, bx, Wh, bh):
             if w.dtype != x.dtype:
                 raise TypeError("weights must have the dtype of x (%s), got %s" % (x.dtype, w.dtype))
@@ -550,6 +552,7 @@ def lstm_persistent_fwd_stack2(x, h0a, c0a, Wx0, bx0, Wh0, bh0, h0b, c0b, Wx1, b
     H = Wh0.shape[1]
     assert x.is_contiguous() and Wh0.is_contiguous() and Wh1.is_contiguous()
     assert Wx0.shape == (4 * H, I) and Wh0.shape == (4 * H, H) and Wx1.shape == (4 * H, H) and Wh1.shape == (4 * H, H)
+    assert bx0.numel() == bh0.numel() == bx1.numel() == bh1.numel() == 4 * H
     for w in (Wx0, bx0, Wh0, bh0, Wx1, bx1, Wh1, bh1):
         if w.dtype != x.dtype:
             raise TypeError("weights must have the dtype of x (%s), got %s" % (x.dtype, w.dtype))
@@ -770,6 +773,7 @@ def lstm_persistent_fwd_pair(xa, h0a, c0a, Wxa, bxa, Wha, bha, xb, h0b, c0b, Wxb
     assert xb.shape == xa.shape and xb.dtype == xa.dtype and xa.is_contiguous() and xb.is_contiguous()
     assert Wha.is_contiguous() and Whb.is_contiguous()
     assert Wxa.shape == (4 * H, I) and Wxb.shape == (4 * H, I) and Wha.shape == (4 * H, H) and Whb.shape == (4 * H, H)
+    assert bxa.numel() == bha.numel() == bxb.numel() == bhb.numel() == 4 * H
     for w in (Wxa, bxa, Wha, bha, Wxb, bxb, Whb, bhb):
         if w.dtype != xa.dtype:
             raise TypeError("weights must have the dtype of x (%s), got %s" % (xa.dtype, w.dtype))
@@ -1236,6 +1240,14 @@ class _TakeRows(torch.autograd.Function):
 _LAYER_PARAMETERS = ("weight_ih_l", "bias_ih_l", "weight_hh_l", "bias_hh_l")   # in the order of _layer_operands
 
 
+@functools.lru_cache(maxsize=256)
+def _parameter_shapes(L, D, I, H, bias):
+    """((name, shape), ...) in the order of FastLSTM._operand_list.  The forms that hand the parameters' addresses on as they are
+    look at the shapes: a module may have been given other parameters."""
+    return tuple((name + str(k // D) + ("_reverse" if k % D else ""), torch.Size((4 * H,) if name[0] == "b" else (4 * H, H) if "hh" in name else (4 * H, I if k < D else D * H)))
+                 for k in range(L * D) for name in (_LAYER_PARAMETERS if bias else _LAYER_PARAMETERS[::2]))
+
+
 class FastLSTM(nn.Module):
     """nn.LSTM-compatible parameters (names, shapes, order, seeded values) and the
     reference's forward contract (fastlstm/lstm.py:586-698): sequence-first input
@@ -1448,15 +1460,14 @@ class FastLSTM(nn.Module):
                 if type(t) is not torch.Tensor or t.dtype != dt or t.shape != (L, B, H) or t.get_device() != idx or not t.is_contiguous():
                     return None
             h0, c0 = h_0.data_ptr(), c_0.data_ptr()
-        params, pointers = self._parameters, []
-        for layer in range(L):
-            for name in _LAYER_PARAMETERS if self.bias else _LAYER_PARAMETERS[::2]:
-                p = params.get(name + str(layer))   # (missing: parametrized, say; then the general path asks for the attribute)
-                if p is None or p.dtype != dt or p.get_device() != idx or not p.is_contiguous():
-                    return None
-                pointers.append(p.data_ptr())
-                if not self.bias:
-                    pointers.append(None)
+        params, pointers, bias = self._parameters, [], self.bias
+        for name, shape in _parameter_shapes(L, 1, I, H, bias):
+            p = params.get(name)   # (missing: parametrized, say; then the general path asks for the attribute)
+            if p is None or p.dtype is not dt or p.get_device() != idx or p.shape != shape or not p.is_contiguous():
+                return None
+            pointers.append(p.data_ptr())
+            if not bias:
+                pointers.append(None)
         if idx != torch.cuda.current_device():
             with torch.cuda.device(idx):
                 return self._forward_short(x, h_c_0)

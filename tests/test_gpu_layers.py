@@ -140,3 +140,18 @@ def test_sorted_indices_changed_in_place_after_forward_are_an_error():
     x.sorted_indices.copy_(torch.arange(4, device="cuda"))
     with pytest.raises(RuntimeError, match="inplace"):
         y.data.sum().backward()
+
+
+@pytest.mark.parametrize("grads,kw,name", [(False, dict(num_layers=2), "weight_hh_l1"), (False, dict(), "bias_ih_l0"), (True, dict(num_layers=2), "weight_ih_l1"),
+                                           (True, dict(num_layers=2, bidirectional=True), "weight_hh_l0_reverse")])
+def test_parameters_of_another_shape_are_refused(grads, kw, name):
+    """A parameter replaced by one of another shape: no form that takes addresses reads past it."""
+    m = FastLSTM(24, 72, **kw).cuda()
+    x = torch.randn(2, 3, 24, device="cuda")
+    with torch.set_grad_enabled(grads):
+        m(x)
+        old = getattr(m, name)
+        setattr(m, name, torch.nn.Parameter(torch.zeros(*old.shape[:-1], old.shape[-1] // 2, device="cuda")))
+        assert layers.plan(m, x, None) is None and (grads or m._forward_short(x, None) is None)
+        with pytest.raises((AssertionError, RuntimeError)):
+            m(x)

@@ -11,7 +11,7 @@ import numpy as np
 import pytest
 import torch
 
-from fastlstm_amd import FastLSTM, PersistentLSTMfn, _lib
+from fastlstm_amd import FastLSTM, PersistentLSTMfn, _lib, lstm
 from helpers import make_problem, to_np
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -285,3 +285,11 @@ def test_device_status_without_a_planned_device_is_ok():
     lib = _lib.load()
     assert lib.fastlstm_device_status(-1, 0) == _lib.OK
     assert lib.fastlstm_device_status(0, 1) == _lib.OK
+
+
+def test_parameter_shapes_follow_the_operand_list():
+    for kw in (dict(num_layers=3), dict(num_layers=2, bidirectional=True, bias=False), dict(num_layers=2, bidirectional=True)):
+        m = FastLSTM(5, 7, **kw)
+        got = lstm._parameter_shapes(m.num_layers, 2 if m.bidirectional else 1, 5, 7, m.bias)
+        assert [s for _, s in got] == [p.shape for p in m._operand_list()]
+        assert [n for n, _ in got] == m._operand_names
