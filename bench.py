@@ -5,14 +5,14 @@
                     [--stage all|fwd_recurrence|gemms|fwd_layer|bwd_layer]
 
 A "step" is one pass of the workload's hot path over one batch of synthetic input
-(already resident in HBM).  The default workload is BASELINE.json's headline
+(already resident in HBM).  The default workload is the headline
 configuration B: single-layer fp16 FORWARD, batch 64, seq_len 512, input = hidden =
 1024 (x ~ N(0,1), h0,c0 ~ N(0,0.1), weights U(+-1/32), seeded).  Prints ONE JSON
 line: metric/value = batch*timesteps per second of that step, plus
   roofline      for the dominant kernel (the launch that holds the persistent recurrence), timed with
                 HIP events on the launch stream: its algorithmic flops against the MFMA peak and, in
                 roofline.latency_bound, its time per timestep against the measured latency floor of a
-                step (barrier round trip + exchange of h_t, fastlstm_diag_step_probe),
+                step (exchange of h_t as the kernel does it, fastlstm_diag_step_probe),
   kernels       per-stage timings (input-projection GEMM, recurrence, and for the
                 forward+backward pass: reverse recurrence, dx GEMM, weight-gradient GEMMs),
   fwd / fwd_bwd the workload timed forward and forward+backward (hot loop, mean of --steps calls),
@@ -430,12 +430,15 @@ def main():
             pk, members, rows = 1, H // 16, 64
         else:
             pk, members, rows = 1, plan_f.n_htiles, min(64, max(16, plan_f.bt // 16 * 16))
-        while H % members:
+        while H % (4 * members if pk == 0 else members):
             members -= 1
         steps_p = 512
         ws_p = torch.zeros(lib.fastlstm_diag_step_probe_bytes(steps_p, H, rows), dtype=torch.uint8, device=dev)
         probe = {}
-        for pm, name in ((0, "empty_barrier_us"), (1, "barrier_plus_publish_us"), (2, "barrier_publish_fetch_us")):
+        modes = [(0, "empty_barrier_us"), (1, "barrier_plus_publish_us"), (2, "barrier_publish_fetch_us")]
+        if pk == 0:   # what the XCD-local kernels do instead: the data carries the synchronisation
+            modes.append((3, "exchange_without_barrier_us"))
+        for pm, name in modes:
             def run(pm=pm):
                 _lib.check(lib.fastlstm_diag_step_probe(pk, pm, members, H, rows, steps_p, ws_p.data_ptr(), ws_p.numel(),
                                                         stream), "step probe")
@@ -443,7 +446,7 @@ def main():
         torch.cuda.synchronize()
         _lib.check(lib.fastlstm_ws_status(ws_p[:64].cpu().numpy().tobytes()), "step probe status")
         mfma_us = 2.0 * B * H * 4 * H / (PEAK_TFLOPS[dname] * 1e12) * 1e6
-        bound = probe["barrier_publish_fetch_us"]
+        bound = probe[modes[-1][1]]
         per_step = t_dom * 1e3 / T
         roofline["latency_bound"] = {
             "bound": "latency", "per_step_bound_us": bound, "achieved_us_per_step": round(per_step, 3),
@@ -451,10 +454,10 @@ def main():
             "recurrence_alone_us_per_step": round(t_rec * 1e3 / T, 3),
             "frac_recurrence_alone": round(bound / (t_rec * 1e3 / T), 4),
             "mfma_time_per_step_at_peak_us": round(mfma_us, 3),
-            "probe": dict(probe, group="XCD-local, L2 counters" if pk == 0 else "flag group over all XCDs",
+            "probe": dict(probe, group="XCD-local" if pk == 0 else "flag group over all XCDs",
                           members=members, rows=rows, steps=steps_p),
-            "note": "per_step_bound_us = publish h_t + barrier round trip + fetch of the group's h_t, timed with the "
-                    "kernels' own code and no arithmetic (fastlstm_diag_step_probe mode 2); frac = bound / achieved"}
+            "note": "per_step_bound_us = publish h_t, wait for the group's h_t and fetch it, timed with the kernels' own code "
+                    "and no arithmetic (fastlstm_diag_step_probe mode %d); frac = bound / achieved" % modes[-1][0]}
 
     res = {
         "metric": "lstm_%s_batch_timesteps_per_s" % mode, "value": round(value, 1), "unit": "batch*timesteps/s",

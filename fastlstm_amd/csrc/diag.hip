@@ -10,10 +10,11 @@
 //   mode 1  + every member stores its share of a `rows`-row h tile into the step's exchange slot (slot t % 2)
 //   mode 2  + every wave fetches its operand blocks of the step with the loads the real kernels use (they go
 //           past the L1 to the L2: a slot is rewritten every second step)
-//   mode 3, 4  (kind 0) the same exchange WITHOUT a barrier: a ring of 4 slots whose unwritten values hold
-//           a sentinel bit pattern (all ones: a NaN no gate output produces); a member stores its share
-//           of h_{t+1}, resets its share of the slot two versions back, and every wave polls its operand
-//           blocks with loads that bypass the L1 (mode 3: sc1, mode 4: sc0 sc1) until no sentinel is left
+//   mode 3  (kind 0) the exchange of the XCD-local kernels, whose data carries the synchronisation: four slots, a member
+//           stores its share of h_t, every wave repeats the loads of its operand blocks until all of them have been
+//           written, and behind a workgroup barrier the member marks the slot before as unwritten (poll_blocks,
+//           written_word of recurrent_fwd_xcd.hpp); mode 4 the same with loads past every cache (sc0 sc1).  Modes 0 to 2 are the
+//           counter barrier that these kernels use once per launch, and per step no more
 // group kinds:
 //   0  XCD-local group: `members` (<= 32) workgroups of ONE XCD, counters in its L2, polled with
 //      scalar loads (recurrent_fwd_xcd.hpp)
@@ -56,59 +57,37 @@ __global__ __launch_bounds__(kWave *kProbeWaves) void step_probe_kernel(const Pr
     int *my_counter = p.counters + (j % kXcdReplicas) * kXcdCounterStride;
     unsigned acc = 0;
     if (p.mode >= 3) {
-        // ring of 4 slots, all sentinel at launch (host); slot v % 4 holds version v
-        constexpr int R = 4;
-        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(p.xbuf, 0, (unsigned)(R * xslot), 0x00020000);
-        long long t0 = 0;
+        // as lstm_fwd_xcd_kernel: all slots unwritten and one counter barrier, then per step the member's share of h_t, the
+        // wave's blocks until none of their words is unwritten, a workgroup barrier, the slot of h_{t-1} unwritten again
         bool dead = false;
-        for (int t = 0; t < p.steps && !dead; ++t) {
-            const unsigned wslot = (unsigned)(((t + 1) % R) * xslot), rslot = (unsigned)(((t + 3) % R) * xslot);
-            for (int it = tid; it < items; it += kWave * kProbeWaves) {
-                const unsigned off = ((it >> 4) / HT) * p.KS * kFragBytes + frag_offset<T>(it & 15, j * HT + (it >> 4) % HT);
-                __builtin_amdgcn_raw_buffer_store_b16((unsigned short)((t + it) & 0x7fff), rs, wslot + off, 0, 0);
-                if (t >= 1) __builtin_amdgcn_raw_buffer_store_b16((unsigned short)0xffffu, rs, rslot + off, 0, 0);
-            }
-            // poll version t + 1
+        auto slot_of = [&](int v) { return XchgL2(p.xbuf + (size_t)(v % kXchgSlots) * xslot, (unsigned)xslot); };
+        auto put = [&](const XchgL2 &x, unsigned w) {   // four units of a row at a time, w in every word
+            for (int it = tid; it < items / 4; it += kWave * kProbeWaves)
+                x.store8(((it >> 4) / (HT / 4)) * p.KS * kFragBytes + frag_offset<T>(it & 15, j * HT + (it >> 4) % (HT / 4) * 4), u32x2{w, w});
+        };
+        for (int v = 0; v < kXchgSlots; ++v) put(slot_of(v), kUnwritten);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        if (tid < kXcdReplicas)
+            __hip_atomic_fetch_add(p.counters + tid * kXcdCounterStride, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        if (wave == 0) wait_counter(my_counter, p.members, p.hdr, p.spin_limit, 0, 0);
+        __syncthreads();
+        auto poll = [&](auto blocks, const XchgL2 &x, int nt, int t) {   // wave w: k-steps w, w + 8, ... (past the end: any block)
+            u32x4 v[decltype(blocks)::value];
+            poll_blocks(v, [&](int i) {
+                const unsigned off = (unsigned)((nt * p.KS + min(wave + kProbeWaves * i, p.KS - 1)) * kWave + lane) * 16u;
+                return p.mode == 3 ? x.load16_l2(off) : __builtin_amdgcn_raw_buffer_load_b128(x.rsrc, off, 0, 17);
+            }, dead, p.hdr, p.spin_limit, 0, t);
+            acc ^= v[0][0] ^ v[decltype(blocks)::value - 1][3];
+        };
+        for (int t = 0; t < p.steps; ++t) {
+            put(slot_of(t), written_word((unsigned)t));
             for (int nt = 0; nt < p.NT; ++nt) {
-                int polls = 0;
-                for (;;) {
-                    u32x4 v[8];
-#pragma unroll
-                    for (int ki = 0; ki < 8; ++ki) {
-                        const int ks = min(wave % shares + shares * ki, p.KS - 1);
-                        const unsigned off = wslot + (unsigned)((nt * p.KS + ks) * kWave + lane) * 16u;
-                        v[ki] = p.mode == 3 ? __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 16)
-                                            : __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 17);
-                    }
-                    unsigned bad = 0;
-#pragma unroll
-                    for (int ki = 0; ki < 8; ++ki)
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            const unsigned w = v[ki][e];
-                            bad |= ((w & 0xffffu) == 0xffffu) | ((w >> 16) == 0xffffu);
-                            acc ^= w;
-                        }
-                    if (!__any(bad)) break;
-                    if (++polls >= 64) {
-                        polls = 0;
-                        if (__hip_atomic_load(&p.hdr->abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) { dead = true; break; }
-                        const long long now = (long long)wall_clock64();
-                        if (t0 == 0) t0 = now;
-                        else if (now - t0 > p.spin_limit) {
-                            if (lane == 0) {
-                                p.hdr->timeout_group = 0;
-                                p.hdr->timeout_step = t;
-                                __hip_atomic_store(&p.hdr->abort_flag, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-                            }
-                            dead = true;
-                            break;
-                        }
-                    }
-                }
-                if (dead) break;
+                if (p.KS <= 32) poll(std::integral_constant<int, 4>{}, slot_of(t), nt, t);
+                else poll(std::integral_constant<int, 8>{}, slot_of(t), nt, t);
             }
-            dead = __syncthreads_or(dead);   // (also keeps the waves of a member within a step of each other, as the real kernels' barriers do)
+            __syncthreads();
+            if (t > 0) put(slot_of(t + kXchgSlots - 1), kUnwritten);
         }
         if (acc == 0x9e3779b9u) p.sink[blockIdx.x] = acc;
         return;
@@ -174,7 +153,7 @@ int fastlstm_diag_step_probe(int kind, int mode, int members, int H, int rows, i
                              void *stream) {
     if (!ws) return FASTLSTM_ERR_NULL;
     if (kind < 0 || kind > 1 || mode < 0 || mode > 4 || (mode >= 3 && kind != 0) || members <= 0 || steps <= 0 || H <= 0 || H % 32 || H % members ||
-        H / members < 4 || members > (kind == 0 ? 32 : 256) || H > 8 * 8 * 32 || rows < 16 || rows > 64 || rows % 16)
+        H / members < 4 || (mode >= 3 && H / members % 4) || members > (kind == 0 ? 32 : 256) || H > 8 * 8 * 32 || rows < 16 || rows > 64 || rows % 16)
         return FASTLSTM_ERR_DIM;
     if (!aligned16(ws)) return FASTLSTM_ERR_ALIGN;
     if (ws_bytes < fastlstm_diag_step_probe_bytes(steps, H, rows)) return FASTLSTM_ERR_WORKSPACE;

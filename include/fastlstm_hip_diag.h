@@ -48,12 +48,11 @@ void fastlstm_set_recurrent_trace(void *buf);
  * that no arithmetic throughput removes, with the recurrent kernels' own barrier and exchange code:
  * mode 0 = the empty barrier (publish + wait), 1 = + every member stores its share of a `rows`-row fp16 h
  * tile into the step's exchange slot (slot t % 2), 2 = + every wave fetches its operand blocks of the step
- * (loads that go past the L1, as in the kernels); 3, 4 (kind 0 only) = the exchange without a barrier:
- * consumers poll the data itself, unwritten values hold an all-ones sentinel, loads bypass the L1 (sc1 /
- * sc0 sc1); the exchange slots of ws (everything from byte 66560 on) must then hold 0xFF bytes.
+ * (loads that go past the L1, as in the kernels); 3, 4 (kind 0 only) = the exchange of the XCD-local kernels:
+ * no barrier, a wave repeats the loads of its operand blocks (sc1 / sc0 sc1) until all of them have been written.
  * kind 0 = an XCD-local group of `members` <= 32 workgroups (counters in that XCD's L2), kind 1 = a flag
  * group of `members` <= 256 workgroups over all XCDs (device-scope flags).  H <= 2048, a multiple of 32 and of
- * `members`; rows = 16, 32, 48 or 64 batch rows per group.  The caller times the launch (its duration /
+ * `members` (modes 3, 4: of 4 `members`); rows = 16, 32, 48 or 64 batch rows per group.  The caller times the launch (its duration /
  * steps = microseconds per round); ws: zeroed device memory of fastlstm_diag_step_probe_bytes.  No
  * counterpart in the reference. */
 int fastlstm_diag_step_probe(int kind, int mode, int members, int H, int rows, int steps, void *ws,

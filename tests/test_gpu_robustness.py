@@ -295,3 +295,17 @@ def test_values_that_look_like_an_unwritten_exchange_word(T, B, I, H, dt):
         assert torch.equal(a.view(-1, B, a.shape[-1])[:, others], b.view(-1, B, b.shape[-1])[:, others])
     assert grads[0][:at + 1, rows].isnan().all() and grads[1][rows].isnan().all() and grads[2][rows].isnan().all()
     assert torch.equal(grads[0][at + 1:], clean[0][at + 1:])
+
+
+@pytest.mark.parametrize("H,rows,members", [(1024, 16, 32), (2048, 32, 32), (96, 64, 8)])
+def test_step_probe_ends_in_every_mode(H, rows, members):
+    """fastlstm_diag_step_probe, on a workspace whose exchange slots hold anything: every mode ends and reports no time-out."""
+    lib, steps = _lib.load(), 20
+    n = lib.fastlstm_diag_step_probe_bytes(steps, H, rows)
+    for kind, mode in ((0, 0), (0, 1), (0, 2), (0, 3), (0, 4), (1, 0), (1, 1), (1, 2)):
+        ws = torch.randint(0, 256, (n,), dtype=torch.uint8, device="cuda")
+        ws[:70000].zero_()
+        assert lib.fastlstm_diag_step_probe(kind, mode, members, H, rows, steps, ws.data_ptr(), n, torch.cuda.current_stream().cuda_stream) == _lib.OK
+        torch.cuda.synchronize()
+        assert lib.fastlstm_ws_status(ws[:64].cpu().numpy().tobytes()) == _lib.OK, (kind, mode)
+    assert lib.fastlstm_diag_step_probe(0, 3, 16, 96, 16, steps, ws.data_ptr(), n, None) == _lib.ERR_DIM   # six units per member
