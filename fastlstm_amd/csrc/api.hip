@@ -375,9 +375,16 @@ struct SecondLayer {
 };
 
 // Products inside a recurrent launch overlap with it chunk by chunk, all but the first chunk (forward: the time loop starts behind
-// it) or the last one (reverse).  A layer of fewer than four chunks (reverse: of one) has little to overlap, and launches of
-// their own are the better tiles (T = 35, B = 20, I = H = 704, one chunk: forward 134 us inside, 103 as two launches).
-constexpr int kMinChunks = 4;
+// it) or the last one (reverse).  With few chunks there is little to overlap, and launches of their own are the better tiles.
+// fp16, us inside / as launches of their own:
+//   forward, chunks 1, 2, 3, 4, 6: B = 64, I = H = 1024 145/107, 200/168, 253/244, 301/309, 417/461; B = 32, I = 512, H = 768
+//   298/262, 539/497, 763/784, 983/1040, 1463/1457; B = 48, I = 256, H = 896 179/148, 286/258, 400/370, 507/491, 735/734;
+//   reverse, chunks 2, 4, 8 (smaller chunks: a prologue and the weight gradients' tiles to pay for): B = 64, I = H = 1024 173/133,
+//   212/190, 283/293; B = 32, I = 512, H = 768 171/143, 248/226, 403/390, 25 chunks 1109/1186; B = 16, I = H = 1024
+//   256/226, 389/374, 667/669, 14 chunks 1105/1185; B = 20, I = H = 704 407/391, 726/725, 1375/1369, 9 chunks 1534/1602.
+// By time the line of the reverse pass would lie at eight; it lies at two because dx of a layer call has to be the bits of
+// fastlstm_bwd_stack2's, whose launch has it inside, and the launch of its own may add in another order (split along K).
+constexpr int kMinChunks = 4, kMinChunksReverse = 2;
 
 bool plan_k1_helpers(const XcdCfg &c, const void *x, const void *Wx, const void *bx, const void *bh, void *ifgo, int T,
                      int B, int I, int H, int dtype, FwdXcdParams *p, const SecondLayer *second = nullptr) {
@@ -831,7 +838,7 @@ bool plan_bwd_helpers(const XcdCfg &c, const void *d_ifgo, const BwdExtras &e, i
         lower_wgrad_inside = all_ms <= upper_ms;
     }
     while (cdiv(tiles_m, ct) > max_chunks) ct += base;
-    if (!lower && cdiv(tiles_m, ct) < 2) return false;   // (see kMinChunks)
+    if (!lower && cdiv(tiles_m, ct) < kMinChunksReverse) return false;
     p->n_layers = layers;
     if (lower) {
         if (e.I != H) return false;   // the upper layer's dx is the lower layer's dout
@@ -1745,9 +1752,13 @@ int fastlstm_fwd_layer_infer(const void *x, const void *Wx, const void *bx, cons
 // ---- a few timesteps of inference, one kernel per step (recurrent_step.hpp) ----------------------------------
 // 1 where that is the faster form.  A launch takes about 3 us plus the operands its workgroups read through the L2s at about
 // 7.5 TB/s; the persistent path about 40 us per layer (its small launches and the host's work for them) and 0.6 us
-// per step more.  Measured on either side of the line, us per call of the module, persistent / one kernel per step:
-// 1 layer, B = 1, I = 80, H = 128 fp16 T = 8 52 / 34, T = 16 51 / 65; 2 layers, B = 4, I = H = 512 T = 16 108 / 91, T = 24
-// 108 / 134; B = 64, I = 1024, H = 2048 T = 1 53 / 22, T = 4 59 / 86.
+// per step more.  Both are on the low side (a persistent call of one layer takes 50 to 70 us with the host, and its GPU part
+// 20 to 80 us plus 1 to 5 us per step), so that the line errs towards the persistent form and holds with a faster host.
+// Measured on either side of it, us per call of the module, persistent / one kernel per step: 1 layer, B = 1, I = 80,
+// H = 128 fp16 T = 12 67 / 50, T = 16 67 / 66; 2 layers, B = 4, I = H = 512 fp16 T = 16 113 / 92, T = 24 116 / 136; 2 layers, B = 8,
+// I = 96, H = 256 fp32 T = 16 123 / 106, T = 24 146 / 155; 3 layers, B = 16, I = 256, H = 768 bf16 T = 8 159 / 102, T = 12 159 / 148,
+// T = 16 175 / 192; 1 layer, B = 64, I = 1024, H = 2048 fp16 T = 1 67 / 23, T = 2 67 / 45, T = 4 67 / 88; 1 layer, B = 32, I = 512,
+// H = 1024 fp32 T = 1 78 / 17, T = 2 88 / 33, T = 6 111 / 95.
 int fastlstm_infer_short_applies(int layers, int T, int B, int I, int H, int dtype) {
     if (layers <= 0 || !dtype_ok(dtype) || check_dims(T, B, I, H)) return 0;
     if (T > 64 || B > 64) return 0;

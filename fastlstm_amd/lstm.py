@@ -290,9 +290,15 @@ def stack_wavefront_chunks(L, T, B, H, dtype, device, backward=False):
 
 
 def _stack2_overlaps(T, B):
-    """Two layers in one launch follow each other in chunks of up to 64 timesteps that are whole tiles of 256 rows: with fewer
-    than four chunks they hardly overlap, and launches per layer are faster (T = 35, B = 20, 2 x 704 units, one chunk:
-    forward 214, reverse 416 us in one launch, 178 and 285 layer by layer)."""
+    """Two layers in one launch follow each other in chunks of up to 64 timesteps that are whole tiles of 256 rows (at an odd B
+    256 timesteps).  With fewer than four chunks they hardly overlap.  What this decides is the calls of fewer than 128
+    timesteps, which run layer by layer then; from 128 on, where the two layers also fit a wavefront
+    (stack2_wavefront_chunks), lstm_persistent_fwd_stack2 takes the one launch however few its chunks are, so that such a
+    call keeps the bits of one layer after the other.  fp16, us forward + reverse in one launch / as a wavefront / layer by
+    layer: B = 20, 2 x 704 units T = 64 346 + 580 / - / 286 + 463, T = 96 411 + 683 / - / 397 + 679, T = 128 500 + 772 /
+    432 + 727 / 505 + 823, T = 192 617 + 974 / 574 + 956 / 733 + 1151, T = 512 1225 + 1860 / 1264 + 2234 / 1805 + 2735; B = 32,
+    2 x 1024 T = 64 390 + 700 / - / 312 + 533, T = 128 513 + 906 / 479 + 877 / 539 + 818, T = 256 759 + 1265 / 849 + 1489 /
+    1105 + 1403; B = 5, 2 x 704 (chunks of 256) T = 256 1061 + 1569 / 687 + 1076 / 911 + 1302."""
     least = 256 // math.gcd(256, B)
     return T > 3 * max(least, 64 // least * least)
 
@@ -561,7 +567,7 @@ def lstm_persistent_fwd_stack2(x, h0a, c0a, Wx0, bx0, Wh0, bh0, h0b, c0b, Wx1, b
     lib = _lib.load()
     with torch.cuda.device(x.device):
         n = stack2_wavefront_chunks(T, B, H, x.dtype, x.device)
-        # (the library's own two-layer launch, with the GEMMs inside, wins wherever it applies)
+        # (the library's own two-layer launch, with the GEMMs inside, wherever it applies)
         if n and not stack2_runs_in_one_launch(T, B, I, H, x.dtype, x.device):
             return _fwd_stack2_wavefront(x, h0a, c0a, Wx0, bx0, Wh0, bh0, h0b, c0b, Wx1, bx1, Wh1, bh1, n, keep_activations)
         bufs = []
