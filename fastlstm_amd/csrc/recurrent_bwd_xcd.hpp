@@ -242,8 +242,13 @@ __device__ __forceinline__ void bwd_helper(const BwdXcdParams &p, unsigned char 
                 gemm16_mainloop<T, true, true, 256, 256, 2, WVM, WVN, 2>(wp, wm0, wn0, kb, ke, smem, acc, salt);
             }
         }
-        for (int i = k * per_chunk + ((h - k * per_chunk) % n_helpers + n_helpers) % n_helpers; i < (k + 1) * per_chunk;
-             i += n_helpers) {
+        // Around the call 28 registers of the accumulators have to go to memory: stored once per chunk, loaded behind the
+        // call.  That a helper takes few tiles of a chunk is said to the compiler: where it took this loop to run as often as
+        // the k loop above, it moved them there and back in every pass of that one, in one instantiation or another (16 bits,
+        // T = 256, I = H = 512, the reverse call: B = 32 2.21 -> 0.56 ms, B = 64 4.19 -> 0.61; I = H = 1024, B = 64 0.85 -> 0.83.
+        // With a probability of 0.5 they are stored with each tile: 0.88).
+        for (int i = k * per_chunk + ((h - k * per_chunk) % n_helpers + n_helpers) % n_helpers;
+             __builtin_expect_with_probability(i < (k + 1) * per_chunk, 1, 0.9); i += n_helpers) {
             const int r = i - k * per_chunk;
             const int rt = c * p.k5_chunk_tiles + r / p.k5_tiles_n, ct = r % p.k5_tiles_n;
             if (rt >= p.k5_tiles_m || !p.k5.C) continue;   // (no dx wanted: the helpers only accumulate weight gradients)

@@ -1,4 +1,4 @@
-"""Wait states around the matrix instructions, in the machine code of the library as built.
+"""Wait states around the matrix instructions, and what their loops spill, in the machine code of the library as built.
 
 The compiler keeps the distances that the hardware does not wait for by itself -- around its own MFMAs; those that are inline
 assembly (recurrent_fwd_big.hpp, gemm16.hpp) it does not see inside.  What it puts between its own for gfx950, and what is
@@ -116,6 +116,20 @@ def violations(code):
     return bad
 
 
+def scratch_in_matrix_loops(code):
+    """Scratch accesses in the innermost loops that hold MFMAs: [(first pc, MFMAs, accesses)]."""
+    index = {ins[0]: k for k, ins in enumerate(code)}
+    loops = [(index[ins[7]], k) for k, ins in enumerate(code) if ins[7] is not None and ins[7] <= ins[0]]
+    found = []
+    for a, b in loops:
+        if any((c, d) != (a, b) and a <= c and d <= b for c, d in loops):
+            continue
+        mfma, scratch = (sum(ins[2].startswith(what) for ins in code[a:b + 1]) for what in ("v_mfma", "scratch_"))
+        if mfma and scratch:
+            found.append((code[a][0], mfma, scratch))
+    return found
+
+
 def kernels_of(path, tmp):
     for n, blob in enumerate(code_objects(path, str(tmp))):
         if b"lstm_" not in blob and b"gemm" not in blob:
@@ -144,13 +158,33 @@ def test_the_check_sees_what_it_looks_for():
     assert violations(back)                                                 # round a loop
 
 
-@pytest.mark.skipif(not os.path.exists(OBJDUMP), reason="no disassembler")
-def test_distances_around_the_matrix_instructions(tmp_path):
-    checked = big = 0
-    for fn, code in kernels_of(_lib.LIB_PATH, tmp_path):
-        if not any(ins[5] for ins in code):
-            continue
-        checked += 1
-        big += "_big_kernel" in fn
-        assert not violations(code), (fn, violations(code)[:3])
-    assert checked > 100 and big == 80
+def test_the_scratch_check_sees_what_it_looks_for():
+    def listing(*body):
+        return parse(["0000000000000000 <k>:"] + ["\t%s // %012X: 00000000%s" % (b, 8 * i, t) for i, (b, t) in enumerate(body)])["k"]
+
+    mfma = ("v_mfma_f32_16x16x32_f16 v[0:3], a[0:3], v[8:11], v[0:3]", "")
+    load, back = ("scratch_load_dwordx4 v[0:3], off, off", ""), ("s_cbranch_scc1 65530", " <k+0x8>")
+    assert scratch_in_matrix_loops(listing(load, mfma, load, back)) == [(8, 1, 1)]
+    assert not scratch_in_matrix_loops(listing(load, mfma, back, load))
+
+
+@pytest.fixture(scope="module")
+def built(tmp_path_factory):
+    """(kernel, wait states broken, scratch accesses in its matrix loops) of every kernel with MFMAs."""
+    if not os.path.exists(OBJDUMP):
+        pytest.skip("no disassembler")
+    return [(fn, violations(code), scratch_in_matrix_loops(code))
+            for fn, code in kernels_of(_lib.LIB_PATH, tmp_path_factory.mktemp("code")) if any(ins[2].startswith("v_mfma") for ins in code)]
+
+
+def test_distances_around_the_matrix_instructions(built):
+    assert sum("_big_kernel" in fn for fn, _, _ in built) == 80 and len(built) > 100
+    for fn, broken, _ in built:
+        assert not broken, (fn, broken[:3])
+
+
+def test_matrix_loops_stay_out_of_scratch(built):
+    """Accumulators moved to scratch and back in every pass of a k loop: the reverse launch with weight gradients took four
+    times as long at 256 <= H <= 512.  (The step loops hold no loop inside and are innermost ones too.)"""
+    spilling = [(fn, s) for fn, _, s in built if s]
+    assert not spilling, spilling
