@@ -308,7 +308,7 @@ struct XcdCfg {
 };
 
 // The XCD-local kernels apply when the device deals workgroups to XCDs in turn, the shape fits
-// and the workspace holds a ring with one slot per exchanged version.
+// and the workspace holds kXchgSlots exchange slots.
 // `launch_rows`: batch rows of this launch (0: all B_all of them).
 // copies > 1: that many recurrences of this shape share the launch, so the unit tile has to leave room for all their
 // groups.
@@ -1878,10 +1878,10 @@ int fastlstm_fwd_layer_noalloc(const void *x, const void *Wx, const void *bx, co
     fastlstm_plan pl;
     if (int rc = plan_device(-1, B, H, dtype, 0, &pl, false)) return rc;
     // the smallest workspace of this shape has to fit; beyond that the call uses as much of the array
-    // as a ring with one slot per timestep would take (more slots = the faster kernels, as with any workspace)
+    // as the faster kernels of this shape take, as with any workspace
     if (pl.ws_bytes > kNoAllocScratchBytes) return FASTLSTM_ERR_WORKSPACE;
-    const size_t ring = fastlstm_recurrent_workspace_bytes(&pl, T, H, dtype, 0);
-    const size_t use = std::min(kNoAllocScratchBytes, std::max(ring, pl.ws_bytes));
+    const size_t full = fastlstm_recurrent_workspace_bytes(&pl, T, H, dtype, 0);
+    const size_t use = std::min(kNoAllocScratchBytes, std::max(full, pl.ws_bytes));
     unsigned char *ptr = nullptr;
     if (int rc = scratch_of_current_device(&ptr)) return rc;
     // the array keeps the last call's contents: clear what this call needs zeroed (a fill kernel, so the

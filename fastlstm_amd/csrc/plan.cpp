@@ -62,11 +62,11 @@ int bwd_lds_bytes(int H, int dtype, int ht, int bt, int split, bool sync) {
 }
 
 // Workspace layout: header (1 KiB) | L2 barrier counters (64 KiB) | flags of every batch chunk |
-// exchange ring of every chunk.  Without a cross-CU barrier: the header only.
+// exchange slots of every chunk.  Without a cross-CU barrier: the header only.
 size_t recurrent_flags_bytes(int n_bt, int n_ht) {
     return align_up((size_t)n_bt * align_up((size_t)n_ht, 64) * sizeof(int), 1024);
 }
-// One ring slot = the exchange data of one timestep of one launch.
+// One slot = the exchange data of one timestep of one launch.
 size_t recurrent_slot_bytes(int H, int dtype, int bt, int n_bt, bool backward) {
     const int KS = backward ? cdiv(4 * H, kstep_of(dtype)) : cdiv(H, kstep_of(dtype));
     return (size_t)n_bt * (bt / 16) * KS * kFragBytes;
@@ -224,7 +224,7 @@ extern "C" size_t fastlstm_recurrent_workspace_bytes(const fastlstm_plan *plan, 
     const size_t slot = recurrent_slot_bytes(H, dtype, plan->bt, plan->n_btiles, backward != 0);
     const int slots = kXchgSlots;   // whatever T is
     size_t ws = plan->ws_bytes;
-    // the XCD-local kernels lay their ring out for batch tiles of 16 or 32 rows, which covers at most
+    // the XCD-local kernels lay their slots out for batch tiles of 16 or 32 rows, which covers at most
     // 16 rows (one operand block per k-step) more than the tiles of the plan
     // (the kernels for H = 1280 ... 2048 use tiles of 64 rows: at most 48 rows more)
     const int KS = cdiv(backward ? 4 * H : H, kstep_of(dtype));

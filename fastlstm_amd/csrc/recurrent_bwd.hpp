@@ -394,7 +394,7 @@ __global__ __launch_bounds__((bwd_threads<SPLIT, VIO, CW>())) void lstm_bwd_pers
         prefetch(3, std::integral_constant<int, 3>{});
     }
 
-    int slot = 0;  // ring slot of this step's d_ifgo
+    int slot = 0;  // exchange slot of this step's d_ifgo
     // One hidden tile per workgroup: the lane's UPL units of the current step's tile rows (4 gates,
     // c_{t-1}, dout), read a step ahead
     using NxV = typename VecBytes<(SPLIT == 2 ? NI : 4) * E::BYTES>::type;

@@ -1,11 +1,13 @@
 // Persistent reverse-time kernel for hidden sizes whose W_h does not fit the CUs of one XCD
-// (H = 1536, 2048 with 16-bit elements): the counterpart of lstm_fwd_wide_kernel.  Same mathematics
-// and results as lstm_bwd_persistent_kernel (which replaces fastlstm/kernels.py:1201-1409).
+// (H = 640 ... 1024 in fp32, 1280 ... 2048 with 16-bit elements): the counterpart of lstm_fwd_wide_kernel.  Same mathematics
+// and results as lstm_bwd_persistent_kernel (which replaces fastlstm/kernels.py:1201-1409).  In 16 bits lstm_bwd_big_kernel is
+// faster at every size (us per step, here and there: H = 2048, 128 rows 11.0, 8.6; 32 rows 6.4, 5.3; a pair of H = 2048, B = 32
+// 9.8, 6.5); this form remains for calls whose workspace has no room for the partial sums of its teams.
 //
 // A workgroup of 8 waves owns 16 hidden units and up to 64 batch rows and keeps Wh[:, units]^T (K = 4H
 // rows of (unit, gate) pairs, 256 KiB for H = 2048) in registers: the waves split K eight ways.
 // A barrier group has H / 16 workgroups on xpg = H / 512 whole XCDs (placement, flags and exchange
-// ring as in the forward kernel).  Per step every workgroup has to read the d_ifgo[t] of its group,
+// slots as in the forward kernel).  Per step every workgroup has to read the d_ifgo[t] of its group,
 // 64 rows x 4H (1 MiB for H = 2048): the step is bound by that stream.  Registers cannot hold enough
 // of it in flight next to the weights, so the operand blocks travel L2 -> LDS with LDS-direct loads
 // into a ring of kRing blocks per wave (nobody else touches a wave's ring: no workgroup barrier, the

@@ -12,13 +12,9 @@
 // flags are polled with device-scope loads.  That keeps the per-step critical path free
 // of whole-L2 write-backs and invalidates: a producer drains its own exchange stores
 // (s_waitcnt vmcnt(0)), the workgroup meets at a barrier, one thread raises the flag.
-// The exchange DATA is read in one of two ways:
-//  * history ring (default): every timestep writes a fresh slot of the exchange buffer, so
-//    no cache can hold a stale copy of an address before its only write; consumers use
-//    ordinary cached loads and the 32 CUs of an XCD share one fetch through their L2
-//    (the data crosses the fabric once per XCD instead of once per CU);
-//  * coherent loads (sc1, miss the non-coherent cache levels): used when the workspace is
-//    too small for T+1 slots, or when two workgroups write parts of the same 128-byte line.
+// The exchange data lies in two slots that are written in turn and is read with coherent loads (sc1, past the
+// non-coherent cache levels): a member writes a slot again only behind the flags of the step in between, which every
+// reader raised after reading.  (The XCD-local kernels keep data and synchronisation in one XCD's L2: recurrent_fwd_xcd.hpp.)
 // Every wait is bounded: after `spin_limit` ticks of the 100 MHz clock it raises an
 // abort flag in the workspace header that ends every other wait as well, so the grid
 // always drains.

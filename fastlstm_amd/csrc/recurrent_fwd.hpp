@@ -463,7 +463,7 @@ __global__ __launch_bounds__((fwd_threads<SPLIT, VIO, CW>())) void lstm_fwd_pers
         prefetch(3, std::integral_constant<int, 3>{});
     }
 
-    int slot_r = 0;  // ring slot that holds h_{t-1}
+    int slot_r = 0;  // exchange slot that holds h_{t-1}
     if constexpr (IOW) __syncthreads();   // the gates tile of step 0 is in LDS (every later one is moved a step ahead)
     // One timestep; u = t % PD selects the prefetch ring entry at compile time.
     auto step = [&](const int t, auto uc) __attribute__((always_inline)) {

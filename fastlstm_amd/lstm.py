@@ -132,8 +132,8 @@ def _plan_cached(idx, B, H, code, backward):
 def _workspace(plan, T, H, code, backward, device):
     """Recurrence workspace, with the part the kernels need zeroed (header, counters, flags; everything
     when the exchange blocks have padding).  Its size does not depend on T: every kernel exchanges
-    h_t / d_ifgo[t] through two slots (a few hundred KiB; plans that stream W_h add one packed copy of it,
-    which the call itself writes)."""
+    h_t / d_ifgo[t] through two or four slots (up to a few MiB; plans that stream W_h add one packed copy of it,
+    which the call itself writes, and the 16-bit reverse pass from H = 1280 on 8 MiB for partial sums)."""
     n = _lib.load().fastlstm_recurrent_workspace_bytes(plan, T, H, code, 1 if backward else 0)
     ws = torch.empty(n, dtype=torch.uint8, device=device)
     ws[:(n if plan.ring_needs_zero else min(n, plan.ws_zero_bytes))].zero_()

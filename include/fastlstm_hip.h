@@ -213,7 +213,7 @@ int fastlstm_fwd_stack2_infer(const void *x, const void *Wx0, const void *bx0, c
  * layers run in ONE launch: the idle workgroups compute both input projections, the second one
  * chunk by chunk behind the first layer's recurrence, and the second layer's recurrence follows a
  * chunk of timesteps behind the first -- the wall time of one layer instead of two.  Otherwise the
- * layers run one after the other.  ws: fastlstm_stack2_workspace_bytes (ring slots for both layers),
+ * layers run one after the other.  ws: fastlstm_stack2_workspace_bytes (exchange slots for both layers),
  * zeroed like any recurrent workspace.  Replaces two iterations of the layer loop at
  * fastlstm/lstm.py:685-696 (which the reference runs strictly one after the other, README.md:94). */
 int fastlstm_fwd_stack2(const void *x, const void *Wx0, const void *bx0, const void *bh0, const void *Wh0,
@@ -351,7 +351,7 @@ int fastlstm_bwd_stack2_fused(int T, int B, int I, int H, int dtype, size_t ws_b
 /* Which kernel fastlstm_fwd_persistent (backward = 0) / fastlstm_bwd_persistent (1) will launch on
  * the current device for this shape and a workspace of ws_bytes: 0 = the general kernel
  * (exchange through device memory), 1 = the XCD-local kernel (barrier group on one XCD,
- * exchange through its L2; needs the ring workspace of fastlstm_recurrent_workspace_bytes and a
+ * exchange through its L2; needs the workspace of fastlstm_recurrent_workspace_bytes and a
  * device that fastlstm_plan_device has probed; a batch with more tiles than one launch holds runs as
  * several launches over ranges of rows), 2 = the register-resident kernel for H = 1280, 1536, 1792,
  * 2048 with 16-bit elements (barrier groups of H / 16 workgroups over several XCDs, 64 batch rows

@@ -1,14 +1,14 @@
-"""BASELINE.json's long configurations at their FULL sequence length against the fp32 CPU oracle
+"""The benchmark's long workloads at their FULL sequence length against the fp32 CPU oracle
 (run with -m gpu on an MI355X).
 
 Config B (fp16, B=64, T=512, I=H=1024: forward and backward) is the headline configuration.  Config C
 (bf16, B=128, T=256, I=H=2048) and config E (fp16, two stacked layers, B=32, T=2048,
-I=H=1024) are the two configurations whose time-dependent host code (exchange ring sizes, chunk
+I=H=1024) are the two configurations whose time-dependent host code (chunk sizes, chunk
 hand-over between the stacked layers, which kernel a workspace size selects) only shows at the real
 T.  The 16-bit GPU results are compared with the oracle evaluated in fp32 WITHOUT any 16-bit
 rounding on the same (16-bit representable) inputs and weights: the tolerance therefore bounds the
 error growth of the 16-bit path over all T steps, 2e-2 of the reference's largest magnitude for
-every output and gradient (north star: <= 2e-2 relative in fp16/bf16 with fp32 accumulation).
+every output and gradient (bar: <= 2e-2 relative in fp16/bf16 with fp32 accumulation).
 The oracle needs about half a minute per configuration on the box's 16 host cores.
 """
 import numpy as np

@@ -1,7 +1,7 @@
 """GPU parity tests (run with -m gpu on an MI355X).  Everything goes through the C ABI
 of libfastlstm_hip.so via the Python mirror of the reference's interface.
 
-Tolerances (north star): fp32 rtol = atol = 1e-4 against torch.nn.LSTM with identical
+Tolerances: fp32 rtol = atol = 1e-4 against torch.nn.LSTM with identical
 weights; fp16/bf16 <= 2e-2 relative (error max-norm / reference max-norm) against an
 fp32/fp64 evaluation with the same 16-bit-rounded weights and inputs.
 """
@@ -1740,7 +1740,7 @@ def test_training_step_replays_from_a_captured_graph(T, B, I, H, layers, dt):
 
 
 # --------------------------------------------------------------------------------------
-# 4. BASELINE.json configurations at their real shapes
+# 4. the benchmark's workloads at their real shapes
 # --------------------------------------------------------------------------------------
 def _module_pair(I, H, layers, dt, seed):
     torch.manual_seed(seed)
