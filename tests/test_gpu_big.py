@@ -101,3 +101,30 @@ def test_pair_of_reverse_recurrences_equals_two_calls(T, B, H, dt, whole):
     for g, w, dg, dw in zip(got, want, d_got, d_want):
         assert torch.equal(dg, dw) and torch.equal(g["dh"], w["dh"]) and torch.equal(g["dc"], w["dc"])
         assert torch.isfinite(dg.float()).all()
+
+
+@pytest.mark.parametrize("B,H", [(1, 1280), (4, 2048), (17, 1536), (3, 2560)])
+def test_rows_past_the_batch_leave_no_trace(B, H):
+    """The reverse kernel computes the gates of rows past the batch on whatever its LDS and the exchange blocks hold: a call behind
+    one that left NaN in both, on a workspace of NaN, is the same bits as one behind zeros."""
+    lib, T, st = _lib.load(), 3, torch.cuda.current_stream().cuda_stream
+    torch.manual_seed(H + B)
+    results = []
+    for fill in (0.0, float("nan")):
+        for rows in (32, B):
+            plan = _lib.Plan()
+            _lib.check(lib.fastlstm_plan_device(0, rows, H, 1, 1, plan), "plan")
+            n = lib.fastlstm_recurrent_workspace_bytes(plan, T, H, 1, 1)
+            ws = torch.full((n,), 0xff if fill != fill else 0, dtype=torch.uint8, device="cuda")
+            ws[:(n if rows == 32 else plan.ws_zero_bytes)] = 0
+            torch.manual_seed(H + rows)
+            dout, dh, dc, ifgo, cell, Wh = (torch.randn(*s, device="cuda").half() * k for s, k in (
+                ((T, rows, H), 1), ((rows, H), 1), ((rows, H), 1), ((T, rows, 4 * H), 1), ((T + 1, rows, H), 1), ((4 * H, H), H ** -.5)))
+            if rows == 32:
+                dout, dh, dc, ifgo, cell = (torch.full_like(t, fill) for t in (dout, dh, dc, ifgo, cell))
+            d = torch.zeros_like(ifgo)
+            _lib.check(lib.fastlstm_bwd_persistent(*(t.data_ptr() for t in (dout, dh, dc, ifgo, cell, d, Wh)), ws.data_ptr(), n, T, rows, H,
+                                                   1, st), "bwd")
+        results.append((d, dh, dc))
+    for clean, dirty in zip(*results):
+        assert torch.isfinite(clean).all() and torch.equal(clean, dirty)
