@@ -103,28 +103,32 @@ def test_pair_of_reverse_recurrences_equals_two_calls(T, B, H, dt, whole):
         assert torch.isfinite(dg.float()).all()
 
 
-@pytest.mark.parametrize("B,H", [(1, 1280), (4, 2048), (17, 1536), (3, 2560)])
-def test_rows_past_the_batch_leave_no_trace(B, H):
-    """The reverse kernel computes the gates of rows past the batch on whatever its LDS and the exchange blocks hold: a call behind
-    one that left NaN in both, on a workspace of NaN, is the same bits as one behind zeros."""
+@pytest.mark.parametrize("B,H,backward", [(1, 1280, True), (4, 2048, True), (17, 1536, True), (3, 2560, True),
+                                          (33, 2048, False), (34, 1280, False), (1, 4096, False)])
+def test_rows_past_the_batch_leave_no_trace(B, H, backward):
+    """The gates of rows past the batch are computed on whatever LDS and the exchange blocks hold: a call behind one that left NaN
+    in both, on a workspace of NaN, is the same bits as one behind zeros."""
     lib, T, st = _lib.load(), 3, torch.cuda.current_stream().cuda_stream
-    torch.manual_seed(H + B)
     results = []
     for fill in (0.0, float("nan")):
-        for rows in (32, B):
+        for rows in (64, B):
             plan = _lib.Plan()
-            _lib.check(lib.fastlstm_plan_device(0, rows, H, 1, 1, plan), "plan")
-            n = lib.fastlstm_recurrent_workspace_bytes(plan, T, H, 1, 1)
+            _lib.check(lib.fastlstm_plan_device(0, rows, H, 1, int(backward), plan), "plan")
+            n = lib.fastlstm_recurrent_workspace_bytes(plan, T, H, 1, int(backward))
             ws = torch.full((n,), 0xff if fill != fill else 0, dtype=torch.uint8, device="cuda")
-            ws[:(n if rows == 32 else plan.ws_zero_bytes)] = 0
+            ws[:(n if rows == 64 else plan.ws_zero_bytes)] = 0
             torch.manual_seed(H + rows)
-            dout, dh, dc, ifgo, cell, Wh = (torch.randn(*s, device="cuda").half() * k for s, k in (
-                ((T, rows, H), 1), ((rows, H), 1), ((rows, H), 1), ((T, rows, 4 * H), 1), ((T + 1, rows, H), 1), ((4 * H, H), H ** -.5)))
-            if rows == 32:
-                dout, dh, dc, ifgo, cell = (torch.full_like(t, fill) for t in (dout, dh, dc, ifgo, cell))
-            d = torch.zeros_like(ifgo)
-            _lib.check(lib.fastlstm_bwd_persistent(*(t.data_ptr() for t in (dout, dh, dc, ifgo, cell, d, Wh)), ws.data_ptr(), n, T, rows, H,
-                                                   1, st), "bwd")
-        results.append((d, dh, dc))
+            draw = lambda *shape: torch.full(shape, fill, device="cuda").half() if rows == 64 else torch.randn(*shape, device="cuda").half()
+            Wh = (torch.randn(4 * H, H, device="cuda") * H ** -.5).half()
+            ifgo, cell = draw(T, rows, 4 * H), draw(T + 1, rows, H)
+            if backward:
+                d = torch.zeros_like(ifgo)
+                moved = [draw(T, rows, H), draw(rows, H), draw(rows, H), ifgo, cell, d, Wh]
+                entry, got = lib.fastlstm_bwd_persistent, moved[1:3] + [d]
+            else:
+                moved = [ifgo, draw(T + 1, rows, H), cell, Wh]
+                entry, got = lib.fastlstm_fwd_persistent, moved[:3]
+            _lib.check(entry(*(t.data_ptr() for t in moved), ws.data_ptr(), n, T, rows, H, 1, st), "recurrence")
+        results.append(got)
     for clean, dirty in zip(*results):
         assert torch.isfinite(clean).all() and torch.equal(clean, dirty)
