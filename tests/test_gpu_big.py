@@ -104,7 +104,8 @@ def test_pair_of_reverse_recurrences_equals_two_calls(T, B, H, dt, whole):
 
 
 @pytest.mark.parametrize("B,H,backward", [(1, 1280, True), (4, 2048, True), (17, 1536, True), (3, 2560, True),
-                                          (33, 2048, False), (34, 1280, False), (1, 4096, False)])
+                                          (33, 2048, False), (34, 1280, False), (1, 4096, False),
+                                          (2, 1280, False), (17, 2048, False)])   # the last two: the 16-unit form
 def test_rows_past_the_batch_leave_no_trace(B, H, backward):
     """The gates of rows past the batch are computed on whatever LDS and the exchange blocks hold: a call behind one that left NaN
     in both, on a workspace of NaN, is the same bits as one behind zeros."""
