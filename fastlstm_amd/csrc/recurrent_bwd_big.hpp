@@ -189,11 +189,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
         const unsigned xs = (unsigned)(s & 1) * xslot;
 
         // ---- point-wise gate backward of this lane's cells --------------------------
-        // (Rows past the batch too, on whatever their LDS rows hold; nothing of them is stored outside.  With at most 4 of 16
-        // lanes active this passage takes some CUs two to three times as long, and the group waits for the slowest: so does
-        // a bare chain of v_exp and v_rcp behind a wait, 860 cycles with 16 lanes of 16, up to 2700 with one.  us per step with
-        // them masked and here: H = 1280, 4 rows 5.6 -> 4.5, H = 2048 6.5 -> 5.2; 5 ... 16 rows no difference.)
-        if (mine) {
+        // (Rows past the batch too, unless the tile holds nothing else, on whatever their LDS rows hold; nothing of them is stored
+        // outside.  With at most 4 of 16 lanes active this passage takes some CUs two to three times as long, and the group waits
+        // for the slowest: so does a bare chain of v_exp and v_rcp behind a wait, 860 cycles with 16 lanes of 16, up to 2700 with
+        // one.  us per step with them masked and here: H = 1280, 4 rows 5.6 -> 4.5, H = 2048 6.5 -> 5.2; 5 ... 16 rows no difference.)
+        if (mine && b0 + ci * 16 < B) {
             u32x2 d[4];   // [gate]: the four units
             const unsigned char *gl_ = tiles + goff;
             const f32x4 pi = halves(*reinterpret_cast<const u32x2 *>(gl_)), pf = halves(*reinterpret_cast<const u32x2 *>(gl_ + GSEG));

@@ -252,6 +252,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
                     for (int pp = 1; pp < NWV; ++pp) s += red[(pp * ST + tl) * kWave + lane];
                     // (Rows past the batch too, see lstm_bwd_big_kernel; nothing of them leaves the workgroup.  us per step with
                     // them masked and here: H = 2048, 33 rows in groups of 16 5.5 -> 3.9, H = 1280 4.3 -> 3.3, H = 4096, 1 row 5.1 -> 4.6.)
+                    if (b0 + i * 16 >= B) continue;
                     T *gl_ = reinterpret_cast<T *>(tiles + i * 16 * GROW + goff) + h * NWV * 4;
                     const float pi = E::to_f32(gl_[0]) + s[0];
                     const float pf = E::to_f32(gl_[HT]) + s[1];

@@ -243,7 +243,7 @@ __global__ __launch_bounds__(kWave * 8) void lstm_fwd_wide_kernel(const FwdXcdPa
             // (16 bits: rows past the batch too, see lstm_bwd_big_kernel; nothing of them leaves the workgroup.  us per step with
             // them masked and here: H = 1280, 1 row 3.9 -> 3.0, H = 2048, 2 rows 4.2 -> 3.4, 17 rows 4.4 -> 3.6.  In fp32 few rows
             // cost nothing, and a training step of H = 1024, T = 128, B = 64 took 3.36 ms without the mask, 3.34 with it.)
-            if (E::BYTES == 2 || valid[m]) {
+            if (E::BYTES == 2 ? b0 + tile % NT * 16 < B : valid[m]) {
                 T *gl_ = reinterpret_cast<T *>(gt + goff[m]);   // the item's 4 gates in the LDS tile
                 const float pi = E::to_f32(gl_[0]) + s[0];
                 const float pf = E::to_f32(gl_[HT]) + s[1];
