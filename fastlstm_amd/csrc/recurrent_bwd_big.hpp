@@ -101,6 +101,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
     const int ut = wave % UT, ci = wave / UT;
     const int b = b0 + ci * 16 + n;
     const bool mine = ci < NT, valid = mine && b < B;
+    // (H > 2048: few rows cost nothing, and the other bound 0.6 % of a step with 64 rows)
+    const bool live = mine && ci * 16 + n < (UT > 1 ? rows_computed(B - b0) : B - b0);
     const size_t off_h = valid ? (size_t)b * H + u0 + 16 * ut + 4 * q : (size_t)b0 * H + u0;
     f32x4 dc_state = {0.f, 0.f, 0.f, 0.f}, dh_rec = {0.f, 0.f, 0.f, 0.f};
     u32x2 c1v = {0u, 0u};   // cell[t + 1] of the four units
@@ -189,42 +191,40 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
         const unsigned xs = (unsigned)(s & 1) * xslot;
 
         // ---- point-wise gate backward of this lane's cells --------------------------
-        // (Rows past the batch too, unless the tile holds nothing else, on whatever their LDS rows hold; nothing of them is stored
-        // outside.  With at most 4 of 16 lanes active this passage takes some CUs two to three times as long, and the group waits
-        // for the slowest: so does a bare chain of v_exp and v_rcp behind a wait, 860 cycles with 16 lanes of 16, up to 2700 with
-        // one.  us per step with them masked and here: H = 1280, 4 rows 5.6 -> 4.5, H = 2048 6.5 -> 5.2; 5 ... 16 rows no difference.)
-        if (mine && b0 + ci * 16 < B) {
-            u32x2 d[4];   // [gate]: the four units
-            const unsigned char *gl_ = tiles + goff;
-            const f32x4 pi = halves(*reinterpret_cast<const u32x2 *>(gl_)), pf = halves(*reinterpret_cast<const u32x2 *>(gl_ + GSEG));
-            const f32x4 pg = halves(*reinterpret_cast<const u32x2 *>(gl_ + 2 * GSEG)), po = halves(*reinterpret_cast<const u32x2 *>(gl_ + 3 * GSEG));
-            const u32x2 c0v = *reinterpret_cast<const u32x2 *>(stc + soff);
-            const f32x4 c0 = halves(c0v), c1 = halves(c1v), dh = dh_rec + halves(*reinterpret_cast<const u32x2 *>(std_ + soff));
-            f32x4 di, df, dg, do_;
+        if (mine) {
+            u32x2 d[4] = {};   // [gate]: the four units
+            if (live) {   // (us per step with rows past the batch masked and so: 4 rows, H = 1280 5.6 -> 4.5, H = 2048 6.5 -> 5.2)
+                const unsigned char *gl_ = tiles + goff;
+                const f32x4 pi = halves(*reinterpret_cast<const u32x2 *>(gl_)), pf = halves(*reinterpret_cast<const u32x2 *>(gl_ + GSEG));
+                const f32x4 pg = halves(*reinterpret_cast<const u32x2 *>(gl_ + 2 * GSEG)), po = halves(*reinterpret_cast<const u32x2 *>(gl_ + 3 * GSEG));
+                const u32x2 c0v = *reinterpret_cast<const u32x2 *>(stc + soff);
+                const f32x4 c0 = halves(c0v), c1 = halves(c1v), dh = dh_rec + halves(*reinterpret_cast<const u32x2 *>(std_ + soff));
+                f32x4 di, df, dg, do_;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float si = sigmoidf_<false>(pi[e]), sf = sigmoidf_<false>(pf[e]), tg = tanhf_<false>(pg[e]), so = sigmoidf_<false>(po[e]);
-                const float tc = tanhf_<false>(c1[e]);
-                const float dc1 = dc_state[e] + dh[e] * so * (1.f - tc * tc);
-                do_[e] = dh[e] * tc * so * (1.f - so);
-                df[e] = dc1 * c0[e] * sf * (1.f - sf);
-                di[e] = dc1 * tg * si * (1.f - si);
-                dg[e] = dc1 * si * (1.f - tg * tg);
-                dc_state[e] = dc1 * sf;
-            }
-            c1v = c0v;   // c_{t-1} is the next step's c_t
-            d[0] = packed(di);
-            d[1] = packed(df);
-            d[2] = packed(dg);
-            d[3] = packed(do_);
+                for (int e = 0; e < 4; ++e) {
+                    const float si = sigmoidf_<false>(pi[e]), sf = sigmoidf_<false>(pf[e]), tg = tanhf_<false>(pg[e]), so = sigmoidf_<false>(po[e]);
+                    const float tc = tanhf_<false>(c1[e]);
+                    const float dc1 = dc_state[e] + dh[e] * so * (1.f - tc * tc);
+                    do_[e] = dh[e] * tc * so * (1.f - so);
+                    df[e] = dc1 * c0[e] * sf * (1.f - sf);
+                    di[e] = dc1 * tg * si * (1.f - si);
+                    dg[e] = dc1 * si * (1.f - tg * tg);
+                    dc_state[e] = dc1 * sf;
+                }
+                c1v = c0v;   // c_{t-1} is the next step's c_t
+                d[0] = packed(di);
+                d[1] = packed(df);
+                d[2] = packed(dg);
+                d[3] = packed(do_);
 #pragma unroll
-            for (int gt = 0; gt < 4; ++gt) *reinterpret_cast<u32x2 *>(tiles + goff + gt * GSEG) = d[gt];
-            // exchange copy: k = (unit, gate 0..3): 16 consecutive k of the lane, 8 per operand-block lane
+                for (int gt = 0; gt < 4; ++gt) *reinterpret_cast<u32x2 *>(tiles + goff + gt * GSEG) = d[gt];
+                // exchange copy: k = (unit, gate 0..3): 16 consecutive k of the lane, 8 per operand-block lane
 #pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const unsigned if0 = __builtin_amdgcn_perm(d[1][h], d[0][h], 0x05040100u), if1 = __builtin_amdgcn_perm(d[1][h], d[0][h], 0x07060302u);
-                const unsigned go0 = __builtin_amdgcn_perm(d[3][h], d[2][h], 0x05040100u), go1 = __builtin_amdgcn_perm(d[3][h], d[2][h], 0x07060302u);
-                if (valid) xch.store16(xs + x_off + h * 256u, u32x4{if0, go0, if1, go1});
+                for (int h = 0; h < 2; ++h) {
+                    const unsigned if0 = __builtin_amdgcn_perm(d[1][h], d[0][h], 0x05040100u), if1 = __builtin_amdgcn_perm(d[1][h], d[0][h], 0x07060302u);
+                    const unsigned go0 = __builtin_amdgcn_perm(d[3][h], d[2][h], 0x05040100u), go1 = __builtin_amdgcn_perm(d[3][h], d[2][h], 0x07060302u);
+                    xch.store16(xs + x_off + h * 256u, u32x4{if0, go0, if1, go1});
+                }
             }
         }
         publish_version(grp_flags + j, s + 1);   // waits for the stores, workgroup barrier, raises the flag

@@ -126,9 +126,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
 
     // ---- this lane's cells: unit tiles wave + 4 h, row 16 i + n of batch tile i -------------
     float c_state[NT][TPW];
+    bool live[NT];
 #pragma unroll
     for (int i = 0; i < NT; ++i) {
         const int b = b0 + i * 16 + n;
+        live[i] = i * 16 + n < rows_computed(B - b0);
 #pragma unroll
         for (int h = 0; h < TPW; ++h)
             c_state[i][h] = b < B ? E::to_f32(cell[(size_t)b * H + u0 + (wave + NWV * h) * 4 + q]) : 0.f;
@@ -250,25 +252,24 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))
                     f32x4 s = red[tl * kWave + lane];
 #pragma unroll
                     for (int pp = 1; pp < NWV; ++pp) s += red[(pp * ST + tl) * kWave + lane];
-                    // (Rows past the batch too, see lstm_bwd_big_kernel; nothing of them leaves the workgroup.  us per step with
-                    // them masked and here: H = 2048, 33 rows in groups of 16 5.5 -> 3.9, H = 1280 4.3 -> 3.3, H = 4096, 1 row 5.1 -> 4.6.)
-                    if (b0 + i * 16 >= B) continue;
-                    T *gl_ = reinterpret_cast<T *>(tiles + i * 16 * GROW + goff) + h * NWV * 4;
-                    const float pi = E::to_f32(gl_[0]) + s[0];
-                    const float pf = E::to_f32(gl_[HT]) + s[1];
-                    const float pg = E::to_f32(gl_[2 * HT]) + s[2];
-                    const float po = E::to_f32(gl_[3 * HT]) + s[3];
-                    const float c1 = sigmoidf_<false>(pf) * c_state[i][h] + sigmoidf_<false>(pi) * tanhf_<false>(pg);
-                    const float h1 = sigmoidf_<false>(po) * tanhf_<false>(c1);
-                    c_state[i][h] = c1;
-                    if (keep) {
-                        gl_[0] = E::from_f32(pi);
-                        gl_[HT] = E::from_f32(pf);
-                        gl_[2 * HT] = E::from_f32(pg);
-                        gl_[3 * HT] = E::from_f32(po);
+                    if (live[i]) {   // (us per step with rows past the batch masked and so: H = 2048, 33 rows 5.5 -> 3.9, H = 4096, 1 row 5.1 -> 4.6)
+                        T *gl_ = reinterpret_cast<T *>(tiles + i * 16 * GROW + goff) + h * NWV * 4;
+                        const float pi = E::to_f32(gl_[0]) + s[0];
+                        const float pf = E::to_f32(gl_[HT]) + s[1];
+                        const float pg = E::to_f32(gl_[2 * HT]) + s[2];
+                        const float po = E::to_f32(gl_[3 * HT]) + s[3];
+                        const float c1 = sigmoidf_<false>(pf) * c_state[i][h] + sigmoidf_<false>(pi) * tanhf_<false>(pg);
+                        const float h1 = sigmoidf_<false>(po) * tanhf_<false>(c1);
+                        c_state[i][h] = c1;
+                        if (keep) {
+                            gl_[0] = E::from_f32(pi);
+                            gl_[HT] = E::from_f32(pf);
+                            gl_[2 * HT] = E::from_f32(pg);
+                            gl_[3 * HT] = E::from_f32(po);
+                        }
+                        *(reinterpret_cast<T *>(sth + i * 16 * SROW + soff) + h * NWV * 4) = E::from_f32(h1);
+                        *(reinterpret_cast<T *>(stc + i * 16 * SROW + soff) + h * NWV * 4) = E::from_f32(c1);
                     }
-                    *(reinterpret_cast<T *>(sth + i * 16 * SROW + soff) + h * NWV * 4) = E::from_f32(h1);
-                    *(reinterpret_cast<T *>(stc + i * 16 * SROW + soff) + h * NWV * 4) = E::from_f32(c1);
                 }
                 __syncthreads();   // `red` is read; behind the last tile: the state tiles are complete
             }

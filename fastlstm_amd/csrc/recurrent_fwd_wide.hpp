@@ -96,13 +96,14 @@ __global__ __launch_bounds__(kWave * 8) void lstm_fwd_wide_kernel(const FwdXcdPa
     float c_state[IPT];
     size_t off_h[IPT];
     int xoff[IPT], goff[IPT], soff[IPT];   // xoff: prologue only
-    bool valid[IPT];
+    bool valid[IPT], live[IPT];
 #pragma unroll
     for (int m = 0; m < IPT; ++m) {
         const int tile = wave + NWV * m;
         const int mt = tile / NT, nt = tile % NT;
         const int unit = u0 + mt * 4 + q, b = b0 + nt * 16 + n;
         valid[m] = tile < TILES && b < B;
+        live[m] = tile < TILES && (E::BYTES == 2 ? nt * 16 + n < rows_computed(B - b0) : b < B);   // (fp32: few rows cost nothing)
         off_h[m] = valid[m] ? (size_t)b * H + unit : (size_t)b0 * H + u0;
         xoff[m] = nt * KS * kFragBytes + frag_offset<T>(n, unit);
         goff[m] = (nt * 16 + n) * GROW + (mt * 4 + q) * E::BYTES;
@@ -240,10 +241,7 @@ __global__ __launch_bounds__(kWave * 8) void lstm_fwd_wide_kernel(const FwdXcdPa
             f32x4 s = red[tile * kWave + lane];
 #pragma unroll
             for (int pp = 1; pp < NWV; ++pp) s += red[(pp * TILES + tile) * kWave + lane];
-            // (16 bits: rows past the batch too, see lstm_bwd_big_kernel; nothing of them leaves the workgroup.  us per step with
-            // them masked and here: H = 1280, 1 row 3.9 -> 3.0, H = 2048, 2 rows 4.2 -> 3.4, 17 rows 4.4 -> 3.6.  In fp32 few rows
-            // cost nothing, and a training step of H = 1024, T = 128, B = 64 took 3.36 ms without the mask, 3.34 with it.)
-            if (E::BYTES == 2 ? b0 + tile % NT * 16 < B : valid[m]) {
+            if (live[m]) {   // (us per step with rows past the batch masked and so: H = 1280, 1 row 3.9 -> 3.0, H = 2048, 2 rows 4.2 -> 3.4)
                 T *gl_ = reinterpret_cast<T *>(gt + goff[m]);   // the item's 4 gates in the LDS tile
                 const float pi = E::to_f32(gl_[0]) + s[0];
                 const float pf = E::to_f32(gl_[HT]) + s[1];
