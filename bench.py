@@ -558,7 +558,7 @@ def main():
         el = oracle_run(ts)
         res["cpu_oracle"] = {"value": round(B * ts / el, 1), "unit": "batch*timesteps/s",
                              "threads": int(os.environ.get("OMP_NUM_THREADS", os.cpu_count() or 1)),
-                             "sample": "C/OpenMP fp32 oracle (the parity checker), layer 0, first %d of %d timesteps, %s; "
+                             "sample": "C/OpenMP fp32 oracle of the parity tests, layer 0, first %d of %d timesteps, %s; "
                                        "one pass of %.1f s" % (ts, T, mode, el)}
 
     print(json.dumps(res))

@@ -98,7 +98,7 @@ void FN(oracle_lstm_fwd)(int T, int B, int I, int H, const REAL *x, const REAL *
  * is also what the recurrent product and the weight-gradient sums consume).
  * The carried dc and dh_rec stay unrounded (the reference's default kernel
  * rounds them through 16-bit buffers every step, kernels.py:1337-1342,
- * 1388-1390; the HIP path keeps them in fp32 registers, so the checker does too).
+ * 1388-1390; the HIP path keeps them in fp32 registers, so the oracle does too).
  */
 void FN(oracle_lstm_bwd)(int T, int B, int I, int H, const REAL *dout, const REAL *dh_n,
                          const REAL *dc_n, const REAL *x, const REAL *out, const REAL *cell,
