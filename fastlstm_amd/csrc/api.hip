@@ -1066,11 +1066,13 @@ static int gemm_dx_impl(const void *d_ifgo, const void *Wx, void *dx, int T, int
     int tile, splits;
     gemm_plan(dtype, p.M, p.N, p.K, p.lda, p.ldb, false, true, scratch != nullptr, &tile, &splits);
     if (splits > 1) {
-        const int bk = tile ? 64 : gemm_bk(dtype);
+        const int bk = tile ? 64 : gemm_bk();
         const int kps = cdiv(cdiv(p.K, splits), bk) * bk;
         splits = cdiv(p.K, kps);
         if (splits > 1 && (size_t)splits * p.M * p.N * sizeof(float) <= scratch_bytes) {
             p.splits = splits; p.k_per_split = kps; p.Cpart = static_cast<float *>(scratch);
+        } else {
+            gemm_plan(dtype, p.M, p.N, p.K, p.lda, p.ldb, false, true, false, &tile, &splits);
         }
     }
     return launch_gemm_tiled(dtype, p, false, true, tile, static_cast<hipStream_t>(stream)) == hipSuccess
@@ -1099,7 +1101,7 @@ int fastlstm_gemm_dx_split(const void *d_ifgo, const void *Wx, void *dx, int T, 
 // tile and split-K factor of a weight-gradient product C[M,N] = A^T.B with reduction length K
 static void wgrad_plan(int M, int N, int K, int dtype, int *tile, int *splits, int *k_per_split) {
     gemm_plan(dtype, M, N, K, M, N, true, true, true, tile, splits);
-    const int bk = *tile ? 64 : gemm_bk(dtype);
+    const int bk = *tile ? 64 : gemm_bk();
     *k_per_split = cdiv(cdiv(K, *splits), bk) * bk;
     *splits = cdiv(K, *k_per_split);
 }
@@ -1114,7 +1116,13 @@ size_t fastlstm_wgrad_workspace_bytes(int T, int B, int I, int H, int dtype) {
     size_t part = std::max(sx > 1 ? (size_t)sx * M * I : 0, sh > 1 ? (size_t)sh * M * H : 0) * sizeof(float);
     size_t cs = (size_t)colsum_chunks(K) * M * sizeof(float);
     const size_t small = small_bwd_eligible(dtype, K, I, H) ? small_bwd_workspace(K, I, H) : 0;
-    return std::max(std::max(align_up(cs, 256) + align_up(part, 256), wgrad_merged_workspace(dtype, M, I, H, K)), small) + 256;
+    size_t dx = 0;   // fp32: room for dx's parts (its sums over K are meant to be short, gemm_f32_plan)
+    if (dtype == FASTLSTM_FP32) {
+        int dx_tile, dx_splits;
+        gemm_plan(dtype, K, I, M, M, I, false, true, true, &dx_tile, &dx_splits);
+        dx = dx_splits > 1 ? (size_t)dx_splits * K * I * sizeof(float) : 0;
+    }
+    return std::max({align_up(cs, 256) + align_up(part, 256), wgrad_merged_workspace(dtype, M, I, H, K), small, dx}) + 256;
 }
 
 int fastlstm_gemm_wgrad(const void *d_ifgo, const void *x, const void *h, void *dWx, void *dWh, void *db,

@@ -1,12 +1,23 @@
 // Host launchers for the MFMA GEMM stages (K1, K5, K8, K9) and the db column sum.
 #include "gemm.hpp"
 #include "gemm16.hpp"
+#include "gemm_f32.hpp"
 #include <atomic>
 #include "internal.hpp"
 
 namespace fastlstm {
 
 namespace {
+
+// C = the sum over the parts of a split product
+template <typename T> hipError_t launch_splitk_reduce(const GemmParams &p, hipStream_t stream) {
+    const size_t total = (size_t)p.M * p.N;
+    const int slices = p.splits >= 16 ? 4 : 1;     // many splits: four threads per output
+    const int blocks = (int)((total * slices + 255) / 256);
+    hipLaunchKernelGGL(splitk_reduce_kernel<T>, dim3(blocks), dim3(256), 0, stream, p.Cpart, static_cast<T *>(p.C), p.M, p.N,
+                       p.ldc, p.splits, slices);
+    return hipGetLastError();
+}
 
 template <typename T, bool A_KM, bool B_KM>
 hipError_t launch_gemm_t(const GemmParams &p, hipStream_t stream) {
@@ -23,15 +34,7 @@ hipError_t launch_gemm_t(const GemmParams &p, hipStream_t stream) {
     hipLaunchKernelGGL(kern, dim3(grid), dim3(kThreads), G::LDS_BYTES, stream, p);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    if (p.splits > 1) {
-        const size_t total = (size_t)p.M * p.N;
-        const int slices = p.splits >= 16 ? 4 : 1;     // many splits: four threads per output
-        const int blocks = (int)((total * slices + 255) / 256);
-        hipLaunchKernelGGL(splitk_reduce_kernel<T>, dim3(blocks), dim3(256), 0, stream, p.Cpart,
-                           static_cast<T *>(p.C), p.M, p.N, p.ldc, p.splits, slices);
-        e = hipGetLastError();
-    }
-    return e;
+    return p.splits > 1 ? launch_splitk_reduce<T>(p, stream) : hipSuccess;
 }
 
 std::atomic<int> g_gemm_baseline{0};   // diagnostics: 1 = stand-alone 16-bit 256 x 256 launches run gemm16_onetile_kernel
@@ -73,15 +76,7 @@ hipError_t launch_gemm16_t(const GemmParams &p, hipStream_t stream) {
     if (!baseline) hipLaunchKernelGGL(kern, dim3(grid), dim3(C::THREADS), C::LDS_BYTES, stream, p);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    if (p.splits > 1) {
-        const size_t total = (size_t)p.M * p.N;
-        const int slices = p.splits >= 16 ? 4 : 1;     // many splits: four threads per output
-        const int blocks = (int)((total * slices + 255) / 256);
-        hipLaunchKernelGGL(splitk_reduce_kernel<T>, dim3(blocks), dim3(256), 0, stream, p.Cpart,
-                           static_cast<T *>(p.C), p.M, p.N, p.ldc, p.splits, slices);
-        e = hipGetLastError();
-    }
-    return e;
+    return p.splits > 1 ? launch_splitk_reduce<T>(p, stream) : hipSuccess;
 }
 
 template <typename T, int BM, int BN, int NS, int WVM, int WVN, int KSPT>
@@ -132,8 +127,8 @@ hipError_t launch_colsum_t(const void *in, void *out, float *part, int R, int C,
 // The 16-bit fast kernel needs: K range of every split a multiple of 64, 16-byte aligned
 // rows, operands addressable with 32-bit byte offsets.
 bool gemm16_eligible(int dtype, int M, int N, int K, int lda, int ldb, bool a_km, bool b_km) {
-    // (fp32 runs on the 256 x 256 tile only: see gemm_plan)
-    const int es = dtype == FASTLSTM_FP32 ? 4 : 2, epc = 16 / es;
+    if (dtype == FASTLSTM_FP32) return false;
+    const int es = 2, epc = 16 / es;
     // K-major x K-major (the weight gradients, K = T*B rows): any K -- the loop runs to the next multiple of 64 and the
     // rows past K lie outside both operands' buffer ranges, where loads return zero
     if ((K % 64 != 0 && !(a_km && b_km)) || lda % epc != 0 || ldb % epc != 0) return false;
@@ -145,12 +140,17 @@ bool gemm16_eligible(int dtype, int M, int N, int K, int lda, int ldb, bool a_km
 // Tile edge (256 or 128; 0 = generic kernel) and split-K factor for a product.
 void gemm_plan(int dtype, int M, int N, int K, int lda, int ldb, bool a_km, bool b_km, bool allow_split,
                int *tile, int *splits) {
+    if (dtype == FASTLSTM_FP32) {
+        int kps;
+        gemm_f32_plan(M, N, 0, K, allow_split, tile, splits, &kps);
+        return;
+    }
     *splits = 1;
     if (!gemm16_eligible(dtype, M, N, K, lda, ldb, a_km, b_km)) {
         *tile = 0;
         const int tiles = cdiv(M, kBM) * cdiv(N, kBN);
         if (allow_split && tiles < 128) {
-            const int bk = gemm_bk(dtype);
+            const int bk = gemm_bk();
             *splits = std::max(1, std::min(std::min(cdiv(512, tiles), std::max(1, K / (4 * bk))), 1024));
         }
         return;
@@ -162,15 +162,6 @@ void gemm_plan(int dtype, int M, int N, int K, int lda, int ldb, bool a_km, bool
     } else if (std::min(256 / t256, max_split) * t256 >= 192) {   // (one round of workgroups: the factor rounded down)
         *tile = 256;
         *splits = std::min(256 / t256, max_split);
-    } else if (dtype == FASTLSTM_FP32) {
-        // true-fp32 MFMA runs at 1/16 of the 16-bit rate: a product too small to fill the device with 256 x 256 tiles is
-        // left to the generic 128 x 128 kernel (two workgroups per CU), planned as above
-        *tile = 0;
-        const int tiles = cdiv(M, kBM) * cdiv(N, kBN);
-        if (allow_split && tiles < 128) {
-            const int bk = gemm_bk(dtype);
-            *splits = std::max(1, std::min(std::min(cdiv(512, tiles), std::max(1, K / (4 * bk))), 1024));
-        }
     } else {
         *tile = 128;
         if (t128 < 192) *splits = std::max(1, std::min(cdiv(512, t128), max_split));
@@ -178,12 +169,18 @@ void gemm_plan(int dtype, int M, int N, int K, int lda, int ldb, bool a_km, bool
 }
 
 // ---- both weight gradients + the bias gradient on the tile kernel (gemm16_wgrad_kernel) ------------------------
-// Taken for 16-bit products that the 256 x 256 tile kernel holds.  *merged: both products as one tile grid with
+// Taken for fp32 (gemm_f32.hpp) and for 16-bit products that the 256 x 256 tile kernel holds.  *merged: both products as one tile grid with
 // one split factor (K = T*B is split so that the tiles of both together fill the device); otherwise each product
 // fills the device on its own and they run as two launches of one round of tiles each, the bias gradient with
 // the first (a second round of tiles starts out of step with its neighbours and shares less in the L2:
 // M = 8192, I = H = 2048, K = 32768: 1.85 ms merged against 2 x 0.86).
 bool wgrad_merged_plan(int dtype, int M, int I, int H, int K, int *splits, int *k_per_split, bool *merged) {
+    if (dtype == FASTLSTM_FP32) {   // any shape, always one grid
+        int tile;
+        *merged = true;
+        gemm_f32_plan(M, I, H, K, true, &tile, splits, k_per_split);
+        return true;
+    }
     if (!gemm16_eligible(dtype, M, I, K, M, I, true, true) || !gemm16_eligible(dtype, M, H, K, M, H, true, true)) return false;
     if (M < 256 || I < 128 || H < 128) return false;   // thin outputs: the 128 x 128 tiles waste less
     const int tx = cdiv(M, 256) * cdiv(I, 256), th = cdiv(M, 256) * cdiv(H, 256);
@@ -191,9 +188,6 @@ bool wgrad_merged_plan(int dtype, int M, int I, int H, int K, int *splits, int *
     int sp = 1;
     // (rounded down: one round of at most 256 workgroups; 60 tiles x 5 splits would be a full round and a sixth of one)
     if (*merged && tx + th < 192) sp = std::max(1, std::min(256 / (tx + th), K / 512));   // >= 8 k-tiles per split
-    // true-fp32 MFMA runs at 1/16 of the 16-bit rate: products that do not fill the device with 256 x 256 tiles stay
-    // with the generic 128 x 128 kernel and its finer split (T*B = 2048, 4H = 1024, I = H = 256: 0.06 against 0.15 ms)
-    if (dtype == FASTLSTM_FP32 && (tx + th) * sp < 192) return false;
     const int kps = cdiv(cdiv(K, sp), 64) * 64;
     *k_per_split = kps;
     *splits = cdiv(K, kps);
@@ -225,6 +219,16 @@ static hipError_t launch_wgrad_kernel_t(const WgradParams &w, hipStream_t s) {
     return hipGetLastError();
 }
 
+template <typename T> static hipError_t launch_wgrad_reduce(const WgradParams &w, void *db, int db_parts, hipStream_t s) {
+    const int M = w.x.M, splits = w.x.splits;
+    const int ri = splits > 1 ? w.x.N : 0, rh = splits > 1 ? w.h.N : 0;   // the products need no pass without a split
+    const size_t threads = (size_t)M * ri / 4 + (size_t)M * rh / 4 + M;
+    hipLaunchKernelGGL(wgrad_reduce_kernel<T>, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, w.x.Cpart,
+                       static_cast<T *>(w.x.C), w.h.Cpart, static_cast<T *>(w.h.C), w.db_part, static_cast<T *>(db), M, ri, rh,
+                       splits, db_parts);
+    return hipGetLastError();
+}
+
 template <typename T>
 static hipError_t launch_wgrad_merged_t(const WgradParams &w, bool merged, void *db, hipStream_t s) {
     const int M = w.x.M, I = w.x.N, H = w.h.N, splits = w.x.splits;
@@ -233,23 +237,25 @@ static hipError_t launch_wgrad_merged_t(const WgradParams &w, bool merged, void 
         if (hipError_t e = launch_wgrad_kernel_t<T>(w, s)) return e;
         db_parts = splits * (w.tiles_nx + cdiv(H, 256));
     } else {   // the x product with the bias gradient, then the h product alone
-        WgradParams a = w, b = w;
+        WgradParams a = w;
         a.h.N = 0;
-        b.x = w.h; b.h.N = 0; b.tiles_nx = cdiv(H, 256); b.db_part = nullptr;
         if (hipError_t e = launch_wgrad_kernel_t<T>(a, s)) return e;
-        if constexpr (sizeof(T) == 2) {   // one round of tiles, both operands K-major: the symmetric loop (gemm16_onetile_kernel)
-            if (hipError_t e = launch_onetile_t<T, true, true>(w.h, s)) return e;
-        } else {
-            if (hipError_t e = launch_wgrad_kernel_t<T>(b, s)) return e;
-        }
+        // one round of tiles, both operands K-major: the symmetric loop (gemm16_onetile_kernel)
+        if (hipError_t e = launch_onetile_t<T, true, true>(w.h, s)) return e;
         db_parts = splits * w.tiles_nx;
     }
-    const int ri = splits > 1 ? I : 0, rh = splits > 1 ? H : 0;   // the products need no pass without a split
-    const size_t threads = (size_t)M * ri / 4 + (size_t)M * rh / 4 + M;
-    hipLaunchKernelGGL(wgrad_reduce_kernel<T>, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, s, w.x.Cpart,
-                       static_cast<T *>(w.x.C), w.h.Cpart, static_cast<T *>(w.h.C), w.db_part, static_cast<T *>(db), M, ri, rh,
-                       splits, db_parts);
-    return hipGetLastError();
+    return launch_wgrad_reduce<T>(w, db, db_parts, s);
+}
+
+// The fp32 products (gemm_f32.hpp): one grid over both, the bias gradient with the first column of tiles.
+static hipError_t launch_wgrad_f32(const WgradParams &w, int tile, void *db, hipStream_t s) {
+    GemmF32Params g{};
+    g.p = w.x;
+    g.B2 = w.h.B; g.C2 = w.h.C; g.Cpart2 = w.h.Cpart; g.N2 = w.h.N; g.ldb2 = w.h.ldb; g.ldc2 = w.h.ldc;
+    g.tiles_n1 = cdiv(w.x.N, tile);
+    g.db_part = w.db_part;
+    if (hipError_t e = launch_gemm_f32(g, true, true, tile, s)) return e;
+    return launch_wgrad_reduce<float>(w, db, w.x.splits, s);
 }
 
 hipError_t launch_wgrad_merged(int dtype, const void *d_ifgo, const void *x, const void *h, void *dWx, void *dWh, void *db,
@@ -267,8 +273,12 @@ hipError_t launch_wgrad_merged(int dtype, const void *d_ifgo, const void *x, con
     w.h = g; w.h.B = h; w.h.C = dWh; w.h.N = H; w.h.ldb = H; w.h.ldc = H; w.h.Cpart = part_x + (size_t)sp * M * I;
     w.tiles_nx = cdiv(I, 256);
     w.db_part = db_part;
-    return dtype == FASTLSTM_FP32 ? launch_wgrad_merged_t<float>(w, merged, db, s)
-           : dtype == FASTLSTM_FP16 ? launch_wgrad_merged_t<_Float16>(w, merged, db, s)
+    if (dtype == FASTLSTM_FP32) {
+        int tile;
+        gemm_f32_plan(M, I, H, K, true, &tile, &sp, &kps);
+        return launch_wgrad_f32(w, tile, db, s);
+    }
+    return dtype == FASTLSTM_FP16 ? launch_wgrad_merged_t<_Float16>(w, merged, db, s)
                                     : launch_wgrad_merged_t<__bf16>(w, merged, db, s);
 }
 
@@ -285,8 +295,12 @@ hipError_t launch_gemm_tiled(int dtype, const GemmParams &p_in, bool a_km, bool 
     if (tile == ID)                                                                                         \
         return dtype == FASTLSTM_FP16 ? launch_gemm16_dt<_Float16, BM, BN, NS, WVM, WVN, KSPT>(p, a_km, b_km, s) \
                                       : launch_gemm16_dt<__bf16, BM, BN, NS, WVM, WVN, KSPT>(p, a_km, b_km, s);
-    if (tile == 256 && dtype == FASTLSTM_FP32) return launch_gemm16_dt<float, 256, 256, 2, 2, 4, 2>(p, a_km, b_km, s);
-    if (dtype == FASTLSTM_FP32) return launch_gemm(dtype, p, a_km, b_km, s);
+    if (dtype == FASTLSTM_FP32) {
+        GemmF32Params g{};
+        g.p = p;
+        if (hipError_t e = launch_gemm_f32(g, a_km, b_km, tile, s)) return e;
+        return p.splits > 1 ? launch_splitk_reduce<float>(p, s) : hipSuccess;
+    }
     FASTLSTM_TILE_CASE(128, 128, 128, 2, 2, 2, 2)   // 2 workgroups per CU
     FASTLSTM_TILE_CASE(256, 256, 256, 2, 2, 4, 2)   // 8 waves, 128 x 64 per wave, 2 x 64 KiB stages
 #undef FASTLSTM_TILE_CASE
@@ -295,7 +309,6 @@ hipError_t launch_gemm_tiled(int dtype, const GemmParams &p_in, bool a_km, bool 
 
 hipError_t launch_gemm(int dtype, const GemmParams &p, bool a_km, bool b_km, hipStream_t s) {
     switch (dtype) {
-        case FASTLSTM_FP32: return launch_gemm_dt<float>(p, a_km, b_km, s);
         case FASTLSTM_FP16: return launch_gemm_dt<_Float16>(p, a_km, b_km, s);
         default: return launch_gemm_dt<__bf16>(p, a_km, b_km, s);
     }
@@ -319,6 +332,6 @@ hipError_t launch_colsum_final(int dtype, const float *part, void *out, int C, i
     return hipGetLastError();
 }
 
-int gemm_bk(int dtype) { return dtype == FASTLSTM_FP32 ? GemmTile<float>::BK : GemmTile<_Float16>::BK; }
+int gemm_bk() { return GemmTile<_Float16>::BK; }
 
 }  // namespace fastlstm

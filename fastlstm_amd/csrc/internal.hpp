@@ -7,6 +7,7 @@
 namespace fastlstm {
 
 struct GemmParams;
+struct GemmF32Params;
 struct FwdParams;
 struct BwdParams;
 struct FwdXcdParams;
@@ -16,10 +17,13 @@ hipError_t launch_gemm(int dtype, const GemmParams &p, bool a_km, bool b_km, hip
 // diagnostics: the stand-alone 16-bit tile launches in their earlier form (gemm16_onetile_kernel)
 void set_gemm_baseline(int on);
 int gemm_baseline();
+// fp32 products (gemm_f32.hpp): every shape; tile 256 or 128
+void gemm_f32_plan(int M, int N1, int N2, int K, bool allow_split, int *tile, int *splits, int *k_per_split);
+hipError_t launch_gemm_f32(const GemmF32Params &g, bool a_km, bool b_km, int tile, hipStream_t s);
 hipError_t launch_colsum_final(int dtype, const float *part, void *out, int C, int chunks, hipStream_t s);
 hipError_t launch_colsum(int dtype, const void *in, void *out, float *part, int R, int C, int chunks,
                          hipStream_t s);
-int gemm_bk(int dtype);
+int gemm_bk();
 bool gemm16_eligible(int dtype, int M, int N, int K, int lda, int ldb, bool a_km, bool b_km);
 void set_gemm_trace(long long *buf);
 void gemm_plan(int dtype, int M, int N, int K, int lda, int ldb, bool a_km, bool b_km, bool allow_split,

@@ -1,0 +1,59 @@
+"""The fp32 products (csrc/gemm_f32.hpp): edges of their tiles and k-tiles, and operands that are no finite numbers."""
+import pytest
+import torch
+
+import fastlstm_amd.lstm as L
+from fastlstm_amd import _lib
+
+pytestmark = pytest.mark.gpu
+
+# rows T*B, I, H: one element, below and above the tiles of 128 and 256, k-tiles of 16 with a remainder, rows of 4-byte
+# alignment, split sums, more tiles than compute units
+SHAPES = [(1, 1, 1), (5, 3, 4), (127, 15, 33), (129, 17, 32), (255, 260, 64), (257, 129, 66), (1000, 77, 130), (4099, 256, 256),
+          (2048, 513, 1024)]
+
+
+def products(R, I, H, seed=0, plant=None):
+    """((K1, dx, dWx, dWh, db), the same in 64 bits, the same of magnitudes)"""
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    lib, st = _lib.load(), torch.cuda.current_stream().cuda_stream
+    n = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    x, Wx, bx, bh, d, h = n(1, R, I), n(4 * H, I), n(4 * H), n(4 * H), n(1, R, 4 * H), n(2, R, H)
+    if plant is not None:
+        plant(x, Wx, d)
+    k1, dx = torch.empty(R, 4 * H, device="cuda"), torch.empty(R, I, device="cuda")
+    _lib.check(lib.fastlstm_gemm_ifgo(x.data_ptr(), Wx.data_ptr(), bx.data_ptr(), bh.data_ptr(), k1.data_ptr(), 1, R, I, H, 0, st), "k1")
+    _lib.check(lib.fastlstm_gemm_dx(d.data_ptr(), Wx.data_ptr(), dx.data_ptr(), 1, R, I, H, 0, st), "dx")
+    db, _, dWx, dWh = L.Wgrad(d, x, h)
+
+    def exact(f):
+        X, W, D, Hh = f(x[0].double()), f(Wx.double()), f(d[0].double()), f(h[0].double())
+        return X @ W.T + f(bx.double()) + f(bh.double()), D @ W, D.T @ X, D.T @ Hh, D.sum(0)
+    return (k1, dx, dWx, dWh, db), exact(lambda t: t), exact(torch.abs)
+
+
+@pytest.mark.parametrize("R,I,H", SHAPES)
+def test_products_at_the_edges(R, I, H):
+    got, want, magnitude = products(R, I, H, seed=R + I + H)
+    for a, b, m, terms in zip(got, want, magnitude, (I + 2, 4 * H, R, R, R)):
+        # six roundings of the running sum per 16 terms, the products left out (2^-22 of a term) and one of the result; the sums
+        # of magnitudes bound the running sums
+        bound = m * ((3 + 6 * terms / 16) * 2.0 ** -24 + 2.0 ** -22)
+        assert bool(((a.double() - b).abs() <= bound).all())
+
+
+def test_infinities_and_nans_as_in_the_sum():
+    """inf times a number whose lower parts are zero, of either sign, inf times 0, inf - inf and NaN: in an operand of any product."""
+    def plant(x, Wx, d):
+        inf = float("inf")
+        Wx[0, :4] = torch.tensor([1.0, -0.5, 0.0, 3.0])
+        x[0, 3, 0], x[0, 4, 1], x[0, 5, 2], x[0, 200, 3] = inf, inf, -inf, float("nan")
+        Wx[70, 5] = -inf
+        d[0, 10, 9] = inf
+        d[0, 11, 40], d[0, 12, 40] = inf, -inf
+    got, want, _ = products(300, 40, 130, plant=plant)
+    for a, b in zip(got, want):
+        assert torch.equal(torch.isnan(a), torch.isnan(b))
+        assert torch.equal(torch.isinf(a), torch.isinf(b)) and torch.equal(a[torch.isinf(a)].double(), b[torch.isinf(b)])
+        ok = torch.isfinite(b)
+        assert float((a.double() - b)[ok].abs().max()) < 1e-3 and bool(ok.any()) and not bool(ok.all())
