@@ -1210,6 +1210,13 @@ static int one_tile_row_split(int B, int n_rec, int num_cus) {
     return 0;
 }
 
+// The one-CU kernels: n recurrences of B rows side by side, four rows per workgroup, each on a CU of its own.
+static bool cu_applies(int B, int H, int dtype, int n = 1) {
+    DeviceInfo di;
+    return cu_shape(H, dtype) && (g_families.load() & 1) && device_info(-1, &di) == FASTLSTM_OK &&
+           (long long)n * cdiv(B, 4) <= di.num_cus;
+}
+
 // coalesced tile I/O of the general kernels needs complete, 16-byte aligned row segments and room in LDS
 static bool fwd_tile_io(const fastlstm_plan &pl, int H, int dtype, int *tile_bytes) {
     const int s = elem_bytes(dtype), gseg = pl.ht * s;
@@ -1231,6 +1238,19 @@ static int fwd_persistent_impl(void *ifgo, void *out, void *cell, const void *Wh
     fastlstm_plan pl;
     if (int rc = plan_device(-1, B, H, dtype, 0, &pl, false)) return rc;
     if (ws_bytes < pl.ws_bytes) return FASTLSTM_ERR_WORKSPACE;
+    if (n_others <= 3 && cu_applies(B, H, dtype, 1 + n_others)) {
+        FwdParams p{};
+        p.ifgo = ifgo; p.out = out; p.cell = cell; p.Wh = Wh;
+        p.T = T; p.B = B; p.H = H;
+        p.keep = keep;
+        p.n_rec = 1 + n_others;
+        p.n_bt_launch = cdiv(B, 4);
+        for (int i = 0; i < n_others; ++i) {
+            p.ifgo_x[i] = others[i][0]; p.out_x[i] = others[i][1]; p.cell_x[i] = others[i][2]; p.Wh_x[i] = others[i][3];
+        }
+        return launch_fwd_cu(dtype, p, p.n_rec * p.n_bt_launch, static_cast<hipStream_t>(stream)) == hipSuccess ? FASTLSTM_OK
+                                                                                                                 : FASTLSTM_ERR_HIP;
+    }
     const bool sync = pl.wave_split != 2;
     if (n_others && (sync || n_others > 3)) return FASTLSTM_ERR_DIM;
     // 64 units per workgroup: batch tiles of 4 or 8 rows where that many workgroups still find a CU each
@@ -1390,6 +1410,19 @@ static int bwd_persistent_impl(const void *dout, void *dh, void *dc, const void 
     fastlstm_plan pl;
     if (int rc = plan_device(-1, B, H, dtype, 1, &pl, false)) return rc;
     if (ws_bytes < pl.ws_bytes) return FASTLSTM_ERR_WORKSPACE;
+    if (n_others <= 3 && cu_applies(B, H, dtype, 1 + n_others)) {
+        BwdParams p{};
+        p.dout = dout; p.dh = dh; p.dc = dc; p.ifgo = ifgo; p.cell = cell; p.d_ifgo = d_ifgo; p.Wh = Wh;
+        p.T = T; p.B = B; p.H = H;
+        p.n_rec = 1 + n_others;
+        p.n_bt_launch = cdiv(B, 4);
+        for (int i = 0; i < n_others; ++i) {
+            p.dout_x[i] = others[i][0]; p.dh_x[i] = others[i][1]; p.dc_x[i] = others[i][2]; p.ifgo_x[i] = others[i][3];
+            p.cell_x[i] = others[i][4]; p.d_ifgo_x[i] = others[i][5]; p.Wh_x[i] = others[i][6];
+        }
+        return launch_bwd_cu(dtype, p, p.n_rec * p.n_bt_launch, static_cast<hipStream_t>(stream)) == hipSuccess ? FASTLSTM_OK
+                                                                                                                 : FASTLSTM_ERR_HIP;
+    }
     const bool sync = pl.wave_split != 2;
     if (n_others && (sync || n_others > 3)) return FASTLSTM_ERR_DIM;
     const int kstep = dtype == FASTLSTM_FP32 ? 16 : 32;
@@ -1547,7 +1580,11 @@ static int try_multi(bool backward, int n, void *const (*recs)[7], void *ws, siz
     if (int rc = plan_device(-1, B, H, dtype, backward ? 1 : 0, &pl, false)) return rc;
     if (pl.wave_split == 3) return 1;
     void *const *a = recs[0], *const *b = recs[1];
-    if (pl.wave_split == 2) {   // the one-tile form: no exchange between workgroups, any number of them side by side
+    // no exchange between workgroups, any number of them side by side: the one-tile form, the one-CU kernels (or none together
+    // where they hold one alone: a launch of other kernels would sum in another order)
+    const bool one_cu = cu_applies(B, H, dtype);
+    if (one_cu && !cu_applies(B, H, dtype, n)) return 1;
+    if (pl.wave_split == 2 || one_cu) {
         if (dry_run) return FASTLSTM_OK;
         return backward ? bwd_persistent_impl(a[0], a[1], a[2], a[3], a[4], a[5], a[6], ws, ws_bytes, T, B, H, dtype, stream,
                                               recs + 1, n - 1)
@@ -1729,7 +1766,7 @@ static int fwd_layer_impl(const void *x, const void *Wx, const void *bx, const v
         fastlstm_plan pl;
         if (int rc = plan_device(-1, B, H, dtype, 0, &pl, false)) return rc;
         if (ws_bytes < pl.ws_bytes) return FASTLSTM_ERR_WORKSPACE;
-        if (pl.wave_split != 2) {
+        if (pl.wave_split != 2 && !cu_applies(B, H, dtype)) {
             const int rc = try_fwd_xcd(ifgo, out, cell, Wh, static_cast<unsigned char *>(ws), ws_bytes, T, B, H, dtype,
                                        static_cast<hipStream_t>(stream), x, Wx, bx, bh, I, nullptr, false,
                                        LaunchOpts{keep, 0, 0});
@@ -1911,6 +1948,7 @@ size_t fastlstm_stack2_workspace_bytes(const fastlstm_plan *plan, int T, int H, 
 int fastlstm_fwd_stack2_fused(int T, int B, int I, int H, int dtype, size_t ws_bytes) {
     if (!dtype_ok(dtype)) return FASTLSTM_ERR_DTYPE;
     if (int rc = check_dims(T, B, I, H)) return rc;
+    if (cu_applies(B, H, dtype)) return 0;   // (a layer by itself runs on the one-CU kernels)
     unsigned char *fake = reinterpret_cast<unsigned char *>(static_cast<size_t>(4096));   // never dereferenced
     const SecondLayer second{fake, fake, fake, fake, fake, fake, fake};
     const int rc = try_fwd_xcd(fake, fake, fake, fake, fake, ws_bytes, T, B, H, dtype, nullptr, fake, fake, fake, fake, I,
@@ -1936,7 +1974,7 @@ static int fwd_stack2_impl(const void *x, const void *Wx0, const void *bx0, cons
     if (ws_bytes < pl.ws_bytes) return FASTLSTM_ERR_WORKSPACE;
     hipStream_t s = static_cast<hipStream_t>(stream);
 #ifndef FASTLSTM_TIMELINE
-    if (pl.wave_split != 2) {
+    if (pl.wave_split != 2 && !cu_applies(B, H, dtype)) {
         const SecondLayer second{Wx1, bx1, bh1, Wh1, ifgo1, out1, cell1};
         const int rc = try_fwd_xcd(ifgo0, out0, cell0, Wh0, static_cast<unsigned char *>(ws), ws_bytes, T, B, H, dtype, s, x,
                                    Wx0, bx0, bh0, I, &second, false, LaunchOpts{keep, 0, 0});
@@ -2002,7 +2040,7 @@ static int bwd_layer_impl(const void *dout, void *dh, void *dc, const void *ifgo
     if (ws_bytes < pl.ws_bytes) return FASTLSTM_ERR_WORKSPACE;
     int rc = 1;
     int db_done = 0;
-    if (pl.wave_split != 2 && (dx || want_w)) {
+    if (pl.wave_split != 2 && (dx || want_w) && !cu_applies(B, H, dtype)) {
         // (the weight-gradient workspace is not used by a launch that has the weight gradients inside: it takes the
         // partial sums of the bias gradient)
         float *db_part = want_w && db_part_bytes(B, H) <= wgrad_ws_bytes ? static_cast<float *>(wgrad_ws) : nullptr;
@@ -2069,6 +2107,7 @@ size_t fastlstm_stack2_bwd_wgrad_workspace_bytes(int T, int B, int I, int H, int
 int fastlstm_bwd_stack2_fused(int T, int B, int I, int H, int dtype, size_t ws_bytes) {
     if (!dtype_ok(dtype)) return FASTLSTM_ERR_DTYPE;
     if (int rc = check_dims(T, B, I, H)) return rc;
+    if (cu_applies(B, H, dtype)) return 0;   // (see fastlstm_fwd_stack2_fused)
     unsigned char *fake = reinterpret_cast<unsigned char *>(static_cast<size_t>(4096));   // never dereferenced
     const BwdExtras e{fake, fake, fake, fake, fake, fake, H};
     const LowerLayer lower{fake, fake, fake, fake, fake, fake, fake, fake, I, fake, (size_t)1 << 40, fake, fake, fake, fake};
@@ -2101,7 +2140,7 @@ static int bwd_stack2_impl(const void *dout, void *dh1, void *dc1, const void *i
     hipStream_t s = static_cast<hipStream_t>(stream);
     // the upper layer's input is the lower layer's h: x1 = out0[1:]
     const void *x1 = static_cast<const unsigned char *>(out0) + (size_t)B * H * elem_bytes(dtype);
-    if (pl.wave_split != 2) {
+    if (pl.wave_split != 2 && !cu_applies(B, H, dtype)) {
         // the end of the weight-gradient workspace takes the two layers' partial sums of the bias gradients, the
         // parked weight-gradient tiles come before them
         const size_t dbb = db_part_bytes(B, H);

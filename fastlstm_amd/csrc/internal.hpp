@@ -90,6 +90,11 @@ struct StreamLayout {
 };
 StreamLayout stream_layout(const fastlstm_plan &plan, int H, int dtype, bool backward);
 
+// one-CU kernels (recurrent_cu.hpp): p.B, H, T, keep, n_rec and the operands; four rows per workgroup
+bool cu_shape(int H, int dtype);
+hipError_t launch_fwd_cu(int dtype, const FwdParams &p, int grid, hipStream_t s);
+hipError_t launch_bwd_cu(int dtype, const BwdParams &p, int grid, hipStream_t s);
+
 int fwd_lds_bytes(int H, int dtype, int ht, int bt, int split, bool sync);
 int bwd_lds_bytes(int H, int dtype, int ht, int bt, int split, bool sync);
 size_t recurrent_flags_bytes(int n_bt, int n_ht);
