@@ -1162,14 +1162,15 @@ def _padded_hidden_size_cached(T, B, H, code, device_index, training, families):
         # there is at H = 64 (T = 1024, B = 256, I = H = 64 forward + backward 0.93 ms as it is, 3.4 ms as H = 96):
         # its 64-unit kernels spread the batch over tiles of 4 rows and move whole tiles in both directions, which the
         # narrower forms do not (T = 1024, B = 256, inference forward / forward + backward of a training step with its
-        # loss: H = 32 as it is 0.50 / 3.20 ms, H = 16 0.42 / 2.12, H = 64 0.42 / 1.18).  The same holds in fp32 since
-        # the 4-row tiles spread its true-fp32 MFMAs over four times the CUs (T = 256, B = 64: H = 64 as it is 0.36 /
-        # 0.86 ms, as H = 80 on the XCD-local kernels 0.57 / 1.21; H = 48 as it is 0.74 / 2.40, as 64 0.45 / 0.98), except
-        # that up to 16 units nothing gains (H = 16 0.18 / 1.03 as it is, 0.45 / 0.99 as 64) and up to 32 only a
-        # training step does (H = 32 0.28 / 1.16 as it is, 0.45 / 0.98 as 64).
-        if H == 64 or H <= (16 if fp32 or not training else 0):
+        # loss: H = 32 as it is 0.50 / 3.20 ms, H = 16 0.42 / 2.12, H = 64 0.42 / 1.18); up to 16 units nothing gains without
+        # a reverse pass.  fp32 has the one-CU kernels from 64 units on (0.6 us per step forward where the general ones take 0.5 at
+        # H = 16 and 0.85 at 32; with the reverse pass 1.2 against 2.7 and 3.2), which pay for the copies from about 100
+        # steps on: inference / training, as it is and as 64, H = 32 T = 64 0.079 / 0.279 and 0.089 / 0.357 ms, T = 256
+        # 0.244 / 1.05 and 0.174 / 0.414; H = 16 T = 64 0.054 / 0.256 and 0.088 / 0.355, T = 128 0.087 / 0.459 and
+        # 0.112 / 0.367, T = 1024 0.486 / 2.66 and 0.556 / 1.27.
+        if H == 64 or (H <= 16 and not training):
             return 0
-        if fp32 and H <= 32 and not training:
+        if fp32 and H <= 32 and T < 96:
             return 0
         return 64
     if kind(H) != 0 or fast(H):
