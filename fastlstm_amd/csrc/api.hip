@@ -317,14 +317,15 @@ bool select_xcd(int T, int B_all, int H, int dtype, bool backward, size_t ws_byt
     const int B = launch_rows ? launch_rows : B_all;
     DeviceInfo di;
     if (!(g_families.load() & 1) || device_info(-1, &di) != FASTLSTM_OK || di.xcd_round_robin != 1) return false;
-    const int s = elem_bytes(dtype), kstep = dtype == FASTLSTM_FP32 ? 16 : 32;
+    const bool fp32 = dtype == FASTLSTM_FP32;
+    const int s = elem_bytes(dtype), parts = fp32 ? 3 : 1;   // (fp32: operand blocks per k-step, recurrent_parts.hpp)
     const int K = backward ? 4 * H : H;
-    if (K % kstep || (H * s) % 16) return false;
-    c->ks = K / kstep;
+    if (K % (fp32 ? 16 : 32) || (H * s) % 16) return false;
+    c->ks = cdiv(K, 32);
     const int ways = backward ? 8 : 4;   // K-shares
     const int per = cdiv(c->ks, ways);
-    c->nkw = per <= 4 ? 4 : (per <= 8 ? 8 : ((backward && per <= 16) ? 16 : 0));
-    if (!c->nkw) return false;
+    c->nkw = per <= 2 && fp32 ? 2 : per <= 4 ? 4 : (per <= 8 ? 8 : (per <= 16 ? 16 : 0));
+    if (!c->nkw || c->nkw > (backward ? 16 : 8) / (fp32 ? 2 : 1)) return false;
     // hidden units per workgroup: the smallest tile that puts a group on one XCD and all batch tiles in one launch
     const int hts_f[3] = {8, 16, 32}, hts_b[2] = {16, 32};
     const int *hts = backward ? hts_b : hts_f;
@@ -333,8 +334,8 @@ bool select_xcd(int T, int B_all, int H, int dtype, bool backward, size_t ws_byt
     c->ntw = 0;
     for (int hi = 0; hi < n_hts && !ht; ++hi) {
         const int cand = hts[hi];
-        const int frags = (cand / rows) * c->nkw;   // per wave (forward: halved again by the unit split of 8 waves)
-        if (H % cand || H / cand > 32 || cand * s < 16 || frags > (backward ? 32 : 64)) continue;
+        const int frags = (cand / rows) * c->nkw * parts;   // per wave (forward: halved again by the unit split of 8 waves)
+        if (H % cand || H / cand > 32 || cand * s < 16 || frags > (backward ? (fp32 ? 24 : 32) : (fp32 ? 48 : 64))) continue;
         // groups per XCD: as many as its 32 CUs hold, and no more than the workspace has barrier counters for
         const int groups_max = kNumXcd * std::min(32 / (H / cand), kXcdMaxGroups / kNumXcd);
         if (copies * cdiv(B, 16) <= groups_max) { ht = cand; c->ntw = 1; }
@@ -342,13 +343,13 @@ bool select_xcd(int T, int B_all, int H, int dtype, bool backward, size_t ws_byt
     }
     if (!ht) return false;
     c->mt = ht / rows;
-    c->nwv = backward ? 8 : (c->mt * c->nkw > 32 ? 8 : 4);
+    c->nwv = backward ? 8 : (c->mt * c->nkw * parts > 32 ? 8 : 4);
     c->n_ht = H / ht;
     c->gpx = std::min(32 / c->n_ht, kXcdMaxGroups / kNumXcd);
     const int bt = 16 * c->ntw;
     c->n_groups = cdiv(B, bt);
     if (copies * c->n_groups > kNumXcd * c->gpx) return false;   // (the tile loop above guarantees it; the kernels index counters by group)
-    c->xslot = (size_t)c->n_groups * c->ntw * c->ks * kFragBytes;
+    c->xslot = (size_t)c->n_groups * c->ntw * c->ks * parts * kFragBytes;
     if (ws_bytes < kWsHeaderBytes + kWsCounterBytes + kXchgSlots * (size_t)copies * c->xslot) return false;
     // partial sums of the K-shares, gates tile(s), two state tiles (as the kernels lay them out)
     const int gseg = ht * s, gates = bt * (4 * gseg + 16), states = 2 * bt * (gseg + 16);

@@ -23,6 +23,7 @@
 
 #include "common.hpp"
 #include "gemm.hpp"
+#include "recurrent_parts.hpp"
 
 namespace fastlstm {
 
@@ -46,11 +47,6 @@ template <int BM, int BN, int WM, int WN> struct F32Tile {
     static_assert(BM == BN && BM == THREADS / 2, "half of the threads stage 16 elements each of either operand");
 };
 
-// A value with its lower 16 bits cut off.  (By value: a bit cast of an element of a vector takes the vector's first element.)
-__device__ __forceinline__ float upper_half(float v) { return __builtin_bit_cast(float, __builtin_bit_cast(unsigned, v) & 0xffff0000u); }
-__device__ __forceinline__ unsigned upper_halves(float a, float b) {
-    return __builtin_amdgcn_perm(__builtin_bit_cast(unsigned, b), __builtin_bit_cast(unsigned, a), 0x07060302u);
-}
 // The largest magnitude met (a NaN does not count).
 __device__ __forceinline__ void max_magnitude(float &top, float a, float b) {
 #if defined(__HIP_DEVICE_COMPILE__)

@@ -227,10 +227,11 @@ extern "C" size_t fastlstm_recurrent_workspace_bytes(const fastlstm_plan *plan, 
     // the XCD-local kernels lay their slots out for batch tiles of 16 or 32 rows, which covers at most
     // 16 rows (one operand block per k-step) more than the tiles of the plan
     // (the kernels for H = 1280 ... 2048 use tiles of 64 rows: at most 48 rows more)
-    const int KS = cdiv(backward ? 4 * H : H, kstep_of(dtype));
+    // (fp32: three blocks per 32 k, its numbers' parts, where the general kernels have one per 16)
+    const int K = backward ? 4 * H : H, KS = cdiv(K, kstep_of(dtype)), KX = dtype == FASTLSTM_FP32 ? 3 * cdiv(K, 32) : KS;
     const int margin = (dtype != FASTLSTM_FP32 && H > 1024 && H <= 2048 && H % 256 == 0) ? 3 : 1;
     ws = std::max(ws, kWsHeaderBytes + kWsCounterBytes +
-                          (size_t)slots * (plan->batch_chunks * slot + (size_t)margin * KS * kFragBytes));
+                          (size_t)slots * (plan->batch_chunks * (slot / KS * KX) + (size_t)margin * KX * kFragBytes));
     // the reverse kernel of those hidden sizes exchanges partial sums among teams of workgroups: at most
     // 4 KiB per (receiver, sender), 256 workgroups
     if (backward && margin == 3) ws += (size_t)256 * 8 * 4 * kFragBytes;

@@ -27,11 +27,11 @@ struct BwdXcdParams {
     const void *Wh;     // [4H,H]
     WsHeader *hdr;
     int *counters;         // [groups][kXcdReplicas][kXcdCounterStride], zero at launch (XCD-local kernels: the barrier of their prologue)
-    unsigned char *xbuf;   // [kXchgSlots][groups][NT][KSB] operand blocks; reverse step s uses slot s % kXchgSlots
+    unsigned char *xbuf;   // [kXchgSlots][groups][NT][KSB] operand blocks (fp32: three each); reverse step s uses slot s % kXchgSlots
     int T, B, H;
     int n_ht, gpx, n_groups;
     int b_base;         // first batch row of this launch (a large batch runs as several launches over row ranges)
-    int KSB;            // k-steps covering 4H
+    int KSB;            // k-steps of 32 covering 4H
     // In-kernel dx = d_ifgo . Wx (HELP instantiations, k5_tiles_n > 0): the workgroups without a role
     // in the recurrence compute it in 256 x 256 tiles, latest timesteps first, as soon as the
     // recurrence has finished a chunk of k5_chunk_steps timesteps (k5_chunk_tiles row tiles);
@@ -349,6 +349,8 @@ template <typename T, int MT, int NKW, int NTW, int NWV, int HELP = 0>
 __global__ __launch_bounds__(kWave * NWV) void lstm_bwd_xcd_kernel(const BwdXcdParams p) {
     static_assert(!HELP || (NWV == 8 && sizeof(T) == 2), "the in-kernel GEMM tile is the 8-wave 16-bit one");
     using E = Elem<T>;
+    using X = OperandBlocks<T>;
+    constexpr int P = X::P;                            // parts of a number (recurrent_parts.hpp)
     constexpr bool ACC = (E::DT == FASTLSTM_FP32);
     constexpr int NTHR = kWave * NWV;
     constexpr int NT = NTW, HT = 16 * MT, BT = 16 * NT;
@@ -423,28 +425,25 @@ __global__ __launch_bounds__(kWave * NWV) void lstm_bwd_xcd_kernel(const BwdXcdP
 
     // ---- prologue: this wave's fragments of Wh[:, units]^T (fp32: gathered from global memory) ----
     // fragment (unit tile a, k-step ks): lane (q, r) holds row r = unit u0 + 16a + r and
-    // k = ks*KSTEP + q*EPL + e, e < EPL, with k = 4 * source unit + gate
-    u32x4 wreg[MT][NKW];
+    // k = 32 ks + 8 q + e, e < 8, with k = 4 * source unit + gate
+    u32x4 wreg[MT][NKW][P];
     if constexpr (E::BYTES == 2) {
         load_wh_transposed<T, MT, NKW>(Wh, H, u0, reinterpret_cast<unsigned char *>(red) + wave * MT * kFragBytes, KSB,
                                        [&](int ki) { return wave + NWV * ki; },
-                                       [&](auto ki, auto a, u32x4 f) { wreg[decltype(a)::value][decltype(ki)::value] = f; });
+                                       [&](auto ki, auto a, u32x4 f) { wreg[decltype(a)::value][decltype(ki)::value][0] = f; });
     } else {
 #pragma unroll
         for (int a = 0; a < MT; ++a)
 #pragma unroll
             for (int ki = 0; ki < NKW; ++ki) {
                 const int ks = wave + NWV * ki;
-                T tmp[E::EPL];
+                const int uk = ks * 8 + q * 2;   // source unit
+                const bool ok = ks < KSB && uk < H;   // (H is even)
+                const T *src = Wh + (size_t)(ok ? uk : 0) * H + u0 + a * 16 + r;
+                operand_parts<T>([&](int e) { return src[((size_t)(e & 3) * H + (e >> 2)) * H]; }, wreg[a][ki]);
 #pragma unroll
-                for (int e = 0; e < E::EPL; ++e) {
-                    const int k = ks * E::KSTEP + q * E::EPL + e;
-                    const int uk = k >> 2, gate = k & 3;
-                    const bool ok = ks < KSB && uk < H;
-                    const T v = Wh[ok ? ((size_t)gate * H + uk) * H + u0 + a * 16 + r : 0];
-                    tmp[e] = ok ? v : E::from_f32(0.f);
-                }
-                wreg[a][ki] = *reinterpret_cast<u32x4 *>(tmp);
+                for (int i = 0; i < P; ++i)
+                    if (!ok) wreg[a][ki][i] = u32x4{0u, 0u, 0u, 0u};
             }
     }
 
@@ -462,7 +461,7 @@ __global__ __launch_bounds__(kWave * NWV) void lstm_bwd_xcd_kernel(const BwdXcdP
         const int unit = u0 + ul, b = b0 + nt * 16 + n;
         valid[m] = nt < NT && b < B;
         off_h[m] = valid[m] ? (size_t)b * H + unit : (size_t)b0 * H + u0;
-        xoff[m] = (nt < NT ? nt : 0) * KSB * kFragBytes + frag_offset<T>(n, unit * 4);
+        xoff[m] = (nt < NT ? nt : 0) * KSB * X::BYTES + X::offset(n, unit * 4);
         stores[m] = nt < NT && (E::BYTES == 4 || (ul & 1) == 0);
         const int a = ul >> 4, ur = ul & 15;
         roff[m] = ((a * NT + (nt < NT ? nt : 0)) * kWave + (ur >> 2) * 16 + n) * 4 + (ur & 3);
@@ -473,15 +472,20 @@ __global__ __launch_bounds__(kWave * NWV) void lstm_bwd_xcd_kernel(const BwdXcdP
         c1v[m] = valid[m] ? E::to_f32(cell[(size_t)T_ * BH + off_h[m]]) : 0.f;
     }
 
-    const unsigned xgrp = (unsigned)vg * NT * KSB * kFragBytes;
-    const size_t xslot = (size_t)p.n_groups * n_layers * NT * KSB * kFragBytes;
+    const unsigned xgrp = (unsigned)vg * NT * KSB * X::BYTES;
+    const size_t xslot = (size_t)p.n_groups * n_layers * NT * KSB * X::BYTES;
     auto xslot_of = [&](int v) { return XchgL2(p.xbuf + (size_t)(v % kXchgSlots) * xslot, (unsigned)xslot); };
     int *grp_counters = p.counters + (size_t)vg * kXcdGroupStride;
     bool dead = false;   // the launch has given up (see poll_blocks)
     auto unwrite = [&](const XchgL2 &x) {
 #pragma unroll
         for (int m = 0; m < IPT; ++m)
-            if (stores[m]) x.store16(xgrp + xoff[m], u32x4{kUnwritten, kUnwritten, kUnwritten, kUnwritten});
+            if (stores[m]) {
+                if constexpr (P == 1) x.store16(xgrp + xoff[m], u32x4{kUnwritten, kUnwritten, kUnwritten, kUnwritten});
+                else
+#pragma unroll
+                    for (int i = 0; i < P; ++i) x.store8(xgrp + xoff[m] + i * kFragBytes, u32x2{kUnwritten, kUnwritten});
+            }
     };
     // every member has marked its part of the slots unwritten before any member stores or reads one
     for (int v = 0; v < kXchgSlots; ++v) unwrite(xslot_of(v));
@@ -675,10 +679,12 @@ __global__ __launch_bounds__(kWave * NWV) void lstm_bwd_xcd_kernel(const BwdXcdP
                 other[1] = (unsigned)__shfl_down((int)mine[1], 16);
                 if (stores[m]) xch.store16(xgrp + xoff[m], u32x4{mine[0], mine[1], other[0], other[1]});
             } else {
-                u32x4 mine = *reinterpret_cast<u32x4 *>(st_d);
+                const ThreeParts p0(st_d[0]), p1(st_d[1]), p2(st_d[2]), p3(st_d[3]);
+                if (stores[m])
 #pragma unroll
-                for (int e = 0; e < 4; ++e) mine[e] = written_word(mine[e]);
-                if (stores[m]) xch.store16(xgrp + xoff[m], mine);
+                    for (int i = 0; i < P; ++i)
+                        xch.store8(xgrp + xoff[m] + i * kFragBytes, u32x2{written_word(upper_halves(p0.part(i), p1.part(i))),
+                                                                          written_word(upper_halves(p2.part(i), p3.part(i)))});
             }
         }
         __syncthreads();   // the d_ifgo tile is complete (and everyone has read the partial sums of the step before)
@@ -706,19 +712,28 @@ __global__ __launch_bounds__(kWave * NWV) void lstm_bwd_xcd_kernel(const BwdXcdP
         // fetches per step (128 KiB for 16 rows at H = 1024) keeps its path to the L2 busy for most of the step and every
         // repeated block adds to that: H = 1024, B = 64 / 256, us per step: batches of 4 2.47 / 4.4, of 8 2.56 / 6.6
         // (spilled), of 16 2.88 / 12.8; with a counter barrier before the fetch 3.07 / 6.5.
-        constexpr int KB = 4 / NTW, NBATCH = NKW / KB;
+        // (fp32: six, three with groups of 32 rows: one batch tile at a time, what the registers hold)
+        constexpr int TB = P > 1 ? 1 : NTW, KB = P > 1 ? 2 / NTW : 4 / NTW;   // batch tiles and k-steps of a batch
+        constexpr int NBATCH = NKW / KB * (NTW / TB);
         static_assert(NKW % KB == 0, "whole batches");
-        u32x4 bq[2][KB * NTW];
-        auto block = [&](int k0, int i) {
-            const int ks = min(wave + NWV * (k0 + i / NTW), KSB - 1);   // past the end: any valid block (its weights are zero)
-            return xch.load16_l2(xgrp + (unsigned)(((i % NTW) * KSB + ks) * kWave + lane) * 16u);
+        constexpr int NBQ = KB * TB * P;
+        u32x4 bq[2][NBQ];
+        auto block = [&](int n, int i) {   // block i of batch n
+            const int tile = n % (NTW / TB) * TB + i / P % TB;
+            const int ks = min(wave + NWV * (n / (NTW / TB) * KB + i / (TB * P)), KSB - 1);   // past the end: any valid block (its weights are zero)
+            return xch.load16_l2(xgrp + (unsigned)((tile * KSB + ks) * X::BYTES + i % P * kFragBytes + lane * 16));
         };
+        f32x4 small[MT][NTW];
+#pragma unroll
+        for (int a = 0; a < MT; ++a)
+#pragma unroll
+            for (int i = 0; i < NTW; ++i) small[a][i] = f32x4{0.f, 0.f, 0.f, 0.f};
         poll_blocks(bq[0], [&](int i) { return block(0, i); }, dead, p.hdr, p.spin_limit, vg, s);
 #pragma unroll
         for (int n = 0; n < NBATCH; ++n) {
             if (n + 1 < NBATCH) {
 #pragma unroll
-                for (int i = 0; i < KB * NTW; ++i) bq[(n + 1) & 1][i] = block((n + 1) * KB, i);
+                for (int i = 0; i < NBQ; ++i) bq[(n + 1) & 1][i] = block(n + 1, i);
                 __builtin_amdgcn_sched_barrier(0);
             } else {   // the tile has left for memory: the next step's inputs take its place
                 if (s + 1 < T_) tiles_to_lds();
@@ -729,15 +744,21 @@ __global__ __launch_bounds__(kWave * NWV) void lstm_bwd_xcd_kernel(const BwdXcdP
 #pragma unroll
                 for (int a = 0; a < MT; ++a)
 #pragma unroll
-                    for (int i = 0; i < NTW; ++i) acc[a][i] = mfma_kstep<T>(wreg[a][n * KB + kk], bq[n & 1][kk * NTW + i], acc[a][i]);
+                    for (int i = 0; i < TB; ++i) {
+                        const int tile = n % (NTW / TB) * TB + i;
+                        u32x4 b[P];
+#pragma unroll
+                        for (int pp = 0; pp < P; ++pp) b[pp] = bq[n & 1][(kk * TB + i) * P + pp];
+                        mfma_parts<T, P>(wreg[a][n / (NTW / TB) * KB + kk], b, acc[a][tile], small[a][tile]);
+                    }
             __builtin_amdgcn_sched_barrier(0);
             if (n + 1 < NBATCH && any_unwritten(bq[(n + 1) & 1]))
-                poll_blocks(bq[(n + 1) & 1], [&](int i) { return block((n + 1) * KB, i); }, dead, p.hdr, p.spin_limit, vg, s);
+                poll_blocks(bq[(n + 1) & 1], [&](int i) { return block(n + 1, i); }, dead, p.hdr, p.spin_limit, vg, s);
         }
 #pragma unroll
         for (int a = 0; a < MT; ++a)
 #pragma unroll
-            for (int i = 0; i < NTW; ++i) red[((wave * MT + a) * NT + i) * kWave + lane] = acc[a][i];
+            for (int i = 0; i < NTW; ++i) red[((wave * MT + a) * NT + i) * kWave + lane] = P > 1 ? acc[a][i] + small[a][i] : acc[a][i];
         __syncthreads();
         // Every wave of this workgroup has seen its part of d_ifgo[t].  So every member has stored it, i.e. finished step
         // s-1, where the data of its loads had arrived -- and what each of its waves had stored before those loads

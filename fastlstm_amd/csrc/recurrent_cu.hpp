@@ -17,25 +17,11 @@
 // What bounds a step: its chain of latencies (LDS, MFMAs, gates, barrier).
 // Requirements (host): H a multiple of 16, rows and pointers 16-byte aligned.
 #pragma once
-#include "gemm_f32.hpp"
 #include "recurrent_bwd.hpp"
 #include "recurrent_fwd.hpp"
+#include "recurrent_parts.hpp"
 
 namespace fastlstm {
-
-// The three bf16 parts of a factor of a recurrent product.  A part that is zero where the number is not becomes the least normal
-// number of its sign, and those of an infinity too: infinity times zero would be no number.  Zero stays zero.
-struct ThreeParts {
-    float hi, mid, lo, least;   // (least: that number, for the last four columns)
-    __device__ __forceinline__ explicit ThreeParts(float x) {
-        const float tiny = fminf(fabsf(x), 0x1p-126f), r = x - upper_half(x);
-        least = __builtin_copysignf(tiny, x);
-        hi = __builtin_canonicalizef(x);
-        mid = __builtin_copysignf(fmaxf(fabsf(r), tiny), x);
-        lo = __builtin_copysignf(fmaxf(fabsf(r - upper_half(mid)), tiny), x);
-    }
-    __device__ __forceinline__ float part(int i) const { return i == 0 ? hi : i == 1 ? mid : i == 2 ? lo : least; }
-};
 
 template <typename T, int CW> struct CuShape {
     static constexpr bool F32 = sizeof(T) == 4;
@@ -48,26 +34,6 @@ template <typename T, int CW> struct CuShape {
     static constexpr int SET = 4 * GROW + 2 * 4 * SROW;                // LDS tiles of a step: gates, two state tiles
     static constexpr int lds_bytes(bool backward) { return 2 * (backward ? KB : KF) * kFragBytes + 2 * SET; }
 };
-
-// 16 bytes of operand block: 8 consecutive elements of k -> the 16-bit fragment of part i
-template <typename T, typename Get> __device__ __forceinline__ void operand_parts(Get get, u32x4 (&out)[sizeof(T) == 4 ? 3 : 1]) {
-    if constexpr (sizeof(T) == 4) {
-#pragma unroll
-        for (int d = 0; d < 4; ++d) {
-            const ThreeParts a(get(2 * d)), b(get(2 * d + 1));
-#pragma unroll
-            for (int i = 0; i < 3; ++i) out[i][d] = upper_halves(a.part(i), b.part(i));
-        }
-    } else {
-        T t[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e) t[e] = get(e);
-        __builtin_memcpy(&out[0], t, 16);
-    }
-}
-
-// the 16-bit type whose MFMAs multiply
-template <typename T> using CuOperand = typename std::conditional<sizeof(T) == 4, __bf16, T>::type;
 
 // One value per lane: tile j's columns 0 .. 3 for lanes 4j .. 4j + 3.  fp32: the four groups of columns are
 // added first, in all lanes: two additions with a rotation each, then the lanes of a tile only have to pick.
@@ -133,7 +99,7 @@ template <typename T, int CW>
 __global__ __launch_bounds__((CuShape<T, CW>::THREADS)) void lstm_fwd_cu_kernel(const FwdParams p) {
     using C = CuShape<T, CW>;
     using E = Elem<T>;
-    using O = CuOperand<T>;
+    using O = OperandType<T>;
     constexpr int H = C::H, KS = C::KF, P = C::P, PD = 4;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     unsigned char *const xl = smem, *const tiles = smem + 2 * KS * kFragBytes;   // operand blocks of h_t; tile sets of two steps
@@ -272,7 +238,7 @@ template <typename T, int CW>
 __global__ __launch_bounds__((CuShape<T, CW>::THREADS)) void lstm_bwd_cu_kernel(const BwdParams p) {
     using C = CuShape<T, CW>;
     using E = Elem<T>;
-    using O = CuOperand<T>;
+    using O = OperandType<T>;
     constexpr int H = C::H, KS = C::KB, P = C::P, PD = 4;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     unsigned char *const xl = smem, *const tiles = smem + 2 * KS * kFragBytes;   // operand blocks of d_ifgo[t]; tile sets of two steps

@@ -29,13 +29,16 @@
 //    (32 CUs x 160 KiB < 8 MiB for H = 1024): every wave keeps its K-share of the slice, MT x NKW
 //    operand fragments, in registers (up to 256 of the 512 per lane).
 // Requirements (host): H a multiple of the tile width and of 16 bytes' worth of elements,
-// H / (4*MT) <= 32 members, ceil(H / KSTEP) <= 4*NKW k-steps, all batch tiles in one launch.
+// H / (4*MT) <= 32 members, ceil(H / 32) <= 4*NKW k-steps, all batch tiles in one launch.
+//  * fp32: numbers travel and multiply as their three bf16 parts (recurrent_parts.hpp), split by the member that computes them: six
+//    MFMAs of 16 cycles per 16 x 16 x 32, where v_mfma_f32_16x16x4_f32 took 256 cycles, for half as many bytes again to exchange.
 #pragma once
 #include <type_traits>
 
 #include "gemm.hpp"
 #include "gemm16.hpp"
 #include "recurrent_common.hpp"
+#include "recurrent_parts.hpp"
 
 namespace fastlstm {
 
@@ -52,13 +55,13 @@ struct FwdXcdParams {
     const void *Wh;    // [4H,H]
     WsHeader *hdr;
     int *counters;        // [groups][kXcdReplicas][kXcdCounterStride], zero at launch (XCD-local kernels: the barrier of their prologue)
-    unsigned char *xbuf;  // [kXchgSlots][groups][NT][KS] operand blocks; h_v lives in slot v % kXchgSlots
+    unsigned char *xbuf;  // [kXchgSlots][groups][NT][KS] operand blocks (fp32: three each); h_v lives in slot v % kXchgSlots
     int T, B, H;
     int n_ht;          // members of a barrier group (<= 32)
     int gpx;           // groups per XCD (32 / n_ht)
     int n_groups;      // batch tiles of this launch (<= 8 * gpx)
     int b_base;        // first batch row of this launch (a large batch runs as several launches over row ranges)
-    int KS;            // k-steps covering H
+    int KS;            // k-steps of 32 covering H
     // In-kernel input projection (HELP instantiations, k1_tiles_n > 0): the workgroups without a
     // role in the recurrence compute ifgo = x.Wx^T + b in 256 x 256 tiles, earliest timesteps first;
     // k1_done[c] counts the finished tiles of chunk c (k1_chunk_tiles row tiles = k1_chunk_steps
@@ -107,7 +110,6 @@ struct XchgL2 {
         if constexpr (sizeof(T) == 2) __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, v), rsrc, off, 0, 0);
         else __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), rsrc, off, 0, 0);
     }
-    __device__ __forceinline__ void store4(unsigned off, unsigned v) const { __builtin_amdgcn_raw_buffer_store_b32(v, rsrc, off, 0, 0); }
     __device__ __forceinline__ void store8(unsigned off, u32x2 v) const { __builtin_amdgcn_raw_buffer_store_b64(v, rsrc, off, 0, 0); }
     __device__ __forceinline__ void store16(unsigned off, u32x4 v) const { __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, off, 0, 0); }
 };
@@ -296,6 +298,8 @@ __global__ __launch_bounds__(kWave * NWV) void lstm_fwd_xcd_kernel(const FwdXcdP
     static_assert(NWV == 4 || NWV == 8, "4 or 8 waves");
     static_assert(MT % MW == 0, "unit tiles divide among the waves of a K-share");
     using E = Elem<T>;
+    using X = OperandBlocks<T>;
+    constexpr int P = X::P;                            // parts of a number (recurrent_parts.hpp)
     constexpr bool ACC = (E::DT == FASTLSTM_FP32);
     constexpr int NT = NTW, TILES = MT * NT;
     constexpr int IPT = (TILES + NWV - 1) / NWV;     // (tile, lane) items per thread
@@ -356,20 +360,28 @@ __global__ __launch_bounds__(kWave * NWV) void lstm_fwd_xcd_kernel(const FwdXcdP
 
     // ---- prologue 1: this wave's fragments of the W_h slice, global -> registers ---------
     // fragment (m-tile a, k-step ks): lane (q, r) holds row r = (unit a*4 + r/4, gate r%4),
-    // k = ks*KSTEP + q*EPL .. + EPL-1, i.e. 16 contiguous bytes of W_h
+    // k = 32 ks + 8 q .. + 7 (16-bit: 16 contiguous bytes of W_h)
     const int kq = wave % SH, mh = wave / SH;        // K-share and M-part of this wave
-    u32x4 wreg[MTW][NKS];
+    u32x4 wreg[MTW][NKS][P];
 #pragma unroll
     for (int a = 0; a < MTW; ++a)
 #pragma unroll
         for (int ki = 0; ki < NKS; ++ki) {
             const int ks = kq + SH * ki;
             const int unit = u0 + (mh * MTW + a) * 4 + (n >> 2), gate = n & 3;
-            const int k0 = ks * E::KSTEP + q * E::EPL;
-            const bool ok = ks < KS && k0 < H;   // H % EPL == 0: a piece is inside or outside as a whole
+            const int k0 = ks * X::KSTEP + q * 8;
+            const bool ok = ks < KS && k0 < H;   // H % 8 == 0: a piece is inside or outside as a whole
             const size_t off = ok ? ((size_t)gate * H + unit) * H + k0 : 0;
-            const u32x4 v = *reinterpret_cast<const u32x4 *>(Wh + off);
-            wreg[a][ki] = ok ? v : u32x4{0u, 0u, 0u, 0u};
+            if constexpr (P == 1) {
+                wreg[a][ki][0] = *reinterpret_cast<const u32x4 *>(Wh + off);
+            } else {
+                const f32x4 lo = *reinterpret_cast<const f32x4 *>(Wh + off), hi = *reinterpret_cast<const f32x4 *>(Wh + off + 4);
+                const float w[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
+                operand_parts<T>([&](int e) { return w[e]; }, wreg[a][ki]);
+            }
+#pragma unroll
+            for (int i = 0; i < P; ++i)
+                if (!ok) wreg[a][ki][i] = u32x4{0u, 0u, 0u, 0u};
         }
 
     // ---- per-thread items: (tile = wave + NWV m, lane) -> (unit, batch row) -------------
@@ -384,38 +396,41 @@ __global__ __launch_bounds__(kWave * NWV) void lstm_fwd_xcd_kernel(const FwdXcdP
         const int unit = u0 + mt * 4 + q, b = b0 + nt * 16 + n;
         valid[m] = (tile < TILES) && b < B;
         off_h[m] = valid[m] ? (size_t)b * H + unit : (size_t)b0 * H + u0;
-        // the exchange word(s) of the item: fp32 its own, 16-bit types the four units of a tile row by lanes 0 .. 15
-        xoff[m] = nt * KS * kFragBytes + frag_offset<T>(n, E::BYTES == 4 ? unit : u0 + mt * 4);
+        // the exchange words of the item: the four units of a tile row by lanes 0 .. 15
+        xoff[m] = nt * KS * X::BYTES + X::offset(n, u0 + mt * 4);
         goff[m] = (nt * 16 + n) * GROW + (mt * 4 + q) * E::BYTES;
         soff[m] = (nt * 16 + n) * SROW + (mt * 4 + q) * E::BYTES;
         c_state[m] = valid[m] ? E::to_f32(cell[off_h[m]]) : 0.f;
     }
 
-    const unsigned xgrp = (unsigned)vg * NT * KS * kFragBytes;
-    const size_t xslot = (size_t)p.n_groups * n_layers * NT * KS * kFragBytes;
+    const unsigned xgrp = (unsigned)vg * NT * KS * X::BYTES;
+    const size_t xslot = (size_t)p.n_groups * n_layers * NT * KS * X::BYTES;
     auto xslot_of = [&](int v) { return XchgL2(p.xbuf + (size_t)(v % kXchgSlots) * xslot, (unsigned)xslot); };
     int *grp_counters = p.counters + (size_t)vg * kXcdGroupStride;
     bool dead = false;   // the launch has given up (see poll_blocks)
 
     // this wave's part of a slot: the words of its tiles
     auto store_h = [&](const XchgL2 &x, int m, T h) {
-        if constexpr (E::BYTES == 4) {
-            x.store4(xgrp + xoff[m], written_word(__builtin_bit_cast(unsigned, h)));
-        } else {   // the four lane groups hold units 0 .. 3 of the tile: lanes 0 .. 15 get all four of their row
-            const unsigned mine = __builtin_bit_cast(unsigned short, h);
+        auto store = [&](unsigned mine, int part) {   // the four lane groups hold units 0 .. 3 of the tile: lanes 0 .. 15 get all four of their row
             const auto s16 = __builtin_amdgcn_permlane16_swap(mine, mine, false, false);
             const unsigned pair = written_word(s16[0] | (s16[1] << 16));
             const auto s32 = __builtin_amdgcn_permlane32_swap(pair, pair, false, false);
-            if (q == 0) x.store8(xgrp + xoff[m], u32x2{s32[0], s32[1]});
+            if (q == 0) x.store8(xgrp + xoff[m] + part * kFragBytes, u32x2{s32[0], s32[1]});
+        };
+        if constexpr (P == 1) {
+            store(__builtin_bit_cast(unsigned short, h), 0);
+        } else {
+            const ThreeParts s(h);
+#pragma unroll
+            for (int i = 0; i < P; ++i) store(__builtin_bit_cast(unsigned, s.part(i)) >> 16, i);
         }
     };
     auto unwrite = [&](const XchgL2 &x) {
 #pragma unroll
         for (int m = 0; m < IPT; ++m)
-            if (wave + NWV * m < TILES) {
-                if constexpr (E::BYTES == 4) x.store4(xgrp + xoff[m], kUnwritten);
-                else if (q == 0) x.store8(xgrp + xoff[m], u32x2{kUnwritten, kUnwritten});
-            }
+            if (wave + NWV * m < TILES && q == 0)
+#pragma unroll
+                for (int i = 0; i < P; ++i) x.store8(xgrp + xoff[m] + i * kFragBytes, u32x2{kUnwritten, kUnwritten});
     };
 
     // ---- prologue 2: h_0 into slot 0 (zeros for rows past the batch), the other slots unwritten; every member waits
@@ -424,6 +439,11 @@ __global__ __launch_bounds__(kWave * NWV) void lstm_fwd_xcd_kernel(const FwdXcdP
     for (int m = 0; m < IPT; ++m)
         if (wave + NWV * m < TILES) store_h(xslot_of(0), m, valid[m] ? out[off_h[m]] : E::from_f32(0.f));
     for (int v = 1; v < kXchgSlots; ++v) unwrite(xslot_of(v));
+    if (P > 1 && H % X::KSTEP != 0 && j == 0 && tid < 32) {   // (fp32) the upper half of the last k-step is nobody's: zeros, for good
+        for (int v = 0; v < kXchgSlots; ++v)
+            for (int i = 0; i < NT * P; ++i)
+                xslot_of(v).store16(xgrp + (unsigned)((i / P * KS + KS - 1) * X::BYTES + i % P * kFragBytes + 512 + tid * 16), u32x4{0u, 0u, 0u, 0u});
+    }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's exchange stores have reached the L2
     __syncthreads();
     if (tid < kXcdReplicas)
@@ -535,13 +555,19 @@ __global__ __launch_bounds__(kWave * NWV) void lstm_fwd_xcd_kernel(const FwdXcdP
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (the workgroup barrier of step 0 orders it before the tile's use)
     }
 
+#if defined(__HIP_DEVICE_COMPILE__)
+    // The loop starts 28 bytes behind a multiple of 32 (two instructions follow these): its step depends on where it lies against the
+    // 32 bytes of an instruction fetch.  T = 512, B = 64, I = H = 1024 fp16 inference at 28, 16, 24, 8, 0: 0.965, 0.978, 0.988, 1.003,
+    // 1.003 ms; the other residues lie between.
+    if constexpr (HELP && NTW == 1) asm volatile(".p2align 6\n\t.rept 5\n\ts_nop 0\n\t.endr" ::: "memory");
+#endif
     for (int t = 0; t < T_; ++t) {
         // ---- h_t: this wave's operand blocks, as soon as their members have stored them --------------------------
         const XchgL2 xr = xslot_of(t);
-        u32x4 bq[NKS * NTW];
+        u32x4 bq[NKS * NTW * P];
         poll_blocks(bq, [&](int i) {
-            const int ks = min(kq + SH * (i / NTW), KS - 1);   // past the end: any valid block (its weights are zero)
-            return xr.load16_l2(xgrp + (unsigned)(((i % NTW) * KS + ks) * kWave + lane) * 16u);
+            const int ks = min(kq + SH * (i / (NTW * P)), KS - 1);   // past the end: any valid block (its weights are zero)
+            return xr.load16_l2(xgrp + (unsigned)((i / P % NTW * KS + ks) * X::BYTES + i % P * kFragBytes + lane * 16));
         }, dead, p.hdr, p.spin_limit, vg, t);
         if (t + 1 < T_) tile_to_lds(t + 1);
         fetch_tile(t + PD);   // (its chunk has landed: wave 0 has waited for it behind an earlier workgroup barrier)
@@ -558,10 +584,21 @@ __global__ __launch_bounds__(kWave * NWV) void lstm_fwd_xcd_kernel(const FwdXcdP
             for (int a = 0; a < MTW; ++a) {
 #pragma unroll
                 for (int i = 0; i < NTW; ++i) acc[a][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+                f32x4 small[NTW];
+#pragma unroll
+                for (int i = 0; i < NTW; ++i) small[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int ki = 0; ki < NKS; ++ki)
 #pragma unroll
-                    for (int i = 0; i < NTW; ++i) acc[a][i] = mfma_kstep<T>(wreg[a][ki], bq[ki * NTW + i], acc[a][i]);
+                    for (int i = 0; i < NTW; ++i) {
+                        u32x4 b[P];
+#pragma unroll
+                        for (int pp = 0; pp < P; ++pp) b[pp] = bq[(ki * NTW + i) * P + pp];
+                        mfma_parts<T, P>(wreg[a][ki], b, acc[a][i], small[i]);
+                    }
+                if constexpr (P > 1)
+#pragma unroll
+                    for (int i = 0; i < NTW; ++i) acc[a][i] += small[i];
                 __builtin_amdgcn_sched_barrier(0);
                 if (a > 0) {
                     put(a - 1);

@@ -1,0 +1,48 @@
+"""fp32 recurrences whose numbers travel and multiply as three bf16 parts (csrc/recurrent_parts.hpp): half k-steps (H = 16 mod 32), every
+unit tile and batch tile of the XCD-local kernels, against float64; numbers that are not finite."""
+import numpy as np
+import pytest
+import torch
+
+from fastlstm_amd import _lib
+from helpers import nn_lstm_reference
+from test_gpu_one_cu import operands, run
+
+pytestmark = pytest.mark.gpu
+
+
+# (B, H): 16- and 32-row groups, one and two unit tiles, half and whole last k-steps, rows over several launches
+@pytest.mark.parametrize("B,H", [(3, 112), (17, 144), (5, 208), (33, 256), (150, 256), (300, 272), (9, 400), (128, 512), (140, 512), (600, 320)])
+def test_against_float64(B, H):
+    T = 7
+    p, g = operands(T, B, H, torch.float32, seed=H + B)
+    want = nn_lstm_reference({k: v.double() for k, v in p.items()})
+    out, cell, ifgo, d_ifgo, dh, dc = run(g)
+    dx = d_ifgo.double().view(T * B, -1) @ g["Wx"].double()
+    for name, a, b in (("out", out[1:], want["out"]), ("c_n", cell[-1], want["c_n"]), ("dh0", dh, want["dh0"]), ("dc0", dc, want["dc0"]),
+                       ("dx", dx, want["dx"].reshape(T * B, -1))):
+        a, b = a.double().cpu().numpy(), b.numpy()
+        assert np.linalg.norm(a - b) <= 1e-6 * np.linalg.norm(b), name   # (2-norm: some 2e-7 from the rounding of every step's results)
+
+
+@pytest.mark.parametrize("B,H", [(9, 112), (40, 512)])
+@pytest.mark.parametrize("weight", [False, True])
+def test_numbers_that_are_not_finite(B, H, weight):
+    """As test_gpu_one_cu's: the general kernels' entries are infinite, NaN and finite where these are."""
+    g = operands(4, B, H, torch.float32, seed=3)[1]
+    inf = float("inf")
+    g["h0"][2, 5], g["h0"][3, 6], g["h0"][4, 7], g["dh_n"][6, 4] = inf, -inf, float("nan"), inf
+    g["Wh"][7, 5], g["Wh"][8, 6] = 0.5, 0.0
+    if weight:
+        g["Wh"][H + 3, 11] = inf
+    lib = _lib.load()
+    fast = run(g)
+    lib.fastlstm_set_kernel_families(0)
+    try:
+        slow = run(g)
+    finally:
+        lib.fastlstm_set_kernel_families(7)
+    for a, b in list(zip(fast, slow))[:3 if weight else 6]:
+        assert torch.equal(torch.isnan(a), torch.isnan(b)) and torch.equal(torch.isinf(a), torch.isinf(b))
+        ok = torch.isfinite(b)
+        assert bool(ok.any()) and not bool(ok.all()) and float((a - b)[ok].abs().max()) < 1e-4
