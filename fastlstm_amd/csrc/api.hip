@@ -549,12 +549,12 @@ static bool clear_xcd_counters(unsigned char *wsb, hipStream_t s) {
 }
 
 // Shape of a launch of the register-resident kernels whose barrier groups span several XCDs
-// (recurrent_fwd_wide.hpp): 16 units x 16 nt batch rows per workgroup, H / 16 workgroups per group; or, 16-bit, 32 units per
-// workgroup (recurrent_fwd_big.hpp).
+// (recurrent_fwd_wide.hpp): 16 units x 16 nt batch rows per workgroup, H / 16 workgroups per group; or (recurrent_fwd_big.hpp)
+// 32 units per workgroup, in fp32 16.
 struct WideCfg {
     int nkw, n_ht, xpg, n_groups, ks, lds;
     int nt;   // batch tiles of 16 rows per group: the smallest of 1, 2, 4 with which the launch holds the batch
-    int big;  // batch tiles per group of the kernels with 32 units per workgroup (recurrent_fwd_big.hpp), else 0
+    int big;  // batch tiles per group of the whole-CU kernels (recurrent_fwd_big.hpp), else 0
     size_t xslot;
 };
 // copies > 1: that many recurrences of this shape share the launch (groups of 16 or 32 rows only).
@@ -565,10 +565,27 @@ bool select_wide(int T, int B_all, int H, int dtype, bool backward, size_t ws_by
         return false;
     // a weight row of 2.5 ... 4 KiB in steps of 512 bytes: H = 1280, 1536, 1792, 2048 with 16-bit elements,
     // 640, 768, 896, 1024 with fp32
-    const int es = elem_bytes(dtype), kstep = dtype == FASTLSTM_FP32 ? 16 : 32;
+    const int es = elem_bytes(dtype);
     if ((H * es) % 512 || H * es <= 2048 || H * es > 4096) return false;
-    c->ks = (backward ? 4 * H : H) / kstep;
+    c->ks = (backward ? 4 * H : H) / 32;
     c->big = 0;
+    if (dtype == FASTLSTM_FP32) {
+        // The whole-CU kernels with 16 units per workgroup, numbers as three parts; two recurrences side by side at most.  us
+        // per step of lstm_fwd_wide_kernel and lstm_bwd_wide_kernel on fp32 operands (forward up to 32 rows: of the general
+        // kernel) and here, forward, reverse: H = 1024, B = 128 11.1 -> 7.9, 12.4 -> 10.4; B = 16 5.1 -> 3.9, 6.6 -> 5.9.
+        const int n_ht = H / 16, max_groups = kNumXcd * 32 / n_ht;
+        const int nt = copies * cdiv(B, 16) <= max_groups ? 1 : 2, groups = cdiv(B, 16 * nt);
+        const size_t xslot = (size_t)groups * nt * c->ks * 3 * kFragBytes;
+        const size_t partials = backward ? (size_t)groups * n_ht * kBigTeam * nt * kFragBytes : 0;
+        if (copies > 2 || copies * groups > std::min(max_groups, kNumXcd) ||
+            ws_bytes < kWsHeaderBytes + kWsCounterBytes + copies * (2 * xslot + partials))
+            return false;
+        c->big = nt;
+        c->n_ht = n_ht;
+        c->n_groups = groups;
+        c->xslot = xslot;
+        return true;
+    }
     // Two recurrences side by side: the reverse kernel of a call by itself for a pair too (other kernels take the sums in another
     // order: dh_0 and dc_0 of the two ways would differ in their last bits), where the forward pass of the pair is one launch
     // (below: groups of at most 32 rows of the 16-unit form) -- a caller finds a pair fused in both directions or in neither.
@@ -603,15 +620,8 @@ bool select_wide(int T, int B_all, int H, int dtype, bool backward, size_t ws_by
     // CU then fetches a quarter or half of the operand bytes per step
     c->nt = copies * cdiv(B, 16) * c->xpg <= kNumXcd ? 1 : copies * cdiv(B, 32) * c->xpg <= kNumXcd ? 2 : 4;
     if (copies > 1 && c->nt == 4) return false;
-    // fp32 multiplies at 1/16 of the 16-bit rate: 16 units x 64 rows per CU are more MFMA time than a step of the
-    // general kernels, which spread 4 units x all rows over every CU
-    if (dtype == FASTLSTM_FP32 && c->nt == 4) return false;
     c->n_groups = cdiv(B, 16 * c->nt);
     if (copies * c->n_groups * c->xpg > kNumXcd) return false;
-    // ... and a small fp32 batch leaves most CUs without a share of the forward product (B = 32, H = 1024: 6.0
-    // instead of 5.7 us per step; the reverse step, with four times the operand bytes, gains at every size)
-    // (a remainder of rows behind full launches still runs here: the general kernel would take the whole batch)
-    if (dtype == FASTLSTM_FP32 && !backward && copies * c->n_groups * c->xpg < 6 && B == B_all) return false;
     c->xslot = (size_t)c->n_groups * c->nt * c->ks * kFragBytes;
     if (ws_bytes < kWsHeaderBytes + kWsCounterBytes + 2 * (size_t)copies * c->xslot) return false;
     const int gr = 16 * c->nt;
@@ -622,12 +632,13 @@ bool select_wide(int T, int B_all, int H, int dtype, bool backward, size_t ws_by
 }
 
 // Rows per launch (see xcd_rows_per_launch) for the register-resident kernels: full launches of 64-row groups
-// (fp32: 32-row groups) on all XCDs.
+// (whole-CU kernels: of 32-row groups) on all XCDs.
 static int wide_rows_per_launch(int T, int B, int H, int dtype, bool backward, size_t ws_bytes) {
     const int xpg = cdiv(H / 16, 32);
-    const int rows = backward && dtype != FASTLSTM_FP32 && H >= 32 && (g_families.load() & 4)
+    const int rows = dtype == FASTLSTM_FP32 ? 32 * std::min(kNumXcd, kNumXcd * 32 / std::max(1, H / 16))   // (two batch tiles per group)
+                     : backward && H >= 32 && (g_families.load() & 4)
                          ? 32 * (kNumXcd * 32 / (H / 32))   // (groups of the 32-unit form)
-                         : (dtype == FASTLSTM_FP32 ? 32 : 64) * (kNumXcd / std::max(1, xpg));
+                         : 64 * (kNumXcd / std::max(1, xpg));
     if (rows >= B || rows <= 0) return 0;
     WideCfg c;
     if (!select_wide(T, B, H, dtype, backward, ws_bytes, &c, rows)) return 0;
@@ -654,11 +665,14 @@ int try_fwd_wide(void *ifgo, void *out, void *cell, const void *Wh, unsigned cha
         q.b_base = o.row0; q.n_bt = c.n_groups; q.n_ht = c.n_ht;
         q.KS = q.KSP = c.ks;
         q.keep = o.keep;
+        q.n_rec = copies;
+        if (second) { q.ifgo2 = second->ifgo; q.out2 = second->out; q.cell2 = second->cell; q.Wh2 = second->Wh; }
         q.spin_limit = spin_limit_ticks();
+        const int mt = dtype == FASTLSTM_FP32 ? 4 : 8;
         int occ = 0;
-        if (launch_fwd_big(dtype, q, H / 128, 8, c.big, 0, nullptr, &occ) != hipSuccess) return FASTLSTM_ERR_HIP;
+        if (launch_fwd_big(dtype, q, H / 128, mt, c.big, 0, nullptr, &occ) != hipSuccess) return FASTLSTM_ERR_HIP;
         if (occ < 1) return 1;
-        if (!dry_run && launch_fwd_big(dtype, q, H / 128, 8, c.big, c.n_groups * c.n_ht, stream, nullptr) != hipSuccess) return FASTLSTM_ERR_HIP;
+        if (!dry_run && launch_fwd_big(dtype, q, H / 128, mt, c.big, copies * c.n_groups * c.n_ht, stream, nullptr) != hipSuccess) return FASTLSTM_ERR_HIP;
         return FASTLSTM_OK;
     }
     FwdXcdParams p{};
@@ -678,7 +692,7 @@ int try_fwd_wide(void *ifgo, void *out, void *cell, const void *Wh, unsigned cha
     p.b_base = o.row0;
     p.spin_limit = spin_limit_ticks();
     p.keep = o.keep;
-    auto launch = dtype == FASTLSTM_FP16 ? launch_fwd_wide_f16 : dtype == FASTLSTM_BF16 ? launch_fwd_wide_bf16 : launch_fwd_wide_f32;
+    auto launch = dtype == FASTLSTM_FP16 ? launch_fwd_wide_f16 : launch_fwd_wide_bf16;
     int occ = 0;
     if (launch(p, c.nkw, c.nt, 0, c.lds, nullptr, &occ) != hipSuccess) return FASTLSTM_ERR_HIP;
     if (occ < 1) return 1;
@@ -713,11 +727,12 @@ int try_bwd_wide(const void *dout, void *dh, void *dc, const void *ifgo, const v
         q.b_base = o.row0; q.n_bt = c.n_groups; q.n_ht = c.n_ht;
         q.KSB = q.KSBP = c.ks;
         q.spin_limit = spin_limit_ticks();
+        const int mt = dtype == FASTLSTM_FP32 ? 4 : 8;
         int occ = 0;
-        if (launch_bwd_big(dtype, q, H / 128, 8, c.big, 0, nullptr, &occ) != hipSuccess) return FASTLSTM_ERR_HIP;
+        if (launch_bwd_big(dtype, q, H / 128, mt, c.big, 0, nullptr, &occ) != hipSuccess) return FASTLSTM_ERR_HIP;
         if (occ < 1) return 1;
         const int grid = kNumXcd * cdiv(copies * c.n_groups * c.n_ht / kBigTeam, kNumXcd) * kBigTeam;
-        if (!dry_run && launch_bwd_big(dtype, q, H / 128, 8, c.big, grid, stream, nullptr) != hipSuccess) return FASTLSTM_ERR_HIP;
+        if (!dry_run && launch_bwd_big(dtype, q, H / 128, mt, c.big, grid, stream, nullptr) != hipSuccess) return FASTLSTM_ERR_HIP;
         return FASTLSTM_OK;
     }
     BwdXcdParams p{};
@@ -739,7 +754,7 @@ int try_bwd_wide(const void *dout, void *dh, void *dc, const void *ifgo, const v
     p.n_ht = c.n_ht; p.gpx = c.xpg; p.n_groups = c.n_groups; p.KSB = c.ks;
     p.b_base = o.row0;
     p.spin_limit = spin_limit_ticks();
-    auto launch = dtype == FASTLSTM_FP16 ? launch_bwd_wide_f16 : dtype == FASTLSTM_BF16 ? launch_bwd_wide_bf16 : launch_bwd_wide_f32;
+    auto launch = dtype == FASTLSTM_FP16 ? launch_bwd_wide_f16 : launch_bwd_wide_bf16;
     int occ = 0;
     if (launch(p, c.nkw, c.nt, 0, c.lds, nullptr, &occ) != hipSuccess) return FASTLSTM_ERR_HIP;
     if (occ < 1) return 1;
@@ -2223,7 +2238,8 @@ int fastlstm_recurrent_kernel_kind(int T, int B, int H, int dtype, int backward,
     XcdCfg c;
     if (select_xcd(T, B, H, dtype, backward != 0, ws_bytes, &c)) return 1;
     WideCfg w;
-    if (select_wide(T, B, H, dtype, backward != 0, ws_bytes, &w)) return 2;
+    // (fp32 forward calls of up to 32 rows have always been kind 0 here, and callers choose sizes by that)
+    if (select_wide(T, B, H, dtype, backward != 0, ws_bytes, &w)) return dtype == FASTLSTM_FP32 && !backward && B <= 32 ? 0 : 2;
     if (xcd_rows_per_launch(T, B, H, dtype, backward != 0, ws_bytes)) return 1;
     return wide_rows_per_launch(T, B, H, dtype, backward != 0, ws_bytes) ? 2 : 0;
 }

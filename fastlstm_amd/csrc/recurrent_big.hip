@@ -1,4 +1,4 @@
-// Instantiates the whole-CU kernels (recurrent_fwd_big.hpp, recurrent_bwd_big.hpp) for the 16-bit element types.
+// Instantiates the whole-CU kernels (recurrent_fwd_big.hpp, recurrent_bwd_big.hpp) .
 #include "recurrent_bwd_big.hpp"
 #include "recurrent_launch.hpp"
 
@@ -36,14 +36,32 @@ static hipError_t bwd_big_t(const BwdStreamParams &p, int kw, int mt, int nt, in
     return hipErrorInvalidConfiguration;
 }
 
+// fp32, H = 128 KW in 640 ... 1024: 16 units per workgroup, all weights in registers as three parts
+static hipError_t fwd_big_f32(const FwdStreamParams &p, int kw, int nt, int grid, int lds, hipStream_t s, int *occ) {
+#define CASE(KW, NT) \
+    if (kw == KW && nt == NT) return launch_one(lstm_fwd_big_parts_kernel<float, KW, 4, NT>, p, grid, lds, s, occ)
+    CASE(5, 1); CASE(5, 2); CASE(6, 1); CASE(6, 2); CASE(7, 1); CASE(7, 2); CASE(8, 1); CASE(8, 2);
+#undef CASE
+    return hipErrorInvalidConfiguration;
+}
+static hipError_t bwd_big_f32(const BwdStreamParams &p, int kw, int nt, int grid, int lds, hipStream_t s, int *occ) {
+#define CASE(KW, NT) \
+    if (kw == KW && nt == NT) return launch_one(lstm_bwd_big_parts_kernel<float, KW, 4, NT>, p, grid, lds, s, occ)
+    CASE(5, 1); CASE(5, 2); CASE(6, 1); CASE(6, 2); CASE(7, 1); CASE(7, 2); CASE(8, 1); CASE(8, 2);
+#undef CASE
+    return hipErrorInvalidConfiguration;
+}
+
 hipError_t launch_fwd_big(int dtype, const FwdStreamParams &p, int kw, int mt, int nt, int grid, hipStream_t s, int *occ) {
-    const int lds = big_lds_bytes(kw, mt, nt);
+    const int lds = big_lds_bytes(kw, mt, nt, elem_bytes(dtype));
+    if (dtype == FASTLSTM_FP32) return fwd_big_f32(p, kw, nt, grid, lds, s, occ);
     if (dtype == FASTLSTM_FP16) return fwd_big_t<_Float16>(p, kw, mt, nt, grid, lds, s, occ);
     return fwd_big_t<__bf16>(p, kw, mt, nt, grid, lds, s, occ);
 }
 
 hipError_t launch_bwd_big(int dtype, const BwdStreamParams &p, int kw, int mt, int nt, int grid, hipStream_t s, int *occ) {
-    const int lds = big_lds_bytes(kw, mt, nt);
+    const int lds = big_lds_bytes(kw, mt, nt, elem_bytes(dtype));
+    if (dtype == FASTLSTM_FP32) return bwd_big_f32(p, kw, nt, grid, lds, s, occ);
     if (dtype == FASTLSTM_FP16) return bwd_big_t<_Float16>(p, kw, mt, nt, grid, lds, s, occ);
     return bwd_big_t<__bf16>(p, kw, mt, nt, grid, lds, s, occ);
 }

@@ -1,7 +1,6 @@
 // Persistent reverse-time kernel for hidden sizes whose W_h does not fit the CUs of one XCD
-// (H = 640 ... 1024 in fp32, 1280 ... 2048 with 16-bit elements): the counterpart of lstm_fwd_wide_kernel.  Same mathematics
-// and results as lstm_bwd_persistent_kernel (which replaces fastlstm/kernels.py:1201-1409).  In 16 bits lstm_bwd_big_kernel is
-// faster at every size (us per step, here and there: H = 2048, 128 rows 11.0, 8.6; 32 rows 6.4, 5.3; a pair of H = 2048, B = 32
+// (1280 ... 2048, 16-bit elements): the counterpart of lstm_fwd_wide_kernel.  Same mathematics and results as
+// lstm_bwd_persistent_kernel (which replaces fastlstm/kernels.py:1201-1409).  lstm_bwd_big_kernel is faster at every size (us per step, here and there: H = 2048, 128 rows 11.0, 8.6; 32 rows 6.4, 5.3; a pair of H = 2048, B = 32
 // 9.8, 6.5); this form remains for calls whose workspace has no room for the partial sums of its teams.
 //
 // A workgroup of 8 waves owns 16 hidden units and up to 64 batch rows and keeps Wh[:, units]^T (K = 4H
@@ -29,7 +28,8 @@ constexpr int kWideRing = 12;   // LDS blocks (1 KiB) per wave for operand block
 template <typename T, int NKW, int NT>
 __global__ __launch_bounds__(kWave * 8) void lstm_bwd_wide_kernel(const BwdXcdParams p) {
     using E = Elem<T>;
-    constexpr bool ACC = E::BYTES == 4;                // fp32: refined reciprocal in the gates
+    constexpr bool ACC = false;                        // gates: the hardware's reciprocal
+    static_assert(E::BYTES == 2, "fp32: lstm_bwd_big_kernel");
     constexpr int NWV = 8, NTHR = kWave * NWV;
     constexpr int HT = 16, BT = 16 * NT;
     constexpr int IPT = (HT * BT + NTHR - 1) / NTHR;   // (unit, batch row) items per thread
@@ -221,18 +221,13 @@ __global__ __launch_bounds__(kWave * 8) void lstm_bwd_wide_kernel(const BwdXcdPa
 #pragma unroll
                 for (int gt = 0; gt < 4; ++gt) st_d[gt] = E::from_f32(0.f);
             }
-            // exchange copy: 4 consecutive k = (unit, gate 0..3), 16 bytes per unit with fp32; with 16-bit
-            // elements lanes l and l+16 own units u and u+1 of the same batch row and the even-unit lane
-            // writes both (16 bytes, write-through)
-            if constexpr (E::BYTES == 4) {
-                if (valid[m]) xch.store16(xgrp + xoff[m], *reinterpret_cast<u32x4 *>(st_d));
-            } else {
-                const u32x2 mine = *reinterpret_cast<u32x2 *>(st_d);
-                u32x2 other;
-                other[0] = (unsigned)__shfl_down((int)mine[0], 16);
-                other[1] = (unsigned)__shfl_down((int)mine[1], 16);
-                if (pair_lead[m]) xch.store16(xgrp + xoff[m], u32x4{mine[0], mine[1], other[0], other[1]});
-            }
+            // exchange copy: 4 consecutive k = (unit, gate 0..3), 8 bytes: lanes l and l + 16 own units u and u + 1 of the same
+            // batch row and the even-unit lane writes both (16 bytes, write-through)
+            const u32x2 mine = *reinterpret_cast<u32x2 *>(st_d);
+            u32x2 other;
+            other[0] = (unsigned)__shfl_down((int)mine[0], 16);
+            other[1] = (unsigned)__shfl_down((int)mine[1], 16);
+            if (pair_lead[m]) xch.store16(xgrp + xoff[m], u32x4{mine[0], mine[1], other[0], other[1]});
         }
         publish_version(grp_flags + j, s + 1);   // waits for the stores, workgroup barrier, raises the flag
         tile_to_global(t);

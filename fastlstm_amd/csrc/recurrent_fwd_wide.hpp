@@ -34,7 +34,8 @@ namespace fastlstm {
 template <typename T, int NKW, int NT>
 __global__ __launch_bounds__(kWave * 8) void lstm_fwd_wide_kernel(const FwdXcdParams p) {
     using E = Elem<T>;
-    constexpr bool ACC = E::BYTES == 4;                      // fp32: refined reciprocal in the gates
+    constexpr bool ACC = false;                              // gates: the hardware's reciprocal
+    static_assert(E::BYTES == 2, "fp32: lstm_fwd_big_kernel");
     constexpr int NWV = 8, NTHR = kWave * NWV;
     constexpr int MT = 4, TILES = MT * NT;                   // unit tiles, batch tiles of 16 rows
     constexpr int IPT = (TILES + NWV - 1) / NWV;             // (tile, lane) items per thread
@@ -103,7 +104,7 @@ __global__ __launch_bounds__(kWave * 8) void lstm_fwd_wide_kernel(const FwdXcdPa
         const int mt = tile / NT, nt = tile % NT;
         const int unit = u0 + mt * 4 + q, b = b0 + nt * 16 + n;
         valid[m] = tile < TILES && b < B;
-        live[m] = tile < TILES && (E::BYTES == 2 ? nt * 16 + n < rows_computed(B - b0) : b < B);   // (fp32: few rows cost nothing)
+        live[m] = tile < TILES && nt * 16 + n < rows_computed(B - b0);
         off_h[m] = valid[m] ? (size_t)b * H + unit : (size_t)b0 * H + u0;
         xoff[m] = nt * KS * kFragBytes + frag_offset<T>(n, unit);
         goff[m] = (nt * 16 + n) * GROW + (mt * 4 + q) * E::BYTES;

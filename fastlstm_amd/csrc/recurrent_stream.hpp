@@ -38,6 +38,10 @@ struct FwdStreamParams {
     WsHeader *hdr;
     int *flags;        // [n_bt][flag_stride]
     unsigned char *xbuf;   // [2 slots][n_bt][NT][KSP] operand blocks
+    // lstm_fwd_big_parts_kernel: n_rec = 2: a second, independent recurrence of this shape side by side
+    int n_rec;
+    void *ifgo2, *out2, *cell2;
+    const void *Wh2;
     int T, B, H;
     int b_base, n_bt, n_ht, flag_stride;
     int KS, KSP;       // k-steps covering H, padded

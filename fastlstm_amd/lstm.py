@@ -1145,9 +1145,10 @@ def _padded_hidden_size_cached(T, B, H, code, device_index, training, families):
     follows, whose kernels count too."""
     fp32 = code == _DTYPE_CODE[torch.float32]
     kind = lambda h: _recurrent_kind(T, B, h, code, device_index)
-    # fp32 with up to 32 rows keeps the general forward kernel at H = 640 ... 1024, but its reverse pass is twice as
-    # fast on the register-resident kernel (T = 256, B = 8, I = 256, forward + backward: H = 576 3.8 ms, H = 640 2.9)
-    fast = lambda h: kind(h) in (1, 2) or (training and fp32 and _recurrent_kind(T, B, h, code, device_index, True) in (1, 2))
+    # a forward call of up to 32 fp32 rows is reported as general whatever runs it, so fp32 sizes go by the reverse pass,
+    # whose kernels take the same sizes (T = 256, B = 8, I = 256, H = 576 as it is / as 640: inference 1.21 / 0.96 ms,
+    # forward + backward 3.43 / 2.47; B = 32, H = 960 as 1024: 1.62 / 1.19, 5.00 / 3.36; T = 40, B = 1: 0.21 / 0.19)
+    fast = lambda h: kind(h) in (1, 2) or (fp32 and _recurrent_kind(T, B, h, code, device_index, True) in (1, 2))
     # The launches that pad and cut cost ~0.1 ms forward and ~0.2 ms forward + backward whatever the shape: a few steps
     # repay them only with many rows and units (T = 16, B = 128, H = 1150 bf16 forward + backward 0.82 ms as it is,
     # 0.59 ms as 1280; B = 64, H = 650 0.48 against 0.68).

@@ -1,18 +1,19 @@
 """fp32 recurrences whose numbers travel and multiply as three bf16 parts (csrc/recurrent_parts.hpp): half k-steps (H = 16 mod 32), every
-unit tile and batch tile of the XCD-local kernels, against float64; numbers that are not finite."""
+unit tile and batch tile of the XCD-local and the whole-CU kernels, against float64; numbers that are not finite."""
 import numpy as np
 import pytest
 import torch
 
 from fastlstm_amd import _lib
 from helpers import nn_lstm_reference
-from test_gpu_one_cu import operands, run
+from test_gpu_one_cu import backward, operands, run
 
 pytestmark = pytest.mark.gpu
 
 
-# (B, H): 16- and 32-row groups, one and two unit tiles, half and whole last k-steps, rows over several launches
-@pytest.mark.parametrize("B,H", [(3, 112), (17, 144), (5, 208), (33, 256), (150, 256), (300, 272), (9, 400), (128, 512), (140, 512), (600, 320)])
+# (B, H): 16- and 32-row groups, one and two unit tiles, half and whole last k-steps, rows over several launches; 640 on: whole-CU kernels
+@pytest.mark.parametrize("B,H", [(3, 112), (17, 144), (5, 208), (33, 256), (150, 256), (300, 272), (9, 400), (128, 512), (140, 512), (600, 320),
+                                 (3, 640), (90, 640), (33, 768), (20, 896), (70, 1024), (300, 1024)])
 def test_against_float64(B, H):
     T = 7
     p, g = operands(T, B, H, torch.float32, seed=H + B)
@@ -25,7 +26,16 @@ def test_against_float64(B, H):
         assert np.linalg.norm(a - b) <= 1e-6 * np.linalg.norm(b), name   # (2-norm: some 2e-7 from the rounding of every step's results)
 
 
-@pytest.mark.parametrize("B,H", [(9, 112), (40, 512)])
+@pytest.mark.parametrize("B,H", [(19, 640), (40, 1024)])
+def test_side_by_side_are_the_bits_of_calls_by_themselves(B, H):
+    gs = [operands(5, B, H, torch.float32, seed=s)[1] for s in range(2)]
+    alone = [run(g) for g in gs]
+    recs = [(g, a[1], a[2], g["dh_n"].clone(), g["dc_n"].clone()) for g, a in zip(gs, alone)]
+    for d, r, a in zip(backward(recs), recs, alone):
+        assert torch.equal(d, a[3]) and torch.equal(r[3], a[4]) and torch.equal(r[4], a[5])
+
+
+@pytest.mark.parametrize("B,H", [(9, 112), (40, 512), (40, 768)])
 @pytest.mark.parametrize("weight", [False, True])
 def test_numbers_that_are_not_finite(B, H, weight):
     """As test_gpu_one_cu's: the general kernels' entries are infinite, NaN and finite where these are."""
