@@ -137,7 +137,7 @@ bool gemm16_eligible(int dtype, int M, int N, int K, int lda, int ldb, bool a_km
     return a_bytes < (1ull << 32) && b_bytes < (1ull << 32);
 }
 
-// Tile edge (256 or 128; 0 = generic kernel) and split-K factor for a product.
+// Tile edge (256, 128 or 64; 0 = generic kernel) and split-K factor for a product.
 void gemm_plan(int dtype, int M, int N, int K, int lda, int ldb, bool a_km, bool b_km, bool allow_split,
                int *tile, int *splits) {
     if (dtype == FASTLSTM_FP32) {
@@ -155,7 +155,15 @@ void gemm_plan(int dtype, int M, int N, int K, int lda, int ldb, bool a_km, bool
         }
         return;
     }
-    const int t256 = cdiv(M, 256) * cdiv(N, 256), t128 = cdiv(M, 128) * cdiv(N, 128);
+    const int t256 = cdiv(M, 256) * cdiv(N, 256), t128 = cdiv(M, 128) * cdiv(N, 128), t64 = cdiv(M, 64) * cdiv(N, 64);
+    // At most two 64 x 64 tiles per CU: a k-tile takes them 0.22 us, the 128 x 128 tile 0.55, and four times as many CUs work (us with
+    // 64 and 128: M = 700, N = 2816, K = 704, 484 tiles, 8.7 and 9.9; M = N = 700, K = 2816 14.4 and 25.2; with 768 tiles, M = 1024,
+    // N = 3072, K = 512, 9.7 and 8.1).  Parts from 64 k-tiles on, of 16 or more: adding them up costs ~5 us.
+    if (t64 <= 2 * kNumXcd * 32) {
+        *tile = 64;
+        if (allow_split && K >= 4096) *splits = std::max(1, std::min(2 * kNumXcd * 32 / t64, K / 1024));
+        return;
+    }
     const int max_split = allow_split ? std::max(1, K / 512) : 1;  // >= 8 k-tiles per split
     if (t256 >= 192) {
         *tile = 256;
@@ -301,7 +309,13 @@ hipError_t launch_gemm_tiled(int dtype, const GemmParams &p_in, bool a_km, bool 
         if (hipError_t e = launch_gemm_f32(g, a_km, b_km, tile, s)) return e;
         return p.splits > 1 ? launch_splitk_reduce<float>(p, s) : hipSuccess;
     }
-    FASTLSTM_TILE_CASE(128, 128, 128, 2, 2, 2, 2)   // 2 workgroups per CU
+    // 8 waves each (gemm16_mainloop, SHORT).  Four stages of 32 KiB where a CU has one of the 128 x 128 tiles, two where it has two
+    // (us with four and two: M = 1280, N = 2048, K = 8192 in one pass, 160 tiles, 65.5 and 86.6; M = 4096, N = 2048, K = 256, 512 tiles,
+    // 11.9 and 10.4); four of 16 KiB for the 64 x 64 tiles, of which a CU takes two.
+    if (tile == 128 && cdiv(p.M, 128) * cdiv(p.N, 128) * p.splits <= kNumXcd * 32) tile = 4 * 128;
+    FASTLSTM_TILE_CASE(64, 64, 64, 4, 2, 4, 2)
+    FASTLSTM_TILE_CASE(128, 128, 128, 2, 2, 4, 2)
+    FASTLSTM_TILE_CASE(4 * 128, 128, 128, 4, 2, 4, 2)
     FASTLSTM_TILE_CASE(256, 256, 256, 2, 2, 4, 2)   // 8 waves, 128 x 64 per wave, 2 x 64 KiB stages
 #undef FASTLSTM_TILE_CASE
     return launch_gemm(dtype, p, a_km, b_km, s);

@@ -5,9 +5,8 @@
 // that every benchmark configuration of the LSTM hits.
 //
 // Design for gfx950
-//  * BM x BN x 64 workgroup tile (256 x 256 for large problems), 4 waves in 2 x 2, each
-//    wave BM/2 x BN/2 as MFMA 16x16x32 tiles -> up to 256 fp32 accumulators per lane;
-//    one LDS byte feeds 128 MACs, so LDS reads run at half the MFMA rate.
+//  * BM x BN x 64 workgroup tile (256 x 256 for large problems, 128 x 128 and 64 x 64 where those would be few), 8 waves in 2 x 4, each
+//    wave BM/2 x BN/4 as MFMA 16x16x32 tiles.
 //  * K-contiguous operands are stored in LDS directly in MFMA operand order: a fragment is
 //    one linear, conflict-free ds_read_b128.
 //  * K-major operands (d_ifgo, x and h in the weight-gradient products) stay in memory order
@@ -160,6 +159,7 @@ __device__ __forceinline__ void gemm16_mainloop(const GemmParams &p, const int m
     using C = Gemm16Cfg<BM, BN, NS, WVM, WVN, KSPT>;
     constexpr int NWAVES = C::NWAVES;
     constexpr int BK = C::BK, TM = C::TM, TN = C::TN;
+    constexpr bool SHORT = BM <= 128;   // (the products of few tiles)
     // tid_salt is zero.  A caller inside a loop passes one the compiler cannot see through, so that the
     // per-lane address arithmetic below is redone per call instead of being kept in registers (or
     // spilled and reloaded inside the k loop) across the caller's loop.
@@ -177,7 +177,10 @@ __device__ __forceinline__ void gemm16_mainloop(const GemmParams &p, const int m
     // XOR swizzle of the 16-byte column chunk index of a K-major tile, as a function of the
     // k-row: the 4 rows x 32 bytes one 16-lane group of a transposing read touches (k & 3),
     // and the rows of neighbouring lane groups (k & 8), land in different banks.
-    auto swz = [](int k) { return ((k & 3) << 1) ^ (((k >> 3) & 1) << 3); };
+    // (64 columns: a row is half of the banks, rows k and k + 1 fill them.)
+    auto swz = [](int k, int chunks) {
+        return chunks == 8 ? (k & 2) ^ (((k >> 3) & 1) << 2) : ((k & 3) << 1) ^ (((k >> 3) & 1) << 3);
+    };
 
     // K-contiguous operand tile in LDS: rows of BK elements (LPR 16-byte chunks), chunk c of row r
     // at position c ^ kswz(r % 16): the 16 lanes of a fragment read (16 rows, one chunk index) hit
@@ -201,7 +204,7 @@ __device__ __forceinline__ void gemm16_mainloop(const GemmParams &p, const int m
         goff_a = (unsigned)(((size_t)(m0 + row) * p.lda + kb + k) * 2);
     } else {
         constexpr int CPR = BM / 8;
-        const int P = wave * 64 + lane, k = P / CPR, mc = (P % CPR) ^ swz(k);
+        const int P = wave * 64 + lane, k = P / CPR, mc = (P % CPR) ^ swz(k, CPR);
         goff_a = (unsigned)(((size_t)(kb + k) * p.lda + m0 + mc * 8) * 2);
     }
     if constexpr (!B_KM) {
@@ -209,7 +212,7 @@ __device__ __forceinline__ void gemm16_mainloop(const GemmParams &p, const int m
         goff_b = (unsigned)(((size_t)(n0 + row) * p.ldb + kb + k) * 2);
     } else {
         constexpr int CPR = BN / 8;
-        const int P = wave * 64 + lane, k = P / CPR, nc = (P % CPR) ^ swz(k);
+        const int P = wave * 64 + lane, k = P / CPR, nc = (P % CPR) ^ swz(k, CPR);
         goff_b = (unsigned)(((size_t)(kb + k) * p.ldb + n0 + nc * 8) * 2);
     }
     const unsigned a_istep = (unsigned)(A_KM ? NWAVES * 64 / (BM / 8) : NWAVES * RPB) * p.lda * 2;  // bytes per block index
@@ -239,14 +242,14 @@ __device__ __forceinline__ void gemm16_mainloop(const GemmParams &p, const int m
         constexpr int LD = decltype(ld_)::value, ld = LD;
         if constexpr (!km) {
             const unsigned char *src = tile + ((tile16 * 16 + r) * LPR + ((ks * 4 + q) ^ kswz(r))) * 16;
-            if constexpr (A_KM || B_KM) return lds_read_b128_asm<0>(src);   // see the streamed loop below
+            if constexpr (A_KM || B_KM || SHORT) return lds_read_b128_asm<0>(src);   // see the loops below
             else return *reinterpret_cast<const u32x4 *>(src);
         } else {
             // lane (a, b) of a 16-lane group addresses 4 consecutive m of k-row a; rows k and
             // k + 4 (second read) share k & 3 and k & 8, hence the swizzle
             const int a = r >> 2, b = r & 3;
             const int k = ks * 32 + q * 8 + a;
-            const unsigned char *base = tile + k * ld + (((tile16 * 2 + (b >> 1)) ^ swz(k)) * 16) + (b & 1) * 8;
+            const unsigned char *base = tile + k * ld + (((tile16 * 2 + (b >> 1)) ^ swz(k, LD / 16)) * 16) + (b & 1) * 8;
             const u32x2 lo = lds_read_tr16<0>(base), hi = lds_read_tr16<4 * LD>(base);
             return u32x4{lo[0], lo[1], hi[0], hi[1]};
         }
@@ -270,7 +273,62 @@ __device__ __forceinline__ void gemm16_mainloop(const GemmParams &p, const int m
         else wait_vm_at_most<0>();                             // tail: fewer tiles behind this one
         __builtin_amdgcn_s_barrier();
     };
-    if constexpr (A_KM || B_KM) {
+    if constexpr (SHORT) {
+        // Few tiles, one or two workgroups per CU: what bounds them is the chain of a k-tile, LDS reads, multiplications, barrier.  8 waves
+        // on a 128 x 128 or 64 x 64 tile, the fragments of a whole k-step requested while the one before is multiplied.  With 4 waves and
+        // one fragment ahead (the loop below) a k-tile of 128 x 128 took 0.85 us whatever the prefetch depth of the global loads, two
+        // thirds of it LDS latency; here 0.55, and 0.22 with 64 x 64.  us, M, N, K: 700, 2816, 704 12.5 -> 8.7; 700, 704, 2816 42 -> 14.4;
+        // 256, 4096, 1024 14.7 -> 7.7; 1280, 2048, 8192 113 -> 66.  The sums are taken in the same order (k upwards).
+        constexpr int READS = TM * (A_KM ? 2 : 1) + TN * (B_KM ? 2 : 1);   // LDS instructions per k-step
+        static_assert(KSPT == 2 && READS < 16, "lgkmcnt counts to 15");
+        u32x4 fa[2][TM], fb[2][TN];
+        auto read = [&](int kt, auto ksc) __attribute__((always_inline)) {
+            constexpr int ks = decltype(ksc)::value;
+            const unsigned char *tile = smem + (kt % NS) * C::STAGE;
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+                fb[ks][j] = frag(tile + C::A_BYTES, std::bool_constant<B_KM>{}, std::integral_constant<int, C::B_LD>{}, wn * TN + j, ks);
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+                fa[ks][i] = frag(tile, std::bool_constant<A_KM>{}, std::integral_constant<int, C::A_LD>{}, wm * TM + i, ks);
+        };
+        auto landed_but = [&](auto nc, auto ksc) __attribute__((always_inline)) {   // the fragments of a k-step, n younger reads in flight
+            constexpr int ks = decltype(ksc)::value;
+#pragma unroll
+            for (int j = 0; j < TN; ++j) lds_reads_landed_but<decltype(nc)::value>(fb[ks][j]);
+#pragma unroll
+            for (int i = 0; i < TM; ++i) lds_reads_landed_but<decltype(nc)::value>(fa[ks][i]);
+        };
+        auto multiply = [&](auto ksc) __attribute__((always_inline)) {
+            constexpr int ks = decltype(ksc)::value;
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) acc[i][j] = mfma_kstep<T>(fb[ks][j], fa[ks][i], acc[i][j]);
+        };
+        const std::integral_constant<int, 0> k0;
+        const std::integral_constant<int, 1> k1;
+#pragma unroll
+        for (int d = 0; d < D; ++d)
+            if (d < nkt) gload(d, d, 0, 1);
+        tile_ready(0);
+        read(0, k0);
+        for (int kt = 0; kt < nkt; ++kt) {
+            if (kt + D < nkt) gload(kt + D, (kt + D) % NS, 0, 1);   // into the stage the last barrier freed
+            read(kt, k1);
+            landed_but(std::integral_constant<int, READS>{}, k0);
+            multiply(k0);
+            landed_but(std::integral_constant<int, 0>{}, k1);
+            if (kt + 1 < nkt) {
+                tile_ready(kt + 1);
+                read(kt + 1, k0);
+            }
+            multiply(k1);
+        }
+        __syncthreads();
+        return;
+    }
+    else if constexpr (A_KM || B_KM) {
         // Products with a K-major operand: all fragment reads are inline assembly (see
         // lds_read_tr16) and this loop counts them itself.  Registers: the B fragments of both
         // k-steps of a k-tile (TN each) and two registers through which the A fragments stream, one
@@ -283,7 +341,7 @@ __device__ __forceinline__ void gemm16_mainloop(const GemmParams &p, const int m
         //       the stage to the global loads, and requests the next k-tile's first fragments, whose
         //       latency the remaining two iterations' multiplications cover.
         static_assert(KSPT == 2, "two k-steps per k-tile");
-        static_assert(TM % TN == 0 && TM >= 4, "B fragments are read every TM / TN-th iteration");
+        static_assert(TM % TN == 0, "B fragments are read every TM / TN-th iteration");
         constexpr int NA = A_KM ? 2 : 1, NB = B_KM ? 2 : 1, EVERY = TM / TN;   // LDS instructions per fragment
         u32x4 fs[2], fb[2][TN];
         auto rd_a = [&](int kt, int ks, int i) {
@@ -335,19 +393,15 @@ __device__ __forceinline__ void gemm16_mainloop(const GemmParams &p, const int m
                 if constexpr (i == TM - 2)
                     if (more) fs[0] = rd_a(kt + 1, 0, 0);
             };
-            static_assert(TM == 4 || TM == 8, "wave tile rows");
+            static_assert(TM == 8, "wave tile rows");
             step0(std::integral_constant<int, 0>{}); step0(std::integral_constant<int, 1>{});
             step0(std::integral_constant<int, 2>{}); step0(std::integral_constant<int, 3>{});
-            if constexpr (TM == 8) {
-                step0(std::integral_constant<int, 4>{}); step0(std::integral_constant<int, 5>{});
-                step0(std::integral_constant<int, 6>{}); step0(std::integral_constant<int, 7>{});
-            }
+            step0(std::integral_constant<int, 4>{}); step0(std::integral_constant<int, 5>{});
+            step0(std::integral_constant<int, 6>{}); step0(std::integral_constant<int, 7>{});
             step1(std::integral_constant<int, 0>{}); step1(std::integral_constant<int, 1>{});
             step1(std::integral_constant<int, 2>{}); step1(std::integral_constant<int, 3>{});
-            if constexpr (TM == 8) {
-                step1(std::integral_constant<int, 4>{}); step1(std::integral_constant<int, 5>{});
-                step1(std::integral_constant<int, 6>{}); step1(std::integral_constant<int, 7>{});
-            }
+            step1(std::integral_constant<int, 4>{}); step1(std::integral_constant<int, 5>{});
+            step1(std::integral_constant<int, 6>{}); step1(std::integral_constant<int, 7>{});
         }
         __syncthreads();   // every wave has read its last fragments (waited for above)
         return;
