@@ -646,6 +646,31 @@ static int wide_rows_per_launch(int T, int B, int H, int dtype, bool backward, s
     return rows;
 }
 
+// fp32, H = 1280, 1536, 1792, 2048 (plan: streamed weights): the whole-CU kernels with 8 units per workgroup hold all of W_h, as three
+// bf16 parts; one group of 16 to 64 rows per launch, one launch per range of 64 rows (at any batch size faster than streaming them:
+// figures in recurrent_fwd_big.hpp, recurrent_bwd_big.hpp).
+static bool big_half_applies(const fastlstm_plan &pl, int H, int dtype) {
+    DeviceInfo di;
+    return dtype == FASTLSTM_FP32 && pl.wave_split == 3 && H % 256 == 0 && H > 1024 && H <= 2048 && (g_families.load() & 2) &&
+           device_info(-1, &di) == FASTLSTM_OK && di.xcd_round_robin == 1 && di.num_cus >= kNumXcd * 32;
+}
+constexpr int kBigHalfRows = 64;
+static int big_half_tiles(int rows) { return rows <= 16 ? 1 : rows <= 32 ? 2 : 4; }   // batch tiles of a launch
+// Sets what both directions share; returns batch tiles, 0 if the workspace behind the counters does not hold the exchange.
+template <typename P> static int big_half_params(P &p, unsigned char *wsb, size_t ws_bytes, int rows, int H, bool backward) {
+    const int nt = big_half_tiles(rows), ks = (backward ? 4 * H : H) / 32;
+    const size_t xchg = 2 * (size_t)nt * ks * 3 * kFragBytes;
+    const size_t partials = backward ? (size_t)(H / 8) * kBigTeamHalf * nt * kFragBytes : 0;
+    if (ws_bytes < kWsHeaderBytes + kWsCounterBytes + xchg + partials) return 0;
+    p.hdr = reinterpret_cast<WsHeader *>(wsb);
+    p.flags = reinterpret_cast<int *>(wsb + kWsHeaderBytes);
+    p.flag_stride = kXcdGroupStride;
+    p.xbuf = wsb + kWsHeaderBytes + kWsCounterBytes;
+    p.n_bt = p.n_rec = 1;
+    p.n_ht = H / 8;
+    return nt;
+}
+
 // Returns 1 when the kernel does not apply, else a fastlstm_status.
 // `second` (+ o.more): independent recurrences of the same shape side by side in the launch, as try_fwd_xcd takes them.
 int try_fwd_wide(void *ifgo, void *out, void *cell, const void *Wh, unsigned char *wsb, size_t ws_bytes, int T, int B,
@@ -1289,6 +1314,20 @@ static int fwd_persistent_impl(void *ifgo, void *out, void *cell, const void *Wh
         p.KS = l.KS; p.KSP = l.KSP;
         p.keep = keep;
         p.spin_limit = spin_limit_ticks();
+        if (big_half_applies(pl, H, dtype)) {
+            FwdStreamParams h = p;
+            const int nt_all = big_half_params(h, wsb, ws_bytes, std::min(B, kBigHalfRows), H, false);
+            int occ = 0;
+            if (nt_all && launch_fwd_big(dtype, h, H / 128, 2, nt_all, 0, nullptr, &occ) != hipSuccess) return FASTLSTM_ERR_HIP;
+            for (int r0 = 0; occ >= 1 && r0 < B; r0 += kBigHalfRows) {
+                if (r0 && !clear_xcd_counters(wsb, s)) return FASTLSTM_ERR_HIP;
+                const int nt = big_half_params(h, wsb, ws_bytes, std::min(B - r0, kBigHalfRows), H, false);
+                h.KS = h.KSP = H / 32;
+                h.b_base = r0;
+                if (launch_fwd_big(dtype, h, H / 128, 2, nt, h.n_ht, s, nullptr) != hipSuccess) return FASTLSTM_ERR_HIP;
+            }
+            if (occ >= 1) return FASTLSTM_OK;
+        }
         // 16-bit up to H = 4096: the slice of 16 units of a workgroup stays on its CU for the whole launch
         bool resident = dtype != FASTLSTM_FP32 && pl.ht == 16 && H % 16 == 0 && l.KSP >= 80 && l.KSP <= 128 && (g_families.load() & 2);
         if (resident) {
@@ -1455,6 +1494,24 @@ static int bwd_persistent_impl(const void *dout, void *dh, void *dc, const void 
         p.flag_stride = (int)align_up((size_t)pl.n_htiles, 64);
         p.KSB = l.KS; p.KSBP = l.KSP;
         p.spin_limit = spin_limit_ticks();
+        if (big_half_applies(pl, H, dtype)) {
+            BwdStreamParams h = p;
+            h.Wh = Wh;
+            const int nt_all = big_half_params(h, wsb, ws_bytes, std::min(B, kBigHalfRows), H, true);
+            int occ = 0;
+            if (nt_all && launch_bwd_big(dtype, h, H / 128, 4, nt_all, 0, nullptr, &occ) != hipSuccess) return FASTLSTM_ERR_HIP;
+            for (int r0 = 0; occ >= 1 && r0 < B; r0 += kBigHalfRows) {
+                if (r0 && !clear_xcd_counters(wsb, s)) return FASTLSTM_ERR_HIP;
+                const int nt = big_half_params(h, wsb, ws_bytes, std::min(B - r0, kBigHalfRows), H, true);
+                h.KSB = h.KSBP = 4 * H / 32;
+                h.b_base = r0;
+                h.team_flags = h.flags + kXcdGroupStride;
+                h.partials = h.xbuf + 2 * (size_t)nt * h.KSB * 3 * kFragBytes;
+                const int grid = kNumXcd * cdiv(h.n_ht / kBigTeamHalf, kNumXcd) * kBigTeamHalf;
+                if (launch_bwd_big(dtype, h, H / 128, 4, nt, grid, s, nullptr) != hipSuccess) return FASTLSTM_ERR_HIP;
+            }
+            if (occ >= 1) return FASTLSTM_OK;
+        }
         // 16-bit up to H = 4096: teams of 4 workgroups keep the slices of 64 units on their CUs for the whole launch; the
         // place of the packed weights holds the team's partial sums
         DeviceInfo di;

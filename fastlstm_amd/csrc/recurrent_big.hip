@@ -1,4 +1,4 @@
-// Instantiates the whole-CU kernels (recurrent_fwd_big.hpp, recurrent_bwd_big.hpp) .
+// Instantiates the 16-bit whole-CU kernels (recurrent_fwd_big.hpp, recurrent_bwd_big.hpp); launches of all of them.
 #include "recurrent_bwd_big.hpp"
 #include "recurrent_launch.hpp"
 
@@ -36,21 +36,9 @@ static hipError_t bwd_big_t(const BwdStreamParams &p, int kw, int mt, int nt, in
     return hipErrorInvalidConfiguration;
 }
 
-// fp32, H = 128 KW in 640 ... 1024: 16 units per workgroup, all weights in registers as three parts
-static hipError_t fwd_big_f32(const FwdStreamParams &p, int kw, int nt, int grid, int lds, hipStream_t s, int *occ) {
-#define CASE(KW, NT) \
-    if (kw == KW && nt == NT) return launch_one(lstm_fwd_big_parts_kernel<float, KW, 4, NT>, p, grid, lds, s, occ)
-    CASE(5, 1); CASE(5, 2); CASE(6, 1); CASE(6, 2); CASE(7, 1); CASE(7, 2); CASE(8, 1); CASE(8, 2);
-#undef CASE
-    return hipErrorInvalidConfiguration;
-}
-static hipError_t bwd_big_f32(const BwdStreamParams &p, int kw, int nt, int grid, int lds, hipStream_t s, int *occ) {
-#define CASE(KW, NT) \
-    if (kw == KW && nt == NT) return launch_one(lstm_bwd_big_parts_kernel<float, KW, 4, NT>, p, grid, lds, s, occ)
-    CASE(5, 1); CASE(5, 2); CASE(6, 1); CASE(6, 2); CASE(7, 1); CASE(7, 2); CASE(8, 1); CASE(8, 2);
-#undef CASE
-    return hipErrorInvalidConfiguration;
-}
+// fp32 (recurrent_big_fwd_f32.hip, recurrent_big_bwd_f32.hip)
+hipError_t fwd_big_f32(const FwdStreamParams &p, int kw, int nt, int grid, int lds, hipStream_t s, int *occ);
+hipError_t bwd_big_f32(const BwdStreamParams &p, int kw, int nt, int grid, int lds, hipStream_t s, int *occ);
 
 hipError_t launch_fwd_big(int dtype, const FwdStreamParams &p, int kw, int mt, int nt, int grid, hipStream_t s, int *occ) {
     const int lds = big_lds_bytes(kw, mt, nt, elem_bytes(dtype));

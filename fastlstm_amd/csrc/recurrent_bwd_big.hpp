@@ -1,4 +1,4 @@
-// Persistent reverse-time kernel for 16-bit elements and 1280 <= H <= 4096, and for fp32 and 640 <= H <= 1024: weights on the CU for the whole launch, as in
+// Persistent reverse-time kernel for 16-bit elements and 1280 <= H <= 4096, and for fp32 and 640 <= H <= 2048: weights on the CU for the whole launch, as in
 // lstm_fwd_big_kernel, and the product split over K among teams.  Same mathematics and results as
 // lstm_bwd_persistent_kernel (which replaces fastlstm/kernels.py:1201-1409); the sums over K are taken in another order.
 //
@@ -23,7 +23,11 @@
 // fp32 (lstm_bwd_big_parts_kernel, MT = 4): d_ifgo[t] is exchanged as the three bf16 parts of its numbers, the weights' are all in
 // registers; bounds as in 16 bits with 1.5 times the bytes per number.  H = 1024, us per step of the kernel on the fp32 matrix
 // instructions and here: B = 128 12.4 -> 10.4, B = 16 6.6 -> 5.9.
-// Requirements (host): H a multiple of 16 MT (fp32: of 128), workgroup ids dealt to the XCDs in turn, all teams co-resident.
+// Above H = 1024 a workgroup has 8 units, half a unit tile: teams of 8 own 64 units, members 2 v and 2 v + 1 share tile v's sums, and
+// a member reads an eighth of d_ifgo[t] (teams of 4 with two unit tiles would read a quarter; hence the multiples of 256).  T = 100,
+// I = 512, training step with lstm_bwd_stream_kernel and here (the forward pass as in recurrent_fwd_big.hpp): H = 2048, B = 1
+// 4.05 -> 1.48 ms, 16 4.85 -> 1.91, 64 12.9 -> 4.74, 200 30.3 -> 15.1; H = 1280, B = 16 3.09 -> 1.52, 100 8.63 -> 5.38.
+// Requirements (host): H a multiple of 16 MT (fp32: of 128, above 1024 of 256), workgroup ids dealt to the XCDs in turn, all teams co-resident.
 #pragma once
 #include <type_traits>
 
@@ -31,13 +35,14 @@
 
 namespace fastlstm {
 
-constexpr int kBigTeam = 4;
+constexpr int kBigTeam = 4, kBigTeamHalf = 8;   // members of a team; with half a unit tile each
 
 template <typename T, int KW, int MT, int NT>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))) void lstm_bwd_big_kernel(const BwdStreamParams p) {
+    constexpr int V = kBigTeam;
 #include "recurrent_bwd_big.inc"
 }
-template <typename T, int KW, int MT, int NT>
+template <typename T, int KW, int MT, int NT, int V>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1, 1))) void lstm_bwd_big_parts_kernel(const BwdStreamParams p) {
 #include "recurrent_bwd_big.inc"
 }

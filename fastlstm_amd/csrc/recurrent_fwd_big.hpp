@@ -1,5 +1,5 @@
-// Persistent forward kernel for 16-bit elements and 1280 <= H <= 4096, and for fp32 and 640 <= H <= 1024: a workgroup keeps up to
-// 512 KiB of weights -- those of 16 hidden units, or of 32 where H <= 2048 in 16 bits -- on its CU for the whole launch, up to 384 KiB of
+// Persistent forward kernel for 16-bit elements and 1280 <= H <= 4096, and for fp32 and 640 <= H <= 2048: a workgroup keeps up to
+// 512 KiB of weights -- those of 16 hidden units, or of 32 where H <= 2048 in 16 bits, or of 8 where H > 1024 in fp32 -- on its CU for the whole launch, up to 384 KiB of
 // them in registers, the rest in LDS.
 //
 // Same mathematics, stored values and rounding points as lstm_fwd_persistent_kernel (which replaces
@@ -22,6 +22,9 @@
 // workgroup all in registers, h_t exchanged as parts; the largest of the six products has a sum of its own.  What bounds it: at two
 // batch tiles the 96 H bytes of operand blocks of each (H = 1024: 384 KiB per CU and step), at one the exchange.  H = 1024,
 // us per step of the kernels on the fp32 matrix instructions (1/16 of the rate) and here: B = 128 11.1 -> 7.9, B = 16 5.1 -> 3.9.
+// Above H = 1024 a workgroup holds 8 units (MT = 2: 384 KiB at H = 2048), one group of up to 64 rows is a launch, and every CU reads the
+// 6 H bytes of each of its rows every step.  T = 100, I = 512, inference with lstm_fwd_stream_kernel and here: H = 2048, B = 1
+// 1.66 -> 0.60 ms, 16 1.74 -> 0.70, 64 4.37 -> 1.65, 200 (four launches) 9.05 -> 5.38; H = 1280, B = 16 1.14 -> 0.57, 100 3.18 -> 2.13.
 // Requirements (host): H a multiple of MT * 4 (and of 8; fp32: of 128), the workgroups of all groups co-resident.
 #pragma once
 #include <type_traits>

@@ -1158,6 +1158,12 @@ def _padded_hidden_size_cached(T, B, H, code, device_index, training, families):
         return -(-H // 64) * 64 if T >= 16 else 0
     if T < 32 and (H <= 64 or T * B * H < (1_200_000 if fp32 else 2_000_000)):
         return 0
+    # fp32 between 1024 and 2048: the kernels that keep all of W_h on chip take multiples of 256, any other size runs on the general
+    # or the streamed kernels (T = 100, I = 512, inference / training as it is and padded: H = 1030, B = 1 0.79 / 2.16 and 0.56 / 1.31 ms,
+    # B = 256 6.17 / 22.1 and 4.41 / 11.5; H = 1900, B = 16 1.66 / 4.68 and 0.73 / 1.95; T = 32, B = 1, H = 1100 0.32 / 0.84 and
+    # 0.26 / 0.54; T = 16, B = 128 0.65 / 1.93 and 0.45 / 1.15)
+    if fp32 and families & 2 and 1024 < H < 2048:
+        return -(-H // 256) * 256 if H % 256 else 0
     if H <= 64:
         # The general kernels' one-tile form (no exchange between workgroups at all).  In 16 bits it is the fastest
         # there is at H = 64 (T = 1024, B = 256, I = H = 64 forward + backward 0.93 ms as it is, 3.4 ms as H = 96):

@@ -11,9 +11,11 @@ from test_gpu_one_cu import backward, operands, run
 pytestmark = pytest.mark.gpu
 
 
-# (B, H): 16- and 32-row groups, one and two unit tiles, half and whole last k-steps, rows over several launches; 640 on: whole-CU kernels
+# (B, H): 16- and 32-row groups, one and two unit tiles, half and whole last k-steps, rows over several launches; 640 on: whole-CU kernels,
+# 1280 on with half a unit tile per workgroup, in launches of up to 64 rows
 @pytest.mark.parametrize("B,H", [(3, 112), (17, 144), (5, 208), (33, 256), (150, 256), (300, 272), (9, 400), (128, 512), (140, 512), (600, 320),
-                                 (3, 640), (90, 640), (33, 768), (20, 896), (70, 1024), (300, 1024)])
+                                 (3, 640), (90, 640), (33, 768), (20, 896), (70, 1024), (300, 1024), (1, 1280), (66, 1280), (17, 1536), (150, 1792),
+                                 (16, 2048), (33, 2048), (64, 2048)])
 def test_against_float64(B, H):
     T = 7
     p, g = operands(T, B, H, torch.float32, seed=H + B)
@@ -35,7 +37,7 @@ def test_side_by_side_are_the_bits_of_calls_by_themselves(B, H):
         assert torch.equal(d, a[3]) and torch.equal(r[3], a[4]) and torch.equal(r[4], a[5])
 
 
-@pytest.mark.parametrize("B,H", [(9, 112), (40, 512), (40, 768)])
+@pytest.mark.parametrize("B,H", [(9, 112), (40, 512), (40, 768), (40, 1536)])
 @pytest.mark.parametrize("weight", [False, True])
 def test_numbers_that_are_not_finite(B, H, weight):
     """As test_gpu_one_cu's: the general kernels' entries are infinite, NaN and finite where these are."""
