@@ -142,7 +142,7 @@ void gemm_plan(int dtype, int M, int N, int K, int lda, int ldb, bool a_km, bool
                int *tile, int *splits) {
     if (dtype == FASTLSTM_FP32) {
         int kps;
-        gemm_f32_plan(M, N, 0, K, allow_split, tile, splits, &kps);
+        gemm_f32_plan(M, N, 0, K, allow_split, a_km && b_km, tile, splits, &kps);
         return;
     }
     *splits = 1;
@@ -186,7 +186,7 @@ bool wgrad_merged_plan(int dtype, int M, int I, int H, int K, int *splits, int *
     if (dtype == FASTLSTM_FP32) {   // any shape, always one grid
         int tile;
         *merged = true;
-        gemm_f32_plan(M, I, H, K, true, &tile, splits, k_per_split);
+        gemm_f32_plan(M, I, H, K, true, true, &tile, splits, k_per_split);
         return true;
     }
     if (!gemm16_eligible(dtype, M, I, K, M, I, true, true) || !gemm16_eligible(dtype, M, H, K, M, H, true, true)) return false;
@@ -283,7 +283,7 @@ hipError_t launch_wgrad_merged(int dtype, const void *d_ifgo, const void *x, con
     w.db_part = db_part;
     if (dtype == FASTLSTM_FP32) {
         int tile;
-        gemm_f32_plan(M, I, H, K, true, &tile, &sp, &kps);
+        gemm_f32_plan(M, I, H, K, true, true, &tile, &sp, &kps);
         return launch_wgrad_f32(w, tile, db, s);
     }
     return dtype == FASTLSTM_FP16 ? launch_wgrad_merged_t<_Float16>(w, merged, db, s)

@@ -27,14 +27,15 @@ template <bool A_KM, bool B_KM, int T, bool TWO> hipError_t launch_t(const GemmF
 // A k-tile of 16 takes a 256 x 256 tile 2.2 us and two 128 x 128 tiles of a CU 1.35 us (0.7 us one alone); a tile takes 5 and 4 us
 // besides (start, epilogue); partial sums are written and read back at 3.5 TB/s, by a launch of 4 us.
 // M = 16384, N = 4096, K = 1024: 256 0.69 ms, 128 0.75; M = 2048, N = 1024, K = 256: 256 0.051 ms, 128 0.023.
-// K is cut at least so that the parts fill the device: the sums over them stay short, and so does what they are rounded by.
-void gemm_f32_plan(int M, int N1, int N2, int K, bool allow_split, int *tile, int *splits, int *k_per_split) {
+// K is cut at least so that the parts fill the device: the sums over them stay short, and so does what they are rounded by.  two: the
+// 128 x 128 tile has sums of its own for the small products whether K is cut or not (the weight gradients), and need not be cut for it.
+void gemm_f32_plan(int M, int N1, int N2, int K, bool allow_split, bool two, int *tile, int *splits, int *k_per_split) {
     double best = 0.;
     *splits = 0;
     for (int t = 256; t >= 128; t /= 2) {
         const long long tiles = (long long)cdiv(M, t) * (cdiv(N1, t) + cdiv(N2, t));
         const int most = !allow_split ? 1 : std::max(1, std::min(64, K / (N2 ? 128 : 160)));
-        const int least = (int)std::min<long long>(most, t == 256 ? 256 / tiles : tiles >= 512 ? 1 : std::max<long long>(2, (255 + tiles) / tiles));
+        const int least = (int)std::min<long long>(most, t == 256 ? 256 / tiles : tiles >= 512 ? 1 : std::max<long long>(two ? 1 : 2, (255 + tiles) / tiles));
         for (int sp = std::max(1, least); sp <= most; ++sp) {
             const int kps = sp == 1 ? K : cdiv(cdiv(K, sp), 64) * 64;
             if (sp > least && cdiv(K, kps) != sp) continue;

@@ -18,7 +18,7 @@ hipError_t launch_gemm(int dtype, const GemmParams &p, bool a_km, bool b_km, hip
 void set_gemm_baseline(int on);
 int gemm_baseline();
 // fp32 products (gemm_f32.hpp): every shape; tile 256 or 128
-void gemm_f32_plan(int M, int N1, int N2, int K, bool allow_split, int *tile, int *splits, int *k_per_split);
+void gemm_f32_plan(int M, int N1, int N2, int K, bool allow_split, bool two, int *tile, int *splits, int *k_per_split);
 hipError_t launch_gemm_f32(const GemmF32Params &g, bool a_km, bool b_km, int tile, hipStream_t s);
 hipError_t launch_colsum_final(int dtype, const float *part, void *out, int C, int chunks, hipStream_t s);
 hipError_t launch_colsum(int dtype, const void *in, void *out, float *part, int R, int C, int chunks,
