@@ -159,7 +159,11 @@ void gemm_plan(int dtype, int M, int N, int K, int lda, int ldb, bool a_km, bool
     // At most two 64 x 64 tiles per CU: a k-tile takes them 0.22 us, the 128 x 128 tile 0.55, and four times as many CUs work (us with
     // 64 and 128: M = 700, N = 2816, K = 704, 484 tiles, 8.7 and 9.9; M = N = 700, K = 2816 14.4 and 25.2; with 768 tiles, M = 1024,
     // N = 3072, K = 512, 9.7 and 8.1).  Parts from 64 k-tiles on, of 16 or more: adding them up costs ~5 us.
-    if (t64 <= 2 * kNumXcd * 32) {
+    // Not for weight gradients of very many rows: what bounds those is reading the operands, a 64 x 64 tile twice as often (us with 64
+    // and 128, thin products of T*B rows, I, H: 173400, 1024, 64 312 and 182; 65536, 64, 256 171 and 123; 32768, 80, 512 204 and 147,
+    // 16384 106 and 102, 8192 65 and 81; 32768, 96, 96 49 and 44, 16384 33 and 37).
+    const bool many_rows = a_km && b_km && (K >= 32768 || (long long)t64 * K > 1 << 21);
+    if (t64 <= 2 * kNumXcd * 32 && !many_rows) {
         *tile = 64;
         if (allow_split && K >= 4096) *splits = std::max(1, std::min(2 * kNumXcd * 32 / t64, K / 1024));
         return;

@@ -50,3 +50,16 @@ def test_products(T, B, I, H, dt):
         assert float((d.double() - want).norm()) <= EPS[dt] * float(want.norm())
     m = (T * B + 1) // 2   # other tiles, the same bits
     assert torch.equal(ifgo(x[:m], Wx, b, 1, m, I, H), y[:m]) and torch.equal(dx(g[:m], Wx, 1, m, I, H), whole[:m])
+
+
+# (rows, I, H) of thin weight gradients: 64 x 64 tiles in one part and in several, 128 x 128 ones from 32768 rows or 2^21 rows x tiles on
+@pytest.mark.parametrize("R,I,H", [(500, 80, 96), (16500, 96, 96), (8200, 80, 512), (32767, 192, 64), (32768, 192, 64)])
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+def test_weight_gradients(R, I, H, dt):
+    gen = torch.Generator(device="cuda").manual_seed(R + H)
+    d, x, h = (torch.randn(s, generator=gen, device="cuda").mul_(R ** -0.5).to(dt) for s in ((1, R, 4 * H), (1, R, I), (2, R, H)))
+    db, _, dWx, dWh = L.Wgrad(d, x, h)
+    D = d[0].double()
+    # fp32 sums: at most R roundings of a running sum, in practice their square root; the bound of the results' rounding leaves room
+    for got, want in ((dWx, D.t() @ x[0].double()), (dWh, D.t() @ h[0].double()), (db, D.sum(0))):
+        assert float((got.double() - want).norm()) <= EPS[dt] * float(want.norm())
