@@ -354,8 +354,8 @@ int fastlstm_bwd_stack2_fused(int T, int B, int I, int H, int dtype, size_t ws_b
  * exchange through its L2; needs the workspace of fastlstm_recurrent_workspace_bytes and a
  * device that fastlstm_plan_device has probed; a batch with more tiles than one launch holds runs as
  * several launches over ranges of rows), 2 = the register-resident kernel for H = 1280, 1536, 1792,
- * 2048 with 16-bit elements (barrier groups of H / 16 workgroups over several XCDs, 64 batch rows
- * each; same needs as 1), 3 = the streamed-weights kernel of a hidden size whose W_h does not fit on chip (more
+ * 2048 with 16-bit elements, 640, 768, 896, 1024 in fp32 (barrier groups over several XCDs; same
+ * needs as 1), 3 = the streamed-weights kernel of a hidden size whose W_h does not fit on chip (more
  * than 32 MiB: the reference's RELOAD_WEIGHTS case, fastlstm/lstm.py:70-72).  Negative: fastlstm_status.
  * Diagnostics; no counterpart in the reference. */
 int fastlstm_recurrent_kernel_kind(int T, int B, int H, int dtype, int backward, size_t ws_bytes);
