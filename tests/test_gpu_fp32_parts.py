@@ -4,7 +4,8 @@ import numpy as np
 import pytest
 import torch
 
-from fastlstm_amd import _lib
+import fastlstm_amd.lstm as L
+from fastlstm_amd import FastLSTM, _lib
 from helpers import nn_lstm_reference
 from test_gpu_one_cu import backward, operands, run
 
@@ -58,3 +59,23 @@ def test_numbers_that_are_not_finite(B, H, weight):
         assert torch.equal(torch.isnan(a), torch.isnan(b)) and torch.equal(torch.isinf(a), torch.isinf(b))
         ok = torch.isfinite(b)
         assert bool(ok.any()) and not bool(ok.all()) and float((a - b)[ok].abs().max()) < 1e-4
+
+
+@pytest.mark.parametrize("T,B,H,padded", [(32, 5, 1100, 1280), (31, 5, 1100, 0), (33, 3, 1800, 2048), (40, 2, 1536, 0)])
+def test_module_between_the_sizes(T, B, H, padded):
+    """1024 < H < 2048 in the module: padded to a multiple of 256 from 32 steps on; outputs and gradients against float64."""
+    assert L._padded_hidden_size(T, B, H, 0, 0, True) == padded
+    torch.manual_seed(T + H)
+    want = torch.nn.LSTM(24, H).double()
+    got = FastLSTM(24, H, device="cuda", dtype=torch.float32)
+    got.load_state_dict(want.state_dict())   # (rounds)
+    want.load_state_dict(got.state_dict())
+    x, d = torch.randn(T, B, 24), torch.randn(T, B, H)
+    xg, xw = x.cuda().requires_grad_(), x.double().requires_grad_()
+    y, (h, c) = got(xg)
+    y.backward(d.cuda())
+    yw, (hw, cw) = want(xw)
+    yw.backward(d.double())
+    pairs = [(y, yw), (h, hw), (c, cw), (xg.grad, xw.grad)] + [(p.grad, q.grad) for p, q in zip(got.parameters(), want.parameters())]
+    for i, (a, b) in enumerate(pairs):   # (2-norm: rounding of every step's results and of sums of fp32 products)
+        assert a.shape == b.shape and float((a.double().cpu() - b).norm()) <= 2e-6 * float(b.norm()), i
