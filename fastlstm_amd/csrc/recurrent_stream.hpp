@@ -3,8 +3,8 @@
 //
 // The reference does the same above H = 64 (fp32) / 128 (16-bit): RELOAD_WEIGHTS, fastlstm/lstm.py:70-72,
 // fastlstm/kernels.py:464, 550-626 (forward) and 1362-1383 (reverse, always).  Here the resident kernels
-// cover everything up to 32 MiB of W_h (H = 2048 in 16 bits, 1024 in fp32) and, in 16 bits, multiples of 64 up to H = 4096
-// (recurrent_fwd_big.hpp, recurrent_bwd_big.hpp); these kernels take the rest, so that no hidden size is refused.
+// cover everything up to 32 MiB of W_h (H = 2048 in 16 bits, 1024 in fp32) and, in 16 bits, multiples of 64 up to H = 4096,
+// in fp32 multiples of 256 up to 2048 (recurrent_fwd_big.hpp, recurrent_bwd_big.hpp); these kernels take the rest, so that no hidden size is refused.
 // Mathematics, stored values and rounding points are those of lstm_fwd_persistent_kernel / lstm_bwd_persistent_kernel.
 //
 // What bounds a step here is the stream itself: all of W_h (4H x H elements) crosses the memory system once
