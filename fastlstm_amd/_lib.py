@@ -70,6 +70,7 @@ SIGNATURES = {
     "fastlstm_gemm_dx_wgrad": (_i, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _sz, _i, _i, _i, _i, _i, _vp]),
     "fastlstm_diag_step_probe": (_i, [_i, _i, _i, _i, _i, _i, _vp, _sz, _vp]),
     "fastlstm_diag_step_probe_bytes": (_sz, [_i, _i, _i]),
+    "fastlstm_diag_xcd_shape": (_i, [_i, _i, _i, _i, _i, _vp]),
     "fastlstm_ws_status": (_i, [_vp]),
     "fastlstm_device_status": (_i, [_i, _i]),
     "fastlstm_prepare_forward": (_i, [_vp, _sz, _vp, _vp, _vp, _vp, _i, _i, _i, _vp]),

@@ -12,6 +12,7 @@
 #include "recurrent_fwd_xcd.hpp"
 #include "recurrent_step.hpp"
 #include "recurrent_bwd_big.hpp"
+#include "recurrent_xcd_cases.hpp"
 
 using namespace fastlstm;
 
@@ -307,16 +308,9 @@ struct XcdCfg {
     size_t xslot;              // bytes of one exchange slot (of kXchgSlots)
 };
 
-// The XCD-local kernels apply when the device deals workgroups to XCDs in turn, the shape fits
-// and the workspace holds kXchgSlots exchange slots.
-// `launch_rows`: batch rows of this launch (0: all B_all of them).
-// copies > 1: that many recurrences of this shape share the launch, so the unit tile has to leave room for all their
-// groups.
-bool select_xcd(int T, int B_all, int H, int dtype, bool backward, size_t ws_bytes, XcdCfg *c, int launch_rows = 0,
-                int copies = 1) {
-    const int B = launch_rows ? launch_rows : B_all;
-    DeviceInfo di;
-    if (!(g_families.load() & 1) || device_info(-1, &di) != FASTLSTM_OK || di.xcd_round_robin != 1) return false;
+// Shape of the launch that holds `copies` recurrences of B rows (their unit tile leaves room for all their groups); false if none does.
+// Whether there is a kernel of that shape is for the caller to ask (xcd_instance_exists).
+static bool xcd_shape(int B, int H, int dtype, bool backward, int copies, XcdCfg *c) {
     const bool fp32 = dtype == FASTLSTM_FP32;
     const int s = elem_bytes(dtype), parts = fp32 ? 3 : 1;   // (fp32: operand blocks per k-step, recurrent_parts.hpp)
     const int K = backward ? 4 * H : H;
@@ -350,12 +344,24 @@ bool select_xcd(int T, int B_all, int H, int dtype, bool backward, size_t ws_byt
     c->n_groups = cdiv(B, bt);
     if (copies * c->n_groups > kNumXcd * c->gpx) return false;   // (the tile loop above guarantees it; the kernels index counters by group)
     c->xslot = (size_t)c->n_groups * c->ntw * c->ks * parts * kFragBytes;
-    if (ws_bytes < kWsHeaderBytes + kWsCounterBytes + kXchgSlots * (size_t)copies * c->xslot) return false;
     // partial sums of the K-shares, gates tile(s), two state tiles (as the kernels lay them out)
     const int gseg = ht * s, gates = bt * (4 * gseg + 16), states = 2 * bt * (gseg + 16);
     const int shares = backward || (c->nwv == 8 && c->ntw == 1) ? 8 : 4;
     c->lds = shares * c->mt * c->ntw * kFragBytes + (backward ? c->ntw * (gates + states) : 2 * gates + states);
     return true;
+}
+
+// The XCD-local kernels apply when the device deals workgroups to XCDs in turn, the shape fits
+// and the workspace holds kXchgSlots exchange slots.
+// `launch_rows`: batch rows of this launch (0: all B_all of them).
+// copies > 1: that many recurrences of this shape share the launch.
+bool select_xcd(int T, int B_all, int H, int dtype, bool backward, size_t ws_bytes, XcdCfg *c, int launch_rows = 0,
+                int copies = 1) {
+    DeviceInfo di;
+    if (!(g_families.load() & 1) || device_info(-1, &di) != FASTLSTM_OK || di.xcd_round_robin != 1) return false;
+    if (!xcd_shape(launch_rows ? launch_rows : B_all, H, dtype, backward, copies, c)) return false;
+    if (!xcd_instance_exists(dtype == FASTLSTM_FP32, backward, c->mt, c->nkw, c->ntw, c->nwv)) return false;
+    return ws_bytes >= kWsHeaderBytes + kWsCounterBytes + kXchgSlots * (size_t)copies * c->xslot;
 }
 
 // GEMM work of `flop` on `n_helpers` CUs inside a recurrent launch of about rec_ms: worth while when the launch, which
@@ -2346,6 +2352,17 @@ int fastlstm_device_status(int device, int clear) {
     if (!di.status_host || __atomic_load_n(di.status_host, __ATOMIC_RELAXED) == 0) return FASTLSTM_OK;
     if (clear) __atomic_store_n(di.status_host, 0, __ATOMIC_RELAXED);
     return FASTLSTM_ERR_TIMEOUT;
+}
+
+int fastlstm_diag_xcd_shape(int B, int H, int dtype, int backward, int copies, int *shape) {
+    if (!shape) return FASTLSTM_ERR_NULL;
+    if (!dtype_ok(dtype)) return FASTLSTM_ERR_DTYPE;
+    if (B <= 0 || H <= 0 || copies < 1 || copies > kMaxSideBySide) return FASTLSTM_ERR_DIM;
+    XcdCfg c;
+    if (!xcd_shape(B, H, dtype, backward != 0, copies, &c)) return 0;
+    const int v[5] = {c.mt, c.nkw, c.ntw, c.nwv, c.lds};
+    std::copy(v, v + 5, shape);
+    return xcd_instance_exists(dtype == FASTLSTM_FP32, backward != 0, c.mt, c.nkw, c.ntw, c.nwv) ? 1 : 2;
 }
 
 void fastlstm_set_gemm_baseline(int on) { fastlstm::set_gemm_baseline(on); }

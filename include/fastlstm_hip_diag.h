@@ -59,6 +59,11 @@ int fastlstm_diag_step_probe(int kind, int mode, int members, int H, int rows, i
                              size_t ws_bytes, void *stream);
 size_t fastlstm_diag_step_probe_bytes(int steps, int H, int rows);
 
+/* Diagnostics: which XCD-local kernel `copies` recurrences of B rows and H units side by side would run on a device of 8 XCDs with 32
+ * compute units (no device is asked).  0 = none, 1 = the one in shape[0 .. 3] (unit tiles of a workgroup, k-steps of a wave, batch tiles,
+ * waves) with shape[4] bytes of LDS, 2 = the rule yields a shape that no kernel is compiled for; negative: fastlstm_status. */
+int fastlstm_diag_xcd_shape(int B, int H, int dtype, int backward, int copies, int *shape);
+
 #ifdef __cplusplus
 }
 #endif

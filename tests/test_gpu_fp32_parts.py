@@ -1,5 +1,7 @@
 """fp32 recurrences whose numbers travel and multiply as three bf16 parts (csrc/recurrent_parts.hpp): half k-steps (H = 16 mod 32), every
 unit tile and batch tile of the XCD-local and the whole-CU kernels, against float64; numbers that are not finite."""
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -27,6 +29,38 @@ def test_against_float64(B, H):
                        ("dx", dx, want["dx"].reshape(T * B, -1))):
         a, b = a.double().cpu().numpy(), b.numpy()
         assert np.linalg.norm(a - b) <= 1e-6 * np.linalg.norm(b), name   # (2-norm: some 2e-7 from the rounding of every step's results)
+
+
+# 32 units per workgroup, forward: groups of 16 rows and of 32
+@pytest.mark.parametrize("B,H,shape", [(520, 256, (8, 2, 2, 8)), (1024, 224, (8, 2, 2, 8)), (600, 192, (8, 2, 1, 8)), (1100, 128, (8, 2, 2, 8)),
+                                       (1500, 96, (8, 2, 2, 8))])
+def test_32_units_per_workgroup(B, H, shape):
+    got = (ctypes.c_int * 5)()
+    assert _lib.load().fastlstm_diag_xcd_shape(B, H, 0, 0, 1, got) == 1 and tuple(got)[:4] == shape
+    test_against_float64(B, H)
+
+
+@pytest.mark.parametrize("B,H,n", [(300, 256, 2), (165, 256, 3)])
+def test_32_units_per_workgroup_side_by_side(B, H, n):
+    """One forward launch, the results of calls by themselves to rounding (those have 16 units per workgroup: other sums)."""
+    lib, code, T = _lib.load(), 0, 5
+    gs = [operands(T, B, H, torch.float32, seed=s)[1] for s in range(n)]
+    plan = L._plan(gs[0]["x"].device, B, H, code, False)
+    size = lib.fastlstm_multi_workspace_bytes(plan, n, T, H, code, 0)
+    assert lib.fastlstm_multi_fused(n, T, B, H, code, 0, size) == 1
+    ws = torch.zeros(size, dtype=torch.uint8, device="cuda")
+    bufs = []
+    for g in gs:
+        out, cell = (torch.zeros(T + 1, B, H, device="cuda") for _ in range(2))
+        out[0], cell[0] = g["h0"], g["c0"]
+        bufs.append((g["x"] @ g["Wx"].t() + g["bx"] + g["bh"], out, cell, g["Wh"]))
+    arr = lambda i: (ctypes.c_void_p * n)(*[b[i].data_ptr() for b in bufs])
+    _lib.check(lib.fastlstm_fwd_persistent_multi(n, arr(0), arr(1), arr(2), arr(3), ws.data_ptr(), size, T, B, H, code, 1,
+                                                 torch.cuda.current_stream().cuda_stream), "fwd multi")
+    for g, (_, out, cell, _) in zip(gs, bufs):
+        o, c, _ = L.lstm_persistent_fwd(g["x"], g["h0"], g["c0"], g["Wx"], g["bx"], g["Wh"], g["bh"])
+        for a, b in ((out, o), (cell, c)):
+            assert float((a.double() - b.double()).norm()) <= 1e-6 * float(b.double().norm())   # (some 2e-7 for either from rounding)
 
 
 @pytest.mark.parametrize("B,H", [(19, 640), (40, 1024)])
