@@ -6,11 +6,11 @@ namespace fastlstm {
 
 namespace {
 
-template <bool A_KM, bool B_KM, int T, bool TWO> hipError_t launch_t(const GemmF32Params &g, hipStream_t s) {
+template <bool A_KM, bool B_KM, int T, bool TWO, bool ALL = false> hipError_t launch_t(const GemmF32Params &g, hipStream_t s) {
     constexpr int WN = T / 64;
     using F = F32Tile<T, T, 2, WN>;
     static bool attr_set = false;
-    auto kern = gemm_f32_kernel<A_KM, B_KM, T, T, 2, WN, TWO>;
+    auto kern = gemm_f32_kernel<A_KM, B_KM, T, T, 2, WN, TWO, ALL>;
     if (!attr_set) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, F::LDS_BYTES);
         if (e != hipSuccess) return e;
@@ -32,7 +32,7 @@ template <bool A_KM, bool B_KM, int T, bool TWO> hipError_t launch_t(const GemmF
 void gemm_f32_plan(int M, int N1, int N2, int K, bool allow_split, bool two, int *tile, int *splits, int *k_per_split) {
     double best = 0.;
     *splits = 0;
-    for (int t = 256; t >= 128; t /= 2) {
+    for (int t = K > kF32AllK ? 256 : 128; t >= 128; t /= 2) {
         const long long tiles = (long long)cdiv(M, t) * (cdiv(N1, t) + cdiv(N2, t));
         const int most = !allow_split ? 1 : std::max(1, std::min(64, K / (N2 ? 128 : 160)));
         const int least = (int)std::min<long long>(most, t == 256 ? 256 / tiles : tiles >= 512 ? 1 : std::max<long long>(two ? 1 : 2, (255 + tiles) / tiles));
@@ -54,6 +54,10 @@ void gemm_f32_plan(int M, int N1, int N2, int K, bool allow_split, bool two, int
 }
 
 hipError_t launch_gemm_f32(const GemmF32Params &g, bool a_km, bool b_km, int tile, hipStream_t s) {
+    if (g.p.K <= kF32AllK && tile == 128 && g.p.splits == 1) {
+        if (a_km && b_km) return launch_t<true, true, 128, true, true>(g, s);
+        if (!a_km) return b_km ? launch_t<false, true, 128, true, true>(g, s) : launch_t<false, false, 128, true, true>(g, s);
+    }
     if (a_km && b_km) return tile == 256 ? launch_t<true, true, 256, false>(g, s) : launch_t<true, true, 128, true>(g, s);
     if (a_km || (!b_km && g.p.splits > 1)) return hipErrorInvalidValue;
     if (!b_km) return tile == 256 ? launch_t<false, false, 256, false>(g, s) : launch_t<false, false, 128, false>(g, s);

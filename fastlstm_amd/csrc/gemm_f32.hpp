@@ -2,18 +2,22 @@
 //     C[m][n] = sum_k A(m,k) * B(n,k)   [+ bias0[n] + bias1[n]]
 // the contraction of gemm.hpp for every shape, with each operand K-contiguous or K-major.
 //
-// An fp32 number is the exact sum of three bf16 numbers of 8 significant bits each (cut off, not rounded: the cuts keep the sign,
-// cannot overflow, and what is left after two of them fits the third).  Of the nine products of two such sums the three smallest
-// (below 2^-22 of the largest) are left out; the other six go to v_mfma_f32_32x32x16_bf16, which runs at 16 times the rate of the
-// fp32 MFMA, and are added in fp32, the small ones first.  Six roundings of the sum per 16 products: against 64 bits the results are
-// nearer than those of v_mfma_f32_16x16x4_f32 in tiles of the same size were (relative error of x.Wx^T at K = 1024 5.7e-7 -> 4.9e-7,
-// of d.Wx at K = 4096 1.15e-6 -> 1.01e-6; over thirteen shapes of a layer every result and gradient at 0.2 ... 1.0 times what it was).
+// An fp32 number is the exact sum of three bf16 numbers: the nearest one, the one nearest to what is left, and the rest, which is at
+// most half a step of the second and fits 8 bits.  The products of two such sums go to v_mfma_f32_32x32x16_bf16, which runs at 16 times
+// the rate of the fp32 MFMA, and are added in fp32, the small ones first.
+//  * K > 64: six of the nine.  Left out are the three smallest, each below 2^-24 of the largest and of either sign.  (Parts that are cut
+//    off instead of rounded all have the number's sign: results came out 4e-8 low, and x.Wx^T of K = 4096 terms of one sign, where the
+//    MFMA drops what lies far below the running sum, 1e-5.)  Six roundings of the sum per 16 terms: fewer than v_mfma_f32_16x16x4_f32's.
+//  * K <= 64: all nine, the eight small ones in sums of their own, so that the large ones are rounded once per 16 terms.
+//  Error against 64 bits (2-norm over that of the result) in tiles of v_mfma_f32_16x16x4_f32 and here, x.Wx^T: K = 1 2.5e-8, 2.5e-8; 2 3.1e-8,
+//  2.6e-8; 8 5.4e-8, 2.8e-8; 64 1.4e-7, 4.9e-8; 65 1.5e-7, 1.2e-7; 1024 5.7e-7, 4.9e-7; 16384 2.3e-6, 2.1e-6; terms of one sign: K = 64 1.2e-7,
+//  4.1e-8; 1024 4.7e-7, 3.2e-7; 16384 1.9e-6, 1.2e-6.
 //  * what bounds it: the matrix units (16-bit products at 1.65 PFLOP/s are what they reach on random data; that is 275 here) and, next
 //    to them, the LDS (half of its cycles) and the conversions, which lie among the MFMAs, three vector instructions to each (behind
-//    them instead: 205).  TFLOP/s of fp32, before and here: M = 8192, N = 8192, K = 2048 x.Wx^T 136 -> 213, d.Wx 136 -> 231, weight
+//    them instead: 205).  TFLOP/s of fp32, on the fp32 MFMA and here: M = 8192, N = 8192, K = 2048 x.Wx^T 136 -> 213, d.Wx 136 -> 231, weight
 //    gradients 133 -> 235; M = 16384, I = H = 1024 weight gradients 131 -> 229; M = 8192, I = 512, H = 1024 97 -> 195.  (Parts below 2^-133, the least bf16 number, are lost.)
-//  * infinities: inf - inf of the cut is no number.  A workgroup that has met one computes its tile again with the fp32 MFMA
-//    (at the end of the kernel), so that they come out as they do there.  (A NaN stays one either way.)
+//  * infinities: what is left of one is no number, as of a finite one that is rounded to one.  A workgroup with a sum that is not finite
+//    computes its tile again with the fp32 MFMA (at the end of the kernel), so that the results are those of that.
 //  * staging: global -> registers, a k-tile ahead of the conversion -> three bf16 planes in LDS, in MFMA operand order, double
 //    buffered; one barrier per k-tile of 16.  Half of the waves stage A, the others B.
 //  * a K-major operand is transposed on the way: a thread loads 4 k x 4 rows and stores 4 rows x 4 k; rows are stored at
@@ -30,6 +34,7 @@ namespace fastlstm {
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kF32BK = 16;   // k of a stage: one MFMA k-step
+constexpr int kF32AllK = 64;   // up to this K all nine products are added (see above)
 
 struct GemmF32Params {
     GemmParams p;
@@ -47,31 +52,34 @@ template <int BM, int BN, int WM, int WN> struct F32Tile {
     static_assert(BM == BN && BM == THREADS / 2, "half of the threads stage 16 elements each of either operand");
 };
 
-// The largest magnitude met (a NaN does not count).
-__device__ __forceinline__ void max_magnitude(float &top, float a, float b) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    asm("v_max3_f32 %0, %0, abs(%1), abs(%2)" : "+v"(top) : "v"(a), "v"(b));
-#endif
+// Two values, rounded to bf16 and packed in order; and the values of such a pair.
+__device__ __forceinline__ unsigned bf16_pair(float a, float b) {
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(unsigned, __builtin_convertvector(f32x2{a, b}, bf16x2));
 }
+__device__ __forceinline__ float pair_first(unsigned p) { return __builtin_bit_cast(float, p << 16); }
+__device__ __forceinline__ float pair_second(unsigned p) { return __builtin_bit_cast(float, p & 0xffff0000u); }
 
 // Four values -> their three bf16 parts, packed in order.
 struct F32Planes {
-    float x[4], r[4];
+    float r[4];
     u32x2 hi, mid, lo;
-    __device__ __forceinline__ void cut(const f32x4 v, float &top) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const float f = v[e];
-            x[e] = f;
-            r[e] = f - upper_half(f);
-        }
-        max_magnitude(top, x[0], x[1]);
-        max_magnitude(top, x[2], x[3]);
+    __device__ __forceinline__ void cut(const f32x4 v) {
+        const float x[4] = {v[0], v[1], v[2], v[3]};
+        split(x, hi);
     }
     __device__ __forceinline__ void pack() {
-        hi = u32x2{upper_halves(x[0], x[1]), upper_halves(x[2], x[3])};
-        mid = u32x2{upper_halves(r[0], r[1]), upper_halves(r[2], r[3])};
-        lo = u32x2{upper_halves(r[0] - upper_half(r[0]), r[1] - upper_half(r[1])), upper_halves(r[2] - upper_half(r[2]), r[3] - upper_half(r[3]))};
+        split(r, mid);
+        lo = u32x2{bf16_pair(r[0], r[1]), bf16_pair(r[2], r[3])};
+    }
+    __device__ __forceinline__ void split(const float *x, u32x2 &part) {   // x -> its first part, and what is left of it in r
+        part = u32x2{bf16_pair(x[0], x[1]), bf16_pair(x[2], x[3])};
+#pragma unroll
+        for (int e = 0; e < 4; e += 2) {
+            r[e] = x[e] - pair_first(part[e / 2]);
+            r[e + 1] = x[e + 1] - pair_second(part[e / 2]);
+        }
     }
 };
 
@@ -113,9 +121,9 @@ template <int BM> struct F32Stager {
     }
     // piece i of a thread into the three planes of a stage's operand, [row tile of 32][plane][lane: k half, row][8 k], in three
     // parts that the main loop deals out among its MFMAs
-    template <bool KM> __device__ __forceinline__ void store(int part, int i, unsigned char *op, const f32x4 (&v)[4], F32Planes &w, float &top) const {
+    template <bool KM> __device__ __forceinline__ void store(int part, int i, unsigned char *op, const f32x4 (&v)[4], F32Planes &w) const {
         if (part == 0) {
-            w.cut(KM ? f32x4{v[0][i], v[1][i], v[2][i], v[3][i]} : v[i], top);
+            w.cut(KM ? f32x4{v[0][i], v[1][i], v[2][i], v[3][i]} : v[i]);
         } else if (part == 1) {
             w.pack();
         } else {
@@ -135,10 +143,11 @@ __device__ __forceinline__ void lds_barrier() {
 #endif
 }
 
-// TWO: the five small products have sums of their own, so that the large ones are rounded once per 16 k instead of six times (an error
+// TWO: the small products have sums of their own, so that the large ones are rounded once per 16 k instead of six times (an error
 // 2.6 times smaller: fewer parts of K for the same one).  Only where the sums are split anyway: without a split the two tile sizes add up
 // in the same order, so that a range of rows has the bits that it has within the whole.
-template <bool A_KM, bool B_KM, int BM, int BN, int WM, int WN, bool TWO>
+// ALL: nine products (K <= kF32AllK).
+template <bool A_KM, bool B_KM, int BM, int BN, int WM, int WN, bool TWO, bool ALL>
 __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_kernel(const GemmF32Params g) {
     using F = F32Tile<BM, BN, WM, WN>;
     constexpr int TA = F::TA, TB = F::TB;
@@ -167,7 +176,6 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_kernel(const GemmF32
     const F32Stager<BM> st{stages_a ? A : B, stages_a ? p.lda : p.ldb, stages_a ? p.M - m0 : p.N - n0, ke, tid & (F::THREADS / 2 - 1)};
     const bool sums = A_KM && g.db_part && nt == 0 && stages_a;
     f32x4 dsum = {0.f, 0.f, 0.f, 0.f}, dsum16 = {0.f, 0.f, 0.f, 0.f};   // (of the last up to 16 k-tiles, of those before)
-    float top = 0.f;
 
     f32x16 acc[TA][TB], acc2[TWO ? TA : 1][TWO ? TB : 1];
     auto clear = [&](auto &c) {
@@ -208,27 +216,30 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_kernel(const GemmF32
             for (int b = 0; b < TB; ++b)
 #pragma unroll
                 for (int s = 0; s < 3; ++s) fb[b][s] = frag(sb, wn * TB + b, s);
-            constexpr int pa[6] = {2, 0, 1, 1, 0, 0}, pb[6] = {0, 2, 1, 0, 1, 0}, SPP = 6 * TA / 4;   // (SPP: products per piece)
+            // (the parts of A and B that a product takes; the twelve steps of the conversion are spread over the products of the tile)
+            constexpr int pa[9] = {2, 2, 1, 2, 0, 1, 1, 0, 0}, pb[9] = {2, 1, 2, 0, 2, 1, 0, 1, 0}, P0 = ALL ? 0 : 3, NP = 9 - P0;
+            constexpr auto slot_of = [](int step) { return step * NP * TA / 12; };
+            int step = 0;
 #pragma unroll
-            for (int sl = 0; sl < 6 * TA; ++sl) {
-                const int a = sl / 6, i = sl % 6;
+            for (int sl = 0; sl < NP * TA; ++sl) {
+                const int a = sl / NP, i = sl % NP;
                 if (i == 2 && a + 1 < TA)
 #pragma unroll
                     for (int s = 0; s < 3; ++s) fa[(a + 1) & 1][s] = frag(sa, wm * TA + a + 1, s);
 #pragma unroll
                 for (int b = 0; b < TB; ++b) {
-                    f32x16 &c = TWO && i < 5 ? acc2[TWO ? a : 0][TWO ? b : 0] : acc[a][b];
-                    c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[b][pb[i]], fa[a & 1][pa[i]], c, 0, 0, 0);
+                    f32x16 &c = TWO && i < NP - 1 ? acc2[TWO ? a : 0][TWO ? b : 0] : acc[a][b];
+                    c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[b][pb[P0 + i]], fa[a & 1][pa[P0 + i]], c, 0, 0, 0);
                 }
                 if constexpr (NEXT)
-                    if (sl % SPP % (SPP / 3) == 0) st.template store<KM>(sl % SPP / (SPP / 3), sl / SPP, op, v, w, top);
+                    for (; step < 12 && slot_of(step) == sl; ++step) st.template store<KM>(step % 3, step / 3, op, v, w);
                 __builtin_amdgcn_sched_barrier(0);
             }
         };
         st.template load<KM>(kb, v);
         sum(0);
 #pragma unroll
-        for (int i = 0; i < 12; ++i) st.template store<KM>(i % 3, i / 3, smem + (stages_a ? 0 : F::A_BYTES), v, w, top);
+        for (int i = 0; i < 12; ++i) st.template store<KM>(i % 3, i / 3, smem + (stages_a ? 0 : F::A_BYTES), v, w);
         if (nkt > 1) st.template load<KM>(kb + kF32BK, v);
         lds_barrier();
         for (int kt = 0; kt + 1 < nkt; ++kt) {
@@ -249,7 +260,14 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_kernel(const GemmF32
 
     // lane: row m = lane % 32 of a tile, columns 8 (i / 4) + 4 (lane / 32) + i % 4
     const int ml = lane & 31, q = lane >> 5;
-    if (__syncthreads_or(top == __builtin_inff())) {   // (see above)
+    float zero = 0.f;   // (not if one of the sums is infinite or no number)
+#pragma unroll
+    for (auto &row : acc)
+#pragma unroll
+        for (auto &t : row)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) zero = __builtin_fmaf(t[i], 0.f, zero);
+    if (__syncthreads_or(zero != 0.f)) {   // (see above)
         clear(acc);
         for (int k = kb; k < ke; k += 2) {
             const bool in = k + q < ke;

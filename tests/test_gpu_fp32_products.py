@@ -57,3 +57,44 @@ def test_infinities_and_nans_as_in_the_sum():
         assert torch.equal(torch.isinf(a), torch.isinf(b)) and torch.equal(a[torch.isinf(a)].double(), b[torch.isinf(b)])
         ok = torch.isfinite(b)
         assert float((a.double() - b)[ok].abs().max()) < 1e-3 and bool(ok.any()) and not bool(ok.all())
+
+
+def chain(A, B):
+    """A.B^T as a chain of fp32 multiply-adds (each rounded once; the product in 64 bits is exact)."""
+    acc = torch.zeros(A.shape[0], B.shape[0], device=A.device)
+    for k in range(A.shape[1]):
+        acc = (acc.double() + A[:, k, None].double() * B[None, :, k].double()).float()
+    return acc
+
+
+def each_product(A, B):
+    """A[M,K].B[N,K]^T with N a multiple of 4, by every product that has this K: x.Wx^T, d.Wx, the weight gradients."""
+    lib, st = _lib.load(), torch.cuda.current_stream().cuda_stream
+    (M, K), N = A.shape, B.shape[0]
+    y, z = torch.empty(M, N, device="cuda"), torch.zeros(N, device="cuda")
+    _lib.check(lib.fastlstm_gemm_ifgo(A.data_ptr(), B.data_ptr(), z.data_ptr(), z.data_ptr(), y.data_ptr(), 1, M, K, N // 4, 0, st), "k1")
+    yield "x.Wx^T", y
+    if K % 4 == 0:
+        dx, W, ws = torch.empty(M, N, device="cuda"), B.t().contiguous(), torch.empty(32 << 20, dtype=torch.uint8, device="cuda")
+        _lib.check(lib.fastlstm_gemm_dx_split(A.data_ptr(), W.data_ptr(), dx.data_ptr(), 1, M, N, K // 4, 0, ws.data_ptr(), ws.numel(), st), "dx")
+        yield "d.Wx", dx
+    d = A.t().contiguous()[None]
+    yield "d^T.x", L.Wgrad(d, B.t().contiguous()[None], torch.zeros(2, K, M // 4, device="cuda"))[2]
+
+
+@pytest.mark.parametrize("K", [1, 2, 3, 4, 5, 8, 16, 17, 64, 65, 128, 4096])
+@pytest.mark.parametrize("sign", [False, True])
+def test_no_further_off_than_a_chain_of_multiply_adds(K, sign):
+    """Short contractions, where every rounding shows, the two sides of the line between nine products and six, and a long sum; terms of
+    one sign, whose errors add up if they have one."""
+    g = torch.Generator(device="cuda").manual_seed(K)
+    A, B = (torch.randn(128, K, generator=g, device="cuda") for _ in range(2))
+    if sign:
+        A, B = A.abs() + 0.25, B.abs() + 0.25
+    want = A.double() @ B.double().t()
+    allowed = float((chain(A, B).double() - want).norm())
+    for name, got in each_product(A, B):
+        # (128 x 128 results: 2-norms of rounding errors differ by less than 1 % from sample to sample, K = 1: the same roundings)
+        assert float((got.double() - want).norm()) <= 1.02 * allowed, name
+        if sign and K <= 128:   # the mean of 16384 unbiased roundings of up to 6e-8 is some 3e-10; what the MFMA drops below its sum, K / 16 times
+            assert abs(float(((got.double() - want) / want).mean())) <= 1e-9 + K / 16 * 1e-9, name
