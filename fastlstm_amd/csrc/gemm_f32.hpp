@@ -15,7 +15,10 @@
 //  * what bounds it: the matrix units (16-bit products at 1.65 PFLOP/s are what they reach on random data; that is 275 here) and, next
 //    to them, the LDS (half of its cycles) and the conversions, which lie among the MFMAs, three vector instructions to each (behind
 //    them instead: 205).  TFLOP/s of fp32, on the fp32 MFMA and here: M = 8192, N = 8192, K = 2048 x.Wx^T 136 -> 213, d.Wx 136 -> 231, weight
-//    gradients 133 -> 235; M = 16384, I = H = 1024 weight gradients 131 -> 229; M = 8192, I = 512, H = 1024 97 -> 195.  (Parts below 2^-133, the least bf16 number, are lost.)
+//    gradients 133 -> 235; M = 16384, I = H = 1024 weight gradients 131 -> 229; M = 8192, I = 512, H = 1024 97 -> 195.
+//  * small numbers: the operands are taken times 2^24, which makes the last bit of the least fp32 number a normal bf16 number, and the
+//    sums times 2^-48.  (Without that the parts of numbers below 2^-110 lose bits: of an operand of 1e-36 the products were off by 6e-5, of
+//    1e-38 by 1e-2.)  A sum beyond 2^80, or an operand beyond 2^104, is dealt with as an infinity:
 //  * infinities: what is left of one is no number, as of a finite one that is rounded to one.  A workgroup with a sum that is not finite
 //    computes its tile again with the fp32 MFMA (at the end of the kernel), so that the results are those of that.
 //  * staging: global -> registers, a k-tile ahead of the conversion -> three bf16 planes in LDS, in MFMA operand order, double
@@ -35,6 +38,7 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 constexpr int kF32BK = 16;   // k of a stage: one MFMA k-step
 constexpr int kF32AllK = 64;   // up to this K all nine products are added (see above)
+constexpr float kF32Scale = 0x1p24f, kF32Unscale = 0x1p-48f;   // of an operand, of a product of two
 
 struct GemmF32Params {
     GemmParams p;
@@ -66,7 +70,7 @@ struct F32Planes {
     float r[4];
     u32x2 hi, mid, lo;
     __device__ __forceinline__ void cut(const f32x4 v) {
-        const float x[4] = {v[0], v[1], v[2], v[3]};
+        const float x[4] = {v[0] * kF32Scale, v[1] * kF32Scale, v[2] * kF32Scale, v[3] * kF32Scale};
         split(x, hi);
     }
     __device__ __forceinline__ void pack() {
@@ -267,7 +271,9 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_kernel(const GemmF32
         for (auto &t : row)
 #pragma unroll
             for (int i = 0; i < 16; ++i) zero = __builtin_fmaf(t[i], 0.f, zero);
+    float unscale = kF32Unscale;
     if (__syncthreads_or(zero != 0.f)) {   // (see above)
+        unscale = 1.f;
         clear(acc);
         for (int k = kb; k < ke; k += 2) {
             const bool in = k + q < ke;
@@ -310,7 +316,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_kernel(const GemmF32
             for (int i = 0; i < 4; ++i) {
                 const int n = n0 + (wn * TB + b) * 32 + 8 * i + 4 * q;
                 if (n >= p.N) continue;
-                f32x4 r = {acc[a][b][4 * i], acc[a][b][4 * i + 1], acc[a][b][4 * i + 2], acc[a][b][4 * i + 3]};
+                f32x4 r = f32x4{acc[a][b][4 * i], acc[a][b][4 * i + 1], acc[a][b][4 * i + 2], acc[a][b][4 * i + 3]} * unscale;
                 if (bias0 && !part)
 #pragma unroll
                     for (int e = 0; e < 4; ++e)

@@ -98,3 +98,16 @@ def test_no_further_off_than_a_chain_of_multiply_adds(K, sign):
         assert float((got.double() - want).norm()) <= 1.02 * allowed, name
         if sign and K <= 128:   # the mean of 16384 unbiased roundings of up to 6e-8 is some 3e-10; what the MFMA drops below its sum, K / 16 times
             assert abs(float(((got.double() - want) / want).mean())) <= 1e-9 + K / 16 * 1e-9, name
+
+
+@pytest.mark.parametrize("a,b", [(2.0 ** -107, 1.0), (2.0 ** -113, 1.0), (2.0 ** -126, 1.0), (2.0 ** -126, 2.0 ** 20), (2.0 ** -140, 2.0 ** 30),
+                                 (2.0 ** -60, 2.0 ** -60), (2.0 ** 79, 1.0), (2.0 ** 100, 2.0 ** -3), (2.0 ** 120, 2.0 ** -30), (2.0 ** 127, 2.0 ** -10)])
+def test_small_and_large_numbers(a, b):
+    """Magnitudes over the whole range of fp32, numbers below its least normal one too (exact in the comparison: they are drawn as such)."""
+    for K in (8, 100):
+        g = torch.Generator(device="cuda").manual_seed(K)
+        A, B = ((torch.rand(128, K, generator=g, device="cuda") * 2 - 1) * s for s in (a, b))
+        want = A.double() @ B.double().t()
+        allowed = float((chain(A, B).double() - want).norm())   # (2-norms of 16384 errors: as above)
+        for name, got in each_product(A, B):
+            assert float((got.double() - want).norm()) <= 1.05 * allowed, name
