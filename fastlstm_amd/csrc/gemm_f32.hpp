@@ -302,35 +302,48 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_kernel(const GemmF32
             g.db_part[(size_t)split * p.M + m0 + tid] = (red[tid] + red[BM + tid]) + (red[2 * BM + tid] + red[3 * BM + tid]);
     }
 
+    // C leaves by rows: a wave's 32 rows go through its part of the LDS (rows padded by 16 bytes), 16 lanes store 256 bytes of a row.
+    // Straight from the accumulators an instruction stores 32 bytes of every row: with few k that was most of the time.  x.Wx^T, us:
+    // T*B = 40000, I = 64, H = 256 102 -> 63, H = 1024 383 -> 250; 280000, 64, 256 682 -> 453; 16384, 1024, 1024 685 -> 627.
+    constexpr int CN = TB * 32, CROW = CN * 4 + 16, LPR = CN / 4, RPI = 64 / LPR;   // columns of a wave, lanes per row, rows per instruction
+    static_assert(F::WAVES * 32 * CROW <= F::LDS_BYTES, "a row tile of every wave");
     const float *bias0 = static_cast<const float *>(p.bias0), *bias1 = static_cast<const float *>(p.bias1);
     const bool part = p.splits > 1;
     float *C = part ? p.Cpart + (size_t)split * p.M * p.N : static_cast<float *>(p.C);
     const int ldc = part ? p.N : p.ldc;
+    unsigned char *const mine = smem + wave * 32 * CROW;
+    const int n = n0 + wn * CN + lane % LPR * 4;
+    f32x4 bias = {0.f, 0.f, 0.f, 0.f};
+    if (bias0 && !part)
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (n + e < p.N) bias[e] = bias0[n + e] + (bias1 ? bias1[n + e] : 0.f);
+    __syncthreads();   // the last k-tile (and the sums of A) are read
 #pragma unroll
     for (int a = 0; a < TA; ++a) {
-        const int m = m0 + (wm * TA + a) * 32 + ml;
-        if (m >= p.M) continue;
 #pragma unroll
         for (int b = 0; b < TB; ++b)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int n = n0 + (wn * TB + b) * 32 + 8 * i + 4 * q;
-                if (n >= p.N) continue;
-                f32x4 r = f32x4{acc[a][b][4 * i], acc[a][b][4 * i + 1], acc[a][b][4 * i + 2], acc[a][b][4 * i + 3]} * unscale;
-                if (bias0 && !part)
+            for (int i = 0; i < 4; ++i)
+                *reinterpret_cast<f32x4 *>(mine + ml * CROW + (b * 32 + 8 * i + 4 * q) * 4) =
+                    f32x4{acc[a][b][4 * i], acc[a][b][4 * i + 1], acc[a][b][4 * i + 2], acc[a][b][4 * i + 3]} * unscale;
+        __builtin_amdgcn_wave_barrier();   // (a wave's LDS accesses are done in order)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (n + e < p.N) r[e] += bias0[n + e] + (bias1 ? bias1[n + e] : 0.f);
-                float *dst = C + (size_t)m * ldc + n;
-                typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
-                if (n + 3 < p.N) {   // (non-temporal: GemmParams::keep_c)
-                    if (part || p.keep_c) *reinterpret_cast<f32x4u *>(dst) = r;
-                    else __builtin_nontemporal_store(r, reinterpret_cast<f32x4u *>(dst));
-                } else
+        for (int k = 0; k < 32 / RPI; ++k) {
+            const int row = lane / LPR + RPI * k, m = m0 + (wm * TA + a) * 32 + row;
+            const f32x4 r = *reinterpret_cast<const f32x4 *>(mine + row * CROW + lane % LPR * 16) + bias;
+            if (m >= p.M || n >= p.N) continue;
+            float *dst = C + (size_t)m * ldc + n;
+            typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
+            if (n + 3 < p.N) {   // (non-temporal: GemmParams::keep_c)
+                if (part || p.keep_c) *reinterpret_cast<f32x4u *>(dst) = r;
+                else __builtin_nontemporal_store(r, reinterpret_cast<f32x4u *>(dst));
+            } else
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        if (n + e < p.N) dst[e] = r[e];
-            }
+                for (int e = 0; e < 4; ++e)
+                    if (n + e < p.N) dst[e] = r[e];
+        }
+        __builtin_amdgcn_wave_barrier();
     }
 }
 
