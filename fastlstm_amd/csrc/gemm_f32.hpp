@@ -102,11 +102,16 @@ template <int BM> struct F32Stager {
             if (whole) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i) __builtin_memcpy(&v[i], base + k0 + at[i], 16);
-            } else {
+            } else {   // (clamped, so that all loads are under way together; what lies past the end is dropped behind them)
+                const int last = ke - 1 - k0;
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) v[i][e] = k + e < ke ? base[k0 + at[i] + e] : 0.f;
+                    for (int e = 0; e < 4; ++e) v[i][e] = base[k0 + at[i] - (th & 3) * 4 + min((th & 3) * 4 + e, last)];
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[i][e] = k + e < ke ? v[i][e] : 0.f;
             }
         } else {               // piece i: k (th / (BM / 4)) * 4 + i, rows (th % (BM / 4)) * 4 ..
             const int c = th % (BM / 4) * 4, k = th / (BM / 4) * 4;
@@ -115,11 +120,15 @@ template <int BM> struct F32Stager {
 #pragma unroll
                 for (int i = 0; i < 4; ++i) __builtin_memcpy(&v[i], src + ((unsigned)(k + i) * (unsigned)ld + (c < rows ? c : 0)), 16);
             } else {
+                const int last = ke - 1 - k0;
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        v[i][e] = k0 + k + i < ke ? src[(unsigned)(k + i) * (unsigned)ld + min(c + e, rows - 1)] : 0.f;
+                    for (int e = 0; e < 4; ++e) v[i][e] = src[(unsigned)min(k + i, last) * (unsigned)ld + min(c + e, rows - 1)];
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[i][e] = k + i <= last ? v[i][e] : 0.f;
             }
         }
     }
