@@ -1034,6 +1034,24 @@ template <typename T> __global__ __launch_bounds__(512) void gemm16_wgrad_kernel
     }
 }
 
+// fp32: the sum of n values `stride` floats apart, in eight sums (what they are rounded by stays in the result), 16 loads in flight
+// (a thread of a thin gradient waits for little else: 128 parts of T*B = 40000, I = 1, H = 16, us, four in flight 43, 16 17).
+template <typename V> __device__ __forceinline__ V sum_of_parts(const float *p, size_t stride, int n) {
+    V s[8] = {};
+    auto add = [&](int k, auto count) __attribute__((always_inline)) {   // (past the end: the last value, which is not added)
+        constexpr int N = decltype(count)::value;
+        V v[N];
+#pragma unroll
+        for (int u = 0; u < N; ++u) v[u] = *reinterpret_cast<const V *>(p + (size_t)min(k + u, n - 1) * stride);
+#pragma unroll
+        for (int u = 0; u < N; ++u) s[u % 8] += k + u < n ? v[u] : V{};
+    };
+    int k = 0;
+    for (; n - k > 8; k += 16) add(k, std::integral_constant<int, 16>{});
+    if (k < n) add(k, std::integral_constant<int, 8>{});
+    return ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+}
+
 // Finishes a weight-gradient launch: out = the sum over splits of the fp32 partials, in split order, for dWx
 // (M x I) and dWh (M x H) -- not called for with splits == 1, then I = H = 0 here -- and db (M) = the sum of its
 // db_parts partial sums.  A thread owns four consecutive elements of a matrix (I and H are multiples of 8) or
@@ -1051,12 +1069,8 @@ __global__ void wgrad_reduce_kernel(const float *part_x, T *dWx, const float *pa
     else {
         i -= qx + qh;
         if (i >= (size_t)M || !db) return;
-        if constexpr (sizeof(T) == 4) {   // (eight sums: what they are rounded by stays in the result)
-            float s[8] = {};
-            for (int k = 0; k < db_parts; k += 8)
-#pragma unroll
-                for (int u = 0; u < 8; ++u) s[u] += k + u < db_parts ? part_db[(size_t)(k + u) * M + i] : 0.f;
-            db[i] = ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
+        if constexpr (sizeof(T) == 4) {
+            db[i] = sum_of_parts<float>(part_db + i, (size_t)M, db_parts);
         } else {
             float s = 0.f;
             for (int k = 0; k < db_parts; ++k) s += part_db[(size_t)k * M + i];
@@ -1064,11 +1078,11 @@ __global__ void wgrad_reduce_kernel(const float *part_x, T *dWx, const float *pa
         }
         return;
     }
-    f32x4 s = {0.f, 0.f, 0.f, 0.f};
-    for (int k = 0; k < splits; ++k) s += *reinterpret_cast<const f32x4 *>(part + (size_t)k * total + i * 4);
     if constexpr (sizeof(T) == 4) {
-        *reinterpret_cast<f32x4 *>(out + i * 4) = s;
+        *reinterpret_cast<f32x4 *>(out + i * 4) = sum_of_parts<f32x4>(part + i * 4, total, splits);
     } else {
+        f32x4 s = {0.f, 0.f, 0.f, 0.f};
+        for (int k = 0; k < splits; ++k) s += *reinterpret_cast<const f32x4 *>(part + (size_t)k * total + i * 4);
         T o[4] = {Elem<T>::from_f32(s[0]), Elem<T>::from_f32(s[1]), Elem<T>::from_f32(s[2]), Elem<T>::from_f32(s[3])};
         *reinterpret_cast<u32x2 *>(out + i * 4) = *reinterpret_cast<u32x2 *>(o);
     }

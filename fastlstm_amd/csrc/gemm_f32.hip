@@ -34,7 +34,8 @@ void gemm_f32_plan(int M, int N1, int N2, int K, bool allow_split, bool two, int
     *splits = 0;
     for (int t = K > kF32AllK ? 256 : 128; t >= 128; t /= 2) {
         const long long tiles = (long long)cdiv(M, t) * (cdiv(N1, t) + cdiv(N2, t));
-        const int most = !allow_split ? 1 : std::max(1, std::min(64, K / (N2 ? 128 : 160)));
+        const int cap = (int)std::max<long long>(64, 256 / tiles);   // (one or two tiles: as many parts as fill the device.  T*B = 280000, I = 1, H = 8 with 64 parts 343 us, now 167)
+        const int most = !allow_split ? 1 : std::max(1, std::min(cap, K / (N2 ? 128 : 160)));
         const int least = (int)std::min<long long>(most, t == 256 ? 256 / tiles : tiles >= 512 ? 1 : std::max<long long>(two ? 1 : 2, (255 + tiles) / tiles));
         for (int sp = std::max(1, least); sp <= most; ++sp) {
             const int kps = sp == 1 ? K : cdiv(cdiv(K, sp), 64) * 64;

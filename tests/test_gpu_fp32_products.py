@@ -111,3 +111,15 @@ def test_small_and_large_numbers(a, b):
         allowed = float((chain(A, B).double() - want).norm())   # (2-norms of 16384 errors: as above)
         for name, got in each_product(A, B):
             assert float((got.double() - want).norm()) <= 1.05 * allowed, name
+
+
+@pytest.mark.parametrize("R,I,H", [(9000, 3, 5), (17000, 1, 32), (9000, 40, 16)])
+def test_thin_gradients_of_many_rows(R, I, H):
+    """One or two output tiles: K in more than 64 parts.  Terms of one sign, whose running sum every rounding is relative to."""
+    g = torch.Generator(device="cuda").manual_seed(R + I)
+    d, x, h = (torch.rand(*s, generator=g, device="cuda") + 0.25 for s in ((1, R, 4 * H), (1, R, I), (2, R, H)))
+    db, _, dWx, dWh = L.Wgrad(d, x, h)
+    D = d[0].double()
+    for got, want in ((dWx, D.t() @ x[0].double()), (dWh, D.t() @ h[0].double()), (db, D.sum(0))):
+        # parts of at most some 200 rows: 2e-7 for the sum of one (its 13 roundings of up to 6e-8 each by their square root), as much for the sum of them
+        assert float((got.double() - want).norm()) <= 4e-7 * float(want.norm())
