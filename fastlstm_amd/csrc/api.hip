@@ -1163,12 +1163,10 @@ size_t fastlstm_wgrad_workspace_bytes(int T, int B, int I, int H, int dtype) {
     size_t part = std::max(sx > 1 ? (size_t)sx * M * I : 0, sh > 1 ? (size_t)sh * M * H : 0) * sizeof(float);
     size_t cs = (size_t)colsum_chunks(K) * M * sizeof(float);
     const size_t small = small_bwd_eligible(dtype, K, I, H) ? small_bwd_workspace(K, I, H) : 0;
-    size_t dx = 0;   // fp32: room for dx's parts (its sums over K are meant to be short, gemm_f32_plan)
-    if (dtype == FASTLSTM_FP32) {
-        int dx_tile, dx_splits;
-        gemm_plan(dtype, K, I, M, M, I, false, true, true, &dx_tile, &dx_splits);
-        dx = dx_splits > 1 ? (size_t)dx_splits * K * I * sizeof(float) : 0;
-    }
+    // room for dx's parts, which a call that computes dx too (fastlstm_gemm_dx_wgrad, fastlstm_bwd_layer) puts here first
+    int dx_splits;
+    gemm_plan(dtype, K, I, M, M, I, false, true, true, &tile, &dx_splits);
+    const size_t dx = dx_splits > 1 ? (size_t)dx_splits * K * I * sizeof(float) : 0;
     return std::max({align_up(cs, 256) + align_up(part, 256), wgrad_merged_workspace(dtype, M, I, H, K), small, dx}) + 256;
 }
 

@@ -24,3 +24,10 @@ def test_every_shape_of_the_xcd_local_kernels_is_compiled(dtype, backward):
     # fp32, forward: units per workgroup 8, 16, 32, with batch tiles of 16 and 32 rows each
     if dtype == 0 and not backward:
         assert {(mt, ntw) for mt, _, ntw, _ in used} == {(mt, ntw) for mt in (2, 4, 8) for ntw in (1, 2)}
+
+
+@pytest.mark.parametrize("T,B,I,H,dtype,parts", [(50, 100, 100, 512, 1, 8), (50, 100, 100, 256, 2, 4), (16, 64, 72, 2048, 1, 2), (16, 16, 64, 256, 0, 2)])
+def test_the_weight_gradients_workspace_holds_the_parts_of_dx(T, B, I, H, dtype, parts):
+    """Few output tiles of d.Wx and a long sum: the product is cut into that many parts at least (operands that the tile kernel takes and
+    ones that it does not, I = 100), whose place is this workspace."""
+    assert _lib.load().fastlstm_wgrad_workspace_bytes(T, B, I, H, dtype) >= parts * T * B * I * 4
