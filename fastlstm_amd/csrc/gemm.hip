@@ -137,6 +137,24 @@ bool gemm16_eligible(int dtype, int M, int N, int K, int lda, int ldb, bool a_km
     return a_bytes < (1ull << 32) && b_bytes < (1ull << 32);
 }
 
+// Parts of K for 64 x 64 tiles, the least time: 0.22 us per k-tile of 64, twice that for two tiles of a CU; adding the parts up is a launch of
+// 3.5 us that moves them at 3.5 TB/s.  us, whole and in parts: M = 1000, N = 64, K = 2048 10.3 -> 7.4; 700, 704, 5632 24 -> 18; both weight
+// gradients of T*B = 4004, I = 104, H = 112 47 -> 24; 640, 640, 2048 stays whole (10.9, in two parts 11.8).
+static int parts_of_few_tiles(int M, int N, int K, int t64) {
+    const int kt = cdiv(K, 64), most = std::max(1, std::min({2 * kNumXcd * 32 / t64, kt / 4, 64}));
+    int best = 1;
+    double least = 0.;
+    for (int sp = 1; sp <= most; ++sp) {
+        double us = cdiv(kt, sp) * (t64 * sp > kNumXcd * 32 ? 0.44 : 0.22);
+        if (sp > 1) us += 3.5 + (2. * sp + 1.) * M * N * sizeof(float) / 3.5e6;
+        if (sp == 1 || us < least) {
+            least = us;
+            best = sp;
+        }
+    }
+    return best;
+}
+
 // Tile edge (256, 128 or 64; 0 = generic kernel) and split-K factor for a product.
 void gemm_plan(int dtype, int M, int N, int K, int lda, int ldb, bool a_km, bool b_km, bool allow_split,
                int *tile, int *splits) {
@@ -158,25 +176,39 @@ void gemm_plan(int dtype, int M, int N, int K, int lda, int ldb, bool a_km, bool
     const int t256 = cdiv(M, 256) * cdiv(N, 256), t128 = cdiv(M, 128) * cdiv(N, 128), t64 = cdiv(M, 64) * cdiv(N, 64);
     // At most two 64 x 64 tiles per CU: a k-tile takes them 0.22 us, the 128 x 128 tile 0.55, and four times as many CUs work (us with
     // 64 and 128: M = 700, N = 2816, K = 704, 484 tiles, 8.7 and 9.9; M = N = 700, K = 2816 14.4 and 25.2; with 768 tiles, M = 1024,
-    // N = 3072, K = 512, 9.7 and 8.1).  Parts from 64 k-tiles on, of 16 or more: adding them up costs ~5 us.
+    // N = 3072, K = 512, 9.7 and 8.1).
     // Not for weight gradients of very many rows: what bounds those is reading the operands, a 64 x 64 tile twice as often (us with 64
     // and 128, thin products of T*B rows, I, H: 173400, 1024, 64 312 and 182; 65536, 64, 256 171 and 123; 32768, 80, 512 204 and 147,
     // 16384 106 and 102, 8192 65 and 81; 32768, 96, 96 49 and 44, 16384 33 and 37).
     const bool many_rows = a_km && b_km && (K >= 32768 || (long long)t64 * K > 1 << 21);
+    // With room for parts and more tiles than CUs, a long sum goes to 128 x 128 tiles in as many parts as one round of them holds (us, 64 x
+    // 64 whole and 128 x 128 in parts: M = 2869, N = 408, K = 4096 32 and 28, 14080 108 and 68; 1100, 1000, 8192 58 and 36; 2000, 640, 4096
+    // 25 and 26).
     if (t64 <= 2 * kNumXcd * 32 && !many_rows) {
-        *tile = 64;
-        if (allow_split && K >= 4096) *splits = std::max(1, std::min(2 * kNumXcd * 32 / t64, K / 1024));
+        const int round128 = kNumXcd * 32 / t128;
+        const bool parts128 = allow_split && t64 > kNumXcd * 32 && K >= 4096 && round128 > 1;
+        *tile = parts128 ? 128 : 64;
+        if (allow_split) *splits = parts128 ? round128 : parts_of_few_tiles(M, N, K, t64);
         return;
     }
     const int max_split = allow_split ? std::max(1, K / 512) : 1;  // >= 8 k-tiles per split
+    // d.Wx has a large output beside its sum, and moving parts of that costs: a k-tile takes 256 x 256 1.8 us, 128 x 128 0.55 alone on a CU and
+    // 1.0 two at a time; parts are added up at 5 TB/s (us, whole on 128 x 128 and in parts on 256 x 256: M = 27870, N = 160, K = 1152 22 and
+    // 39; 3267, 1432, 2688 40 and 53; 7725, 1024, 5632 97 and 114).
+    const auto parts_repay = [&](int t, int tiles, int sp) {
+        const double kt = cdiv(K, 64), per_tile = t == 256 ? 1.8 : tiles * sp > 256 ? 1.0 : 0.55;
+        const double whole = cdiv(t128, 512) * kt * (t128 > 256 ? 1.0 : 0.55);
+        return (a_km && b_km) || cdiv(tiles * sp, t == 256 ? 256 : 512) * kt / sp * per_tile + 3.5 + (2. * sp + 1.) * M * N * sizeof(float) / 5e6 < whole;
+    };
+    const int split256 = std::min(256 / t256, max_split), split128 = t128 < 192 ? std::max(1, std::min(cdiv(512, t128), max_split)) : 1;
     if (t256 >= 192) {
         *tile = 256;
-    } else if (std::min(256 / t256, max_split) * t256 >= 192) {   // (one round of workgroups: the factor rounded down)
+    } else if (split256 * t256 >= 192 && (split256 == 1 || parts_repay(256, t256, split256))) {   // (one round of workgroups: the factor rounded down)
         *tile = 256;
-        *splits = std::min(256 / t256, max_split);
+        *splits = split256;
     } else {
         *tile = 128;
-        if (t128 < 192) *splits = std::max(1, std::min(cdiv(512, t128), max_split));
+        if (split128 > 1 && parts_repay(128, t128, split128)) *splits = split128;
     }
 }
 

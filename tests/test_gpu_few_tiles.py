@@ -52,6 +52,14 @@ def test_products(T, B, I, H, dt):
     assert torch.equal(ifgo(x[:m], Wx, b, 1, m, I, H), y[:m]) and torch.equal(dx(g[:m], Wx, 1, m, I, H), whole[:m])
 
 
+# d.Wx in parts: 64 x 64 tiles in several, 128 x 128 in one round of parts from 257 small tiles and K = 4096 on, and one pass where the parts of a
+# large output would cost more
+@pytest.mark.parametrize("T,B,I,H", [(10, 100, 64, 512), (151, 19, 408, 1024), (30, 929, 160, 288), (33, 99, 1432, 672)])
+@pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
+def test_parts_of_dx(T, B, I, H, dt):
+    test_products(T, B, I, H, dt)
+
+
 # (rows, I, H) of thin weight gradients: 64 x 64 tiles in one part and in several, 128 x 128 ones from 32768 rows or 2^21 rows x tiles on
 @pytest.mark.parametrize("R,I,H", [(500, 80, 96), (16500, 96, 96), (8200, 80, 512), (32767, 192, 64), (32768, 192, 64)])
 @pytest.mark.parametrize("dt", [torch.float16, torch.bfloat16])
