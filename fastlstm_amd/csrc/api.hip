@@ -576,14 +576,14 @@ bool select_wide(int T, int B_all, int H, int dtype, bool backward, size_t ws_by
     c->ks = (backward ? 4 * H : H) / 32;
     c->big = 0;
     if (dtype == FASTLSTM_FP32) {
-        // The whole-CU kernels with 16 units per workgroup, numbers as three parts; two recurrences side by side at most.  us
+        // The whole-CU kernels with 16 units per workgroup, numbers as three parts.  us
         // per step of lstm_fwd_wide_kernel and lstm_bwd_wide_kernel on fp32 operands (forward up to 32 rows: of the general
         // kernel) and here, forward, reverse: H = 1024, B = 128 11.1 -> 7.9, 12.4 -> 10.4; B = 16 5.1 -> 3.9, 6.6 -> 5.9.
         const int n_ht = H / 16, max_groups = kNumXcd * 32 / n_ht;
         const int nt = copies * cdiv(B, 16) <= max_groups ? 1 : 2, groups = cdiv(B, 16 * nt);
         const size_t xslot = (size_t)groups * nt * c->ks * 3 * kFragBytes;
         const size_t partials = backward ? (size_t)groups * n_ht * kBigTeam * nt * kFragBytes : 0;
-        if (copies > 2 || copies * groups > std::min(max_groups, kNumXcd) ||
+        if (copies > kMaxSideBySide || copies * groups > std::min(max_groups, kNumXcd) ||
             ws_bytes < kWsHeaderBytes + kWsCounterBytes + copies * (2 * xslot + partials))
             return false;
         c->big = nt;
@@ -698,6 +698,9 @@ int try_fwd_wide(void *ifgo, void *out, void *cell, const void *Wh, unsigned cha
         q.keep = o.keep;
         q.n_rec = copies;
         if (second) { q.ifgo2 = second->ifgo; q.out2 = second->out; q.cell2 = second->cell; q.Wh2 = second->Wh; }
+        for (int i = 0; i < o.n_more; ++i) {
+            q.ifgo_more[i] = o.more[i][0]; q.out_more[i] = o.more[i][1]; q.cell_more[i] = o.more[i][2]; q.Wh_more[i] = o.more[i][3];
+        }
         q.spin_limit = spin_limit_ticks();
         const int mt = dtype == FASTLSTM_FP32 ? 4 : 8;
         int occ = 0;
@@ -753,6 +756,10 @@ int try_bwd_wide(const void *dout, void *dh, void *dc, const void *ifgo, const v
         if (second) {
             q.dout2 = second[0]; q.dh2 = second[1]; q.dc2 = second[2]; q.ifgo2 = second[3]; q.cell2 = second[4];
             q.d_ifgo2 = second[5]; q.Wh2 = second[6];
+        }
+        for (int i = 0; i < o.n_more; ++i) {
+            q.dout_more[i] = o.more[i][0]; q.dh_more[i] = o.more[i][1]; q.dc_more[i] = o.more[i][2]; q.ifgo_more[i] = o.more[i][3];
+            q.cell_more[i] = o.more[i][4]; q.d_ifgo_more[i] = o.more[i][5]; q.Wh_more[i] = o.more[i][6];
         }
         q.T = T; q.B = B; q.H = H;
         q.b_base = o.row0; q.n_bt = c.n_groups; q.n_ht = c.n_ht;

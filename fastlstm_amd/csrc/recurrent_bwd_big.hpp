@@ -17,8 +17,8 @@
 // lstm_bwd_stream_kernel and here: H = 4096, 64 rows 33.6 -> 12.8, 16 rows 21.1 -> 6.7; H = 3072, 32 rows 16.8 -> 7.2;
 // H = 2560, 64 rows 22.6 -> 9.5.  Of the form with 16 units and 8 waves per CU for H <= 2048 and here: H = 2048, 128 rows 11.0 -> 8.6,
 // 64 rows 9.0 -> 6.2, 32 rows 6.4 -> 5.3; H = 1280, 128 rows 8.7 -> 7.0.
-// Up to H = 2048 (and in fp32) a second recurrence of the same shape may share the launch (the directions of a bidirectional layer, the chunks of
-// a wavefront): the sums are those of a launch of its own, bit by bit.  us per step of a pair on lstm_bwd_wide_kernel and here:
+// Up to H = 2048 a second recurrence of the same shape may share the launch, in fp32 up to H = 1024 a third and a fourth too (the directions of a
+// bidirectional layer, the chunks of a wavefront): the sums are those of a launch of its own, bit by bit.  us per step of a pair on lstm_bwd_wide_kernel and here:
 // H = 2048, B = 16 6.8 -> 5.2, B = 32 9.8 -> 6.5; H = 1536, B = 32 7.7 -> 5.6; H = 1280, B = 20 6.6 -> 5.9.
 // fp32 (lstm_bwd_big_parts_kernel, MT = 4): d_ifgo[t] is exchanged as the three bf16 parts of its numbers, the weights' are all in
 // registers; bounds as in 16 bits with 1.5 times the bytes per number.  H = 1024, us per step of the kernel on the fp32 matrix

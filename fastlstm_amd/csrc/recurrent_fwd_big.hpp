@@ -22,6 +22,8 @@
 // workgroup all in registers, h_t exchanged as parts; the largest of the six products has a sum of its own.  What bounds it: at two
 // batch tiles the 96 H bytes of operand blocks of each (H = 1024: 384 KiB per CU and step), at one the exchange.  H = 1024,
 // us per step of the kernels on the fp32 matrix instructions (1/16 of the rate) and here: B = 128 11.1 -> 7.9, B = 16 5.1 -> 3.9.
+// Up to four recurrences share a launch (T = 256, I = 256, inference / training of three layers, two of them in a launch and three: H = 1024,
+// B = 16 2.93 / 8.48 and 2.20 / 7.38 ms; of four, B = 32 4.23 / 13.4 and 3.76 / 12.8; H = 640, B = 16, three 2.37 / 6.49 and 1.78 / 5.40).
 // Above H = 1024 a workgroup holds 8 units (MT = 2: 384 KiB at H = 2048), one group of up to 64 rows is a launch, and every CU reads the
 // 6 H bytes of each of its rows every step.  T = 100, I = 512, inference with lstm_fwd_stream_kernel and here: H = 2048, B = 1
 // 1.66 -> 0.60 ms, 16 1.74 -> 0.70, 64 4.37 -> 1.65, 200 (four launches) 9.05 -> 5.38; H = 1280, B = 16 1.14 -> 0.57, 100 3.18 -> 2.13.

@@ -38,10 +38,10 @@ struct FwdStreamParams {
     WsHeader *hdr;
     int *flags;        // [n_bt][flag_stride]
     unsigned char *xbuf;   // [2 slots][n_bt][NT][KSP] operand blocks
-    // lstm_fwd_big_parts_kernel: n_rec = 2: a second, independent recurrence of this shape side by side
+    // lstm_fwd_big_parts_kernel: n_rec = 2 ... kMaxSideBySide: further, independent recurrences of this shape side by side
     int n_rec;
-    void *ifgo2, *out2, *cell2;
-    const void *Wh2;
+    void *ifgo2, *out2, *cell2, *ifgo_more[2], *out_more[2], *cell_more[2];
+    const void *Wh2, *Wh_more[2];
     int T, B, H;
     int b_base, n_bt, n_ht, flag_stride;
     int KS, KSP;       // k-steps covering H, padded
@@ -59,9 +59,9 @@ struct BwdStreamParams {
     const void *Wh;    // [4H,H]
     int *team_flags;   // [n_rec n_bt][flag_stride]
     unsigned char *partials;   // [n_rec n_bt][n_ht receivers][4 senders][unit tiles][NT] blocks of fp32 sums
-    int n_rec;         // 2: a second, independent recurrence of this shape side by side, its operands here
-    const void *dout2, *ifgo2, *cell2, *Wh2;
-    void *dh2, *dc2, *d_ifgo2;
+    int n_rec;         // 2 (fp32: up to kMaxSideBySide): further, independent recurrences of this shape side by side, their operands here
+    const void *dout2, *ifgo2, *cell2, *Wh2, *dout_more[2], *ifgo_more[2], *cell_more[2], *Wh_more[2];
+    void *dh2, *dc2, *d_ifgo2, *dh_more[2], *dc_more[2], *d_ifgo_more[2];
     WsHeader *hdr;
     int *flags;
     unsigned char *xbuf;   // [2 slots][n_bt][NT][KSBP]

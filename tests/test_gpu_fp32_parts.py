@@ -40,11 +40,10 @@ def test_32_units_per_workgroup(B, H, shape):
     test_against_float64(B, H)
 
 
-@pytest.mark.parametrize("B,H,n", [(300, 256, 2), (165, 256, 3)])
-def test_32_units_per_workgroup_side_by_side(B, H, n):
-    """One forward launch, the results of calls by themselves to rounding (those have 16 units per workgroup: other sums)."""
-    lib, code, T = _lib.load(), 0, 5
-    gs = [operands(T, B, H, torch.float32, seed=s)[1] for s in range(n)]
+def forward_multi(gs):
+    """[(out, cell, gates)] of recurrences in one launch, the inputs' products by torch"""
+    lib, n, code = _lib.load(), len(gs), 0
+    T, B, H = gs[0]["dout"].shape
     plan = L._plan(gs[0]["x"].device, B, H, code, False)
     size = lib.fastlstm_multi_workspace_bytes(plan, n, T, H, code, 0)
     assert lib.fastlstm_multi_fused(n, T, B, H, code, 0, size) == 1
@@ -53,14 +52,35 @@ def test_32_units_per_workgroup_side_by_side(B, H, n):
     for g in gs:
         out, cell = (torch.zeros(T + 1, B, H, device="cuda") for _ in range(2))
         out[0], cell[0] = g["h0"], g["c0"]
-        bufs.append((g["x"] @ g["Wx"].t() + g["bx"] + g["bh"], out, cell, g["Wh"]))
-    arr = lambda i: (ctypes.c_void_p * n)(*[b[i].data_ptr() for b in bufs])
-    _lib.check(lib.fastlstm_fwd_persistent_multi(n, arr(0), arr(1), arr(2), arr(3), ws.data_ptr(), size, T, B, H, code, 1,
+        bufs.append((out, cell, g["x"] @ g["Wx"].t() + g["bx"] + g["bh"]))
+    arr = lambda ts: (ctypes.c_void_p * n)(*[t.data_ptr() for t in ts])
+    _lib.check(lib.fastlstm_fwd_persistent_multi(n, arr([b[2] for b in bufs]), arr([b[0] for b in bufs]), arr([b[1] for b in bufs]),
+                                                 arr([g["Wh"] for g in gs]), ws.data_ptr(), size, T, B, H, code, 1,
                                                  torch.cuda.current_stream().cuda_stream), "fwd multi")
-    for g, (_, out, cell, _) in zip(gs, bufs):
+    return bufs
+
+
+@pytest.mark.parametrize("B,H,n", [(300, 256, 2), (165, 256, 3), (16, 1024, 3), (32, 1024, 4), (20, 640, 3), (9, 768, 4)])
+def test_forward_side_by_side(B, H, n):
+    """One launch, the results of calls by themselves to rounding (the inputs' products are torch's here, and H = 256 alone has 16 units per
+    workgroup: other sums)."""
+    gs = [operands(5, B, H, torch.float32, seed=s)[1] for s in range(n)]
+    for g, (out, cell, _) in zip(gs, forward_multi(gs)):
         o, c, _ = L.lstm_persistent_fwd(g["x"], g["h0"], g["c0"], g["Wx"], g["bx"], g["Wh"], g["bh"])
         for a, b in ((out, o), (cell, c)):
             assert float((a.double() - b.double()).norm()) <= 1e-6 * float(b.double().norm())   # (some 2e-7 for either from rounding)
+
+
+@pytest.mark.parametrize("B,H,n", [(16, 1024, 3), (32, 1024, 4), (20, 640, 3), (9, 768, 4)])
+def test_three_and_four_side_by_side_are_the_bits_of_calls_by_themselves(B, H, n):
+    lib = _lib.load()
+    size = lib.fastlstm_multi_workspace_bytes(L._plan(torch.device("cuda", 0), B, H, 0, True), n, 5, H, 0, 1)
+    assert lib.fastlstm_multi_fused(n, 5, B, H, 0, 1, size) == 1
+    gs = [operands(5, B, H, torch.float32, seed=s)[1] for s in range(n)]
+    alone = [run(g) for g in gs]
+    recs = [(g, a[1], a[2], g["dh_n"].clone(), g["dc_n"].clone()) for g, a in zip(gs, alone)]
+    for d, r, a in zip(backward(recs), recs, alone):
+        assert torch.equal(d, a[3]) and torch.equal(r[3], a[4]) and torch.equal(r[4], a[5])
 
 
 @pytest.mark.parametrize("B,H", [(19, 640), (40, 1024)])
