@@ -679,7 +679,7 @@ __global__ __launch_bounds__(kWave * NWV) void lstm_bwd_xcd_kernel(const BwdXcdP
                 other[1] = (unsigned)__shfl_down((int)mine[1], 16);
                 if (stores[m]) xch.store16(xgrp + xoff[m], u32x4{mine[0], mine[1], other[0], other[1]});
             } else {
-                const ThreeParts p0(st_d[0]), p1(st_d[1]), p2(st_d[2]), p3(st_d[3]);
+                const ThreeParts p0(st_d[0] * kGradScale), p1(st_d[1] * kGradScale), p2(st_d[2] * kGradScale), p3(st_d[3] * kGradScale);
                 if (stores[m])
 #pragma unroll
                     for (int i = 0; i < P; ++i)
@@ -774,7 +774,7 @@ __global__ __launch_bounds__(kWave * NWV) void lstm_bwd_xcd_kernel(const BwdXcdP
             float v = redf[roff[m]];
 #pragma unroll
             for (int pp = 1; pp < NWV; ++pp) v += redf[roff[m] + pp * MT * NT * kWave * 4];
-            dh_rec[m] = v;
+            dh_rec[m] = P > 1 ? v * kGradUnscale : v;
         }
         // the next step's first workgroup barrier orders these reads before the next writes to `red`
     }

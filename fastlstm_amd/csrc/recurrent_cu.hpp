@@ -343,7 +343,7 @@ __global__ __launch_bounds__((CuShape<T, CW>::THREADS)) void lstm_bwd_cu_kernel(
         c1 = c0;   // c_{t-1} is the next step's c_t
         if (valid) {   // (rows past the batch stay zero in the operand blocks): k = 4 unit + gate
             if constexpr (C::F32) {
-                const ThreeParts p0(d[0]), p1(d[1]), p2(d[2]), p3(d[3]);
+                const ThreeParts p0(d[0] * kGradScale), p1(d[1] * kGradScale), p2(d[2] * kGradScale), p3(d[3] * kGradScale);
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
                     *reinterpret_cast<u32x2 *>(x + frag_offset<O>(4 * i + row, 4 * unit)) =
@@ -379,7 +379,7 @@ __global__ __launch_bounds__((CuShape<T, CW>::THREADS)) void lstm_bwd_cu_kernel(
 #pragma unroll
         for (int i = CH - 2; i >= 0; --i) sum += acc[i];
         const float s0 = sum[0], s1 = sum[1], s2 = sum[2], s3 = sum[3];
-        dh_rec = fold_cells<C::F32>(s0, s1, s2, s3);
+        dh_rec = fold_cells<C::F32>(s0, s1, s2, s3) * (C::F32 ? kGradUnscale : 1.f);
     }
     if (valid) {
         dh[off] = E::from_f32(dh_rec);

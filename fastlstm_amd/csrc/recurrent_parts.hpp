@@ -1,4 +1,6 @@
-// fp32 numbers as sums of three bf16 numbers, for products on the bf16 matrix units (gemm_f32.hpp says why that is exact enough).
+// fp32 numbers as sums of three bf16 numbers, for the recurrent products on the bf16 matrix units: of at least 64 terms, so that six of
+// the nine products of two such sums (three roundings per 32 terms) are nearer to 64 bits than the fp32 matrix instructions are, though the
+// parts are cut off and not rounded (gemm_f32.hpp, where that counts).
 #pragma once
 #include <type_traits>
 
@@ -12,12 +14,17 @@ __device__ __forceinline__ unsigned upper_halves(float a, float b) {
     return __builtin_amdgcn_perm(__builtin_bit_cast(unsigned, b), __builtin_bit_cast(unsigned, a), 0x07060302u);
 }
 
-// The three bf16 parts of a factor of a recurrent product.  A part that is zero where the number is not becomes the least normal
-// number of its sign, and those of an infinity too: infinity times zero would be no number.  Zero stays zero.
+// The three bf16 parts of a factor of a recurrent product.  A part that is zero where the number is not becomes the least bf16 number of
+// its sign, 2^-133, and those of an infinity too: infinity times zero would be no number.  Zero stays zero.  (The matrix units take numbers
+// below the least normal one as they are.)
+// What a number is off by for that, 2^-132, is nothing beside the gates that h and the weights make.  The gate gradients of the reverse pass
+// stand alone, and over a sequence they may fade through all magnitudes: they are taken times 2^16, by which every fp32 number's last bit
+// is a bf16 number, and the sum times 2^-16.  Relative error of dx where |dx| is about 1e-33, 1e-36, 1e-38 (fp32 matrix instructions: 2e-6 at
+// all): 1e-5, 2e-3, 2e-1 without, 2e-6 with it.  A gate gradient beyond 2^112 overflows.
 struct ThreeParts {
     float hi, mid, lo, least;   // (least: that number, for the last four columns)
     __device__ __forceinline__ explicit ThreeParts(float x) {
-        const float tiny = fminf(fabsf(x), 0x1p-126f), r = x - upper_half(x);
+        const float tiny = fminf(fabsf(x), 0x1p-133f), r = x - upper_half(x);
         least = __builtin_copysignf(tiny, x);
         hi = __builtin_canonicalizef(x);
         mid = __builtin_copysignf(fmaxf(fabsf(r), tiny), x);
@@ -25,6 +32,8 @@ struct ThreeParts {
     }
     __device__ __forceinline__ float part(int i) const { return i == 0 ? hi : i == 1 ? mid : i == 2 ? lo : least; }
 };
+
+constexpr float kGradScale = 0x1p16f, kGradUnscale = 0x1p-16f;   // of a gate gradient, of the sum (see above)
 
 // 16 bytes of operand block: 8 consecutive elements of k -> the 16-bit fragment of part i
 template <typename T, typename Get> __device__ __forceinline__ void operand_parts(Get get, u32x4 (&out)[sizeof(T) == 4 ? 3 : 1]) {

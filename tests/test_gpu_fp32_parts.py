@@ -133,3 +133,28 @@ def test_module_between_the_sizes(T, B, H, padded):
     pairs = [(y, yw), (h, hw), (c, cw), (xg.grad, xw.grad)] + [(p.grad, q.grad) for p, q in zip(got.parameters(), want.parameters())]
     for i, (a, b) in enumerate(pairs):   # (2-norm: rounding of every step's results and of sums of fp32 products)
         assert a.shape == b.shape and float((a.double().cpu() - b).norm()) <= 2e-6 * float(b.norm()), i
+
+
+@pytest.mark.parametrize("B,H", [(8, 64), (5, 96), (8, 128), (40, 136), (20, 256), (8, 512), (300, 256), (16, 1024), (8, 1280)])
+def test_gradients_that_fade(B, H):
+    """A loss on the last step and gates that forget: the gradients of the steps before fade through all magnitudes.  Down to the least normal
+    numbers their relative error is that of the sums: an input gradient of step T - n has gone through n products, each 1e-6 off at most."""
+    T, I = 60, 16
+    torch.manual_seed(H)
+    want = torch.nn.LSTM(I, H).double()
+    with torch.no_grad():
+        want.bias_ih_l0[H:2 * H] = -3.0
+    got = FastLSTM(I, H, device="cuda", dtype=torch.float32)
+    got.load_state_dict(want.state_dict())   # (rounds)
+    want.load_state_dict(got.state_dict())
+    x = torch.randn(T, B, I)
+    xg, xw = x.cuda().requires_grad_(), x.double().requires_grad_()
+    got(xg)[0][-1].sum().backward()
+    want(xw)[0][-1].sum().backward()
+    a, b, tested = xg.grad.double().cpu(), xw.grad, 0
+    for t in range(T):
+        size = float(b[t].norm()) / (B * I) ** 0.5
+        if size > 1e-37:
+            assert float((a[t] - b[t]).norm()) <= (T - t) * 1e-6 * float(b[t].norm()), (t, size)
+            tested += size < 1e-33
+    assert tested > 2
