@@ -18,9 +18,10 @@
 //    gradients 133 -> 235; M = 16384, I = H = 1024 weight gradients 131 -> 229; M = 8192, I = 512, H = 1024 97 -> 195.
 //  * small numbers: the operands are taken times 2^24, which makes the last bit of the least fp32 number a normal bf16 number, and the
 //    sums times 2^-48.  (Without that the parts of numbers below 2^-110 lose bits: of an operand of 1e-36 the products were off by 6e-5, of
-//    1e-38 by 1e-2.)  A sum beyond 2^80, or an operand beyond 2^104, is dealt with as an infinity:
-//  * infinities: what is left of one is no number, as of a finite one that is rounded to one.  A workgroup with a sum that is not finite
-//    computes its tile again with the fp32 MFMA (at the end of the kernel), so that the results are those of that.
+//    1e-38 by 1e-2.)  A sum beyond 2^80, or one with an operand beyond 2^104, is dealt with as an infinity:
+//  * infinities: what is left of one is no number, as of a finite one that is rounded to one.  Sums that are not finite are taken from
+//    the fp32 MFMA, 32 x 32 results at a time (behind the main loop): they come out as they do there, and the sums beside them keep their
+//    bits.  (One infinity in x or d, T*B = 16384, I = H = 1024: x.Wx^T 0.7 -> 1.1 ms, weight gradients 1.2 -> 3.8; a NaN costs nothing.)
 //  * staging: global -> registers, a k-tile ahead of the conversion -> three bf16 planes in LDS, in MFMA operand order, double
 //    buffered; one barrier per k-tile of 16.  Half of the waves stage A, the others B.
 //  * a K-major operand is transposed on the way: a thread loads 4 k x 4 rows and stores 4 rows x 4 k; rows are stored at
@@ -56,6 +57,13 @@ template <int BM, int BN, int WM, int WN> struct F32Tile {
     static_assert(BM == BN && BM == THREADS / 2, "half of the threads stage 16 elements each of either operand");
 };
 
+// The largest magnitude met (a NaN does not count).
+__device__ __forceinline__ void max_magnitude(float &top, float a, float b) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    asm("v_max3_f32 %0, %0, abs(%1), abs(%2)" : "+v"(top) : "v"(a), "v"(b));
+#endif
+}
+
 // Two values, rounded to bf16 and packed in order; and the values of such a pair.
 __device__ __forceinline__ unsigned bf16_pair(float a, float b) {
     typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
@@ -69,8 +77,10 @@ __device__ __forceinline__ float pair_second(unsigned p) { return __builtin_bit_
 struct F32Planes {
     float r[4];
     u32x2 hi, mid, lo;
-    __device__ __forceinline__ void cut(const f32x4 v) {
+    __device__ __forceinline__ void cut(const f32x4 v, float &top) {
         const float x[4] = {v[0] * kF32Scale, v[1] * kF32Scale, v[2] * kF32Scale, v[3] * kF32Scale};
+        max_magnitude(top, x[0], x[1]);
+        max_magnitude(top, x[2], x[3]);
         split(x, hi);
     }
     __device__ __forceinline__ void pack() {
@@ -134,9 +144,9 @@ template <int BM> struct F32Stager {
     }
     // piece i of a thread into the three planes of a stage's operand, [row tile of 32][plane][lane: k half, row][8 k], in three
     // parts that the main loop deals out among its MFMAs
-    template <bool KM> __device__ __forceinline__ void store(int part, int i, unsigned char *op, const f32x4 (&v)[4], F32Planes &w) const {
+    template <bool KM> __device__ __forceinline__ void store(int part, int i, unsigned char *op, const f32x4 (&v)[4], F32Planes &w, float &top) const {
         if (part == 0) {
-            w.cut(KM ? f32x4{v[0][i], v[1][i], v[2][i], v[3][i]} : v[i]);
+            w.cut(KM ? f32x4{v[0][i], v[1][i], v[2][i], v[3][i]} : v[i], top);
         } else if (part == 1) {
             w.pack();
         } else {
@@ -190,6 +200,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_kernel(const GemmF32
     const bool sums = A_KM && g.db_part && nt == 0 && stages_a;
     f32x4 dsum = {0.f, 0.f, 0.f, 0.f}, dsum16 = {0.f, 0.f, 0.f, 0.f};   // (of the last up to 16 k-tiles, of those before)
 
+    float top = 0.f;
     f32x16 acc[TA][TB], acc2[TWO ? TA : 1][TWO ? TB : 1];
     auto clear = [&](auto &c) {
 #pragma unroll
@@ -245,14 +256,14 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_kernel(const GemmF32
                     c = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[b][pb[P0 + i]], fa[a & 1][pa[P0 + i]], c, 0, 0, 0);
                 }
                 if constexpr (NEXT)
-                    for (; step < 12 && slot_of(step) == sl; ++step) st.template store<KM>(step % 3, step / 3, op, v, w);
+                    for (; step < 12 && slot_of(step) == sl; ++step) st.template store<KM>(step % 3, step / 3, op, v, w, top);
                 __builtin_amdgcn_sched_barrier(0);
             }
         };
         st.template load<KM>(kb, v);
         sum(0);
 #pragma unroll
-        for (int i = 0; i < 12; ++i) st.template store<KM>(i % 3, i / 3, smem + (stages_a ? 0 : F::A_BYTES), v, w);
+        for (int i = 0; i < 12; ++i) st.template store<KM>(i % 3, i / 3, smem + (stages_a ? 0 : F::A_BYTES), v, w, top);
         if (nkt > 1) st.template load<KM>(kb + kF32BK, v);
         lds_barrier();
         for (int kt = 0; kt + 1 < nkt; ++kt) {
@@ -273,36 +284,28 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_kernel(const GemmF32
 
     // lane: row m = lane % 32 of a tile, columns 8 (i / 4) + 4 (lane / 32) + i % 4
     const int ml = lane & 31, q = lane >> 5;
-    float zero = 0.f;   // (not if one of the sums is infinite or no number)
+    // 32 x 32 results (a, b) of this wave on the fp32 MFMA, 16 k under way at a time
+    auto in_fp32 = [&](int a, int b) {
+        const int m = min((wm * TA + a) * 32 + ml, p.M - m0 - 1), n = min((wn * TB + b) * 32 + ml, p.N - n0 - 1);
+        f32x16 c;
 #pragma unroll
-    for (auto &row : acc)
+        for (int i = 0; i < 16; ++i) c[i] = 0.f;
+        for (int k0 = kb; k0 < ke; k0 += 16) {
+            float ea[8], eb[8];
 #pragma unroll
-        for (auto &t : row)
-#pragma unroll
-            for (int i = 0; i < 16; ++i) zero = __builtin_fmaf(t[i], 0.f, zero);
-    float unscale = kF32Unscale;
-    if (__syncthreads_or(zero != 0.f)) {   // (see above)
-        unscale = 1.f;
-        clear(acc);
-        for (int k = kb; k < ke; k += 2) {
-            const bool in = k + q < ke;
-            float ea[TA], eb[TB];
-#pragma unroll
-            for (int a = 0; a < TA; ++a) {
-                const int m = min((wm * TA + a) * 32 + ml, p.M - m0 - 1);
-                ea[a] = in ? (A_KM ? A[(size_t)(k + q) * p.lda + m] : A[(size_t)m * p.lda + k + q]) : 0.f;
+            for (int i = 0; i < 8; ++i) {
+                const int k = min(k0 + 2 * i + q, ke - 1);
+                ea[i] = A_KM ? A[(size_t)k * p.lda + m] : A[(size_t)m * p.lda + k];
+                eb[i] = B_KM ? B[(size_t)k * p.ldb + n] : B[(size_t)n * p.ldb + k];
             }
 #pragma unroll
-            for (int b = 0; b < TB; ++b) {
-                const int n = min((wn * TB + b) * 32 + ml, p.N - n0 - 1);
-                eb[b] = in ? (B_KM ? B[(size_t)(k + q) * p.ldb + n] : B[(size_t)n * p.ldb + k + q]) : 0.f;
+            for (int i = 0; i < 8; ++i) {
+                const bool in = k0 + 2 * i + q < ke;
+                c = __builtin_amdgcn_mfma_f32_32x32x2f32(in ? eb[i] : 0.f, in ? ea[i] : 0.f, c, 0, 0, 0);
             }
-#pragma unroll
-            for (int a = 0; a < TA; ++a)
-#pragma unroll
-                for (int b = 0; b < TB; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_32x32x2f32(eb[b], ea[a], acc[a][b], 0, 0, 0);
         }
-    }
+        return c;
+    };
     if (A_KM && g.db_part && nt == 0) {   // the threads of a column: k (th / (BM / 4)) * 4 .. + 3 of every k-tile each
         float *red = reinterpret_cast<float *>(smem);
         if (stages_a) *reinterpret_cast<f32x4 *>(red + st.th / (BM / 4) * BM + st.th % (BM / 4) * 4) = dsum + dsum16;
@@ -327,15 +330,30 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_f32_kernel(const GemmF32
 #pragma unroll
         for (int e = 0; e < 4; ++e)
             if (n + e < p.N) bias[e] = bias0[n + e] + (bias1 ? bias1[n + e] : 0.f);
-    __syncthreads();   // the last k-tile (and the sums of A) are read
+    // (the last k-tile and the sums of A are read)  Products of scaled operands below 2^64 cannot overflow: a sum that is no number has a NaN among
+    // its operands then, and stays one.
+    const bool large = __syncthreads_or(top >= 0x1p64f);
 #pragma unroll
     for (int a = 0; a < TA; ++a) {
 #pragma unroll
-        for (int b = 0; b < TB; ++b)
+        for (int b = 0; b < TB; ++b) {
+            f32x16 c = acc[a][b];
+            float zero = 0.f, most = 0.f;   // (zero: not if one of the sums is infinite or no number)
+#pragma unroll
+            for (int i = 0; i < 16; ++i) zero = __builtin_fmaf(c[i], 0.f, zero);
+#pragma unroll
+            for (int i = 0; i < 16; i += 2) max_magnitude(most, c[i], c[i + 1]);
+            if (__ballot(most == __builtin_inff() || (large && zero != 0.f))) {   // (see above: those sums are taken from there, the others stay as they are)
+                const f32x16 other = in_fp32(a, b);
+#pragma unroll
+                for (int i = 0; i < 16; ++i) c[i] = c[i] * 0.f == 0.f ? c[i] * kF32Unscale : other[i];
+            } else {
+                c *= kF32Unscale;
+            }
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-                *reinterpret_cast<f32x4 *>(mine + ml * CROW + (b * 32 + 8 * i + 4 * q) * 4) =
-                    f32x4{acc[a][b][4 * i], acc[a][b][4 * i + 1], acc[a][b][4 * i + 2], acc[a][b][4 * i + 3]} * unscale;
+                *reinterpret_cast<f32x4 *>(mine + ml * CROW + (b * 32 + 8 * i + 4 * q) * 4) = f32x4{c[4 * i], c[4 * i + 1], c[4 * i + 2], c[4 * i + 3]};
+        }
         __builtin_amdgcn_wave_barrier();   // (a wave's LDS accesses are done in order)
 #pragma unroll
         for (int k = 0; k < 32 / RPI; ++k) {

@@ -123,3 +123,22 @@ def test_thin_gradients_of_many_rows(R, I, H):
     for got, want in ((dWx, D.t() @ x[0].double()), (dWh, D.t() @ h[0].double()), (db, D.sum(0))):
         # parts of at most some 200 rows: 2e-7 for the sum of one (its 13 roundings of up to 6e-8 each by their square root), as much for the sum of them
         assert float((got.double() - want).norm()) <= 4e-7 * float(want.norm())
+
+
+def test_sums_beside_those_that_are_not_finite_keep_their_bits():
+    def planted(v):
+        def plant(x, Wx, d):
+            if v is not None:
+                x[0, 7, 3], d[0, 9, 11] = v, v
+        return products(300, 40, 130, seed=3, plant=plant)[0]
+    clean = planted(None)
+    for v in (float("nan"), float("inf"), 3e38, 1e20):
+        for i, (a, b) in enumerate(zip(clean, planted(v))):
+            if i < 2:     # x.Wx^T and d.Wx: one row of results has it in its sum, the weight gradients one row or column
+                row = 7 if i == 0 else 9
+                keep = torch.arange(a.shape[0], device="cuda") != row
+                assert torch.equal(a[keep], b[keep]), (v, i)
+            elif i < 4:
+                keep = torch.arange(a.shape[0], device="cuda") != 11
+                cols = torch.arange(a.shape[1], device="cuda") != (3 if i == 2 else -1)
+                assert torch.equal(a[keep][:, cols], b[keep][:, cols]), (v, i)
