@@ -677,6 +677,18 @@ template <typename P> static int big_half_params(P &p, unsigned char *wsb, size_
     return nt;
 }
 
+// 16-bit, plans of streamed weights up to H = 4096: the whole-CU kernels with 16 units per workgroup.
+static bool fwd_resident(const fastlstm_plan &pl, const StreamLayout &l, int H, int dtype) {
+    return dtype != FASTLSTM_FP32 && pl.ht == 16 && H % 16 == 0 && l.KSP >= 80 && l.KSP <= 128 && (g_families.load() & 2);
+}
+static int resident_teams_grid(int H) { return kNumXcd * cdiv(H / (16 * kBigTeam), kNumXcd) * kBigTeam; }
+static bool bwd_resident(const fastlstm_plan &pl, const StreamLayout &l, int H, int dtype) {
+    DeviceInfo di;
+    const int kw = cdiv(l.KS, 64) * 4;
+    return dtype != FASTLSTM_FP32 && pl.ht == 16 && pl.n_btiles == 1 && H % (16 * kBigTeam) == 0 && kw >= 20 && kw <= 32 && (g_families.load() & 2) &&
+           device_info(-1, &di) == FASTLSTM_OK && di.xcd_round_robin == 1 && di.num_cus >= kNumXcd * 32 && resident_teams_grid(H) <= kNumXcd * 32;
+}
+
 // Returns 1 when the kernel does not apply, else a fastlstm_status.
 // `second` (+ o.more): independent recurrences of the same shape side by side in the launch, as try_fwd_xcd takes them.
 int try_fwd_wide(void *ifgo, void *out, void *cell, const void *Wh, unsigned char *wsb, size_t ws_bytes, int T, int B,
@@ -1340,7 +1352,7 @@ static int fwd_persistent_impl(void *ifgo, void *out, void *cell, const void *Wh
             if (occ >= 1) return FASTLSTM_OK;
         }
         // 16-bit up to H = 4096: the slice of 16 units of a workgroup stays on its CU for the whole launch
-        bool resident = dtype != FASTLSTM_FP32 && pl.ht == 16 && H % 16 == 0 && l.KSP >= 80 && l.KSP <= 128 && (g_families.load() & 2);
+        bool resident = fwd_resident(pl, l, H, dtype);
         if (resident) {
             int occ = 0;
             if (launch_fwd_big(dtype, p, l.KSP / 4, 4, pl.bt / 16, 0, nullptr, &occ) != hipSuccess) return FASTLSTM_ERR_HIP;
@@ -1525,11 +1537,8 @@ static int bwd_persistent_impl(const void *dout, void *dh, void *dc, const void 
         }
         // 16-bit up to H = 4096: teams of 4 workgroups keep the slices of 64 units on their CUs for the whole launch; the
         // place of the packed weights holds the team's partial sums
-        DeviceInfo di;
-        const int teams = H / (16 * kBigTeam), grid_big = kNumXcd * cdiv(teams, kNumXcd) * kBigTeam, kw = cdiv(l.KS, 64) * 4;
-        bool resident = dtype != FASTLSTM_FP32 && pl.ht == 16 && pl.n_btiles == 1 && H % (16 * kBigTeam) == 0 && kw >= 20 && kw <= 32 && (g_families.load() & 2) &&
-                        device_info(-1, &di) == FASTLSTM_OK && di.xcd_round_robin == 1 && di.num_cus >= kNumXcd * 32 &&
-                        grid_big <= kNumXcd * 32;
+        const int grid_big = resident_teams_grid(H), kw = cdiv(l.KS, 64) * 4;
+        bool resident = bwd_resident(pl, l, H, dtype);
         if (resident) {
             p.Wh = Wh;
             p.n_rec = 1;
@@ -2306,8 +2315,32 @@ int fastlstm_recurrent_kernel_kind(int T, int B, int H, int dtype, int backward,
     XcdCfg c;
     if (select_xcd(T, B, H, dtype, backward != 0, ws_bytes, &c)) return 1;
     WideCfg w;
-    // (fp32 forward calls of up to 32 rows have always been kind 0 here, and callers choose sizes by that)
+    // (fp32 forward calls of up to 32 rows are kind 0 whatever runs them, see the header)
     if (select_wide(T, B, H, dtype, backward != 0, ws_bytes, &w)) return dtype == FASTLSTM_FP32 && !backward && B <= 32 ? 0 : 2;
+    if (xcd_rows_per_launch(T, B, H, dtype, backward != 0, ws_bytes)) return 1;
+    return wide_rows_per_launch(T, B, H, dtype, backward != 0, ws_bytes) ? 2 : 0;
+}
+
+int fastlstm_recurrent_form(int T, int B, int H, int dtype, int backward, size_t ws_bytes) {
+    if (!dtype_ok(dtype)) return FASTLSTM_ERR_DTYPE;
+    if (T <= 0) return FASTLSTM_ERR_DIM;
+    if (int rc = check_dims(T, B, H, H)) return rc;
+    fastlstm_plan pl;
+    if (int rc = plan_device(-1, B, H, dtype, backward, &pl, false)) return rc;
+    if (ws_bytes < pl.ws_bytes) return FASTLSTM_ERR_WORKSPACE;
+    if (cu_applies(B, H, dtype)) return 4;
+    if (pl.wave_split == 2) return 0;
+    if (pl.wave_split == 3) {
+        const StreamLayout l = stream_layout(pl, H, dtype, backward != 0);
+        BwdStreamParams p{};
+        unsigned char *fake = reinterpret_cast<unsigned char *>(static_cast<size_t>(4096));   // never dereferenced
+        if (big_half_applies(pl, H, dtype)) return big_half_params(p, fake, ws_bytes, std::min(B, kBigHalfRows), H, backward != 0) ? 2 : 3;
+        return (backward ? bwd_resident(pl, l, H, dtype) : fwd_resident(pl, l, H, dtype)) ? 2 : 3;
+    }
+    XcdCfg c;
+    WideCfg w;
+    if (select_xcd(T, B, H, dtype, backward != 0, ws_bytes, &c)) return 1;
+    if (select_wide(T, B, H, dtype, backward != 0, ws_bytes, &w)) return 2;
     if (xcd_rows_per_launch(T, B, H, dtype, backward != 0, ws_bytes)) return 1;
     return wide_rows_per_launch(T, B, H, dtype, backward != 0, ws_bytes) ? 2 : 0;
 }

@@ -1134,21 +1134,35 @@ def _recurrent_kind_cached(T, B, H, code, device_index, backward, families):
         return lib.fastlstm_recurrent_kernel_kind(T, B, H, code, b, lib.fastlstm_recurrent_workspace_bytes(plan, T, H, code, b))
 
 
+def _recurrent_form(T, B, H, code, device_index, backward=False):
+    """fastlstm_recurrent_form of the forward (reverse) call for the workspace this module allocates."""
+    return _recurrent_form_cached(T, B, H, code, device_index, backward, _families())
+
+
+@functools.lru_cache(maxsize=4096)
+def _recurrent_form_cached(T, B, H, code, device_index, backward, families):
+    lib = _lib.load()
+    device = torch.device("cuda", device_index)
+    with torch.cuda.device(device):
+        plan = _plan(device, B, H, code, backward)
+        b = int(backward)
+        return lib.fastlstm_recurrent_form(T, B, H, code, b, lib.fastlstm_recurrent_workspace_bytes(plan, T, H, code, b))
+
+
 def _padded_hidden_size(T, B, H, code, device_index, training=False):
     return _padded_hidden_size_cached(T, B, H, code, device_index, training, _families())
 
 
 @functools.lru_cache(maxsize=4096)
 def _padded_hidden_size_cached(T, B, H, code, device_index, training, families):
-    """The next hidden size above H (within a quarter, in steps of the MFMA k-step) that the XCD-local or the
-    register-resident kernels take, when H itself gets the general kernels; else 0.  `training`: a reverse pass
+    """The next hidden size above H (within a quarter, in steps of the MFMA k-step) that the XCD-local, the
+    register-resident or the one-CU kernels take, when H itself gets the general kernels; else 0.  `training`: a reverse pass
     follows, whose kernels count too."""
     fp32 = code == _DTYPE_CODE[torch.float32]
-    kind = lambda h: _recurrent_kind(T, B, h, code, device_index)
-    # a forward call of up to 32 fp32 rows is reported as general whatever runs it, so fp32 sizes go by the reverse pass,
-    # whose kernels take the same sizes (T = 256, B = 8, I = 256, H = 576 as it is / as 640: inference 1.21 / 0.96 ms,
-    # forward + backward 3.43 / 2.47; B = 32, H = 960 as 1024: 1.62 / 1.19, 5.00 / 3.36; T = 40, B = 1: 0.21 / 0.19)
-    fast = lambda h: kind(h) in (1, 2) or (fp32 and _recurrent_kind(T, B, h, code, device_index, True) in (1, 2))
+    form = lambda h: _recurrent_form(T, B, h, code, device_index)
+    # (fp32, T = 256, B = 8, I = 256, H = 576 as it is / as 640: inference 1.21 / 0.96 ms, forward + backward 3.43 / 2.47; B = 32, H = 960
+    # as 1024: 1.62 / 1.19, 5.00 / 3.36; T = 40, B = 1: 0.21 / 0.19)
+    fast = lambda h: form(h) in (1, 2, 4) or (fp32 and _recurrent_form(T, B, h, code, device_index, True) in (1, 2, 4))
     # The launches that pad and cut cost ~0.1 ms forward and ~0.2 ms forward + backward whatever the shape: a few steps
     # repay them only with many rows and units (T = 16, B = 128, H = 1150 bf16 forward + backward 0.82 ms as it is,
     # 0.59 ms as 1280; B = 64, H = 650 0.48 against 0.68).
@@ -1162,8 +1176,9 @@ def _padded_hidden_size_cached(T, B, H, code, device_index, training, families):
     # or the streamed kernels (T = 100, I = 512, inference / training as it is and padded: H = 1030, B = 1 0.79 / 2.16 and 0.56 / 1.31 ms,
     # B = 256 6.17 / 22.1 and 4.41 / 11.5; H = 1900, B = 16 1.66 / 4.68 and 0.73 / 1.95; T = 32, B = 1, H = 1100 0.32 / 0.84 and
     # 0.26 / 0.54; T = 16, B = 128 0.65 / 1.93 and 0.45 / 1.15)
-    if fp32 and families & 2 and 1024 < H < 2048:
-        return -(-H // 256) * 256 if H % 256 else 0
+    if fp32 and 1024 < H < 2048:
+        up = -(-H // 256) * 256
+        return up if up != H and form(up) == 2 else 0
     if H <= 64:
         # The general kernels' one-tile form (no exchange between workgroups at all).  In 16 bits it is the fastest
         # there is at H = 64 (T = 1024, B = 256, I = H = 64 forward + backward 0.93 ms as it is, 3.4 ms as H = 96):
@@ -1180,7 +1195,9 @@ def _padded_hidden_size_cached(T, B, H, code, device_index, training, families):
         if fp32 and H <= 32 and T < 96:
             return 0
         return 64
-    if kind(H) != 0 or fast(H):
+    # (the one-CU kernels take 16-bit multiples of 16, as they are / padded to 32: T = 256, B = 64, H = 80 inference 0.163 / 0.179, training
+    # 0.365 / 0.450 ms; H = 144 0.240 / 0.251, 0.534 / 0.567; T = 40, B = 8, H = 112 0.058 / 0.100, 0.287 / 0.403)
+    if form(H) != 0 or fast(H):
         return 0
     step = 16 if fp32 else 32
     for Hp in range((H // step + 1) * step, H + H // 4 + step + 1, step):

@@ -348,8 +348,16 @@ size_t fastlstm_stack2_bwd_workspace_bytes(const fastlstm_plan *plan, int T, int
 size_t fastlstm_stack2_bwd_wgrad_workspace_bytes(int T, int B, int I, int H, int dtype);
 int fastlstm_bwd_stack2_fused(int T, int B, int I, int H, int dtype, size_t ws_bytes);
 
-/* Which kernel fastlstm_fwd_persistent (backward = 0) / fastlstm_bwd_persistent (1) will launch on
- * the current device for this shape and a workspace of ws_bytes: 0 = the general kernel
+/* Which kernel fastlstm_fwd_persistent (backward = 0) / fastlstm_bwd_persistent (1) will launch on the current device for this
+ * shape and a workspace of ws_bytes: 0 = the general kernel, 1 = the XCD-local kernel, 2 = a register-resident kernel (all of W_h on
+ * the chip, barrier groups over several XCDs: multiples of 256 up to H = 2048 and, in 16 bits, of 64 up to 4096; fp32 640, 768, 896
+ * too), 3 = the streamed-weights kernel, 4 = the one-CU kernel (a workgroup holds all of W_h and takes four rows: 16-bit H = 80 ...
+ * 160, fp32 64 ... 96, up to 4 rows per CU).  Negative: fastlstm_status.  No counterpart in the reference. */
+int fastlstm_recurrent_form(int T, int B, int H, int dtype, int backward, size_t ws_bytes);
+
+/* The kernel family of this shape among those that exchange between CUs, as callers know it from before some of today's kernels --
+ * fastlstm_recurrent_form says which kernel runs: sizes of the one-CU kernel are 0 or 1 here, hidden sizes whose W_h is larger than
+ * 32 MiB 3 though it may stay on the chip, and fp32 forward calls of up to 32 rows 0 for H = 640 ... 1024.  0 = the general kernel
  * (exchange through device memory), 1 = the XCD-local kernel (barrier group on one XCD,
  * exchange through its L2; needs the workspace of fastlstm_recurrent_workspace_bytes and a
  * device that fastlstm_plan_device has probed; a batch with more tiles than one launch holds runs as

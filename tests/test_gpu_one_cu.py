@@ -94,3 +94,48 @@ def test_numbers_that_are_not_finite(weight):
         assert torch.equal(torch.isnan(a), torch.isnan(b)) and torch.equal(torch.isinf(a), torch.isinf(b))
         ok = torch.isfinite(b)
         assert bool(ok.any()) and not bool(ok.all()) and float((a - b)[ok].abs().max()) < 1e-4
+
+
+@pytest.mark.parametrize("H,dt", [(80, torch.float16), (112, torch.bfloat16), (144, torch.float16), (80, torch.float32)])
+def test_module_leaves_these_sizes_as_they_are(H, dt):
+    """... from 32 steps on too, where sizes between those of the fast kernels are padded: outputs and gradients against float64."""
+    T, B, I, code = 40, 9, 64, L._DTYPE_CODE[dt]
+    assert L._recurrent_form(T, B, H, code, 0) == L._recurrent_form(T, B, H, code, 0, True) == 4
+    assert L._padded_hidden_size(T, B, H, code, 0, True) == L._padded_hidden_size(T, B, H, code, 0, False) == 0
+    torch.manual_seed(H)
+    want = torch.nn.LSTM(I, H).double()
+    got = L.FastLSTM(I, H, device="cuda", dtype=dt)
+    got.load_state_dict(want.state_dict())   # (rounds)
+    want.load_state_dict(got.state_dict())
+    x, d = torch.randn(T, B, I).to(dt), torch.randn(T, B, H).to(dt)
+    xg, xw = x.cuda().requires_grad_(), x.double().requires_grad_()
+    y, (h, c) = got(xg)
+    y.backward(d.cuda())
+    yw, (hw, cw) = want(xw)
+    yw.backward(d.double())
+    tol = {torch.float32: 2e-6, torch.float16: 5e-3, torch.bfloat16: 4e-2}[dt]   # (every step's results are rounded to the type)
+    for i, (a, b) in enumerate([(y, yw), (h, hw), (c, cw), (xg.grad, xw.grad)] + [(p.grad, q.grad) for p, q in zip(got.parameters(), want.parameters())]):
+        a, b = a.detach().double().cpu(), b.detach()
+        assert a.shape == b.shape and float((a - b).norm()) <= tol * float(b.norm()), i
+
+
+def test_padding_goes_by_the_kernels_that_run():
+    pad = lambda T, B, H, code, training: L._padded_hidden_size(T, B, H, code, 0, training)
+    # 16 bits, more rows than the one-CU kernels hold: sizes that the XCD-local kernels do not take go to those they take
+    assert pad(64, 1025, 80, 1, True) == 96 and pad(64, 1024, 80, 1, True) == 0
+    # fp32 between 1024 and 2048: as the next size whose weights stay on the chip, if they do
+    lib = _lib.load()
+    assert pad(64, 5, 1100, 0, True) == 1280 and L._recurrent_form(64, 5, 1280, 0, 0) == 2
+    lib.fastlstm_set_kernel_families(5)
+    try:
+        assert pad(64, 5, 1100, 0, True) == 0 and L._recurrent_form(64, 5, 1280, 0, 0) == 3
+    finally:
+        lib.fastlstm_set_kernel_families(7)
+
+
+def test_form_of_the_kernel_that_runs():
+    form = lambda B, H, code, backward=False: L._recurrent_form(5, B, H, code, 0, backward)
+    assert form(4, 64, 1) == 0 and form(4, 64, 0) == 4 and form(16, 1024, 0) == 2 and form(16, 1024, 1) == 1
+    assert form(16, 576, 0) == 0 and form(16, 2560, 1) == form(16, 2560, 1, True) == 2 and form(16, 2500, 1) == 3 and form(16, 1536, 0, True) == 2
+    assert form(1025, 96, 0) == 1 and form(1024, 96, 0) == 4 and form(700, 1024, 1) == 1
+    assert _lib.load().fastlstm_recurrent_form(5, 16, 1024, 1, 0, 16) == _lib.ERR_WORKSPACE
