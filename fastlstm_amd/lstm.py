@@ -1192,7 +1192,9 @@ def _padded_hidden_size_cached(T, B, H, code, device_index, training, families):
         # 0.112 / 0.367, T = 1024 0.486 / 2.66 and 0.556 / 1.27.
         if H == 64 or (H <= 16 and not training):
             return 0
-        if fp32 and H <= 32 and T < 96:
+        # Batches that the one-CU kernels do not hold run the one-tile form at 64 units too (T = 256, inference / training, H = 32 as it is and
+        # as 64: B = 1100 0.36 / 2.22 and 0.53 / 1.61 ms, 2000 0.45 / 3.05 and 0.64 / 2.06).
+        if fp32 and H <= 32 and (T < 96 or (not training and form(64) != 4)):
             return 0
         return 64
     # (the one-CU kernels take 16-bit multiples of 16, as they are / padded to 32: T = 256, B = 64, H = 80 inference 0.163 / 0.179, training

@@ -123,6 +123,8 @@ def test_padding_goes_by_the_kernels_that_run():
     pad = lambda T, B, H, code, training: L._padded_hidden_size(T, B, H, code, 0, training)
     # 16 bits, more rows than the one-CU kernels hold: sizes that the XCD-local kernels do not take go to those they take
     assert pad(64, 1025, 80, 1, True) == 96 and pad(64, 1024, 80, 1, True) == 0
+    # fp32 up to 32 units: as 64 where the one-CU kernels hold the batch, and in training
+    assert [pad(128, B, 32, 0, training) for B, training in ((1024, False), (1025, False), (1024, True), (1025, True))] == [64, 0, 64, 64]
     # fp32 between 1024 and 2048: as the next size whose weights stay on the chip, if they do
     lib = _lib.load()
     assert pad(64, 5, 1100, 0, True) == 1280 and L._recurrent_form(64, 5, 1280, 0, 0) == 2
