@@ -1212,6 +1212,14 @@ def _padded_hidden_size_cached(T, B, H, code, device_index, training, families):
 def _operand_padding_cached(T, B, I, H, num_layers, bidirectional, whole_rows, code, idx, training, families):
     fp32 = code == _DTYPE_CODE[torch.float32]
     Hp = _padded_hidden_size(T, B, H, code, idx, training) or H
+    # Stacked 16-bit layers of the one-CU kernels read h as the K of their input projection: where the next size makes that a multiple of 64
+    # (see below) and this one does not, the copies pay from some rows on (as they are / padded, inference and training: 3 x (T = 256, B = 800,
+    # H = 112) 0.96 / 0.74, 2.19 / 2.00 ms; 2 x (256, 256, 112) 0.37 / 0.35, 0.88 / 0.87; 3 x (128, 32, 112) 0.29 / 0.28, 0.81 / 0.88; two
+    # directions, 2 x (128, 200, 80) 0.30 / 0.29, 0.91 / 1.00).
+    D, up = 2 if bidirectional else 1, -(-H // 32) * 32
+    if (Hp == H and num_layers > 1 and not fp32 and D * H % 64 and D * up % 64 == 0 and T * B >= (65536 if training else 4096)
+            and _recurrent_form(T, B, H, code, idx) == 4 == _recurrent_form(T, B, up, code, idx)):
+        Hp = up
     # Where H is padded anyway and stacked layers read it as the K of their input projection: a multiple of 64, which
     # the MFMA tile kernel takes (2 x (T = 256, B = 32): H = 704 forward + backward 2.19 ms, H = 672 2.32).  (Two
     # directions make K = 2H; below 512 the projection is too small to matter.)

@@ -141,3 +141,11 @@ def test_form_of_the_kernel_that_runs():
     assert form(16, 576, 0) == 0 and form(16, 2560, 1) == form(16, 2560, 1, True) == 2 and form(16, 2500, 1) == 3 and form(16, 1536, 0, True) == 2
     assert form(1025, 96, 0) == 1 and form(1024, 96, 0) == 4 and form(700, 1024, 1) == 1
     assert _lib.load().fastlstm_recurrent_form(5, 16, 1024, 1, 0, 16) == _lib.ERR_WORKSPACE
+
+
+def test_stacks_of_sizes_off_a_multiple_of_64():
+    """Many rows: padded where that makes the K of the upper layers' projections a multiple of 64."""
+    pad = lambda T, B, H, layers, two, training: L._operand_padding_cached(T, B, 128, H, layers, two, True, 1, 0, training, L._families())
+    assert pad(128, 32, 112, 3, False, False) == (128, 128) and pad(128, 32, 112, 3, False, True) is None and pad(256, 256, 112, 2, False, True) == (128, 128)
+    assert pad(128, 32, 80, 3, False, False) is None and pad(128, 32, 80, 2, True, False) == (96, 128) and pad(128, 32, 112, 1, False, False) is None
+    assert pad(128, 32, 128, 3, False, False) is None
