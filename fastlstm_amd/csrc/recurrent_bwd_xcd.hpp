@@ -448,6 +448,7 @@ __global__ __launch_bounds__(kWave * NWV) void lstm_bwd_xcd_kernel(const BwdXcdP
     }
 
     // ---- per-thread items: it = tid + NTHR*m -> (row n, unit ul, n-tile nt) ----------------
+    constexpr float GS = P > 1 ? kGradScale : 1.f, GU = P > 1 ? kGradUnscale : 1.f;   // (all gradients of the loop: recurrent_parts.hpp)
     float dc_state[IPT], dh_rec[IPT], c1v[IPT];
     size_t off_h[IPT];
     int xoff[IPT], roff[IPT], goff[IPT], soff[IPT];
@@ -467,8 +468,8 @@ __global__ __launch_bounds__(kWave * NWV) void lstm_bwd_xcd_kernel(const BwdXcdP
         roff[m] = ((a * NT + (nt < NT ? nt : 0)) * kWave + (ur >> 2) * 16 + n) * 4 + (ur & 3);
         goff[m] = ((nt < NT ? nt : 0) * 16 + n) * GROW + ul * E::BYTES;
         soff[m] = ((nt < NT ? nt : 0) * 16 + n) * SROW + ul * E::BYTES;
-        dh_rec[m] = valid[m] ? E::to_f32(dh_state[off_h[m]]) : 0.f;
-        dc_state[m] = valid[m] ? E::to_f32(dc_state_buf[off_h[m]]) : 0.f;
+        dh_rec[m] = valid[m] ? GS * E::to_f32(dh_state[off_h[m]]) : 0.f;
+        dc_state[m] = valid[m] ? GS * E::to_f32(dc_state_buf[off_h[m]]) : 0.f;
         c1v[m] = valid[m] ? E::to_f32(cell[(size_t)T_ * BH + off_h[m]]) : 0.f;
     }
 
@@ -648,7 +649,7 @@ __global__ __launch_bounds__(kWave * NWV) void lstm_bwd_xcd_kernel(const BwdXcdP
                 const float so = sigmoidf_<ACC>(E::to_f32(gl_[3 * HT]));
                 const float tc = tanhf_<ACC>(c1v[m]);
                 const float c0 = E::to_f32(*reinterpret_cast<const T *>(set + BT * GROW + soff[m]));
-                const float dh = dh_rec[m] + E::to_f32(*reinterpret_cast<const T *>(set + BT * GROW + BT * SROW + soff[m]));
+                const float dh = dh_rec[m] + GS * E::to_f32(*reinterpret_cast<const T *>(set + BT * GROW + BT * SROW + soff[m]));
                 const float dc1 = dc_state[m] + dh * so * (1.f - tc * tc);
                 const float d_o = dh * tc * so * (1.f - so);
                 const float d_f = dc1 * c0 * sf * (1.f - sf);
@@ -660,10 +661,11 @@ __global__ __launch_bounds__(kWave * NWV) void lstm_bwd_xcd_kernel(const BwdXcdP
                 st_d[1] = E::from_f32(d_f);
                 st_d[2] = E::from_f32(d_g);
                 st_d[3] = E::from_f32(d_o);
-                gl_[0] = st_d[0];
-                gl_[HT] = st_d[1];
-                gl_[2 * HT] = st_d[2];
-                gl_[3 * HT] = st_d[3];
+                auto stored = [](T d) { if constexpr (P > 1) return d * GU; else return d; };
+                gl_[0] = stored(st_d[0]);
+                gl_[HT] = stored(st_d[1]);
+                gl_[2 * HT] = stored(st_d[2]);
+                gl_[3 * HT] = stored(st_d[3]);
             } else {
 #pragma unroll
                 for (int gt = 0; gt < 4; ++gt) st_d[gt] = E::from_f32(0.f);
@@ -679,7 +681,7 @@ __global__ __launch_bounds__(kWave * NWV) void lstm_bwd_xcd_kernel(const BwdXcdP
                 other[1] = (unsigned)__shfl_down((int)mine[1], 16);
                 if (stores[m]) xch.store16(xgrp + xoff[m], u32x4{mine[0], mine[1], other[0], other[1]});
             } else {
-                const ThreeParts p0(st_d[0] * kGradScale), p1(st_d[1] * kGradScale), p2(st_d[2] * kGradScale), p3(st_d[3] * kGradScale);
+                const ThreeParts p0(st_d[0]), p1(st_d[1]), p2(st_d[2]), p3(st_d[3]);
                 if (stores[m])
 #pragma unroll
                     for (int i = 0; i < P; ++i)
@@ -774,7 +776,7 @@ __global__ __launch_bounds__(kWave * NWV) void lstm_bwd_xcd_kernel(const BwdXcdP
             float v = redf[roff[m]];
 #pragma unroll
             for (int pp = 1; pp < NWV; ++pp) v += redf[roff[m] + pp * MT * NT * kWave * 4];
-            dh_rec[m] = P > 1 ? v * kGradUnscale : v;
+            dh_rec[m] = v;
         }
         // the next step's first workgroup barrier orders these reads before the next writes to `red`
     }
@@ -790,8 +792,8 @@ __global__ __launch_bounds__(kWave * NWV) void lstm_bwd_xcd_kernel(const BwdXcdP
 #pragma unroll
     for (int m = 0; m < IPT; ++m)
         if (valid[m]) {
-            dh_state[off_h[m]] = E::from_f32(dh_rec[m]);
-            dc_state_buf[off_h[m]] = E::from_f32(dc_state[m]);
+            dh_state[off_h[m]] = E::from_f32(GU * dh_rec[m]);
+            dc_state_buf[off_h[m]] = E::from_f32(GU * dc_state[m]);
         }
     if constexpr (HELP != 0) {
         if (db_part) {   // sums over the 16 rows of a batch tile (16 neighbouring lanes), one lane writes the four gates

@@ -319,7 +319,8 @@ __global__ __launch_bounds__((CuShape<T, CW>::THREADS)) void lstm_bwd_cu_kernel(
     const bool valid = b0 + row < B;
     const size_t off = valid ? (size_t)(b0 + row) * H + unit : 0;
     const int goff = row * C::GROW + unit * E::BYTES, soff = row * C::SROW + unit * E::BYTES;
-    float dh_rec = valid ? E::to_f32(dh[off]) : 0.f, dc_state = valid ? E::to_f32(dc[off]) : 0.f;
+    constexpr float GS = C::F32 ? kGradScale : 1.f, GU = C::F32 ? kGradUnscale : 1.f;   // (all gradients of the loop: recurrent_parts.hpp)
+    float dh_rec = valid ? GS * E::to_f32(dh[off]) : 0.f, dc_state = valid ? GS * E::to_f32(dc[off]) : 0.f;
     float c1 = valid ? E::to_f32(cell[(size_t)T_ * B * H + off]) : 0.f;
     T nx[6];   // the gates, c_{t-1} and dout of the step, read a step ahead
     auto read_items = [&](const unsigned char *g) __attribute__((always_inline)) {
@@ -335,7 +336,7 @@ __global__ __launch_bounds__((CuShape<T, CW>::THREADS)) void lstm_bwd_cu_kernel(
         unsigned char *x = xl + (s & 1) * KS * kFragBytes, *g = tiles + (s & 1) * C::SET;
         const float si = sigmoidf_<C::F32>(E::to_f32(nx[0])), sf = sigmoidf_<C::F32>(E::to_f32(nx[1]));
         const float tg = tanhf_<C::F32>(E::to_f32(nx[2])), so = sigmoidf_<C::F32>(E::to_f32(nx[3]));
-        const float tc = tanhf_<C::F32>(c1), c0 = E::to_f32(nx[4]), dhv = dh_rec + E::to_f32(nx[5]);
+        const float tc = tanhf_<C::F32>(c1), c0 = E::to_f32(nx[4]), dhv = dh_rec + GS * E::to_f32(nx[5]);
         const float dc1 = dc_state + dhv * so * (1.f - tc * tc);
         const T d[4] = {E::from_f32(dc1 * tg * si * (1.f - si)), E::from_f32(dc1 * c0 * sf * (1.f - sf)), E::from_f32(dc1 * si * (1.f - tg * tg)),
                         E::from_f32(dhv * tc * so * (1.f - so))};
@@ -343,7 +344,7 @@ __global__ __launch_bounds__((CuShape<T, CW>::THREADS)) void lstm_bwd_cu_kernel(
         c1 = c0;   // c_{t-1} is the next step's c_t
         if (valid) {   // (rows past the batch stay zero in the operand blocks): k = 4 unit + gate
             if constexpr (C::F32) {
-                const ThreeParts p0(d[0] * kGradScale), p1(d[1] * kGradScale), p2(d[2] * kGradScale), p3(d[3] * kGradScale);
+                const ThreeParts p0(d[0]), p1(d[1]), p2(d[2]), p3(d[3]);
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
                     *reinterpret_cast<u32x2 *>(x + frag_offset<O>(4 * i + row, 4 * unit)) =
@@ -353,7 +354,10 @@ __global__ __launch_bounds__((CuShape<T, CW>::THREADS)) void lstm_bwd_cu_kernel(
             }
         }
 #pragma unroll
-        for (int i = 0; i < 4; ++i) reinterpret_cast<T *>(g + goff)[i * H] = d[i];
+        for (int i = 0; i < 4; ++i) {
+            if constexpr (C::F32) reinterpret_cast<T *>(g + goff)[i * H] = d[i] * GU;
+            else reinterpret_cast<T *>(g + goff)[i * H] = d[i];
+        }
         __syncthreads();
         // dh_rec(units of this wave, rows) = Wh[:, units]^T . d_ifgo[t](rows, :)^T over K = 4H, in independent sums
         constexpr int CH = P == 3 ? 3 : 2;
@@ -379,11 +383,11 @@ __global__ __launch_bounds__((CuShape<T, CW>::THREADS)) void lstm_bwd_cu_kernel(
 #pragma unroll
         for (int i = CH - 2; i >= 0; --i) sum += acc[i];
         const float s0 = sum[0], s1 = sum[1], s2 = sum[2], s3 = sum[3];
-        dh_rec = fold_cells<C::F32>(s0, s1, s2, s3) * (C::F32 ? kGradUnscale : 1.f);
+        dh_rec = fold_cells<C::F32>(s0, s1, s2, s3);
     }
     if (valid) {
-        dh[off] = E::from_f32(dh_rec);
-        dc[off] = E::from_f32(dc_state);
+        dh[off] = E::from_f32(GU * dh_rec);
+        dc[off] = E::from_f32(GU * dc_state);
     }
 }
 
