@@ -556,8 +556,9 @@ __global__ __launch_bounds__(kWave * NWV) void lstm_fwd_xcd_kernel(const FwdXcdP
     }
 
 #if defined(__HIP_DEVICE_COMPILE__)
-    // The loop starts 28 bytes behind a multiple of 32 (two instructions follow these): its step depends on where it lies against the
-    // 32 bytes of an instruction fetch.  T = 512, B = 64, I = H = 1024 fp16 inference at 28, 16, 24, 8, 0: 0.965, 0.978, 0.988, 1.003,
+    // The step depends on where the loop lies against the 32 bytes of an instruction fetch.  With these and what the compiler (clang 22 of ROCm
+    // 7.2) puts behind them it starts 28 bytes behind a multiple of 32, which nothing but a test enforces (tests/test_code_placement.py): after a
+    // change that moves it, measure again.  T = 512, B = 64, I = H = 1024 fp16 inference at 28, 16, 24, 8, 0: 0.965, 0.978, 0.988, 1.003,
     // 1.003 ms; the other residues lie between.
     if constexpr (HELP && NTW == 1) asm volatile(".p2align 6\n\t.rept 5\n\ts_nop 0\n\t.endr" ::: "memory");
 #endif
