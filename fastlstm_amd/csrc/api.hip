@@ -2352,6 +2352,7 @@ int fastlstm_recurrent_rows_per_launch(int T, int B, int H, int dtype, int backw
         fastlstm_plan pl;
         if (plan_device(-1, B, H, dtype, backward, &pl, false) == FASTLSTM_OK && pl.wave_split == 3) return 0;
     }
+    if (cu_applies(B, H, dtype)) return 0;
     XcdCfg c;
     WideCfg w;
     if (select_xcd(T, B, H, dtype, backward != 0, ws_bytes, &c) || select_wide(T, B, H, dtype, backward != 0, ws_bytes, &w)) return 0;

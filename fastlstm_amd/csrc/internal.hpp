@@ -60,15 +60,18 @@ hipError_t launch_small_k1(int dtype, const void *x, const void *Wx, const void 
     hipError_t launch_fwd_xcd_help_##SUF(const FwdXcdParams &p, int ntw, int grid, int lds, hipStream_t s, \
                                          int *max_blocks_per_cu);                                 \
     hipError_t launch_bwd_xcd_help_##SUF(const BwdXcdParams &p, int mt, int nkw, int ntw, int grid, int lds, \
-                                         hipStream_t s, int *max_blocks_per_cu);                  \
-    hipError_t launch_fwd_wide_##SUF(const FwdXcdParams &p, int nkw, int nt, int grid, int lds, hipStream_t s, \
-                                     int *max_blocks_per_cu);                                    \
-    hipError_t launch_bwd_wide_##SUF(const BwdXcdParams &p, int nkw, int nt, int grid, int lds, hipStream_t s, \
-                                     int *max_blocks_per_cu);
+                                         hipStream_t s, int *max_blocks_per_cu);
 FASTLSTM_DECL_REC(f32)
 FASTLSTM_DECL_REC(f16)
 FASTLSTM_DECL_REC(bf16)
 #undef FASTLSTM_DECL_REC
+// 16-bit kernels over several XCDs (recurrent_fwd_wide.hpp, recurrent_bwd_wide.hpp)
+#define FASTLSTM_DECL_WIDE(SUF)                                                                                             \
+    hipError_t launch_fwd_wide_##SUF(const FwdXcdParams &p, int nkw, int nt, int grid, int lds, hipStream_t s, int *max_blocks_per_cu); \
+    hipError_t launch_bwd_wide_##SUF(const BwdXcdParams &p, int nkw, int nt, int grid, int lds, hipStream_t s, int *max_blocks_per_cu);
+FASTLSTM_DECL_WIDE(f16)
+FASTLSTM_DECL_WIDE(bf16)
+#undef FASTLSTM_DECL_WIDE
 
 // streamed-weights kernels (recurrent_stream.hpp) and the kernels that keep up to 512 KiB of weights per CU
 // (recurrent_fwd_big.hpp, recurrent_bwd_big.hpp)

@@ -29,7 +29,7 @@ template <typename T, int NKW, int NT>
 __global__ __launch_bounds__(kWave * 8) void lstm_bwd_wide_kernel(const BwdXcdParams p) {
     using E = Elem<T>;
     constexpr bool ACC = false;                        // gates: the hardware's reciprocal
-    static_assert(E::BYTES == 2, "fp32: lstm_bwd_big_kernel");
+    static_assert(E::BYTES == 2, "fp32: lstm_bwd_big_parts_kernel");
     constexpr int NWV = 8, NTHR = kWave * NWV;
     constexpr int HT = 16, BT = 16 * NT;
     constexpr int IPT = (HT * BT + NTHR - 1) / NTHR;   // (unit, batch row) items per thread

@@ -35,7 +35,7 @@ template <typename T, int NKW, int NT>
 __global__ __launch_bounds__(kWave * 8) void lstm_fwd_wide_kernel(const FwdXcdParams p) {
     using E = Elem<T>;
     constexpr bool ACC = false;                              // gates: the hardware's reciprocal
-    static_assert(E::BYTES == 2, "fp32: lstm_fwd_big_kernel");
+    static_assert(E::BYTES == 2, "fp32: lstm_fwd_big_parts_kernel");
     constexpr int NWV = 8, NTHR = kWave * NWV;
     constexpr int MT = 4, TILES = MT * NT;                   // unit tiles, batch tiles of 16 rows
     constexpr int IPT = (TILES + NWV - 1) / NWV;             // (tile, lane) items per thread
