@@ -1233,7 +1233,7 @@ int fastlstm_gemm_wgrad(const void *d_ifgo, const void *x, const void *h, void *
 // (gemm_small.hpp), else the two stages one after the other.  dx may be null, and so may dWx, dWh, db (all three).
 static int gemm_dx_wgrad_impl(const void *d_ifgo, const void *Wx, const void *x, const void *h, void *dx, void *dWx,
                               void *dWh, void *db, void *ws, size_t ws_bytes, int T, int B, int I, int H, int dtype,
-                              void *stream) {
+                              void *stream, bool whole_dx = false) {
     const bool want_w = dWx != nullptr;
     if (!dx && !want_w) return FASTLSTM_OK;
     if (small_bwd_eligible(dtype, T * B, I, H) && (!want_w || ws_bytes >= small_bwd_workspace(T * B, I, H)))
@@ -1243,7 +1243,7 @@ static int gemm_dx_wgrad_impl(const void *d_ifgo, const void *Wx, const void *x,
                    : FASTLSTM_ERR_HIP;
     // (the weight-gradient workspace is free until the weight gradients start: scratch for a split along K)
     if (dx)
-        if (int rc = gemm_dx_impl(d_ifgo, Wx, dx, T, B, I, H, dtype, ws, ws_bytes, stream)) return rc;
+        if (int rc = gemm_dx_impl(d_ifgo, Wx, dx, T, B, I, H, dtype, whole_dx ? nullptr : ws, whole_dx ? 0 : ws_bytes, stream)) return rc;
     if (!want_w) return FASTLSTM_OK;
     return fastlstm_gemm_wgrad(d_ifgo, x, h, dWx, dWh, db, ws, ws_bytes, T, B, I, H, dtype, stream);
 }
@@ -2107,6 +2107,13 @@ int fastlstm_fwd_stack2_infer(const void *x, const void *Wx0, const void *bx0, c
 // bytes of the partial sums that a reverse launch leaves of a layer's bias gradient (BwdXcdParams::db_part)
 static size_t db_part_bytes(int B, int H) { return align_up((size_t)cdiv(B, 16) * 4 * H * sizeof(float), 256); }
 
+// A launch of two stacked layers of this shape may compute their dx inside (plan_bwd_helpers).
+static bool stack_may_have_dx_inside(int B, int H, int dtype) {
+    XcdCfg c;
+    return dtype != FASTLSTM_FP32 && xcd_shape(B, H, dtype, true, 1, &c) && ((c.mt == 2 && c.nkw == 16) || (c.mt == 1 && c.nkw == 8)) &&
+           2 * c.n_groups <= kNumXcd * c.gpx;
+}
+
 static int bwd_layer_impl(const void *dout, void *dh, void *dc, const void *ifgo, const void *cell, void *d_ifgo,
                           const void *Wh, const void *Wx, const void *x, const void *h, void *dx, void *dWx, void *dWh,
                           void *db, void *ws, size_t ws_bytes, void *wgrad_ws, size_t wgrad_ws_bytes, int T, int B, int I,
@@ -2155,8 +2162,9 @@ static int bwd_layer_impl(const void *dout, void *dh, void *dc, const void *ifgo
     if (rc != 3) {   // nothing was launched: recurrence, then dx
         if (int r2 = bwd_persistent_impl(dout, dh, dc, ifgo, cell, d_ifgo, Wh, ws, ws_bytes, T, B, H, dtype, stream))
             return r2;
+        // (dx has the bits of a stack's launch, where it is inside and one sum)
         return gemm_dx_wgrad_impl(d_ifgo, Wx, x, h, dx, want_w ? dWx : nullptr, dWh, db, wgrad_ws, wgrad_ws_bytes, T, B, I, H,
-                                  dtype, stream);
+                                  dtype, stream, stack_may_have_dx_inside(B, H, dtype));
     }
     if (!want_w) return FASTLSTM_OK;
     return fastlstm_gemm_wgrad(d_ifgo, x, h, dWx, dWh, db, wgrad_ws, wgrad_ws_bytes, T, B, I, H, dtype, stream);
