@@ -14,8 +14,8 @@
 //  4.1e-8; 1024 4.7e-7, 3.2e-7; 16384 1.9e-6, 1.2e-6.
 //  * what bounds it: the matrix units (16-bit products at 1.65 PFLOP/s are what they reach on random data; that is 275 here) and, next
 //    to them, the LDS (half of its cycles) and the conversions, which lie among the MFMAs, three vector instructions to each (behind
-//    them instead: 205).  TFLOP/s of fp32, on the fp32 MFMA and here: M = 8192, N = 8192, K = 2048 x.Wx^T 136 -> 213, d.Wx 136 -> 231, weight
-//    gradients 133 -> 235; M = 16384, I = H = 1024 weight gradients 131 -> 229; M = 8192, I = 512, H = 1024 97 -> 195.
+//    them instead: 205).  TFLOP/s of fp32, on the fp32 MFMA and here: M = 8192, N = 8192, K = 2048 x.Wx^T 136 -> 235, d.Wx 136 -> 234, weight
+//    gradients 133 -> 235; M = 16384, I = H = 1024 weight gradients 131 -> 229; M = 8192, I = 512, H = 1024 97 -> 205.
 //  * small numbers: the operands are taken times 2^24, which makes the last bit of the least fp32 number a normal bf16 number, and the
 //    sums times 2^-48.  (Without that the parts of numbers below 2^-110 lose bits: of an operand of 1e-36 the products were off by 6e-5, of
 //    1e-38 by 1e-2.)  A sum beyond 2^80, or one with an operand beyond 2^104, is dealt with as an infinity:
