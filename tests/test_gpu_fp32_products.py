@@ -36,9 +36,9 @@ def products(R, I, H, seed=0, plant=None):
 def test_products_at_the_edges(R, I, H):
     got, want, magnitude = products(R, I, H, seed=R + I + H)
     for a, b, m, terms in zip(got, want, magnitude, (I + 2, 4 * H, R, R, R)):
-        # six roundings of the running sum per 16 terms, the products left out (2^-22 of a term) and one of the result; the sums
+        # six roundings of the running sum per 16 terms, the products left out (together 2^-24 of a term) and one of the result; the sums
         # of magnitudes bound the running sums
-        bound = m * ((3 + 6 * terms / 16) * 2.0 ** -24 + 2.0 ** -22)
+        bound = m * ((3 + 6 * terms / 16) * 2.0 ** -24 + 2.0 ** -24)
         assert bool(((a.double() - b).abs() <= bound).all())
 
 
