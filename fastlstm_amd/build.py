@@ -16,7 +16,9 @@ CSRC = os.path.join(HERE, "csrc")
 LIBDIR = os.path.join(HERE, "lib")
 OBJDIR = os.path.join(HERE, "lib", "obj")
 LIB = os.path.join(LIBDIR, "libfastlstm_hip.so")
-SOURCES = ["recurrent_big_bwd_f32.hip", "recurrent_big_fwd_f32.hip", "recurrent_big.hip", "api.hip", "gemm.hip", "gemm_small.hip", "gemm_f32.hip", "diag.hip", "recurrent_stream.hip", "recurrent_step.hip", "recurrent_cu.hip", "copy_blocks.hip", "plan.cpp", "recurrent_f32.hip", "recurrent_f16.hip", "recurrent_bf16.hip",
+SOURCES = ["recurrent_big_fwd_f32.hip", "recurrent_big_fwd_f16.hip", "recurrent_big_fwd_bf16.hip",
+           "recurrent_big_bwd_f32.hip", "recurrent_big_bwd_f16.hip", "recurrent_big_bwd_bf16.hip", "recurrent_big.hip",
+           "api.hip", "gemm.hip", "gemm_small.hip", "gemm_f32.hip", "diag.hip", "recurrent_stream.hip", "recurrent_step.hip", "recurrent_cu.hip", "copy_blocks.hip", "plan.cpp", "recurrent_f32.hip", "recurrent_f16.hip", "recurrent_bf16.hip",
            "recurrent_wreg_f32.hip", "recurrent_wreg_f16.hip", "recurrent_wreg_bf16.hip",
            "recurrent_xcd_f32.hip", "recurrent_xcd_f16.hip", "recurrent_xcd_bf16.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

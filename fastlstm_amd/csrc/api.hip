@@ -584,7 +584,7 @@ bool select_wide(int T, int B_all, int H, int dtype, bool backward, size_t ws_by
         const size_t xslot = (size_t)groups * nt * c->ks * 3 * kFragBytes;
         const size_t partials = backward ? (size_t)groups * n_ht * kBigTeam * nt * kFragBytes : 0;
         if (copies > kMaxSideBySide || copies * groups > std::min(max_groups, kNumXcd) ||
-            ws_bytes < kWsHeaderBytes + kWsCounterBytes + copies * (2 * xslot + partials))
+            ws_bytes < kWsHeaderBytes + kWsCounterBytes + copies * ((backward ? 2 : big_fwd_slots(H / 128, 4, nt, 3)) * xslot + partials))
             return false;
         c->big = nt;
         c->n_ht = n_ht;
@@ -603,14 +603,14 @@ bool select_wide(int T, int B_all, int H, int dtype, bool backward, size_t ws_by
         // pass gains at every batch size (us per step, 16 units / 32: H = 2048, B = 32 6.4 / 5.3, 64 9.0 / 6.2, 128
         // 11.0 / 8.6; H = 1280, B = 128 8.7 / 7.0): groups of 16 rows where the batch fits the launch that way, else of 32.
         // The forward pass gains with groups of 16 rows where the 16-unit form needs more (H = 2048, B = 64 4.57 / 4.39, H = 1280
-        // 3.99 / 3.31); with 32 rows there is no difference (H = 2048, B = 128 7.1 / 7.3), and where 16-row groups of
-        // 16-unit workgroups fit, their half as many products per CU count for more (H = 2048, B = 32 3.4 / 3.8).
+        // 3.99 / 3.31) and with groups of 32 rows (B = 128, H = 2048 7.3 / 6.2, 1792 6.3 / 5.6, 1536 6.2 / 5.0, 1280 5.4 / 4.7); where 16-row
+        // groups of 16-unit workgroups fit, their half as many products per CU count for more (H = 2048, B = 32 3.4 / 3.8).
         const int n_ht = H / 32, max_groups = kNumXcd * 32 / n_ht;
         const int nt = copies * cdiv(B, 16) <= max_groups ? 1 : 2, groups = cdiv(B, 16 * nt);
-        const bool faster = backward || (nt == 1 && cdiv(B, 16) * cdiv(H / 16, 32) > kNumXcd);
+        const bool faster = backward || nt == 2 || cdiv(B, 16) * cdiv(H / 16, 32) > kNumXcd;
         const size_t xslot = (size_t)groups * nt * c->ks * kFragBytes;
         const size_t partials = backward ? (size_t)groups * n_ht * kBigTeam * 2 * nt * kFragBytes : 0;
-        if (faster && copies * groups <= max_groups && ws_bytes >= kWsHeaderBytes + kWsCounterBytes + copies * (2 * xslot + partials)) {
+        if (faster && copies * groups <= max_groups && ws_bytes >= kWsHeaderBytes + kWsCounterBytes + copies * ((backward ? 2 : big_fwd_slots(H / 128, 8, nt, 1)) * xslot + partials)) {
             c->big = nt;
             c->n_ht = n_ht;
             c->n_groups = groups;
@@ -642,7 +642,7 @@ bool select_wide(int T, int B_all, int H, int dtype, bool backward, size_t ws_by
 static int wide_rows_per_launch(int T, int B, int H, int dtype, bool backward, size_t ws_bytes) {
     const int xpg = cdiv(H / 16, 32);
     const int rows = dtype == FASTLSTM_FP32 ? 32 * std::min(kNumXcd, kNumXcd * 32 / std::max(1, H / 16))   // (two batch tiles per group)
-                     : backward && H >= 32 && (g_families.load() & 4)
+                     : H >= 32 && (g_families.load() & 4)
                          ? 32 * (kNumXcd * 32 / (H / 32))   // (groups of the 32-unit form)
                          : 64 * (kNumXcd / std::max(1, xpg));
     if (rows >= B || rows <= 0) return 0;
@@ -665,7 +665,7 @@ static int big_half_tiles(int rows) { return rows <= 16 ? 1 : rows <= 32 ? 2 : 4
 // Sets what both directions share; returns batch tiles, 0 if the workspace behind the counters does not hold the exchange.
 template <typename P> static int big_half_params(P &p, unsigned char *wsb, size_t ws_bytes, int rows, int H, bool backward) {
     const int nt = big_half_tiles(rows), ks = (backward ? 4 * H : H) / 32;
-    const size_t xchg = 2 * (size_t)nt * ks * 3 * kFragBytes;
+    const size_t xchg = (backward ? 2 : big_fwd_slots(H / 128, 2, nt, 3)) * (size_t)nt * ks * 3 * kFragBytes;
     const size_t partials = backward ? (size_t)(H / 8) * kBigTeamHalf * nt * kFragBytes : 0;
     if (ws_bytes < kWsHeaderBytes + kWsCounterBytes + xchg + partials) return 0;
     p.hdr = reinterpret_cast<WsHeader *>(wsb);
@@ -1356,7 +1356,7 @@ static int fwd_persistent_impl(void *ifgo, void *out, void *cell, const void *Wh
         if (resident) {
             int occ = 0;
             if (launch_fwd_big(dtype, p, l.KSP / 4, 4, pl.bt / 16, 0, nullptr, &occ) != hipSuccess) return FASTLSTM_ERR_HIP;
-            resident = (long long)occ * pl.num_cus >= (long long)pl.n_btiles * pl.n_htiles;
+            resident = (long long)occ * pl.num_cus >= (long long)pl.n_btiles * pl.n_htiles && l.wpack_bytes >= kXchgSlots * l.slot_bytes;
         }
         if (!resident && launch_pack_wh(dtype, false, Wh, wsb + l.wpack_off, H, l.KS, l.KSP, l.mt, pl.n_htiles, s) != hipSuccess)
             return FASTLSTM_ERR_HIP;
@@ -1370,6 +1370,7 @@ static int fwd_persistent_impl(void *ifgo, void *out, void *cell, const void *Wh
             const int grid = n_bt * pl.n_htiles;
             int occ = 0;
             if (resident) {
+                p.xbuf = wsb + l.wpack_off;   // (the place of the packed weights: kXchgSlots slots)
                 if (launch_fwd_big(dtype, p, l.KSP / 4, 4, pl.bt / 16, grid, s, nullptr) != hipSuccess) return FASTLSTM_ERR_HIP;
                 continue;
             }

@@ -145,6 +145,40 @@ __device__ __forceinline__ void wait_versions(const int *flags, int n, int targe
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");  // compiler ordering only: the data is read at device scope
 }
 
+// What an exchange word holds that has not been written: no stored value has this bit pattern (written_word).
+constexpr unsigned kUnwritten = 0xffffffffu;
+// The word as it is stored: all ones, which only NaNs can be (two 16-bit ones, or a 32-bit one), becomes another NaN.
+__device__ __forceinline__ unsigned written_word(unsigned w) { return w < kUnwritten - 1 ? w : kUnwritten - 1; }
+
+// Some word of the wave's blocks is kUnwritten (uniform in the wave).
+template <int N> __device__ __forceinline__ bool any_unwritten(const u32x4 (&b)[N]) {
+    unsigned m = 0;   // (the largest unsigned value is kUnwritten)
+#pragma unroll
+    for (int i = 0; i < N; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) m = m > b[i][e] ? m : b[i][e];
+    return __any(m == kUnwritten);
+}
+
+// Behind a round of loads that found kUnwritten: bounded like wait_versions; `dead` (uniform in the wave) is set when the launch has
+// given up: no wait waits any more.
+__device__ __forceinline__ void poll_failed(int &polls, long long &t0, bool &dead, WsHeader *hdr, long long spin_limit, int group, int step) {
+    if (++polls < 64 && spin_limit > 1) return;
+    polls = 0;
+    if (uniform_int(__hip_atomic_load(&hdr->abort_flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))) dead = true;
+    const long long now = (long long)wall_clock64();
+    if (t0 == 0 && spin_limit > 1) {
+        t0 = now;
+    } else if (now - t0 > spin_limit && !dead) {
+        dead = true;
+        if ((threadIdx.x & (kWave - 1)) == 0) {
+            hdr->timeout_group = group;
+            hdr->timeout_step = step;
+            __hip_atomic_store(&hdr->abort_flag, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+        }
+    }
+}
+
 // Called by all threads of the workgroup after they stored the data of `version`.
 __device__ __forceinline__ void publish_version(int *flag, int version) {
     // every wave drains its own (write-through) exchange stores before the workgroup

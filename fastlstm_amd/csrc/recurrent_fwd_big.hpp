@@ -10,18 +10,28 @@
 //    the k-steps so that an LDS read has the MFMAs of the k-steps between to arrive;
 //  * the batch tiles of 16 rows are multiplied one after the other.  Operand blocks go through a ring of R blocks of
 //    registers, refilled as they are consumed, across the tiles of a step;
-//  * behind each tile the four partial sums meet in LDS and the gates of its rows are computed while the next tile's operand
-//    blocks arrive;
-//  * exchange and flags as in lstm_fwd_wide_kernel: device-scope stores of 16-byte pieces, two slots, one flag per workgroup.
-// What bounds a step now: the operand blocks, 512 KiB per CU at H = 4096 and 64 rows (16 MiB through the L2 of an XCD at about
-// 2.1 TB/s), and the exchange.  us per step of lstm_fwd_stream_kernel and here: H = 4096, 64 rows 24.8 -> 11.0, 16 rows
-// 20.9 -> 4.8; H = 3072, 32 rows 14.1 -> 5.5; H = 2560, 64 rows 15.4 -> 8.7; and no packed copy of W_h per call (118 us at 4096).
+//  * behind each tile the four partial sums meet in LDS and the gates of its rows are computed;
+//  * exchange by device-scope stores of whole 16-byte pieces.  What tells a member that they are there goes by big_fwd_data:
+//    - the data itself, as in recurrent_fwd_xcd.hpp (unwritten words, four slots, the same argument for what may be overwritten when), tile by
+//      tile: the rows of a tile are on their way while the next tile is multiplied, and the first blocks of the next step's first tile are
+//      requested behind the last ones of this step's last, so with several tiles nobody waits (of a step of H = 2048 with two tiles 0.7 us are
+//      waits, where the flags and the drains in front of them took 2.5);
+//    - or one flag per workgroup and step, raised behind the acknowledgement of its stores: with one tile everybody would look for blocks
+//      that cannot be there yet, and their loads and the marking of words as unwritten double what the members' L2s have to give up.
+//    us per step, flags and data: bf16 H = 2048, 64 rows (one tile) 4.3 and 4.8, 128 rows (two) 7.3 and 6.2; H = 2560, 16, 32, 64 rows (one, two,
+//    four tiles of half the units) 4.3, 5.7, 8.4 and 3.7, 3.9, 7.4; H = 4096 5.1, 7.0, 11.4 and 4.6, 5.8, 11.3.  fp32, three times the words: H = 1024, 64 rows
+//    (one tile) 4.7 and 5.4, 128 rows (two; the registers do not hold what it takes) 7.2 and 8.0, H = 640, 128 rows 5.8 and 5.3, H = 1280, 16 rows 4.8
+//    and 4.2, H = 2048, 16, 32, 64 rows 5.7, 8.0, 12.6 and 5.9, 7.7, 14.6.
+// What bounds a step now: the operand blocks, 512 KiB per CU at H = 4096 and 64 rows -- a CU takes 90 KB per us from its L2, whatever is in
+// flight --, then the chain behind a tile: sums through LDS, gates (0.2 us per cell of a lane), pieces.  us per step of lstm_fwd_stream_kernel and here:
+// H = 4096, 64 rows 24.8 -> 11.3, 16 rows 20.9 -> 4.6; H = 3072, 32 rows 14.1 -> 4.5; H = 2560, 64 rows 15.4 -> 7.4; and no packed copy of W_h per call (118
+// us at 4096).
 // Up to H = 2048, with 32 units, there are twice as many barrier groups as lstm_fwd_wide_kernel has: half the rows per group, half
 // the operand bytes per CU (H = 1280, B = 64 3.99 -> 3.31).
 // fp32 (lstm_fwd_big_parts_kernel): every number as the sum of three bf16 parts (recurrent_parts.hpp), the weights' 384 H bytes per
 // workgroup all in registers, h_t exchanged as parts; the largest of the six products has a sum of its own.  What bounds it: at two
-// batch tiles the 96 H bytes of operand blocks of each (H = 1024: 384 KiB per CU and step), at one the exchange.  H = 1024,
-// us per step of the kernels on the fp32 matrix instructions (1/16 of the rate) and here: B = 128 11.1 -> 7.9, B = 16 5.1 -> 3.9.
+// batch tiles the 96 H bytes of operand blocks of each (H = 1024: 192 KiB per CU and step), at one the exchange.  H = 1024,
+// us per step of the kernels on the fp32 matrix instructions (1/16 of the rate) and here: B = 128 11.1 -> 7.1, B = 16 5.1 -> 3.9.
 // Up to four recurrences share a launch (T = 256, I = 256, inference / training of three layers, two of them in a launch and three: H = 1024,
 // B = 16 2.93 / 8.48 and 2.20 / 7.38 ms; of four, B = 32 4.23 / 13.4 and 3.76 / 12.8; H = 640, B = 16, three 2.37 / 6.49 and 1.78 / 5.40).
 // Above H = 1024 a workgroup holds 8 units (MT = 2: 384 KiB at H = 2048), one group of up to 64 rows is a launch, and every CU reads the
@@ -40,15 +50,25 @@ namespace fastlstm {
 constexpr int kBigRegBlocks = 96;   // blocks of weights per wave (of 4 registers per lane) that stay in registers,
 constexpr int kBigAccBlocks = 64;   // the first of them in the accumulator half of the register file
 
-constexpr int big_ring(int kw, int mt) {   // operand blocks in flight per wave: what the registers hold
+constexpr int big_ring(int kw, int mt) {   // reverse kernel: operand blocks in flight per wave: what the registers hold
     return mt == 8 ? (kw <= 10 ? 16 : kw <= 12 ? 12 : kw <= 14 ? 6 : 8) : kw <= 20 ? 16 : kw <= 24 ? 12 : 10;
 }
-constexpr int big_lds_steps(int kw, int mt) { return kw > kBigRegBlocks / mt ? kw - kBigRegBlocks / mt : 0; }
+constexpr int big_fwd_ring(int kw, int mt, int nt) {   // forward (a block more and weights move to scratch memory: tests/test_mfma_wait_states.py)
+    return mt == 8 ? (kw <= 10 ? 10 : kw <= 12 ? (nt > 1 ? 8 : 12) : kw <= 14 ? 8 : nt > 1 ? 6 : 8) : kw <= 20 ? 16 : kw <= 24 ? (nt > 1 ? 10 : 12) : kw <= 28 ? (nt > 1 ? 8 : 10) : 8;
+}
+// The data tells that it is there (see above; figures there).
+constexpr bool big_fwd_data(int kw, int mt, int nt, int parts) {
+    return parts == 1 ? nt > 1 || mt == 4 : mt == 2 ? (nt == 1 ? kw <= 12 : nt == 2) : nt == 2 && kw < 8;
+}
+constexpr int big_fwd_slots(int kw, int mt, int nt, int parts) { return big_fwd_data(kw, mt, nt, parts) ? kXchgSlots : 2; }   // exchange slots
+constexpr int big_lds_steps(int kw, int mt) {   // (14 k-steps: there is room for one more, and the ring's registers are worth more)
+    return kw > kBigRegBlocks / mt ? kw - kBigRegBlocks / mt + (kw == 14) : 0;
+}
 // tiles whose partial sums meet in LDS at a time: all, or four where the weights leave room for no more
 constexpr int big_sum_tiles(int kw, int mt) { return 4 * big_lds_steps(kw, mt) * mt > 48 ? 4 : mt; }
 constexpr int big_lds_bytes(int kw, int mt, int nt, int es) {   // (es: bytes per element)
     const int bt = 16 * nt, gseg = 4 * mt * es;
-    return 4 * (big_lds_steps(kw, mt) * mt + big_sum_tiles(kw, mt)) * kFragBytes + bt * (4 * gseg + 16) + 2 * bt * (gseg + 16);
+    return 4 * (big_lds_steps(kw, mt) * mt + big_sum_tiles(kw, mt)) * kFragBytes + (nt == 1 ? 2 : 1) * bt * (4 * gseg + 16) + 2 * bt * (gseg + 16);
 }
 
 // acc (+)= A . B with the A block in the accumulator half of the register file (ACC_HALF) or in the ordinary one.  Inline assembly:

@@ -92,11 +92,6 @@ struct FwdXcdParams {
     long long *trace;  // diagnostic build only
 };
 
-// What an exchange word holds that has not been written: no stored value has this bit pattern (written_word).
-constexpr unsigned kUnwritten = 0xffffffffu;
-// The word as it is stored: all ones, which only NaNs can be (two 16-bit ones, or a 32-bit one), becomes another NaN.
-__device__ __forceinline__ unsigned written_word(unsigned w) { return w < kUnwritten - 1 ? w : kUnwritten - 1; }
-
 // Exchange slots in the L2 of this XCD.
 struct XchgL2 {
     __amdgpu_buffer_rsrc_t rsrc;
@@ -113,16 +108,6 @@ struct XchgL2 {
     __device__ __forceinline__ void store8(unsigned off, u32x2 v) const { __builtin_amdgcn_raw_buffer_store_b64(v, rsrc, off, 0, 0); }
     __device__ __forceinline__ void store16(unsigned off, u32x4 v) const { __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, off, 0, 0); }
 };
-
-// Some word of the wave's blocks is kUnwritten (uniform in the wave).
-template <int N> __device__ __forceinline__ bool any_unwritten(const u32x4 (&b)[N]) {
-    unsigned m = 0;   // (the largest unsigned value is kUnwritten)
-#pragma unroll
-    for (int i = 0; i < N; ++i)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) m = m > b[i][e] ? m : b[i][e];
-    return __any(m == kUnwritten);
-}
 
 // b[i] = load(i), i < N, repeated until no word of them is kUnwritten.  All loads of a round are requested before the
 // first is looked at, and none is in flight behind the loop: what the compiler issues next needs no wait for them.

@@ -133,3 +133,32 @@ def test_rows_past_the_batch_leave_no_trace(B, H, backward):
         results.append(got)
     for clean, dirty in zip(*results):
         assert torch.isfinite(clean).all() and torch.equal(clean, dirty)
+
+
+@pytest.mark.parametrize("T,B,H,dt", [
+    (3, 16, 2576, torch.bfloat16),   # one batch tile, half a k-step past H
+    (4, 33, 2560, torch.float16),    # three tiles of four
+    (3, 64, 4096, torch.bfloat16),
+    (4, 128, 2048, torch.float16),   # groups of two tiles
+    (4, 192, 1280, torch.bfloat16),  # ... six groups in a launch
+    (3, 120, 640, torch.float32),    # two tiles, three words for two numbers
+    (4, 7, 1536, torch.float32),
+    (3, 30, 2048, torch.float32),
+    (3, 64, 1280, torch.float32),    # with flags
+])
+def test_rows_that_are_no_numbers(T, B, H, dt):
+    """A row of NaN whose bits are all ones, which is what a word that has not been written looks like: the launch ends, the row is NaN from
+    its first step on, and no bit of any other row changes."""
+    p = make_problem(T, B, 24, H, seed=T * 100 + H)
+    g = {k: dev(v, dt) for k, v in p.items() if v is not None}
+    bits = torch.int32 if dt == torch.float32 else torch.int16
+    row = B - 1 if B % 16 else B // 2
+    outs = []
+    for h0 in (g["h0"], g["h0"].clone()):
+        if outs:
+            h0.view(bits)[row] = -1
+        outs.append(L.lstm_persistent_fwd(g["x"], h0, g["c0"], g["Wx"], g["bx"], g["Wh"], g["bh"])[:2])
+    others = torch.arange(B, device="cuda") != row
+    for want, got in zip(*outs):
+        assert torch.equal(want[1:, others], got[1:, others])
+        assert got[1:, row].isnan().all()
