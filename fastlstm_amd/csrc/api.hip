@@ -761,7 +761,6 @@ int try_bwd_wide(const void *dout, void *dh, void *dc, const void *ifgo, const v
         q.hdr = reinterpret_cast<WsHeader *>(wsb);
         q.flags = reinterpret_cast<int *>(wsb + kWsHeaderBytes);
         q.flag_stride = kXcdGroupStride;
-        q.team_flags = q.flags + kNumXcd * kXcdGroupStride;
         q.xbuf = wsb + kWsHeaderBytes + kWsCounterBytes;
         q.partials = q.xbuf + 2 * copies * c.xslot;
         q.n_rec = copies;
@@ -1529,7 +1528,6 @@ static int bwd_persistent_impl(const void *dout, void *dh, void *dc, const void 
                 const int nt = big_half_params(h, wsb, ws_bytes, std::min(B - r0, kBigHalfRows), H, true);
                 h.KSB = h.KSBP = 4 * H / 32;
                 h.b_base = r0;
-                h.team_flags = h.flags + kXcdGroupStride;
                 h.partials = h.xbuf + 2 * (size_t)nt * h.KSB * 3 * kFragBytes;
                 const int grid = kNumXcd * cdiv(h.n_ht / kBigTeamHalf, kNumXcd) * kBigTeamHalf;
                 if (launch_bwd_big(dtype, h, H / 128, 4, nt, grid, s, nullptr) != hipSuccess) return FASTLSTM_ERR_HIP;
@@ -1543,7 +1541,6 @@ static int bwd_persistent_impl(const void *dout, void *dh, void *dc, const void 
         if (resident) {
             p.Wh = Wh;
             p.n_rec = 1;
-            p.team_flags = reinterpret_cast<int *>(wsb + kWsHeaderBytes);
             p.partials = wsb + l.wpack_off;
             int occ = 0;
             if (launch_bwd_big(dtype, p, kw, 4, pl.bt / 16, 0, nullptr, &occ) != hipSuccess) return FASTLSTM_ERR_HIP;
@@ -1561,7 +1558,6 @@ static int bwd_persistent_impl(const void *dout, void *dh, void *dc, const void 
             const int grid = n_bt * pl.n_htiles;
             int occ = 0;
             if (resident) {
-                if (c && !clear_xcd_counters(wsb, s)) return FASTLSTM_ERR_HIP;   // (the team flags lie there)
                 if (launch_bwd_big(dtype, p, kw, 4, pl.bt / 16, grid_big, s, nullptr) != hipSuccess) return FASTLSTM_ERR_HIP;
                 continue;
             }

@@ -57,7 +57,6 @@ struct BwdStreamParams {
     const unsigned char *wpack;   // [n_ht][MTB][KSBP] operand blocks of Wh[:, units]^T, K = (unit', gate)
     // lstm_bwd_big_kernel:
     const void *Wh;    // [4H,H]
-    int *team_flags;   // [n_rec n_bt][flag_stride]
     unsigned char *partials;   // [n_rec n_bt][n_ht receivers][4 senders][unit tiles][NT] blocks of fp32 sums
     int n_rec;         // 2 (fp32: up to kMaxSideBySide): further, independent recurrences of this shape side by side, their operands here
     const void *dout2, *ifgo2, *cell2, *Wh2, *dout_more[2], *ifgo_more[2], *cell_more[2], *Wh_more[2];
