@@ -1052,6 +1052,21 @@ template <typename V> __device__ __forceinline__ V sum_of_parts(const float *p, 
     return ((s[0] + s[1]) + (s[2] + s[3])) + ((s[4] + s[5]) + (s[6] + s[7]));
 }
 
+// The sum of n values `stride` floats apart, one after the other, 16 loads in flight: a thread waits for little else.  (The loads of the loop as
+// it was written waited for each other: M = 1152, I = 128, H = 288, 17 parts, 51 of the bias gradient, 13.5 us, so 6.2.)
+template <typename V> __device__ __forceinline__ V sum_in_order(const float *p, size_t stride, int n) {
+    V s{};
+    for (int k = 0; k < n; k += 16) {
+        V v[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) v[u] = *reinterpret_cast<const V *>(p + (size_t)min(k + u, n - 1) * stride);   // (past the end: the last value, which is not added)
+#pragma unroll
+        for (int u = 0; u < 16; ++u)
+            if (k + u < n) s += v[u];
+    }
+    return s;
+}
+
 // Finishes a weight-gradient launch: out = the sum over splits of the fp32 partials, in split order, for dWx
 // (M x I) and dWh (M x H) -- not called for with splits == 1, then I = H = 0 here -- and db (M) = the sum of its
 // db_parts partial sums.  A thread owns four consecutive elements of a matrix (I and H are multiples of 8) or
@@ -1072,17 +1087,14 @@ __global__ void wgrad_reduce_kernel(const float *part_x, T *dWx, const float *pa
         if constexpr (sizeof(T) == 4) {
             db[i] = sum_of_parts<float>(part_db + i, (size_t)M, db_parts);
         } else {
-            float s = 0.f;
-            for (int k = 0; k < db_parts; ++k) s += part_db[(size_t)k * M + i];
-            db[i] = Elem<T>::from_f32(s);
+            db[i] = Elem<T>::from_f32(sum_in_order<float>(part_db + i, (size_t)M, db_parts));
         }
         return;
     }
     if constexpr (sizeof(T) == 4) {
         *reinterpret_cast<f32x4 *>(out + i * 4) = sum_of_parts<f32x4>(part + i * 4, total, splits);
     } else {
-        f32x4 s = {0.f, 0.f, 0.f, 0.f};
-        for (int k = 0; k < splits; ++k) s += *reinterpret_cast<const f32x4 *>(part + (size_t)k * total + i * 4);
+        const f32x4 s = sum_in_order<f32x4>(part + i * 4, total, splits);
         T o[4] = {Elem<T>::from_f32(s[0]), Elem<T>::from_f32(s[1]), Elem<T>::from_f32(s[2]), Elem<T>::from_f32(s[3])};
         *reinterpret_cast<u32x2 *>(out + i * 4) = *reinterpret_cast<u32x2 *>(o);
     }
