@@ -28,7 +28,6 @@ struct Cand {
     double cost;
 };
 
-constexpr int kNoSyncMaxH = 64;  // whole W_h on one CU, barrier compiled out
 
 int kstep_of(int dtype) { return dtype == FASTLSTM_FP32 ? 16 : 32; }
 
