@@ -644,16 +644,16 @@ bool select_wide(int T, int B_all, int H, int dtype, bool backward, size_t ws_by
 // Rows per launch (see xcd_rows_per_launch) for the register-resident kernels: full launches of 64-row groups
 // (whole-CU kernels: of 32-row groups) on all XCDs.
 static int wide_rows_per_launch(int T, int B, int H, int dtype, bool backward, size_t ws_bytes) {
-    const int xpg = cdiv(H / 16, 32);
-    const int rows = dtype == FASTLSTM_FP32 ? 32 * std::min(kNumXcd, kNumXcd * 32 / std::max(1, H / 16))   // (two batch tiles per group)
-                     : H >= 32 && (g_families.load() & 4)
-                         ? 32 * (kNumXcd * 32 / (H / 32))   // (groups of the 32-unit form)
-                         : 64 * (kNumXcd / std::max(1, xpg));
-    if (rows >= B || rows <= 0) return 0;
-    WideCfg c;
-    if (!select_wide(T, B, H, dtype, backward, ws_bytes, &c, rows)) return 0;
-    if (B % rows && !select_wide(T, B, H, dtype, backward, ws_bytes, &c, B % rows)) return 0;
-    return rows;
+    const bool fp32 = dtype == FASTLSTM_FP32;
+    const int big = fp32 ? 32 * std::min(kNumXcd, kNumXcd * 32 / std::max(1, H / 16))   // (two batch tiles per group)
+                    : H >= 32 && (g_families.load() & 4) ? 32 * (kNumXcd * 32 / (H / 32)) : 0;   // (groups of the 32-unit form)
+    auto holds = [&](int rows) {
+        WideCfg c;
+        return rows > 0 && rows < B && select_wide(T, B, H, dtype, backward, ws_bytes, &c, rows) &&
+               (B % rows == 0 || select_wide(T, B, H, dtype, backward, ws_bytes, &c, B % rows));
+    };
+    const int wide = fp32 ? 0 : 64 * (kNumXcd / std::max(1, cdiv(H / 16, 32)));   // (a workspace of two slots holds no more)
+    return holds(big) ? big : holds(wide) ? wide : 0;
 }
 
 // fp32, H = 1280, 1536, 1792, 2048 (plan: streamed weights): the whole-CU kernels with 8 units per workgroup hold all of W_h, as three
