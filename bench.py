@@ -393,7 +393,7 @@ def main():
         alg = "2*B*H*4H*T + 2*T*B*I*4H flop per launch = %.1f GFLOP" % (flops / 1e9)
     else:
         flops, t_dom = rec_flops, t_rec
-        kname = {0: "lstm_fwd_persistent_kernel", 1: "lstm_fwd_xcd_kernel", 2: "lstm_fwd_wide_kernel"}[kind]
+        kname = {0: "lstm_fwd_persistent_kernel", 1: "lstm_fwd_xcd_kernel", 2: "lstm_fwd_big_kernel"}[kind]
         alg = "2*B*H*4H*T flop per launch = %.1f GFLOP" % (flops / 1e9)
         if args.workload == "B":
             traffic, traffic_src = None, None
