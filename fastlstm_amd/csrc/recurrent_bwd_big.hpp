@@ -17,7 +17,7 @@
 // lstm_bwd_stream_kernel and here: H = 4096, 64 rows 33.6 -> 12.8, 16 rows 21.1 -> 6.7; H = 3072, 32 rows 16.8 -> 7.2;
 // H = 2560, 64 rows 22.6 -> 9.5.  Of the form with 16 units and 8 waves per CU for H <= 2048 and here, while the team's sums went by flags:
 // H = 2048, 128 rows 11.0 -> 8.6, 64 rows 9.0 -> 6.2, 32 rows 6.4 -> 5.3; H = 1280, 128 rows 8.7 -> 7.0.  Since then (sums that say themselves that they
-// are there, gate derivatives computed while they travel) 128 rows of H = 2048 9.2 -> 7.6 on one box, fp32 H = 1024, 64 rows 7.4 -> 6.1; forward and
+// are there, gate derivatives computed while they travel) 128 rows of H = 2048 9.2 -> 7.6, fp32 H = 1024, 64 rows 7.4 -> 6.1; forward and
 // reverse pass together, us per timestep of a training call: bf16 H = 1280, 32 rows 8.9 -> 8.2, H = 2048, 32 rows 10.4 -> 9.6, H = 3072, 16 rows 13.0 -> 11.2, H =
 // 4096, 64 rows 33.0 -> 32.0; fp32 H = 640, 16 rows 9.3 -> 8.7, H = 1280, 16 rows 12.8 -> 11.8, H = 2048, 64 rows 43.1 -> 40.4.
 // Up to H = 2048 a second recurrence of the same shape may share the launch, in fp32 up to H = 1024 a third and a fourth too (the directions of a
