@@ -23,7 +23,7 @@ template <bool A_KM, bool B_KM, int T, bool TWO, bool ALL = false> hipError_t la
 
 }  // namespace
 
-// Tile edge (256: one workgroup per CU, 128: two) and parts of K of C[M][N1 | N2]: the least time, put together from measured parts.
+// Tile edge (256: one workgroup per CU, 128: two, 64: few tiles) and parts of K of C[M][N1 | N2]: the least time, put together from measured parts.
 // A k-tile of 16 takes a 256 x 256 tile 2.2 us and two 128 x 128 tiles of a CU 1.35 us (0.7 us one alone); a tile takes 5 and 4 us
 // besides (start, epilogue); partial sums are written and read back at 3.5 TB/s, by a launch of 4 us.
 // M = 16384, N = 4096, K = 1024: 256 0.69 ms, 128 0.75; M = 2048, N = 1024, K = 256: 256 0.051 ms, 128 0.023.
@@ -52,9 +52,18 @@ void gemm_f32_plan(int M, int N1, int N2, int K, bool allow_split, bool two, int
             }
         }
     }
+    // Up to one 64 x 64 tile per CU, each on a CU of its own: a quarter of the products per k-tile and of the rows to store (x.Wx^T, rows, K, N, us
+    // on 128 x 128 and here: 512, 80, 384 8.5 and 6.5; 256, 256, 1024 15.5 and 11.9; 1024, 256, 1024 16.0 and 12.3; 256, 1024, 4096 46 and 36; with 304
+    // tiles, 1000, 300, 1200, 18.7 and 19.1, with 512, 8192, 40, 256, 9.4 and 12.6).
+    if (!two && *tile == 128 && *splits == 1 && (long long)cdiv(M, 64) * (cdiv(N1, 64) + cdiv(N2, 64)) <= 256) *tile = 64;
 }
 
 hipError_t launch_gemm_f32(const GemmF32Params &g, bool a_km, bool b_km, int tile, hipStream_t s) {
+    if (tile == 64) {
+        if (a_km || g.p.splits > 1) return hipErrorInvalidValue;
+        if (g.p.K <= kF32AllK) return b_km ? launch_t<false, true, 64, true, true>(g, s) : launch_t<false, false, 64, true, true>(g, s);
+        return b_km ? launch_t<false, true, 64, false>(g, s) : launch_t<false, false, 64, false>(g, s);
+    }
     if (g.p.K <= kF32AllK && tile == 128 && g.p.splits == 1) {
         if (a_km && b_km) return launch_t<true, true, 128, true, true>(g, s);
         if (!a_km) return b_km ? launch_t<false, true, 128, true, true>(g, s) : launch_t<false, false, 128, true, true>(g, s);

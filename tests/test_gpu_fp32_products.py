@@ -42,6 +42,26 @@ def test_products_at_the_edges(R, I, H):
         assert bool(((a.double() - b).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("I,H,rows", [(40, 64, (1, 63, 65, 4096)), (64, 65, (64, 200)), (65, 96, (31, 129)), (300, 256, (1, 1000)), (1030, 512, (7, 128))])
+def test_a_range_of_rows_has_the_bits_of_the_whole(I, H, rows):
+    """Tiles of 64 (few rows), 128 and 256 add up in the same order: x.Wx^T and d.Wx of the first rows alone."""
+    g = torch.Generator(device="cuda").manual_seed(I + H)
+    lib, st = _lib.load(), torch.cuda.current_stream().cuda_stream
+    n = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    R = 8192
+    x, Wx, bx, bh, d = n(R, I), n(4 * H, I), n(4 * H), n(4 * H), n(R, 4 * H)
+
+    def both(r):
+        y, dx = torch.empty(r, 4 * H, device="cuda"), torch.empty(r, I, device="cuda")
+        _lib.check(lib.fastlstm_gemm_ifgo(x.data_ptr(), Wx.data_ptr(), bx.data_ptr(), bh.data_ptr(), y.data_ptr(), 1, r, I, H, 0, st), "k1")
+        _lib.check(lib.fastlstm_gemm_dx(d.data_ptr(), Wx.data_ptr(), dx.data_ptr(), 1, r, I, H, 0, st), "dx")
+        return y, dx
+    whole = both(R)
+    for r in rows:
+        for a, b in zip(both(r), whole):
+            assert torch.equal(a, b[:r]), r
+
+
 def test_infinities_and_nans_as_in_the_sum():
     """inf times a number whose lower parts are zero, of either sign, inf times 0, inf - inf and NaN: in an operand of any product."""
     def plant(x, Wx, d):
