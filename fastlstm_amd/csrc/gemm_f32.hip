@@ -55,13 +55,13 @@ void gemm_f32_plan(int M, int N1, int N2, int K, bool allow_split, bool two, int
     // Up to one 64 x 64 tile per CU, each on a CU of its own: a quarter of the products per k-tile and of the rows to store (x.Wx^T, rows, K, N, us
     // on 128 x 128 and here: 512, 80, 384 8.5 and 6.5; 256, 256, 1024 15.5 and 11.9; 1024, 256, 1024 16.0 and 12.3; 256, 1024, 4096 46 and 36; with 304
     // tiles, 1000, 300, 1200, 18.7 and 19.1, with 512, 8192, 40, 256, 9.4 and 12.6).
-    if (!two && *tile == 128 && *splits == 1 && (long long)cdiv(M, 64) * (cdiv(N1, 64) + cdiv(N2, 64)) <= 256) *tile = 64;
+    // (K <= 64: the sums of all nine products take more registers than two waves of a SIMD have, for 8.5 -> 8.0.)
+    if (!two && K > kF32AllK && *tile == 128 && *splits == 1 && (long long)cdiv(M, 64) * (cdiv(N1, 64) + cdiv(N2, 64)) <= 256) *tile = 64;
 }
 
 hipError_t launch_gemm_f32(const GemmF32Params &g, bool a_km, bool b_km, int tile, hipStream_t s) {
     if (tile == 64) {
-        if (a_km || g.p.splits > 1) return hipErrorInvalidValue;
-        if (g.p.K <= kF32AllK) return b_km ? launch_t<false, true, 64, true, true>(g, s) : launch_t<false, false, 64, true, true>(g, s);
+        if (a_km || g.p.splits > 1 || g.p.K <= kF32AllK) return hipErrorInvalidValue;
         return b_km ? launch_t<false, true, 64, false>(g, s) : launch_t<false, false, 64, false>(g, s);
     }
     if (g.p.K <= kF32AllK && tile == 128 && g.p.splits == 1) {
