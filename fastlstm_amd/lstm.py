@@ -320,10 +320,12 @@ def _chunk_workspaces(n_bytes, zero_bytes, count, device):
 
 
 def _zero_states(count, like):
-    """`count` zero states of like's shape, dtype and device, each on a 16-byte boundary, by ONE fill."""
-    stride = (like.numel() + 7) // 8 * 8
-    buf = torch.zeros(count * stride, device=like.device, dtype=like.dtype)
-    return [buf[k * stride:k * stride + like.numel()].view(like.shape) for k in range(count)]
+    """`count` zero states of like's shape, dtype and device, cleared by ONE launch.  Each has a storage of its own: they become gradients that a
+    caller keeps or saves one by one."""
+    states = [torch.empty(like.shape, device=like.device, dtype=like.dtype) for _ in range(count)]
+    if states:
+        torch._foreach_zero_(states)
+    return states
 
 
 def _initial_states(bufs, states):

@@ -293,3 +293,15 @@ def test_parameter_shapes_follow_the_operand_list():
         got = lstm._parameter_shapes(m.num_layers, 2 if m.bidirectional else 1, 5, 7, m.bias)
         assert [s for _, s in got] == [p.shape for p in m._operand_list()]
         assert [n for n, _ in got] == m._operand_names
+
+
+def test_zero_states_share_no_storage():
+    """The zero gradients of final states, which come back as dh_0 and dc_0: each is all of its own storage."""
+    import fastlstm_amd.lstm as L
+    like = torch.ones(3, 2, 7)[1]
+    states = L._zero_states(4, like)
+    assert len({s.untyped_storage().data_ptr() for s in states}) == 4
+    for s in states:
+        assert s.shape == like.shape and s.dtype == like.dtype and s.is_contiguous() and not s.any()
+        assert s.untyped_storage().nbytes() == like.numel() * 4 and s._base is None
+    assert L._zero_states(0, like) == []
