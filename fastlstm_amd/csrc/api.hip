@@ -1567,6 +1567,8 @@ static int bwd_persistent_impl(const void *dout, void *dh, void *dc, const void 
             const int grid = n_bt * pl.n_htiles;
             int occ = 0;
             if (resident) {
+                // (the flags are a range's own; the XCD rotation that the launch's workgroups agree on is not, and is another in every launch)
+                if (c && !clear_xcd_counters(wsb, s)) return FASTLSTM_ERR_HIP;
                 if (launch_bwd_big(dtype, p, kw, 4, pl.bt / 16, grid_big, s, nullptr) != hipSuccess) return FASTLSTM_ERR_HIP;
                 continue;
             }

@@ -1,6 +1,8 @@
 """Robustness of the boundary (run with -m gpu): gradients that autograd does not ask for are not computed,
 recurrent calls from several streams are ordered by the library, a failed launch shows in its own results,
 and the host-side dispatch caches follow the kernel-family switch."""
+import ctypes
+
 import pytest
 import torch
 
@@ -309,3 +311,52 @@ def test_step_probe_ends_in_every_mode(H, rows, members):
         torch.cuda.synchronize()
         assert lib.fastlstm_ws_status(ws[:64].cpu().numpy().tobytes()) == _lib.OK, (kind, mode)
     assert lib.fastlstm_diag_step_probe(0, 3, 16, 96, 16, steps, ws.data_ptr(), n, None) == _lib.ERR_DIM   # six units per member
+
+
+class _KernelNode(ctypes.Structure):   # hipKernelNodeParams
+    _fields_ = [("block", ctypes.c_uint * 3), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p), ("grid", ctypes.c_uint * 3),
+                ("args", ctypes.c_void_p), ("shared", ctypes.c_uint)]
+
+
+def _captured_kernels(call):
+    """The functions of the kernels that call() enqueues on the current stream, in order (captured, not run)."""
+    hip = _lib.load()   # (its handle finds the functions of the runtime that it is linked with)
+    graph = torch.cuda.CUDAGraph(keep_graph=True)
+    with torch.cuda.graph(graph):
+        call()
+    raw, n = ctypes.c_void_p(graph.raw_cuda_graph()), ctypes.c_size_t(0)
+    assert hip.hipGraphGetNodes(raw, None, ctypes.byref(n)) == 0
+    nodes = (ctypes.c_void_p * n.value)()
+    assert hip.hipGraphGetNodes(raw, nodes, ctypes.byref(n)) == 0
+    funcs = []
+    for node in nodes:
+        params = _KernelNode()
+        assert hip.hipGraphKernelNodeGetParams(ctypes.c_void_p(node), ctypes.byref(params)) == 0   # (kernels only)
+        funcs.append(params.func)
+    return funcs
+
+
+@pytest.mark.parametrize("B,H,dt,backward", [(65, 4096, torch.bfloat16, 1),    # teams of whole-CU kernels, two launches
+                                             (150, 2560, torch.float16, 1),    # ... three
+                                             (65, 1280, torch.float32, 1),     # ... of half unit tiles
+                                             (129, 2048, torch.bfloat16, 1),   # ... groups of 32 rows
+                                             (300, 1024, torch.float16, 0),    # XCD-local kernels
+                                             (300, 1024, torch.float16, 1)])
+def test_launches_over_row_ranges_start_from_a_clean_header(B, H, dt, backward):
+    """Workgroups of a launch compare the XCD that they run on with what the first one wrote down (check_xcd_placement), which
+    is the same within ONE launch: between two that share a workspace something clears it."""
+    lib, T, code = _lib.load(), 1, {torch.float32: 0, torch.float16: 1, torch.bfloat16: 2}[dt]
+    plan = _lib.Plan()
+    _lib.check(lib.fastlstm_plan_device(0, B, H, code, backward, plan), "plan")
+    n = lib.fastlstm_recurrent_workspace_bytes(plan, T, H, code, backward)
+    ws = torch.zeros(n, dtype=torch.uint8, device="cuda")
+    z = lambda *shape: torch.zeros(shape, device="cuda", dtype=dt)
+    dout, dh, dc, ifgo, cell, d_ifgo, out, Wh = z(T, B, H), z(B, H), z(B, H), z(T, B, 4 * H), z(T + 1, B, H), z(T, B, 4 * H), z(T + 1, B, H), z(4 * H, H)
+    operands = (dout, dh, dc, ifgo, cell, d_ifgo, Wh) if backward else (ifgo, out, cell, Wh)
+    entry = lib.fastlstm_bwd_persistent if backward else lib.fastlstm_fwd_persistent
+    torch.cuda.synchronize()
+    kernels = _captured_kernels(lambda: _lib.check(entry(*(t.data_ptr() for t in operands), ws.data_ptr(), n, T, B, H, code,
+                                                         torch.cuda.current_stream().cuda_stream), "recurrence"))
+    assert len(kernels) >= 4 and len(kernels) % 2 == 0   # launch, (clearing, launch) ..., the status
+    clearing = set(kernels[1:-1:2])
+    assert len(clearing) == 1 and not clearing & set(kernels[0::2]) and kernels[-1] not in kernels[:-1]
