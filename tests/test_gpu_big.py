@@ -5,7 +5,7 @@ import pytest
 import torch
 
 import fastlstm_amd.lstm as L
-from test_gpu_parity import FWD_KEYS, HALF_TOL, RM, dev, make_problem, npy, to_np, within
+from test_gpu_parity import FP32_TOL, FWD_KEYS, HALF_TOL, RM, dev, make_problem, npy, to_np, within
 from fastlstm_amd import FastLSTM, _lib
 
 pytestmark = pytest.mark.gpu
@@ -162,3 +162,110 @@ def test_rows_that_are_no_numbers(T, B, H, dt):
     for want, got in zip(*outs):
         assert torch.equal(want[1:, others], got[1:, others])
         assert got[1:, row].isnan().all()
+
+
+REVERSE = [
+    (3, 16, 2560, torch.bfloat16),   # one unit tile per member, one batch tile
+    (4, 64, 4096, torch.float16),    # four batch tiles
+    (3, 40, 2048, torch.bfloat16),   # two unit tiles per member, groups of 16 rows
+    (4, 128, 2048, torch.float16),   # ... of 32, all CUs
+    (3, 90, 1280, torch.bfloat16),   # ... a ragged group, teams on the XCDs unevenly
+    (4, 64, 1024, torch.float32),    # fp32: teams of four
+    (3, 100, 640, torch.float32),
+    (4, 7, 1280, torch.float32),     # teams of eight: two members share a unit tile, and the place of its sums
+    (3, 50, 2048, torch.float32),
+]
+
+
+def _reverse_call(operands, ws_bytes=None):
+    """fastlstm_bwd_persistent on copies: ([d_ifgo, dh_0, dc_0], status of the workspace)."""
+    dout, dh, dc, ifgo, cell, Wh = operands
+    (T, B, H), code, lib = dout.shape, RM[dout.dtype], _lib.load()
+    plan = _lib.Plan()
+    _lib.check(lib.fastlstm_plan_device(0, B, H, code, 1, plan), "plan")
+    n = ws_bytes or lib.fastlstm_recurrent_workspace_bytes(plan, T, H, code, 1)
+    assert lib.fastlstm_recurrent_form(T, B, H, code, 1, n) == 2
+    ws = torch.full((n,), 0xff, dtype=torch.uint8, device="cuda")
+    ws[:min(n, plan.ws_zero_bytes)] = 0
+    dh, dc, d = dh.clone(), dc.clone(), torch.empty_like(ifgo)
+    _lib.check(lib.fastlstm_bwd_persistent(dout.data_ptr(), dh.data_ptr(), dc.data_ptr(), ifgo.data_ptr(), cell.data_ptr(), d.data_ptr(),
+                                           Wh.data_ptr(), ws.data_ptr(), n, T, B, H, code, torch.cuda.current_stream().cuda_stream), "reverse")
+    torch.cuda.synchronize()
+    return [d, dh, dc], lib.fastlstm_ws_status(ws[:64].cpu().numpy().tobytes())
+
+
+def _reverse_operands(T, B, H, dt):
+    g = torch.Generator(device="cuda").manual_seed(T * 100 + H)
+    n = lambda *s, k=1.0: (torch.randn(*s, device="cuda", generator=g) * k).to(dt)
+    return n(T, B, H), n(B, H), n(B, H), n(T, B, 4 * H), n(T + 1, B, H, k=.5), n(4 * H, H, k=H ** -.5)
+
+
+@pytest.mark.parametrize("T,B,H,dt", REVERSE)
+def test_gradients_that_are_no_numbers(T, B, H, dt):
+    """A row of NaN whose bits are all ones (what a word of the team's sums that has not been written looks like) in each operand of the
+    reverse pass in turn: the launch ends, the row's gradients are NaN from there on, and no bit of any other row changes."""
+    clean_operands = _reverse_operands(T, B, H, dt)
+    clean, status = _reverse_call(clean_operands)
+    assert status == _lib.OK and all(torch.isfinite(t).all() for t in clean)
+    bits, row = torch.int32 if dt == torch.float32 else torch.int16, B - 1 if B % 16 else B // 2
+    others = torch.arange(B, device="cuda") != row
+    for which, name in enumerate(("dout", "dh_n", "dc_n", "ifgo", "cell")):
+        operands = [t.clone() for t in clean_operands]
+        bad = operands[which].view(bits)
+        if bad.dim() == 3:
+            bad[T // 2, row] = -1
+        else:
+            bad[row] = -1
+        got, status = _reverse_call(operands)
+        assert status == _lib.OK, name
+        for a, b in zip(got, clean):
+            assert torch.equal(a[..., others, :], b[..., others, :]), name
+            assert a[..., row, :].view(-1, a.shape[-1])[0].isnan().all(), name   # (d_ifgo: its first timestep)
+
+
+@pytest.mark.parametrize("T,B,H,dt", REVERSE)
+def test_reverse_launches_drain_on_timeout(T, B, H, dt):
+    """A spin limit of one poll, forced from the host: the waits for the group and for the team's sums give up, the grid drains, the
+    call reports it and its results are NaN; the next call is healthy."""
+    lib, operands = _lib.load(), _reverse_operands(T, B, H, dt)
+    want, _ = _reverse_call(operands)
+    try:
+        lib.fastlstm_set_spin_limit(1)
+        got, status = _reverse_call(operands)
+    finally:
+        lib.fastlstm_set_spin_limit(400000000)
+    assert status == _lib.ERR_TIMEOUT and lib.fastlstm_device_status(0, 1) == _lib.ERR_TIMEOUT
+    assert got[0][0].isnan().any() and got[1].isnan().all() and got[2].isnan().all()
+    again, status = _reverse_call(operands)
+    assert status == _lib.OK and all(torch.equal(a, b) for a, b in zip(again, want))
+
+
+@pytest.mark.parametrize("T,B,H,dt", [
+    (3, 128, 1280, torch.float16),    # groups of 64 rows of the 16-unit form: two slots are all there is room for
+    (3, 140, 1280, torch.bfloat16),   # ... over row ranges
+    (3, 128, 2048, torch.bfloat16),
+    (3, 140, 2048, torch.float16),
+    (3, 60, 2048, torch.float16),     # one batch tile per group: needs no more than two
+    (3, 120, 640, torch.float32),     # two batch tiles, parts of numbers: the general kernel
+])
+def test_forward_with_the_smallest_workspace(oracle, T, B, H, dt):
+    """plan.ws_bytes, the least that is accepted, holds two exchange slots: the forms that take four leave the call to another."""
+    lib, code = _lib.load(), RM[dt]
+    p = make_problem(T, B, 24, H, seed=T * 1000 + H + B)
+    pr = {k: (v.to(dt).double() if v is not None else None) for k, v in p.items()}
+    wants = oracle.forward(*to_np(pr, FWD_KEYS), round_mode=RM[dt])
+    plan = _lib.Plan()
+    _lib.check(lib.fastlstm_plan_device(0, B, H, code, 0, plan), "plan")
+    g = {k: dev(v, dt) for k, v in p.items() if v is not None}
+    ifgo, out, cell = (torch.empty(s, device="cuda", dtype=dt) for s in ((T, B, 4 * H), (T + 1, B, H), (T + 1, B, H)))
+    out[0], cell[0] = g["h0"], g["c0"]
+    n = plan.ws_bytes
+    ws = torch.zeros(n + (1 << 20), dtype=torch.uint8, device="cuda")
+    ws[n:] = 0x5a
+    st = torch.cuda.current_stream().cuda_stream
+    _lib.check(lib.fastlstm_fwd_layer(*(t.data_ptr() for t in (g["x"], g["Wx"], g["bx"], g["bh"], g["Wh"], ifgo, out, cell, ws)), n, T, B, 24, H,
+                                      code, st), "forward")
+    torch.cuda.synchronize()
+    assert lib.fastlstm_ws_status(ws[:64].cpu().numpy().tobytes()) == _lib.OK and bool((ws[n:] == 0x5a).all())
+    for name, got, want in zip(("out", "cell", "ifgo"), (out, cell, ifgo), wants):
+        within(got, want, FP32_TOL if dt == torch.float32 else HALF_TOL, name)
