@@ -23,6 +23,8 @@ pytestmark = pytest.mark.gpu
     (2, 15, 1792, torch.float16),    # ... one group of 16 rows, the weights' sums four tiles at a time
     (1, 128, 2048, torch.float16),   # ... all CUs
     (3, 33, 2064, torch.float16),    # no multiple of 64: the forward kernel only
+    (1, 50, 2304, torch.bfloat16),   # four batch tiles, whose results leave behind the products of the next: one step,
+    (2, 36, 2880, torch.float16),    # ... two, with a tile that has no row
 ])
 def test_big_layers_vs_oracle(oracle, T, B, H, dt):
     p = make_problem(T, B, 24, H, seed=T * 1000 + H)
