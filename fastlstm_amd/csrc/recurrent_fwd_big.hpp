@@ -20,8 +20,8 @@
 //      that cannot be there yet, and their loads and the marking of words as unwritten double what the members' L2s have to give up.
 //    us per step, flags and data: bf16 H = 2048, 64 rows (one tile) 4.3 and 4.8, 128 rows (two) 7.3 and 6.2; H = 2560, 16, 32, 64 rows (one, two,
 //    four tiles of half the units) 4.3, 5.7, 8.4 and 3.7, 3.9, 7.4; H = 4096 5.1, 7.0, 11.4 and 4.6, 5.8, 11.3.  fp32, three times the words: H = 1024, 64 rows
-//    (one tile) 4.7 and 5.4, 128 rows (two; the registers do not hold what it takes) 7.2 and 8.0, H = 640, 128 rows 5.8 and 5.3, H = 1280, 16 rows 4.8
-//    and 4.2, H = 2048, 16, 32, 64 rows 5.7, 8.0, 12.6 and 5.9, 7.7, 14.6.
+//    (one tile) 4.7 and 5.4, 128 rows (two; the registers do not hold what it takes) 7.2 and 8.0, H = 640, 128 rows 5.8 and 5.3, H = 768 6.4 and 5.5, H = 896, 80
+//    rows 6.9 and 5.7, H = 1280, 16 rows 4.8 and 4.2, H = 1536 (activations kept) 4.5 and 4.7, H = 2048, 16, 32, 64 rows 5.7, 8.0, 12.6 and 5.9, 7.7, 14.6.
 // What bounds a step now: the operand blocks, 512 KiB per CU at H = 4096 and 64 rows -- a CU takes 90 KB per us from its L2, whatever is in
 // flight --, then the chain behind a tile: sums through LDS, gates (0.2 us per cell of a lane), pieces.  us per step of lstm_fwd_stream_kernel and here:
 // H = 4096, 64 rows 24.8 -> 11.3, 16 rows 20.9 -> 4.6; H = 3072, 32 rows 14.1 -> 4.5; H = 2560, 64 rows 15.4 -> 7.4; and no packed copy of W_h per call (118
@@ -58,7 +58,7 @@ constexpr int big_fwd_ring(int kw, int mt, int nt) {   // forward (a block more 
 }
 // The data tells that it is there (see above; figures there).
 constexpr bool big_fwd_data(int kw, int mt, int nt, int parts) {
-    return parts == 1 ? nt > 1 || mt == 4 : mt == 2 ? (nt == 1 ? kw <= 12 : nt == 2) : nt == 2 && kw < 8;
+    return parts == 1 ? nt > 1 || mt == 4 : mt == 2 ? (nt == 1 ? kw <= 10 : nt == 2) : nt == 2 && kw < 8;
 }
 constexpr int big_fwd_slots(int kw, int mt, int nt, int parts) { return big_fwd_data(kw, mt, nt, parts) ? kXchgSlots : 2; }   // exchange slots
 constexpr int big_lds_steps(int kw, int mt) {   // (14 k-steps: there is room for one more, and the ring's registers are worth more)

@@ -144,7 +144,8 @@ def test_rows_past_the_batch_leave_no_trace(B, H, backward):
     (4, 128, 2048, torch.float16),   # groups of two tiles
     (4, 192, 1280, torch.bfloat16),  # ... six groups in a launch
     (3, 120, 640, torch.float32),    # two tiles, three words for two numbers
-    (4, 7, 1536, torch.float32),
+    (4, 9, 1280, torch.float32),     # ... 8 units per workgroup, one tile
+    (4, 7, 1536, torch.float32),     # with flags
     (3, 30, 2048, torch.float32),
     (3, 64, 1280, torch.float32),    # with flags
 ])
