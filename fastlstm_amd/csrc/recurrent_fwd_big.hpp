@@ -61,14 +61,16 @@ constexpr bool big_fwd_data(int kw, int mt, int nt, int parts) {
     return parts == 1 ? nt > 1 || mt == 4 : mt == 2 ? (nt == 1 ? kw <= 10 : nt == 2) : nt == 2 && kw < 8;
 }
 constexpr int big_fwd_slots(int kw, int mt, int nt, int parts) { return big_fwd_data(kw, mt, nt, parts) ? kXchgSlots : 2; }   // exchange slots
-constexpr int big_lds_steps(int kw, int mt) {   // (14 k-steps: there is room for one more, and the ring's registers are worth more)
-    return kw > kBigRegBlocks / mt ? kw - kBigRegBlocks / mt + (kw == 14) : 0;
+// k-steps of weights in LDS.  (14, forward: there is room for one more, and the ring's registers are worth more; reverse pass, H = 1792, T = 256, us with two
+// and with three: 1 row 1174 and 1201, 16 1119 and 1132, 64 1245 and 1253, 100 1591 and 1614, 128 1614 and 1620, 256 3321 and 3311)
+constexpr int big_lds_steps(int kw, int mt, bool backward) {
+    return kw > kBigRegBlocks / mt ? kw - kBigRegBlocks / mt + (kw == 14 && !backward) : 0;
 }
 // tiles whose partial sums meet in LDS at a time: all, or four where the weights leave room for no more
-constexpr int big_sum_tiles(int kw, int mt) { return 4 * big_lds_steps(kw, mt) * mt > 48 ? 4 : mt; }
-constexpr int big_lds_bytes(int kw, int mt, int nt, int es) {   // (es: bytes per element)
+constexpr int big_sum_tiles(int kw, int mt) { return 4 * big_lds_steps(kw, mt, true) * mt > 48 ? 4 : mt; }
+constexpr int big_lds_bytes(int kw, int mt, int nt, int es, bool backward) {   // (es: bytes per element)
     const int bt = 16 * nt, gseg = 4 * mt * es;
-    return 4 * (big_lds_steps(kw, mt) * mt + big_sum_tiles(kw, mt)) * kFragBytes + (nt == 1 ? 2 : 1) * bt * (4 * gseg + 16) + 2 * bt * (gseg + 16);
+    return 4 * (big_lds_steps(kw, mt, backward) * mt + big_sum_tiles(kw, mt)) * kFragBytes + (nt == 1 ? 2 : 1) * bt * (4 * gseg + 16) + 2 * bt * (gseg + 16);
 }
 
 // acc (+)= A . B with the A block in the accumulator half of the register file (ACC_HALF) or in the ordinary one.  Inline assembly:

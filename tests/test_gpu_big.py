@@ -21,6 +21,7 @@ pytestmark = pytest.mark.gpu
     (2, 97, 1280, torch.float16),    # 32 units per workgroup: groups of 32 rows, the last one ragged
     (3, 161, 1536, torch.bfloat16),  # ... a launch over 160 rows and one row
     (2, 15, 1792, torch.float16),    # ... one group of 16 rows, the weights' sums four tiles at a time
+    (2, 100, 1792, torch.bfloat16),  # ... groups of 32
     (1, 128, 2048, torch.float16),   # ... all CUs
     (3, 33, 2064, torch.float16),    # no multiple of 64: the forward kernel only
     (1, 50, 2304, torch.bfloat16),   # four batch tiles, whose results leave behind the products of the next: one step,
