@@ -387,13 +387,18 @@ def main():
     kind = lib.fastlstm_recurrent_kernel_kind(T, B, H, code, 0, ws_f.numel())
     xcd_local = kind == 1
     fused = xcd_local and t_layer < 0.9 * (t_k1 + t_rec)
+    # 16-bit, H = 1280 ... 2048 (kind 2), groups of 16 rows: of H / 16 workgroups where 8 XCDs hold them, else of H / 32 where 256 CUs do;
+    # else groups of 32 rows, two batch tiles, of H / 32 workgroups, which exchange tile by tile without a flag per step
+    tiles16 = -(-B // 16)
+    whole_cu = kind == 2 and tiles16 * -(-H // 512) > 8
+    by_tiles = whole_cu and tiles16 > 256 // (H // 32)
     traffic, traffic_src = TRAFFIC.get(args.workload, (None, None))
     if fused:
         flops, t_dom, kname = rec_flops + k1_flops, t_layer, "lstm_fwd_xcd_kernel<..., HELP=true> (projection + recurrence)"
         alg = "2*B*H*4H*T + 2*T*B*I*4H flop per launch = %.1f GFLOP" % (flops / 1e9)
     else:
         flops, t_dom = rec_flops, t_rec
-        kname = {0: "lstm_fwd_persistent_kernel", 1: "lstm_fwd_xcd_kernel", 2: "lstm_fwd_big_kernel"}[kind]
+        kname = {0: "lstm_fwd_persistent_kernel", 1: "lstm_fwd_xcd_kernel", 2: "lstm_fwd_big_kernel" if whole_cu else "lstm_fwd_wide_kernel"}[kind]
         alg = "2*B*H*4H*T flop per launch = %.1f GFLOP" % (flops / 1e9)
         if args.workload == "B":
             traffic, traffic_src = None, None
@@ -402,7 +407,9 @@ def main():
                 "peak": PEAK_TFLOPS[dname], "unit": "TFLOP/s", "frac": round(ach / PEAK_TFLOPS[dname], 4),
                 "traffic": traffic, "traffic_source": traffic_src,
                 "algorithmic": alg, "launch_ms": round(t_dom, 4),
-                "note": "the launch is latency-bound, not MFMA-bound: T sequential steps, each a cross-CU exchange "
+                "note": "T sequential steps, each bound by the h that every CU reads from its L2 and by the sums and gates behind a "
+                        "batch tile; the exchange of a tile runs beside the products of the next one" if by_tiles else
+                        "the launch is latency-bound, not MFMA-bound: T sequential steps, each a cross-CU exchange "
                         + ("through the L2 of one XCD" if xcd_local else "through device memory")
                         + "; see latency_bound"}
 
@@ -421,13 +428,13 @@ def main():
                     "launch_ms": round(t_rec, 4),
                     "note": "latency-bound, not HBM-bound: %d independent workgroups (%d batch rows each) walk through "
                             "T sequential steps; us/step is in kernels.recurrent_fwd_us_per_step" % (-(-B // rows_wg), rows_wg)}
-    elif dname != "fp32" and H % 32 == 0 and H <= 2048:
+    elif dname != "fp32" and H % 32 == 0 and H <= 2048 and not by_tiles:
         # ---- the latency floor of a step, measured with the recurrence's own barrier and exchange code ----
         # (fastlstm_diag_step_probe: 16-bit h tiles; one group is timed alone on an otherwise idle device)
         if kind == 1:
             pk, members, rows = 0, min(32, H // 8), 16   # the smallest unit tile that keeps a group on one XCD
         elif kind == 2:
-            pk, members, rows = 1, H // 16, 64
+            pk, members, rows = 1, H // 32 if whole_cu else H // 16, 16
         else:
             pk, members, rows = 1, plan_f.n_htiles, min(64, max(16, plan_f.bt // 16 * 16))
         while H % (4 * members if pk == 0 else members):
