@@ -167,7 +167,7 @@ __device__ __forceinline__ void lds_barrier() {
 }
 
 // TWO: the small products have sums of their own, so that the large ones are rounded once per 16 k instead of six times (an error
-// 2.6 times smaller: fewer parts of K for the same one).  Only where the sums are split anyway: without a split the two tile sizes add up
+// 2.6 times smaller: fewer parts of K for the same one).  Only where the sums are split anyway: without a split tiles of 64, 128 and 256 add up
 // in the same order, so that a range of rows has the bits that it has within the whole.
 // ALL: nine products (K <= kF32AllK).
 template <bool A_KM, bool B_KM, int BM, int BN, int WM, int WN, bool TWO, bool ALL>

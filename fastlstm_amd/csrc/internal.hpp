@@ -85,9 +85,10 @@ hipError_t launch_bwd_stream(int dtype, const BwdStreamParams &p, int mtb, int n
                              int *max_blocks_per_cu);
 hipError_t launch_pack_wh(int dtype, bool backward, const void *Wh, unsigned char *wpack, int H, int KS, int KSP, int mt,
                           int n_ht, hipStream_t s);
-// Workspace layout of a streamed-weights plan: header | counters | per batch chunk: flags, 2 exchange slots | packed W_h
 constexpr int kNoSyncMaxH = 64;  // whole W_h on one CU, barrier compiled out
 
+// Workspace layout of a streamed-weights plan: header | counters | per batch chunk: flags, 2 exchange slots | packed W_h, or where the
+// whole-CU kernels hold W_h on chip: forward kXchgSlots exchange slots (which every chunk's launch uses), reverse the teams' partial sums
 struct StreamLayout {
     int KS, KSP;            // k-steps of the contraction, padded to the K loop's granule
     int mt;                 // operand row tiles of a workgroup's weight slice (forward: ht / 4, reverse: ht / 16)

@@ -28,7 +28,6 @@ struct Cand {
     double cost;
 };
 
-
 int kstep_of(int dtype) { return dtype == FASTLSTM_FP32 ? 16 : 32; }
 
 }  // namespace

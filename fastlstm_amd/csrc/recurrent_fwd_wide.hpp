@@ -30,7 +30,9 @@ namespace fastlstm {
 // NT batch tiles of 16 rows per group: 4 (64 rows; groups x XCDs-per-group <= 8 limits a launch to 128 rows at
 // H = 2048), or 2 or 1 where the batch fits the launch that way: a small batch then spreads over more groups,
 // i.e. more CUs, and a CU fetches a half or a quarter of the operand bytes per step (H = 2048, B = 16:
-// 3.3 instead of 5.8 us per step).
+// 3.3 instead of 5.8 us per step).  With NT = 1 for one recurrence, 1 or 2 for two side by side; larger batches run on
+// lstm_fwd_big_kernel, and here with NT = 2 or 4 only where its four exchange slots do not fit the workspace (plan.ws_bytes) or the
+// kernel-family switch takes it away.
 template <typename T, int NKW, int NT>
 __global__ __launch_bounds__(kWave * 8) void lstm_fwd_wide_kernel(const FwdXcdParams p) {
     using E = Elem<T>;
