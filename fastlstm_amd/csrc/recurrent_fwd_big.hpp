@@ -22,9 +22,11 @@
 //    four tiles of half the units) 4.3, 5.7, 8.4 and 3.7, 3.9, 7.4; H = 4096 5.1, 7.0, 11.4 and 4.6, 5.8, 11.3.  fp32, three times the words: H = 1024, 64 rows
 //    (one tile) 4.7 and 5.4, 128 rows (two; the registers do not hold what it takes) 7.2 and 8.0, H = 640, 128 rows 5.8 and 5.3, H = 768 6.4 and 5.5, H = 896, 80
 //    rows 6.9 and 5.7, H = 1280, 16 rows 4.8 and 4.2, H = 1536 (activations kept) 4.5 and 4.7, H = 2048, 16, 32, 64 rows 5.7, 8.0, 12.6 and 5.9, 7.7, 14.6.
+//    (With 128 rows of H = 2048 these are from whole calls; alone a step takes 5.3 in inference and 5.8 where the activations are kept, within training
+//    calls, whose products hold the clocks down, 6.5.  Of the four tiles: before their results left behind the next products, see the .inc.)
 // What bounds a step now: the operand blocks, 512 KiB per CU at H = 4096 and 64 rows -- a CU takes 90 KB per us from its L2, whatever is in
 // flight --, then the chain behind a tile: sums through LDS, gates (0.2 us per cell of a lane), pieces.  us per step of lstm_fwd_stream_kernel and here:
-// H = 4096, 64 rows 24.8 -> 11.3, 16 rows 20.9 -> 4.6; H = 3072, 32 rows 14.1 -> 4.5; H = 2560, 64 rows 15.4 -> 7.4; and no packed copy of W_h per call (118
+// H = 4096, 64 rows 24.8 -> 10.2, 16 rows 20.9 -> 4.6; H = 3072, 32 rows 14.1 -> 4.5; H = 2560, 64 rows 15.4 -> 6.9; and no packed copy of W_h per call (118
 // us at 4096).
 // Up to H = 2048, with 32 units, there are twice as many barrier groups as lstm_fwd_wide_kernel has: half the rows per group, half
 // the operand bytes per CU (H = 1280, B = 64 3.99 -> 3.31).
